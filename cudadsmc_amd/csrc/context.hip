@@ -21,6 +21,7 @@
 #include "dsmc_internal.hpp"
 #include "fused.hpp"
 #include "plain.hpp"
+#include "readout.hpp"
 
 using namespace dsmc;
 
@@ -155,10 +156,12 @@ struct dsmc_ctx {
     long long *step_dev() const { return step_buf + ssel; }
     unsigned long long *coll_accum = nullptr;
     int *n_dev = nullptr;           // [0], [1]: alive counts; [2]: scratch
+    int *n_host = nullptr;          // pinned copy of n_dev for host reads
+    int *scan_partial = nullptr;    // partials of scans and compactions
     // FP64 form
     PlainPtrs ps[2];
     int2 *start_end = nullptr;
-    int *count = nullptr, *prefix = nullptr, *scan_partial = nullptr, *coll_count = nullptr;
+    int *count = nullptr, *prefix = nullptr, *coll_count = nullptr;
     int *tag = nullptr;
     uint32_t *cmap = nullptr;
     double *evap_pos_d = nullptr, *evap_vel_d = nullptr;
@@ -203,6 +206,7 @@ struct dsmc_ctx {
         if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
         if (graph) (void)hipGraphDestroy(graph);
         for (void *p : allocs) (void)hipFree(p);
+        if (n_host) (void)hipHostFree(n_host);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -384,10 +388,15 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
     x->step_save = x->alloc<long long>(1);
     x->coll_accum = x->alloc<unsigned long long>(n_traps);
     x->n_dev = x->alloc<int>(4);
+    DSMC_HIP(hipHostMalloc((void **)&x->n_host, 4 * sizeof(int), hipHostMallocDefault));
 
     if (!x->fp32) {
         for (int b = 0; b < 2; ++b) {
-            for (int k = 0; k < 9; ++k) x->ps[b].d[k] = x->alloc<double>(N);
+            // one block for the nine arrays (each 256-byte aligned): the
+            // buffer that is not current is also the staging of host reads
+            const size_t pad = ((size_t)N + 31) & ~(size_t)31;
+            double *block = x->alloc<double>(9 * pad);
+            for (int k = 0; k < 9; ++k) x->ps[b].d[k] = block + k * pad;
             x->ps[b].id = x->alloc<int>(N);
             x->ps[b].up = x->alloc<uint8_t>(N);
             for (int k = 0; k < 4; ++k) x->ps[b].psi[k] = c->spin ? x->alloc<double>(N) : nullptr;
@@ -440,6 +449,7 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
         x->rec.cnt = x->alloc<unsigned int>((size_t)n_traps);
         for (int t = 0; t < n_traps; ++t) x->max_trap_atoms = std::max(x->max_trap_atoms, traps[t].n_atoms);
         x->acc2 = x->alloc<double>((size_t)n_traps * kAccK);
+        x->scan_partial = x->alloc<int>(scan_partials(N) + 8);
         x->obs_first = x->alloc<int>((size_t)n_traps);
         x->obs_last = x->alloc<int>((size_t)n_traps);
         x->evap_pos_f = x->alloc<float>(3 * (size_t)N);
@@ -839,46 +849,54 @@ static void do_steps(dsmc_ctx *x, int n)
     for (; k < n; ++k) fused_step(x);
 }
 
-// Sync and read the number of slots of the current state buffer (FP32: alive
-// atoms plus the atoms the last move removed, which keep their slots until
-// the next sort).
-static int host_slots(dsmc_ctx *x)
+// Wait for the stream and read n_dev: n_host[k] = n_dev[k].
+static void read_counts(dsmc_ctx *x)
 {
-    int n = 0;
+    DSMC_HIP(hipMemcpyAsync(x->n_host, x->n_dev, 4 * sizeof(int), hipMemcpyDeviceToHost, x->stream));
     DSMC_HIP(hipStreamSynchronize(x->stream));
-    DSMC_HIP(hipMemcpy(&n, x->fp32 ? x->n_dev + x->cur : x->n_dev, sizeof(int), hipMemcpyDeviceToHost));
-    return n;
 }
 
-// FP32 form: the alive slots of the current state in slot order (all slots
-// when no move has removed atoms since the last sort); returns the slot count.
-static int fused_live(dsmc_ctx *x, std::vector<uint32_t> &live, std::vector<uint32_t> *keys = nullptr)
+// FP32 form: the alive slots of the current state in slot order.  Returns
+// their map (slot of each alive atom), or null when every slot is alive; n
+// and n_slots receive the alive atoms and the slots (alive atoms plus the
+// atoms the last move removed, which keep their slots until the next sort).
+// The map is built on the device, in the re-sort's scratch, which is free
+// between the calls of the C ABI.  When the trap table is valid the alive
+// count is already known (the last sorted move's finalize or k_table_fused
+// left it), so nothing is built if no atom was removed.
+static const uint32_t *fused_live(dsmc_ctx *x, int &n, int &n_slots, bool want_map = true)
 {
-    const int n = host_slots(x);
-    live.clear();
-    std::vector<uint32_t> k;
-    if (x->dead_in_state || keys) {
-        k.resize((size_t)n);
-        if (n) DSMC_HIP(hipMemcpy(k.data(), x->key_a, sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToHost));
+    read_counts(x);
+    n = n_slots = x->n_host[x->cur];
+    if (!x->dead_in_state || n_slots == 0) return nullptr;
+    if (x->tbl_valid) {
+        n = x->n_host[x->cur ^ 1];
+        if (n == n_slots || !want_map) return nullptr;
     }
-    live.reserve((size_t)n);
-    for (int i = 0; i < n; ++i)
-        if (!x->dead_in_state || k[(size_t)i] != x->dead_key) live.push_back((uint32_t)i);
-    if (keys) {
-        keys->resize(live.size());
-        for (size_t j = 0; j < live.size(); ++j) (*keys)[j] = k[live[j]];
+    int *stencil = (int *)x->res.alt_k;
+    uint32_t *map = x->res.alt_v;
+    launch_dead_stencil(x->key_a, x->n_dev + x->cur, n_slots, x->dead_key, stencil, x->stream);
+    compaction_map(stencil, x->n_dev + x->cur, n_slots, map, x->n_dev + 2, x->scan_partial, x->stream,
+                   nullptr);
+    if (!x->tbl_valid) {
+        read_counts(x);
+        n = x->n_host[2];
+        if (n == n_slots) return nullptr;
     }
-    return n;
+    return map;
 }
 
 // Sync and read the current alive count.
 static int host_alive(dsmc_ctx *x)
 {
-    if (!x->fp32) return host_slots(x);
-    if (!x->dead_in_state) return host_slots(x);
-    std::vector<uint32_t> live;
-    (void)fused_live(x, live);
-    return (int)live.size();
+    int n = 0, n_slots = 0;
+    if (x->fp32) {
+        (void)fused_live(x, n, n_slots, false);
+    } else {
+        read_counts(x);
+        n = x->n_host[0];
+    }
+    return n;
 }
 
 // Clears one 64-bit counter (a kernel, not a memset: callers may capture it).
@@ -914,21 +932,13 @@ static void observe_now(dsmc_ctx *x, std::vector<dsmc_observables> &out)
 // transfer goes through the context's own (non-blocking) stream, then waits.
 static void reset_cells(dsmc_ctx *x)
 {
-    std::vector<double> sv(x->n_keys, 0.0);
-    for (int t = 0; t < x->T; ++t)
-        for (int k = 0; k <= x->tdev[t].n_cells; ++k) sv[x->key_base[t] + k] = x->tdev[t].sigvrmax0;
-    const long long zero = 0;
-    int nn[2] = { x->n_cap, x->n_cap };
     hipStream_t st = x->stream;
-    std::vector<float> svf;
-    if (x->fp32) {
-        svf.assign(sv.begin(), sv.end());
-        DSMC_HIP(hipMemcpyAsync(x->sigvrmax_f, svf.data(), sizeof(float) * svf.size(),
-                                hipMemcpyHostToDevice, st));
-    } else {
-        DSMC_HIP(hipMemcpyAsync(x->sigvrmax, sv.data(), sizeof(double) * sv.size(),
-                                hipMemcpyHostToDevice, st));
-    }
+    if (x->fp32)
+        launch_init_sigvrmax(x->d_traps, x->d_key_base, x->T, x->n_keys, x->sigvrmax_f, st);
+    else
+        launch_init_sigvrmax(x->d_traps, x->d_key_base, x->T, x->n_keys, x->sigvrmax, st);
+    const long long zero = 0;
+    const int nn[2] = { x->n_cap, x->n_cap };
     DSMC_HIP(hipMemcpyAsync(x->step_dev(), &zero, sizeof zero, hipMemcpyHostToDevice, st));
     DSMC_HIP(hipMemsetAsync(x->coll_accum, 0, sizeof(unsigned long long) * x->T, st));
     DSMC_HIP(hipMemcpyAsync(x->n_dev, nn, sizeof nn, hipMemcpyHostToDevice, st));
@@ -956,16 +966,10 @@ static InitParams init_params(const dsmc_ctx *x)
     return ip;
 }
 
-// (plane, component) of each axis' value and remainder in the FP32 state
-// records: position x, y, z = (0,0)+(0,3), (0,1)+(2,0), (0,2)+(2,1); velocity
-// x, y, z = (1,0)+(1,3), (1,1)+(2,2), (1,2)+(2,3).
-static const int kRecPosHi[3][2] = { { 0, 0 }, { 0, 1 }, { 0, 2 } };
-static const int kRecPosLo[3][2] = { { 0, 3 }, { 2, 0 }, { 2, 1 } };
-static const int kRecVelHi[3][2] = { { 1, 0 }, { 1, 1 }, { 1, 2 } };
-static const int kRecVelLo[3][2] = { { 1, 3 }, { 2, 2 }, { 2, 3 } };
-
 // ---------------------------------------------------------------------------
-// Host-side field conversion (device layout -> AoS host)
+// Host reads: fields are converted to the host layout on the device, in the
+// state buffer that is not current (scratch between moves: a move overwrites
+// all of it), and copied from there (readout.hip).
 // ---------------------------------------------------------------------------
 template <typename T_>
 static std::vector<T_> d2h(const T_ *d, size_t n)
@@ -975,10 +979,16 @@ static std::vector<T_> d2h(const T_ *d, size_t n)
     return h;
 }
 
-static void interleave(double *dst, const std::vector<double> *cols, int ncols, size_t n)
+static void *stage(dsmc_ctx *x)
 {
-    for (size_t i = 0; i < n; ++i)
-        for (int c = 0; c < ncols; ++c) dst[i * ncols + c] = cols[c][i];
+    return x->fp32 ? (void *)x->fs[x->cur ^ 1].r : (void *)x->ps[x->cur ^ 1].d[0];
+}
+
+static void to_host(dsmc_ctx *x, void *host, const void *dev, size_t bytes)
+{
+    if (!bytes) return;
+    DSMC_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, x->stream));
+    DSMC_HIP(hipStreamSynchronize(x->stream));
 }
 
 static size_t field_size(dsmc_ctx *x, int field, int n)
@@ -1023,87 +1033,63 @@ static void trap_ranges_of(const dsmc_ctx *x, const std::vector<uint32_t> &keys,
 
 static void copy_field(dsmc_ctx *x, int field, void *host, size_t bytes)
 {
-    std::vector<uint32_t> live;
-    const int n_slots = x->fp32 ? fused_live(x, live) : host_slots(x);
-    const int n = x->fp32 ? (int)live.size() : n_slots;
+    int n = 0, n_slots = 0;
+    const uint32_t *live = nullptr;
+    if (x->fp32) live = fused_live(x, n, n_slots);
+    else n = n_slots = host_alive(x);
     const size_t need = field_size(x, field, n);
     // a field of this form has a size at one atom; at no alive atoms it is empty
     if (field_size(x, field, 1) == 0) fail(DSMC_ENOTSUP, "field not available in this form");
     if (need == 0) return;
     if (bytes < need) fail(DSMC_EINVAL, "host buffer too small");
     const size_t N = (size_t)n;
-    double *hd = (double *)host;
-    std::vector<double> cols[4];
+    hipStream_t st = x->stream;
+    double *const sd = (double *)stage(x);
     if (!x->fp32) {
         const PlainPtrs &s = x->ps[x->cur];
         switch (field) {
         case DSMC_FIELD_POS: case DSMC_FIELD_VEL: case DSMC_FIELD_ACC: {
             const int o = field == DSMC_FIELD_POS ? 0 : field == DSMC_FIELD_VEL ? 3 : 6;
-            for (int c = 0; c < 3; ++c) cols[c] = d2h(s.d[o + c], N);
-            interleave(hd, cols, 3, N);
+            launch_pack_columns(s.d + o, 3, n, sd, st);
+            to_host(x, host, sd, need);
             return;
         }
-        case DSMC_FIELD_ATOM_ID: DSMC_HIP(hipMemcpy(host, s.id, N * 4, hipMemcpyDeviceToHost)); return;
+        case DSMC_FIELD_ATOM_ID: to_host(x, host, s.id, need); return;
         case DSMC_FIELD_SPIN:
-            for (int c = 0; c < 4; ++c) cols[c] = d2h(s.psi[c], N);
-            interleave(hd, cols, 4, N);
+            launch_pack_columns(s.psi, 4, n, sd, st);
+            to_host(x, host, sd, need);
             return;
-        case DSMC_FIELD_EVAP_POS:
-            DSMC_HIP(hipMemcpy(host, x->evap_pos_d, need, hipMemcpyDeviceToHost)); return;
-        case DSMC_FIELD_EVAP_VEL:
-            DSMC_HIP(hipMemcpy(host, x->evap_vel_d, need, hipMemcpyDeviceToHost)); return;
-        case DSMC_FIELD_EVAP_TAG: DSMC_HIP(hipMemcpy(host, x->tag, need, hipMemcpyDeviceToHost)); return;
-        case DSMC_FIELD_CELL_START_END:
-            DSMC_HIP(hipMemcpy(host, x->start_end, need, hipMemcpyDeviceToHost)); return;
-        case DSMC_FIELD_CELL_COUNT: DSMC_HIP(hipMemcpy(host, x->count, need, hipMemcpyDeviceToHost)); return;
-        case DSMC_FIELD_CELL_PREFIX: DSMC_HIP(hipMemcpy(host, x->prefix, need, hipMemcpyDeviceToHost)); return;
-        case DSMC_FIELD_COLLISION_COUNT:
-            DSMC_HIP(hipMemcpy(host, x->coll_count, need, hipMemcpyDeviceToHost)); return;
+        case DSMC_FIELD_EVAP_POS: to_host(x, host, x->evap_pos_d, need); return;
+        case DSMC_FIELD_EVAP_VEL: to_host(x, host, x->evap_vel_d, need); return;
+        case DSMC_FIELD_EVAP_TAG: to_host(x, host, x->tag, need); return;
+        case DSMC_FIELD_CELL_START_END: to_host(x, host, x->start_end, need); return;
+        case DSMC_FIELD_CELL_COUNT: to_host(x, host, x->count, need); return;
+        case DSMC_FIELD_CELL_PREFIX: to_host(x, host, x->prefix, need); return;
+        case DSMC_FIELD_COLLISION_COUNT: to_host(x, host, x->coll_count, need); return;
         default: break;
         }
     } else {
         const FusedPtrs &s = x->fs[x->cur];
         switch (field) {
-        case DSMC_FIELD_POS: case DSMC_FIELD_VEL: case DSMC_FIELD_POS_COMP: case DSMC_FIELD_VEL_COMP: {
-            const bool pos = field == DSMC_FIELD_POS || field == DSMC_FIELD_POS_COMP;
-            const bool comp = field == DSMC_FIELD_POS_COMP || field == DSMC_FIELD_VEL_COMP;
-            const std::vector<f4> rec = d2h(s.r, rec_elems((size_t)n_slots));
-            for (int c = 0; c < 3; ++c) {
-                const int *h = pos ? kRecPosHi[c] : kRecVelHi[c], *l = pos ? kRecPosLo[c] : kRecVelLo[c];
-                cols[c].resize(N);
-                for (size_t i = 0; i < N; ++i) {
-                    const f4 *q = rec.data() + rec_index(live[i]);
-                    const float a = q[h[0] * kRecTile][h[1]];
-                    const float b = pos ? rem_value(q[l[0] * kRecTile][l[1]]) : q[l[0] * kRecTile][l[1]];
-                    cols[c][i] = comp ? (double)b : (double)a + (double)b;
-                }
-            }
-            interleave(hd, cols, 3, N);
+        case DSMC_FIELD_POS: case DSMC_FIELD_VEL: case DSMC_FIELD_POS_COMP: case DSMC_FIELD_VEL_COMP:
+            launch_pack_records(field == DSMC_FIELD_POS   ? RecVec::Pos
+                                : field == DSMC_FIELD_VEL ? RecVec::Vel
+                                : field == DSMC_FIELD_POS_COMP ? RecVec::PosRem : RecVec::VelRem,
+                                s, live, n, sd, st);
+            to_host(x, host, sd, need);
             return;
-        }
-        case DSMC_FIELD_ATOM_ID: {   // the labels travel in the position remainders
-            const std::vector<f4> rec = d2h(s.r, rec_elems((size_t)n_slots));
-            int *hi_ = (int *)host;
-            for (size_t i = 0; i < N; ++i) {
-                const f4 *q = rec.data() + rec_index(live[i]);
-                hi_[i] = rec_label(q[0][3], q[2 * kRecTile][0], q[2 * kRecTile][1]);
-            }
+        case DSMC_FIELD_ATOM_ID:   // the labels travel in the position remainders
+            launch_pack_labels(s, live, n, (int *)sd, st);
+            to_host(x, host, sd, need);
             return;
-        }
         case DSMC_FIELD_SPIN:
-            for (int c = 0; c < 3; ++c) {
-                const std::vector<float> a = d2h(s.s[c], (size_t)n_slots);
-                cols[c].resize(N);
-                for (size_t i = 0; i < N; ++i) cols[c][i] = a[live[i]];
-            }
-            interleave(hd, cols, 3, N);
+            launch_pack_columns(s.s, 3, live, n, sd, st);
+            to_host(x, host, sd, need);
             return;
-        case DSMC_FIELD_EVAP_POS: case DSMC_FIELD_EVAP_VEL: {
-            std::vector<float> a = d2h(field == DSMC_FIELD_EVAP_POS ? x->evap_pos_f : x->evap_vel_f,
-                                       (size_t)x->n_cap * 3);
-            for (size_t i = 0; i < a.size(); ++i) hd[i] = a[i];
+        case DSMC_FIELD_EVAP_POS: case DSMC_FIELD_EVAP_VEL:
+            launch_widen(field == DSMC_FIELD_EVAP_POS ? x->evap_pos_f : x->evap_vel_f, 3LL * x->n_cap, sd, st);
+            to_host(x, host, sd, need);
             return;
-        }
         case DSMC_FIELD_CELL_START_END: {
             if (!x->have_sort) fail(DSMC_ESTATE, "the cell table exists between sort and move");
             DSMC_HIP(hipMemsetAsync(x->cell_start, 0xFF, sizeof(uint32_t) * x->n_keys, x->stream));
@@ -1118,16 +1104,24 @@ static void copy_field(dsmc_ctx *x, int field, void *host, size_t bytes)
             return;
         }
         case DSMC_FIELD_TRAP_START: {
-            std::vector<uint32_t> lk;
-            (void)fused_live(x, live, &lk);
+            std::vector<uint32_t> lk(N);
+            const uint32_t *src = x->key_a;
+            if (live) {
+                gather_u32((uint32_t *)sd, x->key_a, live, nullptr, n, st, nullptr);
+                src = (const uint32_t *)sd;
+            }
+            to_host(x, lk.data(), src, sizeof(uint32_t) * N);
             trap_ranges_of(x, lk, (int *)host);
             return;
         }
         case DSMC_FIELD_CELL_ID:
             if (!x->have_sort) {   // keys of the alive slots (unsorted order)
-                const std::vector<uint32_t> a = d2h(x->key_a, (size_t)n_slots);
-                uint32_t *hk = (uint32_t *)host;
-                for (size_t i = 0; i < N; ++i) hk[i] = a[live[i]];
+                const uint32_t *src = x->key_a;
+                if (live) {
+                    gather_u32((uint32_t *)sd, x->key_a, live, nullptr, n, st, nullptr);
+                    src = (const uint32_t *)sd;
+                }
+                to_host(x, host, src, need);
                 return;
             }
             break;
@@ -1140,20 +1134,24 @@ static void copy_field(dsmc_ctx *x, int field, void *host, size_t bytes)
         // sort: the sorted keys (the alive atoms; removed atoms sort last)
         const uint32_t *src = (x->fp32 && !x->have_sort) ? x->key_a : x->sorted_key;
         if (!src) src = x->key_a;
-        DSMC_HIP(hipMemcpy(host, src, N * 4, hipMemcpyDeviceToHost));
+        to_host(x, host, src, need);
         return;
     }
     case DSMC_FIELD_PERM:
         if (!x->perm) fail(DSMC_ESTATE, "no sort has run yet");
-        DSMC_HIP(hipMemcpy(host, x->perm, N * 4, hipMemcpyDeviceToHost));
+        to_host(x, host, x->perm, need);
         return;
     case DSMC_FIELD_SIGVRMAX:
         if (x->fp32) {
-            const std::vector<float> f = d2h(x->sigvrmax_f, (size_t)x->n_keys);
-            double *h = (double *)host;
-            for (int k = 0; k < x->n_keys; ++k) h[k] = (double)f[k];
+            // widened in pieces that fit the staging (48 bytes per atom)
+            const long long piece = std::max<long long>(1, 6LL * x->n_cap);
+            for (long long k = 0; k < x->n_keys; k += piece) {
+                const long long m = std::min<long long>(piece, x->n_keys - k);
+                launch_widen(x->sigvrmax_f + k, m, sd, st);
+                to_host(x, (double *)host + k, sd, sizeof(double) * (size_t)m);
+            }
         } else {
-            DSMC_HIP(hipMemcpy(host, x->sigvrmax, need, hipMemcpyDeviceToHost));
+            to_host(x, host, x->sigvrmax, need);
         }
         return;
     case DSMC_FIELD_TRAP_START: {
@@ -1162,22 +1160,18 @@ static void copy_field(dsmc_ctx *x, int field, void *host, size_t bytes)
         h[1] = n;
         return;
     }
-    case DSMC_FIELD_OBS:
-        DSMC_HIP(hipMemcpy(host, x->obs_log, need, hipMemcpyDeviceToHost));
-        return;
+    case DSMC_FIELD_OBS: to_host(x, host, x->obs_log, need); return;
     case DSMC_FIELD_SPIN_UP: {
         int *h = (int *)host;
         if (x->fp32) {   // the FP32 form removes atoms instead of flipping them
             for (size_t i = 0; i < N; ++i) h[i] = 1;
             return;
         }
-        const std::vector<uint8_t> u = d2h(x->ps[x->cur].up, N);
-        for (size_t i = 0; i < N; ++i) h[i] = u[i] ? 1 : 0;
+        launch_widen(x->ps[x->cur].up, n, (int *)sd, st);
+        to_host(x, host, sd, need);
         return;
     }
-    case DSMC_FIELD_LOCAL_POPS:
-        DSMC_HIP(hipMemcpy(host, x->pops, need, hipMemcpyDeviceToHost));
-        return;
+    case DSMC_FIELD_LOCAL_POPS: to_host(x, host, x->pops, need); return;
     default: break;
     }
     fail(DSMC_EINVAL, "unknown field");
@@ -1314,44 +1308,24 @@ dsmc_status dsmc_set_state(dsmc_ctx *ctx, const double *pos, const double *vel, 
     DSMC_API_BEGIN(ctx)
     if (!pos || !vel || n != ctx->n_cap) fail(DSMC_EINVAL, "set_state needs n_capacity atoms");
     reset_cells(ctx);
+    // the rows go to the other state buffer (reset_cells made 0 current) and
+    // are laid out from there
     const size_t N = (size_t)n;
-    std::vector<int> ids(N);
-    for (size_t i = 0; i < N; ++i) ids[i] = (int)i;
+    double *const sp = (double *)stage(ctx), *const sv = sp + 3 * N;
+    hipStream_t st = ctx->stream;
+    DSMC_HIP(hipMemcpyAsync(sp, pos, 3 * N * sizeof(double), hipMemcpyHostToDevice, st));
+    DSMC_HIP(hipMemcpyAsync(sv, vel, 3 * N * sizeof(double), hipMemcpyHostToDevice, st));
     if (!ctx->fp32) {
         const PlainPtrs &s = ctx->ps[0];
-        std::vector<double> cols(6 * N);
-        for (int c = 0; c < 3; ++c)
-            for (size_t i = 0; i < N; ++i) {
-                cols[c * N + i] = pos[3 * i + c];
-                cols[(3 + c) * N + i] = vel[3 * i + c];
-            }
-        for (int c = 0; c < 6; ++c)
-            DSMC_HIP(hipMemcpyAsync(s.d[c], cols.data() + c * N, N * 8, hipMemcpyHostToDevice,
-                                    ctx->stream));
-        DSMC_HIP(hipMemcpyAsync(s.id, ids.data(), N * 4, hipMemcpyHostToDevice, ctx->stream));
-        DSMC_HIP(hipMemsetAsync(s.up, 1, N, ctx->stream));
-        launch_accel_plain(ctx->tdev[0], s, n, ctx->stream, &ctx->prof);
+        launch_unpack_columns(sp, 3, n, s.d, st);
+        launch_unpack_columns(sv, 3, n, s.d + 3, st);
+        launch_iota(s.id, n, st);
+        DSMC_HIP(hipMemsetAsync(s.up, 1, N, st));
+        launch_accel_plain(ctx->tdev[0], s, n, st, &ctx->prof);
         plain_index(ctx);
     } else {
-        const FusedPtrs &s = ctx->fs[0];
-        std::vector<f4> rec(rec_elems(N), f4{ 0.0f, 0.0f, 0.0f, 0.0f });
-        for (int c = 0; c < 3; ++c) {
-            for (int which = 0; which < 2; ++which) {
-                const double *src = which ? vel : pos;
-                const int *h = which ? kRecVelHi[c] : kRecPosHi[c];
-                const int *l = which ? kRecVelLo[c] : kRecPosLo[c];
-                for (size_t i = 0; i < N; ++i) {
-                    f4 *q = rec.data() + rec_index((uint32_t)i);
-                    const double v = src[3 * i + c];
-                    const float hv = (float)v, lv = (float)(v - (double)hv);
-                    q[h[0] * kRecTile][h[1]] = hv;
-                    // slot i holds atom i: its label in the position remainders
-                    q[l[0] * kRecTile][l[1]] = which ? lv : rem_tag(lv, label_part((int)i, c));
-                }
-            }
-        }
-        DSMC_HIP(hipMemcpyAsync(s.r, rec.data(), rec.size() * sizeof(f4), hipMemcpyHostToDevice,
-                                ctx->stream));
+        // slot i holds atom i: its label in the position remainders
+        launch_unpack_records(sp, sv, n, ctx->fs[0], st);
         fused_index(ctx);
     }
     DSMC_HIP(hipStreamSynchronize(ctx->stream));
@@ -1362,27 +1336,21 @@ dsmc_status dsmc_set_spin(dsmc_ctx *ctx, const double *spin, int n, int componen
 {
     DSMC_API_BEGIN(ctx)
     if (!ctx->cfg.spin) fail(DSMC_ENOTSUP, "spin evolution is off in this context");
-    if (!spin || n != host_alive(ctx)) fail(DSMC_EINVAL, "set_spin needs one row per alive atom");
-    const size_t N = (size_t)n;
-    if (!ctx->fp32) {
-        if (components != 4) fail(DSMC_EINVAL, "the FP64 form stores spinors (4 components)");
-        std::vector<double> col(4 * N);
-        for (int c = 0; c < 4; ++c) {
-            for (size_t i = 0; i < N; ++i) col[c * N + i] = spin[4 * i + c];
-            DSMC_HIP(hipMemcpyAsync(ctx->ps[ctx->cur].psi[c], col.data() + c * N, N * 8,
-                                    hipMemcpyHostToDevice, ctx->stream));
-        }
+    int n_alive = 0, n_slots = 0;
+    const uint32_t *live = nullptr;
+    if (ctx->fp32) live = fused_live(ctx, n_alive, n_slots);
+    else n_alive = host_alive(ctx);
+    if (!spin || n != n_alive) fail(DSMC_EINVAL, "set_spin needs one row per alive atom");
+    double *const sd = (double *)stage(ctx);
+    if (!ctx->fp32 && components != 4) fail(DSMC_EINVAL, "the FP64 form stores spinors (4 components)");
+    if (ctx->fp32 && components != 3) fail(DSMC_EINVAL, "the FP32 form stores Bloch vectors (3 components)");
+    if (n > 0) {
+        DSMC_HIP(hipMemcpyAsync(sd, spin, sizeof(double) * (size_t)components * (size_t)n, hipMemcpyHostToDevice,
+                                ctx->stream));
+        // FP32 form: rows go to the alive slots; slots of removed atoms keep their values
+        if (!ctx->fp32) launch_unpack_columns(sd, 4, n, ctx->ps[ctx->cur].psi, ctx->stream);
+        else launch_unpack_columns(sd, 3, live, n, ctx->fs[ctx->cur].s, ctx->stream);
         DSMC_HIP(hipStreamSynchronize(ctx->stream));
-    } else {
-        if (components != 3) fail(DSMC_EINVAL, "the FP32 form stores Bloch vectors (3 components)");
-        // rows go to the alive slots; slots of removed atoms keep their values
-        std::vector<uint32_t> live;
-        const size_t S = (size_t)fused_live(ctx, live);
-        for (int c = 0; c < 3; ++c) {
-            std::vector<float> col = d2h(ctx->fs[ctx->cur].s[c], S);
-            for (size_t i = 0; i < N; ++i) col[live[i]] = (float)spin[3 * i + c];
-            DSMC_HIP(hipMemcpy(ctx->fs[ctx->cur].s[c], col.data(), S * 4, hipMemcpyHostToDevice));
-        }
     }
     DSMC_API_END(ctx)
 }

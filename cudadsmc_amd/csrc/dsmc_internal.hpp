@@ -149,7 +149,7 @@ inline int scan_partials(int n) { return div_up(n > 0 ? n : 1, kScanTile) + 1; }
 void compaction_map(const int *stencil, const int *n_dev, int n_cap, uint32_t *map,
                     int *n_out_dev, int *partial, hipStream_t stream, Profiler *prof);
 
-// dst[i] = src[map[i]] for i < *n_dev.
+// dst[i] = src[map[i]] for i < *n_dev (i < n_cap when n_dev is null).
 void gather_u32(uint32_t *dst, const uint32_t *src, const uint32_t *map, const int *n_dev,
                 int n_cap, hipStream_t stream, Profiler *prof);
 

@@ -864,17 +864,17 @@ void compaction_map(const int *stencil, const int *n_dev, int n_cap, uint32_t *m
 __global__ __launch_bounds__(256) void k_gather_u32(uint32_t *__restrict__ dst,
                                                     const uint32_t *__restrict__ src,
                                                     const uint32_t *__restrict__ map,
-                                                    const int *__restrict__ n_dev)
+                                                    const int *__restrict__ n_dev, int n)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < *n_dev) dst[i] = src[map[i]];
+    if (i < (n_dev ? *n_dev : n)) dst[i] = src[map[i]];
 }
 
 void gather_u32(uint32_t *dst, const uint32_t *src, const uint32_t *map, const int *n_dev,
                 int n_cap, hipStream_t stream, Profiler *prof)
 {
     DSMC_LAUNCH(prof, "gather_u32", (double)n_cap * 12.0, k_gather_u32, div_up(n_cap > 0 ? n_cap : 1, 256),
-                256, stream, dst, src, map, n_dev);
+                256, stream, dst, src, map, n_dev, n_cap);
 }
 
 // ---------------------------------------------------------------------------

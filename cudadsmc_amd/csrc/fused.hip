@@ -1391,6 +1391,17 @@ void k_move_fused(
     }
 }
 
+// Waits until this thread's earlier stores have completed.  Between blocks of
+// one launch it orders agent-scope atomic stores (which write through the L2)
+// before a later agent-scope atomic of the same thread, without the L2
+// write-back and invalidation that __threadfence() adds on gfx950 for plain
+// stores: with one such fence pair per block, 128 traps x 2 blocks took 31 us
+// where 128 x 1 (no fence) took 7.5.
+__device__ __forceinline__ void stores_done()
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // Grid (P, T): block (p, t) adds the records of every P-th move block of trap
 // t (fixed order) and, when the next sort's trap ranges are asked for, the
 // removal counts of every P-th move block before the trap; the last of the P
@@ -1494,8 +1505,9 @@ __global__ __launch_bounds__(256) void k_obs_finalize(
         for (int q = 0; q < kAccK; ++q)
             __hip_atomic_store(&lvl2[((size_t)t * P + p) * kAccK + q], a[q], __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
-        __threadfence();
-        fin = atomicAdd(&cnt[t], 1u) == (unsigned)(P - 1);
+        stores_done();
+        fin = __hip_atomic_fetch_add(&cnt[t], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+              (unsigned)(P - 1);
     }
     __syncthreads();
     if (!fin) return;   // whole block leaves together
@@ -1503,7 +1515,6 @@ __global__ __launch_bounds__(256) void k_obs_finalize(
         // the last of the trap's P blocks to finish: every partial loaded at
         // once, then thread q sums quantity q in block order (the same order
         // whichever block finishes last)
-        __threadfence();
         for (int e = tid; e < P * kAccK; e += 256)
             part[e] = __hip_atomic_load(&lvl2[(size_t)t * P * kAccK + e], __ATOMIC_RELAXED,
                                         __HIP_MEMORY_SCOPE_AGENT);

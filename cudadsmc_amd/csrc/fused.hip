@@ -26,6 +26,7 @@
 //                           incremental re-sort's first phase
 // Every kernel reads the alive count and the step number from device memory,
 // so the loop can be captured once and replayed as a HIP graph.
+#include "cells_device.hpp"
 #include "fused.hpp"
 #include "resort_device.hpp"
 #include "sincos_f32.hpp"
@@ -539,8 +540,6 @@ __device__ __forceinline__ int cell_trials_wave(const CollideParams &cp, const C
     return count;
 }
 
-constexpr int kCollItems = 8;  // slots per lane scanned for cell heads
-constexpr uint32_t kNoKey = 0xFFFFFFFFu;   // no slot there (keys are below 2^31)
 constexpr int kWaveTrialsDefault = 16;
 
 // Trials of one cell (serial by one lane, or by the whole wave when heavy);
@@ -560,14 +559,13 @@ __device__ __forceinline__ int run_cell(const CollideParams &cp, const CellJob &
 }
 
 // Each wave takes kWave * kCollItems consecutive sorted slots and runs the
-// cells that start there (a cell ends where the next one starts, possibly in
-// the next chunk).  Only cells of two or more atoms are compacted for the
-// lanes (ballot + popcount), one per lane; cells with more than
-// `wave_trials` trials are then run by the whole wave.  When the chunk lies
-// in one trap, its parameters are wave-uniform (scalar loads).  Five waves
-// per SIMD: the kernel is bound by the latency of its dependent loads (key,
-// sigma v_r,max, permutation, velocities).  CB threads per block (one or
-// four waves).
+// cells that start there (wave_list_cells), one cell of two or more atoms per
+// lane; cells with more than `wave_trials` trials are then run by the whole
+// wave.  When the chunk lies in one trap, its parameters are wave-uniform
+// (scalar loads).  Five waves per SIMD: the kernel is bound by the latency of
+// its dependent loads (key, sigma v_r,max, permutation, velocities).  CB
+// threads per block (one or four waves); the waves share nothing but the
+// trap table, which a single trap does without (no block barrier then).
 template <int CB>
 __global__ __launch_bounds__(CB, 5) void k_collide_fused(
     const TrapDev *__restrict__ traps, const int *__restrict__ key_base, int T, CollideParams cp,
@@ -576,119 +574,56 @@ __global__ __launch_bounds__(CB, 5) void k_collide_fused(
     unsigned long long *__restrict__ coll_accum, const long long *__restrict__ step_dev,
     int wave_trials)
 {
-    constexpr int kChunk = kWave * kCollItems;
     extern __shared__ int kb[];
-    __shared__ int heads[CB / kWave][kChunk + 1];
-    __shared__ uint32_t hkey[CB / kWave][kChunk];   // key of each head
-    __shared__ short multi[CB / kWave][kChunk];   // heads index of cells with >= 2 atoms
-    __shared__ short heavy[CB / kWave][kChunk];
+    __shared__ WaveCells cells[CB / kWave];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    const int chunk0 = (blockIdx.x * (CB / kWave) + w) * kChunk;
+    const int chunk0 = (blockIdx.x * (CB / kWave) + w) * kCollChunk;
     const VelGlobal vg = { s.r, perm };
     const uint64_t lt = lanemask_lt();
-    // the chunk's keys, the one before it and the 64 after it (for the end
-    // of its last cell) are loaded with the alive count, the step and the
-    // trap table's first 2 CB entries; kNoKey marks slots past the alive
-    // atoms
+    WaveCells &L = cells[w];
+    // the keys are loaded with the alive count, the step and the trap table's
+    // first 2 CB entries
     const int tb_j = (int)threadIdx.x;
-    const int tb0 = tb_j < T + 1 ? key_base[tb_j] : 0;
-    const int tb1 = tb_j + CB < T + 1 ? key_base[tb_j + CB] : 0;
-    uint32_t kk[kCollItems];
-#pragma unroll
-    for (int it = 0; it < kCollItems; ++it) {
-        const int i = chunk0 + it * kWave + lane;
-        kk[it] = i < n_cap ? key[i] : kNoKey;
+    int tb0 = 0, tb1 = 0;
+    if (T > 1) {
+        tb0 = tb_j < T + 1 ? key_base[tb_j] : 0;
+        tb1 = tb_j + CB < T + 1 ? key_base[tb_j + CB] : 0;
     }
-    const int jp = chunk0 + kChunk + lane;
-    uint32_t pk = jp < n_cap ? key[jp] : kNoKey;
-    uint32_t k_before = chunk0 > 0 && chunk0 <= n_cap ? key[chunk0 - 1] : kNoKey;
+    ChunkKeys ck;
+    chunk_load(key, n_cap, chunk0, ck);
     const int n = *n_dev;
     const uint32_t step = (uint32_t)*step_dev;
-    const int chunk1 = min(n, chunk0 + kChunk);
-#pragma unroll
-    for (int it = 0; it < kCollItems; ++it)
-        if (chunk0 + it * kWave + lane >= n) kk[it] = kNoKey;
-    if (jp >= n) pk = kNoKey;
-    if (chunk0 > n) k_before = kNoKey;
-    const uint32_t k_after = __shfl(pk, 0, kWave);
-    if (tb_j < T + 1) kb[tb_j] = tb0;
-    if (tb_j + CB < T + 1) kb[tb_j + CB] = tb1;
-    for (int j = tb_j + 2 * CB; j < T + 1; j += CB) kb[j] = key_base[j];
-    __syncthreads();
-    int nh = 0, nm = 0;
-    uint32_t klast = 0;   // key of the chunk's last cell head
-#pragma unroll
-    for (int it = 0; it < kCollItems; ++it) {
-        const int i = chunk0 + it * kWave + lane;
-        const uint32_t k = kk[it];
-        // neighbours from the adjacent lanes (and items)
-        uint32_t kp = __shfl_up(k, 1, kWave), kn = __shfl_down(k, 1, kWave);
-        const uint32_t prev_last = it > 0 ? __shfl(kk[it > 0 ? it - 1 : 0], kWave - 1, kWave) : k_before;
-        const uint32_t next_first = it + 1 < kCollItems ? __shfl(kk[it + 1 < kCollItems ? it + 1 : it], 0, kWave)
-                                                        : k_after;
-        if (lane == 0) kp = prev_last;
-        if (lane == kWave - 1) kn = next_first;
-        bool head = false, mult = false;
-        if (i < n) {
-            head = i == 0 || kp != k;
-            mult = head && i + 1 < n && kn == k;
-        }
-        const uint64_t bh = __ballot(head), bm = __ballot(mult);
-        const int pos = nh + __popcll(bh & lt);
-        if (head) { heads[w][pos] = i; hkey[w][pos] = k; }
-        if (mult) multi[w][nm + __popcll(bm & lt)] = (short)pos;
-        if (bh) klast = __shfl(k, 63 - __clzll((long long)bh), kWave);
-        nh += __popcll(bh);
-        nm += __popcll(bm);
+    if (T > 1) {
+        if (tb_j < T + 1) kb[tb_j] = tb0;
+        if (tb_j + CB < T + 1) kb[tb_j + CB] = tb1;
+        for (int j = tb_j + 2 * CB; j < T + 1; j += CB) kb[j] = key_base[j];
+        __syncthreads();
     }
-    // sigma v_r,max of this lane's first cell, loaded now (the load overlaps
-    // the end-of-chunk probe and the barrier); each round loads the next
-    // round's while it runs
-    float sm_next = lane < nm ? sigvrmax[hkey[w][multi[w][lane]]] : 0.0f;
-    if (nh > 0) {
-        // end of the last cell: the first later slot with another key.  The
-        // wave probes the next 64 slots at once; a longer cell (e.g. the
-        // overflow cell of atoms outside the grid) is searched by galloping.
-        const uint64_t bd = __ballot(chunk1 == chunk0 + kChunk && pk != kNoKey && pk != klast);
-        int end = chunk1 + kWave;
-        if (bd) end = chunk1 + __ffsll((unsigned long long)bd) - 1;
-        if (chunk1 + kWave >= n) end = min(end, n);
-        if (lane == 0) {
-            if (!bd && end < n) {
-                int lo = end, stp = 1;
-                while (lo + stp - 1 < n && key[lo + stp - 1] == klast) { lo += stp; stp <<= 1; }
-                int hi = min(n, lo + stp - 1);  // the first other key is in [lo, hi]
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (key[mid] == klast) lo = mid + 1; else hi = mid;
-                }
-                end = lo;
-            }
-            heads[w][nh] = end;
-        }
-    }
+    uint32_t k_first = 0, klast = 0;
+    const int nm = wave_list_cells(key, n, chunk0, ck, L, k_first, klast);
+    if (nm == 0) return;   // whole wave (no block barrier follows)
+    // sigma v_r,max of this lane's first cell, loaded now; each round loads
+    // the next round's while it runs
+    float sm_next = lane < nm ? sigvrmax[L.key[lane]] : 0.0f;
     // traps of the chunk's first and last cells: usually the same
     int t_lo = 0, t_hi = 0;
-    if (nh > 0) {
-        t_lo = __builtin_amdgcn_readfirstlane(last_le(kb, T + 1, (int)__shfl(kk[0], 0, kWave)));
+    if (T > 1) {
+        t_lo = __builtin_amdgcn_readfirstlane(last_le(kb, T + 1, (int)k_first));
         t_hi = __builtin_amdgcn_readfirstlane(last_le(kb, T + 1, (int)klast));
     }
-    __syncthreads();
     int nheavy = 0;
     unsigned long long wave_cnt = 0;   // accepted collisions of trap t_lo (uniform chunks)
     for (int m0 = 0; m0 < nm; m0 += kWave) {
         const int mi = m0 + lane;
         const float sm = sm_next;
-        if (mi + kWave < nm) sm_next = sigvrmax[hkey[w][multi[w][mi + kWave]]];
+        if (mi + kWave < nm) sm_next = sigvrmax[L.key[mi + kWave]];
         CellJob c;
         Trial0 t0;
         bool ok = false;
-        int h = 0;
         uint32_t stream = 0;
         if (mi < nm) {
-            h = multi[w][mi];
-            const int i = heads[w][h], end = heads[w][h + 1];
-            const uint32_t k = hkey[w][h];
+            const int i = chunk0 + L.start[mi], end = L.end[mi];
+            const uint32_t k = L.key[mi];
             auto setup = [&](const TrapDev &tr, int t) {
                 stream = tr.stream;
                 trial0_load(cp, stream, k - (uint32_t)tr.key_base, step, end - i, i, vg, t0);
@@ -703,7 +638,7 @@ __global__ __launch_bounds__(CB, 5) void k_collide_fused(
         }
         const bool is_heavy = ok && c.ncol > wave_trials;
         const uint64_t hb = __ballot(is_heavy);
-        if (is_heavy) heavy[w][nheavy + __popcll(hb & lt)] = (short)mi;
+        if (is_heavy) L.heavy[nheavy + __popcll(hb & lt)] = (short)mi;
         nheavy += __popcll(hb);
         if (ok && !is_heavy) {
             const int cnt = run_cell(cp, c, stream, step, vg, sigvrmax, false, t0);
@@ -711,14 +646,13 @@ __global__ __launch_bounds__(CB, 5) void k_collide_fused(
             else if (cnt) atomicAdd(&coll_accum[c.t], (unsigned long long)cnt);
         }
     }
-    __syncthreads();
+    wave_lds_fence();
     for (int q = 0; q < nheavy; ++q) {
-        const int h = multi[w][heavy[w][q]];
-        const int i = heads[w][h];
-        const uint32_t k = hkey[w][h];
+        const int h = L.heavy[q];
+        const uint32_t k = L.key[h];
         const int t = t_lo == t_hi ? t_lo : last_le(kb, T + 1, (int)k);
         CellJob c;
-        (void)cell_setup(traps[t], t, k, cp, (double)sigvrmax[k], i, heads[w][h + 1], c);
+        (void)cell_setup(traps[t], t, k, cp, (double)sigvrmax[k], chunk0 + L.start[h], L.end[h], c);
         const Trial0 none = { 0u, 0u, 0.0f, 0.0f };
         const int cnt = run_cell(cp, c, traps[t].stream, step, vg, sigvrmax, true, none);
         if (lane == 0) {
@@ -1746,7 +1680,7 @@ void launch_collide_fused(const TrapDev *traps, const int *key_base, int n_traps
     // in LDS, so beyond 511 traps (a 2 KB table) one-wave blocks would put
     // fewer than five waves on a SIMD, and four-wave blocks are used.
     if (n_traps > 1 && n_traps + 1 <= 512)
-        hipLaunchKernelGGL(k_collide_fused<kWave>, dim3(fgrid(n_cap, kWave * kCollItems)),
+        hipLaunchKernelGGL(k_collide_fused<kWave>, dim3(fgrid(n_cap, kCollChunk)),
                            dim3(kWave), lds, st, traps, key_base, n_traps, cp, key, perm, n_dev,
                            n_cap, s, sigvrmax, coll_accum, step_dev, wave_trials);
     else

@@ -24,8 +24,8 @@ LIB = PKG / "libdsmc.so"
 DRIVER = PKG / "bin" / "cudadsmc"
 H5LIB = PKG / "libdsmc_h5.so"
 
-HIP_SOURCES = ["primitives.hip", "plain.hip", "fused.hip", "readout.hip",
-               "context.hip"]
+HIP_SOURCES = ["primitives.hip", "plain.hip", "plain_step.hip", "fused.hip",
+               "readout.hip", "context.hip"]
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",

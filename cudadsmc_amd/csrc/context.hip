@@ -4,8 +4,8 @@
 //
 // Host-side call sequence per motion step (main.cu:412-523 without the dead
 // median, the MCWF spin-flip model and the HDF5 output):
-//   FP64 form:  [index, sort + gather, cell table, collide]  every lpc steps
-//               spin, move, evaporation tag + compaction, FP64 observables
+//   FP64 form:  sort, collide every lpc steps, then the motion substeps up to
+//               the next collision step in one kernel (plain_step.hip)
 //   FP32 form:  sort, table, [collide], fused move           every step
 // No call in the loop synchronises with the host.
 #include <algorithm>
@@ -21,6 +21,7 @@
 #include "dsmc_internal.hpp"
 #include "fused.hpp"
 #include "plain.hpp"
+#include "plain_step.hpp"
 #include "readout.hpp"
 
 using namespace dsmc;
@@ -138,7 +139,7 @@ struct dsmc_ctx {
     uint32_t *srt_k[2] = {nullptr, nullptr}, *srt_v[2] = {nullptr, nullptr};  // FP32 sort outputs
     int srt_cur = 0;                // FP32: srt_*[srt_cur] holds the last sort's result
     int graph_srt = 0;              // srt_cur at graph capture
-    int graph_ssel = 0, graph_tsel = 0;   // step and trap-range buffers at graph capture
+    int graph_ssel = 0, graph_tsel = 0, graph_cur = 0;   // other buffers' parities at graph capture
     bool prepped = false;           // FP32: the last finalize ran the re-sort's first phase
     bool prep_in_finalize = true;   // FP32: run it there (else in the re-sort itself)
     bool split_step = true;         // FP32: dsmc_step runs collide and move as two kernels
@@ -168,6 +169,24 @@ struct dsmc_ctx {
     double *partials = nullptr, *evap_accum = nullptr;
     double *pops = nullptr;                  // spin-flip model: populations by label
     unsigned long long *flips = nullptr;     // spin-flip model: flips of the last call
+    // FP64 form, whole steps (plain_step.hip).  dsmc_step leaves some of what
+    // the single calls and host reads expect to be made when they ask
+    // (plain_settle, plain_need_acc, plain_need_tables).
+    PlainCtl *ctl = nullptr;        // [2]: counters, ctl[csel] current
+    int csel = 0;
+    uint32_t *key_f = nullptr;      // the state's next keys (dead key: removed atoms)
+    uint64_t *mask_d2[2] = {nullptr, nullptr};   // removed atoms; [mpar] the current state's
+    uint64_t *mask_last = nullptr;
+    int mpar = 0;
+    double *rec64 = nullptr;        // per-block sums of a move launch
+    unsigned long long *cc_tagged = nullptr;     // collision step << 32 | collisions, per cell
+    bool ctl_live = false;          // ctl describes the state (else n_dev, step, coll_steps do)
+    bool sorted_ok = false;         // srt_k[srt_cur][i] is the key of slot i, masks and samples too
+    bool keys_ok = false;           // key_f holds the state's keys
+    bool lazy_dead = false;         // removed atoms may still hold slots
+    bool acc_stale = false;         // the accelerations in memory are not the state's
+    bool tables_stale = false;      // cell table and counts are those of an earlier sort
+    int perm_mask = -1;             // perm's slots count the removed atoms of mask_d2[perm_mask]
     // FP32 form
     FusedPtrs fs[2];
     uint32_t *cell_start = nullptr, *cell_end = nullptr;
@@ -389,6 +408,16 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
     x->coll_accum = x->alloc<unsigned long long>(n_traps);
     x->n_dev = x->alloc<int>(4);
     DSMC_HIP(hipHostMalloc((void **)&x->n_host, 4 * sizeof(int), hipHostMallocDefault));
+    // incremental re-sort
+    resort_scratch_bind(x->res, N, x->alloc<char>(resort_scratch_bytes(N), false));
+    // one entry per block of the smallest move block size, whole 2048-slot
+    // tiles (never-written entries stay zero)
+    x->blk_moved = x->alloc<uint32_t>((size_t)div_up(N, 2048) * (2048 / 64) + 64);
+    x->blk_dead = x->alloc<uint32_t>((size_t)div_up(N, 2048) * (2048 / 64) + 64);
+    x->mask_moved = x->alloc<uint64_t>(resort_mask_words(N));
+    x->key_samp = x->alloc<uint32_t>(resort_mask_words(N));
+    // (+ 4: the locate reads the samples in 16-byte pieces)
+    x->key_tsamp = x->alloc<uint32_t>(resort_mask_words(N) / (kResortTile / 64) + 4);
 
     if (!x->fp32) {
         for (int b = 0; b < 2; ++b) {
@@ -417,21 +446,22 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
             x->pops = x->alloc<double>(2 * (size_t)N);
             x->flips = x->alloc<unsigned long long>(1);
         }
+        x->ctl = x->alloc<PlainCtl>(2);
+        x->key_f = x->alloc<uint32_t>(N);
+        for (int b = 0; b < 2; ++b) {
+            x->srt_k[b] = x->alloc<uint32_t>(N);
+            x->srt_v[b] = x->alloc<uint32_t>(N);
+            x->mask_d2[b] = x->alloc<uint64_t>(resort_mask_words(N));
+        }
+        x->mask_last = x->alloc<uint64_t>(resort_mask_words(N));
+        x->rec64 = x->alloc<double>((size_t)std::min(c->lpc, kMaxSub) * kStepRec * step_rec_stride(N));
+        x->cc_tagged = x->alloc<unsigned long long>(C1);
     } else {
         for (int b = 0; b < 2; ++b) {
             x->fs[b].r = x->alloc<f4>(rec_elems(N));
             for (int k = 0; k < 3; ++k) x->fs[b].s[k] = c->spin ? x->alloc<float>(N) : nullptr;
         }
-        resort_scratch_bind(x->res, N, x->alloc<char>(resort_scratch_bytes(N), false));
-        // one entry per block of the smallest move block size, whole 2048-slot
-        // tiles (never-written entries stay zero)
-        x->blk_moved = x->alloc<uint32_t>((size_t)div_up(N, 2048) * (2048 / 64) + 64);
-        x->blk_dead = x->alloc<uint32_t>((size_t)div_up(N, 2048) * (2048 / 64) + 64);
-        x->mask_moved = x->alloc<uint64_t>(resort_mask_words(N));
         x->mask_dead = x->alloc<uint64_t>(resort_mask_words(N));
-        x->key_samp = x->alloc<uint32_t>(resort_mask_words(N));
-        // (+ 4: the locate reads the samples in 16-byte pieces)
-        x->key_tsamp = x->alloc<uint32_t>(resort_mask_words(N) / (kResortTile / 64) + 4);
         x->srt_k[0] = x->key_b; x->srt_v[0] = x->val_b;
         x->srt_k[1] = x->alloc<uint32_t>(N); x->srt_v[1] = x->alloc<uint32_t>(N);
         x->cell_start = x->alloc<uint32_t>(x->n_keys, false);
@@ -476,6 +506,9 @@ static CollideParams collide_params(const dsmc_ctx *x)
 
 static void plain_index(dsmc_ctx *x)
 {
+    // an even number of radix passes sorts in place: the sorted keys are then
+    // the array that the index overwrites
+    if (x->sorted_key && x->passes % 2 == 0) x->sorted_key = x->key_a;
     launch_index_plain(x->tdev[0], x->ps[x->cur], x->key_a, x->n_dev, x->n_cap, x->stream, &x->prof);
 }
 
@@ -488,6 +521,7 @@ static void run_sort(dsmc_ctx *x, const int *n_dev)
     radix_sort(x->key_a, nullptr, ak, av, ok, ov, n_dev, x->key_bits, x->sort, x->stream, &x->prof);
     x->sorted_key = ok;
     x->perm = ov;
+    x->perm_mask = -1;
 }
 
 static void plain_sort(dsmc_ctx *x)
@@ -512,14 +546,20 @@ static void plain_collide(dsmc_ctx *x)
     x->coll_steps++;
 }
 
-static void plain_spin(dsmc_ctx *x)
+static SpinParams spin_params(const dsmc_ctx *x)
 {
     SpinParams sp;
     sp.gs = x->cfg.gs;
     sp.dt = x->cfg.dt;
     sp.substeps = x->cfg.spin_substeps;
-    sp.dt_spin = x->cfg.dt / x->cfg.spin_substeps;
+    sp.dt_spin = x->cfg.spin_substeps > 0 ? x->cfg.dt / x->cfg.spin_substeps : x->cfg.dt;
     sp.interp = x->cfg.spin_interp;
+    return sp;
+}
+
+static void plain_spin(dsmc_ctx *x)
+{
+    const SpinParams sp = spin_params(x);
     launch_spin_plain(x->tdev[0], sp, x->ps[x->cur], x->n_dev, x->n_cap, x->stream, &x->prof);
 }
 
@@ -531,7 +571,7 @@ static void plain_local_pops(dsmc_ctx *x)
                             &x->prof);
 }
 
-static void plain_flip(dsmc_ctx *x)
+static FlipParams flip_params(const dsmc_ctx *x)
 {
     FlipParams fp;
     std::memset(&fp, 0, sizeof fp);
@@ -539,16 +579,28 @@ static void plain_flip(dsmc_ctx *x)
     fp.mass = x->cfg.mass;
     fp.gap = 2.0 * x->tdev[0].mu;
     fp.step = (uint32_t)x->coll_steps;
+    return fp;
+}
+
+static void plain_flip(dsmc_ctx *x)
+{
+    const FlipParams fp = flip_params(x);
     launch_flip_plain(x->tdev[0], fp, x->ps[x->cur], x->pops, x->flips, x->n_dev, x->n_cap,
                       x->stream, &x->prof);
 }
 
-static void plain_decay(dsmc_ctx *x)
+static DecayParams decay_params(const dsmc_ctx *x)
 {
     DecayParams dp;
     dp.dt = x->cfg.lpc * x->cfg.dt;
     dp.sigma = x->cfg.sigma;
     dp.mass = x->cfg.mass;
+    return dp;
+}
+
+static void plain_decay(dsmc_ctx *x)
+{
+    const DecayParams dp = decay_params(x);
     launch_decay_plain(x->tdev[0], dp, x->ps[x->cur], x->n_dev, x->n_cap, x->stream, &x->prof);
 }
 
@@ -588,31 +640,136 @@ static void plain_observe(dsmc_ctx *x, dsmc_observables *slot, long long step)
                          slot, x->coll_accum, x->evap_accum, step, x->stream, &x->prof);
 }
 
-static void plain_step(dsmc_ctx *x)
+// ---------------------------------------------------------------------------
+// FP64 form, whole steps.
+// ---------------------------------------------------------------------------
+// Drops the removed atoms that still hold slots: the state is then that of the
+// reference's compaction after every motion step, with the tags of the last.
+static void plain_settle(dsmc_ctx *x)
 {
-    const int lpc = x->cfg.lpc;
-    if (x->step % lpc == 0) {
-        plain_index(x);
-        plain_sort(x);
-        plain_table(x);
-        plain_collide(x);
-        if (x->cfg.mcwf) plain_local_pops(x);
+    if (!x->lazy_dead) return;
+    const PlainCtl *c = x->ctl + x->csel;
+    int *stencil = (int *)x->res.alt_k;
+    uint32_t *map = x->res.alt_v;
+    launch_prev_dead_stencil(x->key_f, x->mask_last, c, x->n_cap, x->dead_key, stencil, x->stream);
+    compaction_map(stencil, &c->slots, x->n_cap, map, x->n_dev + 2, x->scan_partial, x->stream, nullptr);
+    launch_last_tags(map, x->mask_last, x->n_dev + 2, x->n_cap, x->tag, x->stream);
+    launch_dead_stencil(x->key_f, &c->slots, x->n_cap, x->dead_key, stencil, x->stream);
+    compaction_map(stencil, &c->slots, x->n_cap, x->cmap, x->n_dev, x->scan_partial, x->stream, nullptr);
+    launch_gather_plain(x->ps[x->cur ^ 1], x->ps[x->cur], x->cmap, x->n_dev, x->n_cap, x->cfg.spin,
+                        x->stream, nullptr);
+    x->cur ^= 1;
+    launch_set_ctl(x->ctl + x->csel, x->step, (unsigned)x->coll_steps, x->n_dev, x->stream);
+    x->lazy_dead = false;
+    x->sorted_ok = false;
+    x->keys_ok = false;
+    x->prepped = false;
+}
+
+static void plain_need_acc(dsmc_ctx *x)
+{
+    if (!x->acc_stale) return;
+    launch_accel_plain(x->tdev[0], x->ps[x->cur], x->n_cap, x->stream, nullptr);
+    x->acc_stale = false;
+}
+
+static void plain_need_tables(dsmc_ctx *x)
+{
+    if (!x->tables_stale) return;
+    launch_cell_table_plain(x->sorted_key, x->n_dev + 3, x->n_cap, x->start_end, x->count, x->prefix,
+                            x->scan_partial, x->ncells, x->stream, nullptr);
+    launch_untag_counts(x->cc_tagged, (unsigned)x->coll_steps, x->ncells, x->coll_count, x->stream);
+    x->tables_stale = false;
+}
+
+// Before a single call of the FP64 form: everything in memory as the calls
+// leave it.  What the call changes is not in the order of the last step's sort.
+static void plain_enter(dsmc_ctx *x)
+{
+    plain_settle(x);
+    plain_need_acc(x);
+    plain_need_tables(x);
+    x->ctl_live = false;
+    x->sorted_ok = false;
+    x->keys_ok = false;
+    x->prepped = false;
+}
+
+// Substeps of one launch: their log records are written by different blocks,
+// so no two may share a place of the ring.
+static int max_substeps(const dsmc_ctx *x) { return std::min(kMaxSub, x->obs_cap); }
+
+// L motion substeps from the current one, with the sort and the collisions
+// when a collision step begins (L reaches at most to its end).
+static void plain_substeps(dsmc_ctx *x, int L)
+{
+    const int lpc = x->cfg.lpc, phase = (int)(x->step % lpc);
+    const bool after = phase == 0, resort = resort_supported(x->n_cap);
+    const PlainCtl *c = x->ctl + x->csel;
+    const TrapDev &t = x->tdev[0];
+    if (after) {
+        uint32_t *ok = x->srt_k[x->srt_cur ^ 1], *ov = x->srt_v[x->srt_cur ^ 1];
+        if (x->sorted_ok && resort) {
+            resort_incremental(x->key_f, x->srt_k[x->srt_cur], &c->slots, x->dead_key, x->blk_moved,
+                               x->blk_dead, x->mask_moved, x->mask_d2[x->mpar], x->key_samp,
+                               x->key_tsamp, kStepBlock, x->prepped, x->res, ok, ov, x->stream, &x->prof);
+        } else {
+            if (!x->keys_ok)
+                launch_index_plain(t, x->ps[x->cur], x->key_f, &c->slots, x->n_cap, x->stream, &x->prof);
+            radix_sort(x->key_f, nullptr, x->res.alt_k, x->res.alt_v, ok, ov, &c->slots, x->key_bits,
+                       x->sort, x->stream, &x->prof);
+        }
+        x->srt_cur ^= 1;
+        x->sorted_key = ok;
+        x->perm = ov;
+        x->perm_mask = x->lazy_dead ? x->mpar : -1;
+        x->mpar ^= 1;
+        launch_collide_step(t, collide_params(x), x->ps[x->cur], ok, ov, c, x->n_cap, x->sigvrmax,
+                            x->cc_tagged, x->coll_accum, x->n_dev + 3, x->stream, &x->prof);
     }
-    if (x->cfg.spin) plain_spin(x);
-    launch_move_plain(x->tdev[0], x->cfg.dt, x->ps[x->cur], x->n_dev, x->n_cap, x->stream,
-                      &x->prof);
-    if (x->cfg.evaporation) {
-        plain_evap_tag(x);
-        plain_compact(x);
+    PlainStepParams p;
+    std::memset(&p, 0, sizeof p);
+    p.dt = x->cfg.dt;
+    p.mass = x->cfg.mass;
+    p.spin = spin_params(x);
+    p.flip = flip_params(x);
+    p.decay = decay_params(x);
+    p.spin_loss = (x->cfg.evaporation & DSMC_EVAP_SPIN) ? 1 : 0;
+    p.energy_cut = (x->cfg.evaporation & DSMC_EVAP_ENERGY) ? 1 : 0;
+    p.mcwf = x->cfg.mcwf;
+    p.lpc = lpc;
+    p.phase = phase;
+    p.L = L;
+    p.fast_key = t.nc[0] < (1 << 20) && t.nc[1] < (1 << 20) && t.nc[2] < (1 << 20);
+    p.dead_key = x->dead_key;
+    const bool sorted = after || x->sorted_ok;
+    p.key_prev = sorted ? x->srt_k[x->srt_cur] : nullptr;
+    p.blk_moved = x->blk_moved; p.blk_dead = x->blk_dead;
+    p.mask_moved = x->mask_moved; p.mask_dead = x->mask_d2[x->mpar]; p.mask_last = x->mask_last;
+    p.key_samp = x->key_samp; p.key_tsamp = x->key_tsamp;
+    launch_move_step(x->cfg.spin != 0, x->cfg.mcwf != 0, t, p, x->ps[x->cur],
+                     x->ps[after ? x->cur ^ 1 : x->cur], after ? x->perm : nullptr,
+                     !after && x->lazy_dead ? x->key_f : nullptr, after, c, x->key_f, x->pops,
+                     x->evap_pos_d, x->evap_vel_d, x->rec64, step_rec_stride(x->n_cap), x->n_cap,
+                     x->stream, &x->prof);
+    ResortPrepArgs prep;
+    x->prepped = sorted && resort && phase + L == lpc;
+    if (x->prepped)
+        prep = resort_prep_args(x->res, after ? &c->alive : &c->slots, kStepBlock, x->blk_moved, x->blk_dead,
+                                x->mask_moved, x->mask_d2[x->mpar]);
+    launch_step_finalize(p, after, x->rec64, step_rec_stride(x->n_cap), c, x->ctl + (x->csel ^ 1),
+                         x->coll_accum, x->evap_accum, x->obs_log, x->obs_cap, prep, x->stream, &x->prof);
+    x->csel ^= 1;
+    if (after) {
+        x->cur ^= 1;
+        x->sorted_ok = true;
+        x->tables_stale = true;
+        x->coll_steps++;
     }
-    if (x->cfg.mcwf && (x->step + 1) % lpc == 0) {   // main.cu:501-516
-        plain_flip(x);
-        plain_decay(x);
-    }
-    if (x->cfg.spin && (x->step + 1) % lpc == 0)
-        launch_normalise_plain(x->ps[x->cur], x->n_dev, x->n_cap, x->stream, &x->prof);
-    plain_observe(x, x->obs_log + (x->step % x->obs_cap), x->step);
-    x->step++;
+    x->keys_ok = true;
+    x->lazy_dead = x->cfg.evaporation != 0;
+    if (!x->cfg.mcwf) x->acc_stale = true;
+    x->step += L;
 }
 
 // ---------------------------------------------------------------------------
@@ -778,7 +935,7 @@ static void fused_step(dsmc_ctx *x)
     x->step++;
 }
 
-static bool graph_ok(const dsmc_ctx *x) { return x->fp32 && x->cfg.use_graph && !x->prof.enabled; }
+static bool graph_ok(const dsmc_ctx *x) { return x->cfg.use_graph && !x->prof.enabled; }
 
 // Destroy the captured graph.  Its earlier launches may still be in flight on
 // the stream, so the stream is drained first: an executable graph is not
@@ -793,23 +950,42 @@ static void drop_graph(dsmc_ctx *x)
     x->graph = nullptr;
 }
 
-static void fused_graph_steps(dsmc_ctx *x, int pairs)
+// The steps of one graph: two FP32 steps, or two collision steps of the FP64
+// form.  Every double buffer is back where it was after them.
+static int graph_len(const dsmc_ctx *x) { return x->fp32 ? 2 : 2 * x->cfg.lpc; }
+
+static void graph_body(dsmc_ctx *x)
 {
-    if (x->graph_exec && (x->graph_srt != x->srt_cur || x->graph_ssel != x->ssel ||
-                          x->graph_tsel != x->tsel)) {
+    if (x->fp32) {
+        fused_step(x);
+        fused_step(x);
+        return;
+    }
+    for (int k = 0; k < 2; ++k)
+        for (int done = 0; done < x->cfg.lpc;) {
+            const int L = std::min(x->cfg.lpc - done, max_substeps(x));
+            plain_substeps(x, L);
+            done += L;
+        }
+}
+
+static void graph_steps(dsmc_ctx *x, int times)
+{
+    const int ssel = x->fp32 ? x->ssel : x->csel, tsel = x->fp32 ? x->tsel : x->mpar;
+    if (x->graph_exec && (x->graph_srt != x->srt_cur || x->graph_ssel != ssel ||
+                          x->graph_tsel != tsel || x->graph_cur != x->cur)) {
         // captured with the other sort (step, trap-range) buffer current
         drop_graph(x);
     }
+    const long long step0 = x->step, cs0 = x->coll_steps;
     if (!x->graph_exec) {
-        const int cur0 = x->cur;
         x->graph_srt = x->srt_cur;
-        x->graph_ssel = x->ssel;
-        x->graph_tsel = x->tsel;
-        const long long step0 = x->step, cs0 = x->coll_steps;
+        x->graph_ssel = ssel;
+        x->graph_tsel = tsel;
+        x->graph_cur = x->cur;
         DSMC_HIP(hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
         try {
-            fused_step(x);
-            fused_step(x);
+            graph_body(x);
         } catch (...) {
             hipGraph_t g;
             (void)hipStreamEndCapture(x->stream, &g);
@@ -818,22 +994,40 @@ static void fused_graph_steps(dsmc_ctx *x, int pairs)
         }
         DSMC_HIP(hipStreamEndCapture(x->stream, &x->graph));
         DSMC_HIP(hipGraphInstantiate(&x->graph_exec, x->graph, nullptr, nullptr, 0));
-        x->cur = cur0;
-        x->srt_cur = x->graph_srt;
-        x->ssel = x->graph_ssel;
-        x->tsel = x->graph_tsel;
-        x->step = step0;
-        x->coll_steps = cs0;
     }
-    for (int k = 0; k < pairs; ++k) DSMC_HIP(hipGraphLaunch(x->graph_exec, x->stream));
-    x->step += 2LL * pairs;
-    x->coll_steps += 2LL * pairs;
+    for (int k = 0; k < times; ++k) DSMC_HIP(hipGraphLaunch(x->graph_exec, x->stream));
+    x->step = step0 + (long long)graph_len(x) * times;
+    x->coll_steps = cs0 + 2LL * times;
+    if (!x->fp32) {
+        // as the captured steps leave it
+        x->sorted_key = x->srt_k[x->srt_cur];
+        x->perm = x->srt_v[x->srt_cur];
+        x->perm_mask = x->cfg.evaporation ? x->mpar ^ 1 : -1;
+        x->tables_stale = true;
+        x->acc_stale = !x->cfg.mcwf;
+    }
 }
 
 static void do_steps(dsmc_ctx *x, int n)
 {
     if (!x->fp32) {
-        for (int k = 0; k < n; ++k) plain_step(x);
+        if (n > 0 && !x->ctl_live) {
+            launch_set_ctl(x->ctl + x->csel, x->step, (unsigned)x->coll_steps, x->n_dev, x->stream);
+            x->ctl_live = true;
+        }
+        const bool resort = resort_supported(x->n_cap);
+        while (n > 0) {
+            const int phase = (int)(x->step % x->cfg.lpc), len = graph_len(x);
+            if (graph_ok(x) && phase == 0 && n >= len && ((x->sorted_ok && x->prepped) || !resort)) {
+                const int times = n / len;
+                graph_steps(x, times);
+                n -= times * len;
+                continue;
+            }
+            const int L = std::min(std::min(x->cfg.lpc - phase, n), max_substeps(x));
+            plain_substeps(x, L);
+            n -= L;
+        }
         return;
     }
     if (x->have_sort) fail(DSMC_ESTATE, "a sort is pending: call dsmc_move_atoms first");
@@ -844,7 +1038,7 @@ static void do_steps(dsmc_ctx *x, int n)
         const bool need_srt = x->cfg.sort_mode == DSMC_SORT_INCREMENTAL;
         while (k < n && (x->cur == 1 || (need_srt && !x->srt_valid))) { fused_step(x); ++k; }
         const int pairs = (n - k) / 2;
-        if (pairs > 0) { fused_graph_steps(x, pairs); k += 2 * pairs; }
+        if (pairs > 0) { graph_steps(x, pairs); k += 2 * pairs; }
     }
     for (; k < n; ++k) fused_step(x);
 }
@@ -893,6 +1087,7 @@ static int host_alive(dsmc_ctx *x)
     if (x->fp32) {
         (void)fused_live(x, n, n_slots, false);
     } else {
+        plain_settle(x);
         read_counts(x);
         n = x->n_host[0];
     }
@@ -906,6 +1101,7 @@ static void observe_now(dsmc_ctx *x, std::vector<dsmc_observables> &out)
 {
     out.assign(x->T, dsmc_observables{});
     if (!x->fp32) {
+        plain_settle(x);
         plain_observe(x, x->obs_log + x->obs_cap, x->step);
         DSMC_HIP(hipStreamSynchronize(x->stream));
         DSMC_HIP(hipMemcpy(out.data(), x->obs_log + x->obs_cap, sizeof(dsmc_observables),
@@ -933,6 +1129,13 @@ static void observe_now(dsmc_ctx *x, std::vector<dsmc_observables> &out)
 static void reset_cells(dsmc_ctx *x)
 {
     hipStream_t st = x->stream;
+    if (!x->fp32) {
+        plain_enter(x);   // what host reads see of the earlier run stays readable
+        DSMC_HIP(hipMemsetAsync(x->cc_tagged, 0, sizeof(unsigned long long) * (x->ncells + 1), st));
+        for (int b = 0; b < 2; ++b) DSMC_HIP(hipMemsetAsync(x->ps[b].up, 1, (size_t)x->n_cap, st));
+    }
+    // the double buffers as in a new context: a captured graph stays valid
+    x->ssel = x->tsel = x->srt_cur = x->csel = x->mpar = 0;
     if (x->fp32)
         launch_init_sigvrmax(x->d_traps, x->d_key_base, x->T, x->n_keys, x->sigvrmax_f, st);
     else
@@ -1047,9 +1250,13 @@ static void copy_field(dsmc_ctx *x, int field, void *host, size_t bytes)
     double *const sd = (double *)stage(x);
     if (!x->fp32) {
         const PlainPtrs &s = x->ps[x->cur];
+        if (field == DSMC_FIELD_CELL_START_END || field == DSMC_FIELD_CELL_COUNT ||
+            field == DSMC_FIELD_CELL_PREFIX || field == DSMC_FIELD_COLLISION_COUNT)
+            plain_need_tables(x);
         switch (field) {
         case DSMC_FIELD_POS: case DSMC_FIELD_VEL: case DSMC_FIELD_ACC: {
             const int o = field == DSMC_FIELD_POS ? 0 : field == DSMC_FIELD_VEL ? 3 : 6;
+            if (field == DSMC_FIELD_ACC) plain_need_acc(x);
             launch_pack_columns(s.d + o, 3, n, sd, st);
             to_host(x, host, sd, need);
             return;
@@ -1140,6 +1347,17 @@ static void copy_field(dsmc_ctx *x, int field, void *host, size_t bytes)
     case DSMC_FIELD_PERM:
         if (!x->perm) fail(DSMC_ESTATE, "no sort has run yet");
         to_host(x, host, x->perm, need);
+        if (!x->fp32 && x->perm_mask >= 0) {
+            // slots as they were counted without the removed atoms among them
+            const std::vector<uint64_t> m = d2h(x->mask_d2[x->perm_mask], resort_mask_words(x->n_cap));
+            std::vector<uint32_t> before(m.size() + 1, 0u);
+            for (size_t w = 0; w < m.size(); ++w) before[w + 1] = before[w] + (uint32_t)__builtin_popcountll(m[w]);
+            uint32_t *h = (uint32_t *)host;
+            for (size_t i = 0; i < N; ++i) {
+                const uint32_t v = h[i], w = v >> 6;
+                h[i] = v - before[w] - (uint32_t)__builtin_popcountll(m[w] & ((1ull << (v & 63)) - 1ull));
+            }
+        }
         return;
     case DSMC_FIELD_SIGVRMAX:
         if (x->fp32) {
@@ -1320,7 +1538,6 @@ dsmc_status dsmc_set_state(dsmc_ctx *ctx, const double *pos, const double *vel, 
         launch_unpack_columns(sp, 3, n, s.d, st);
         launch_unpack_columns(sv, 3, n, s.d + 3, st);
         launch_iota(s.id, n, st);
-        DSMC_HIP(hipMemsetAsync(s.up, 1, N, st));
         launch_accel_plain(ctx->tdev[0], s, n, st, &ctx->prof);
         plain_index(ctx);
     } else {
@@ -1362,6 +1579,7 @@ dsmc_status dsmc_index_atoms(dsmc_ctx *ctx)
         if (ctx->have_sort) fail(DSMC_ESTATE, "a sort is pending: call dsmc_move_atoms first");
         fused_index(ctx);
     } else {
+        plain_enter(ctx);
         plain_index(ctx);
     }
     DSMC_API_END(ctx)
@@ -1374,6 +1592,7 @@ dsmc_status dsmc_sort_arrays(dsmc_ctx *ctx)
         if (ctx->have_sort) fail(DSMC_ESTATE, "a sort is pending: call dsmc_move_atoms first");
         fused_sort(ctx);
     } else {
+        plain_enter(ctx);
         plain_sort(ctx);
     }
     DSMC_API_END(ctx)
@@ -1387,6 +1606,7 @@ dsmc_status dsmc_build_cell_table(dsmc_ctx *ctx)
         if (!ctx->have_sort) fail(DSMC_ESTATE, "build the table right after dsmc_sort_arrays");
         fused_table(ctx);
     } else {
+        plain_enter(ctx);
         plain_table(ctx);
     }
     DSMC_API_END(ctx)
@@ -1400,6 +1620,7 @@ dsmc_status dsmc_collide(dsmc_ctx *ctx)
         fused_collide(ctx);
         ctx->coll_steps++;
     } else {
+        plain_enter(ctx);
         plain_collide(ctx);
     }
     DSMC_API_END(ctx)
@@ -1410,6 +1631,7 @@ dsmc_status dsmc_evolve_spin(dsmc_ctx *ctx)
     DSMC_API_BEGIN(ctx)
     if (!ctx->cfg.spin) fail(DSMC_ENOTSUP, "spin evolution is off in this context");
     if (ctx->fp32) fail(DSMC_ENOTSUP, "the FP32 form evolves spins inside dsmc_move_atoms");
+    plain_enter(ctx);
     plain_spin(ctx);
     launch_normalise_plain(ctx->ps[ctx->cur], ctx->n_dev, ctx->n_cap, ctx->stream, &ctx->prof);
     DSMC_API_END(ctx)
@@ -1421,6 +1643,7 @@ dsmc_status dsmc_move_atoms(dsmc_ctx *ctx)
     if (ctx->fp32) {
         fused_move(ctx);
     } else {
+        plain_enter(ctx);
         launch_move_plain(ctx->tdev[0], ctx->cfg.dt, ctx->ps[ctx->cur], ctx->n_dev, ctx->n_cap,
                           ctx->stream, &ctx->prof);
         plain_observe(ctx, ctx->obs_log + (ctx->step % ctx->obs_cap), ctx->step);
@@ -1444,6 +1667,7 @@ dsmc_status dsmc_local_populations(dsmc_ctx *ctx)
 {
     DSMC_API_BEGIN(ctx)
     if (!ctx->pops) fail(DSMC_ENOTSUP, "the spin-flip model is off in this context (cfg.mcwf)");
+    plain_enter(ctx);
     plain_local_pops(ctx);
     DSMC_API_END(ctx)
 }
@@ -1452,6 +1676,7 @@ dsmc_status dsmc_flip_atoms(dsmc_ctx *ctx, long long *n_flipped)
 {
     DSMC_API_BEGIN(ctx)
     if (!ctx->pops) fail(DSMC_ENOTSUP, "the spin-flip model is off in this context (cfg.mcwf)");
+    plain_enter(ctx);
     hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(1), 0, ctx->stream, ctx->flips);
     DSMC_HIP(hipGetLastError());
     plain_flip(ctx);
@@ -1468,6 +1693,7 @@ dsmc_status dsmc_exponential_decay(dsmc_ctx *ctx)
 {
     DSMC_API_BEGIN(ctx)
     if (!ctx->pops) fail(DSMC_ENOTSUP, "the spin-flip model is off in this context (cfg.mcwf)");
+    plain_enter(ctx);
     plain_decay(ctx);
     DSMC_API_END(ctx)
 }
@@ -1476,6 +1702,7 @@ dsmc_status dsmc_evaporation_tag(dsmc_ctx *ctx)
 {
     DSMC_API_BEGIN(ctx)
     if (ctx->fp32) fail(DSMC_ENOTSUP, "the FP32 form tags inside dsmc_move_atoms");
+    plain_enter(ctx);
     plain_evap_tag(ctx);
     DSMC_API_END(ctx)
 }
@@ -1484,6 +1711,7 @@ dsmc_status dsmc_compact(dsmc_ctx *ctx, int *n_alive)
 {
     DSMC_API_BEGIN(ctx)
     if (ctx->fp32) fail(DSMC_ENOTSUP, "the FP32 form compacts inside the sort");
+    plain_enter(ctx);
     plain_compact(ctx);
     if (n_alive) *n_alive = host_alive(ctx);
     DSMC_API_END(ctx)

@@ -9,7 +9,7 @@
 // slot -> atom label map is carried along as `id`.
 #include "dsmc_device.hpp"
 #include "dsmc_internal.hpp"
-#include "plain.hpp"
+#include "plain_device.hpp"
 
 namespace dsmc {
 
@@ -90,55 +90,26 @@ __global__ __launch_bounds__(kBlock) void k_collide_plain(
         // reset it only in cells of two or more atoms (a cell that empties
         // keeps a stale count there)
         if (n <= 1) { coll_count[cell] = 0; continue; }
-        const double Mc = 0.5 * (n - 1) * n;
-        const double X = Mc * t.alpha * lpc * cp.dt * sigvrmax[cell] / cellVolume;
-        const double lambda = ceil(X) / Mc;
-        // reference pair mode keeps collisions.cu:322's truncation of Mc * lambda
-        const int Ncol = cp.pair_mode ? (int)(Mc * lambda) : (int)ceil(X);
+        double lambda;
+        const int Ncol = plain_trials(t, cp, n, sigvrmax[cell], lambda);
         const int base = prefix[cell];
         int count = 0;
         double smax = sigvrmax[cell];
         for (int tr = 0; tr < Ncol; ++tr) {
-            int i = 0, j = 1;
+            int i, j;
             double u_acc;
-            if (cp.pair_mode == 0) {
-                U32x4 o = draw(cp.seed, t.stream, (uint32_t)cell, step, (uint32_t)tr,
-                               kPurposeCollide, 0);
-                i = (int)uint_below(o.x, (uint32_t)n);
-                j = (int)uint_below(o.y, (uint32_t)(n - 1));
-                j += (j >= i);
-                u_acc = u01(o.z, o.w);
-            } else {
-                if (n > 2) {
-                    i = 0; j = 0;
-                    for (uint32_t k = 0; k < 64 && i == j; ++k) {
-                        U32x4 o = draw(cp.seed, t.stream, (uint32_t)cell, step, (uint32_t)tr,
-                                       kPurposeCollide, 16 + k);
-                        i = (int)floor(u01(o.x, o.y) * (n - 1));
-                        j = (int)floor(u01(o.z, o.w) * (n - 1));
-                    }
-                    if (i == j) { i = 0; j = 1; }
-                }
-                U32x4 o = draw(cp.seed, t.stream, (uint32_t)cell, step, (uint32_t)tr,
-                               kPurposeCollide, 1);
-                u_acc = u01(o.x, o.y);
-            }
+            plain_trial(cp, t.stream, (uint32_t)cell, step, tr, n, i, j, u_acc);
             const int a = base + i, b = base + j;
-            const double vax = vx[a], vay = vy[a], vaz = vz[a];
-            const double vbx = vx[b], vby = vy[b], vbz = vz[b];
-            const double dx = vax - vbx, dy = vay - vby, dz = vaz - vbz;
+            D3 va = { vx[a], vy[a], vz[a] }, vb = { vx[b], vy[b], vz[b] };
+            const double dx = va.x - vb.x, dy = va.y - vb.y, dz = va.z - vb.z;
             const double magVrel = sqrt(dx * dx + dy * dy + dz * dz);
             if (magVrel * crossSection > smax) smax = magVrel * crossSection;
             const double ProbCol =
                 t.alpha * lpc * cp.dt / cellVolume * magVrel * crossSection / lambda;
             if (ProbCol > u_acc) {
-                const double cx = 0.5 * (vax + vbx), cy = 0.5 * (vay + vby), cz = 0.5 * (vaz + vbz);
-                double nx, ny, nz;
-                sphere_point(cp.seed, t.stream, (uint32_t)cell, step, (uint32_t)tr,
-                             kPurposeCollide, 2, nx, ny, nz);
-                const double wx = magVrel * nx, wy = magVrel * ny, wz = magVrel * nz;
-                vx[a] = cx - 0.5 * wx; vy[a] = cy - 0.5 * wy; vz[a] = cz - 0.5 * wz;
-                vx[b] = cx + 0.5 * wx; vy[b] = cy + 0.5 * wy; vz[b] = cz + 0.5 * wz;
+                plain_scatter(t, cp, (uint32_t)cell, step, tr, magVrel, va, vb);
+                vx[a] = va.x; vy[a] = va.y; vz[a] = va.z;
+                vx[b] = vb.x; vy[b] = vb.y; vz[b] = vb.z;
                 ++count;
             }
         }
@@ -158,19 +129,11 @@ __global__ __launch_bounds__(kBlock) void k_move_plain(TrapDev t, double dt, Pla
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= *n_dev) return;
-    double x = s.d[0][i], y = s.d[1][i], z = s.d[2][i];
-    double vx = s.d[3][i], vy = s.d[4][i], vz = s.d[5][i];
-    const bool up = s.up[i] != 0;
-    D3 a = { s.d[6][i], s.d[7][i], s.d[8][i] };
-    vx = vx + (0.5 * a.x) * dt; vy = vy + (0.5 * a.y) * dt; vz = vz + (0.5 * a.z) * dt;
-    x = x + vx * dt; y = y + vy * dt; z = z + vz * dt;
-    if (t.periodic) {
-        x = wrap_periodic(x, t.hw[0]); y = wrap_periodic(y, t.hw[1]); z = wrap_periodic(z, t.hw[2]);
-    }
-    a = accel(t, x, y, z, up);
-    vx = vx + (0.5 * a.x) * dt; vy = vy + (0.5 * a.y) * dt; vz = vz + (0.5 * a.z) * dt;
-    s.d[0][i] = x; s.d[1][i] = y; s.d[2][i] = z;
-    s.d[3][i] = vx; s.d[4][i] = vy; s.d[5][i] = vz;
+    D3 p = { s.d[0][i], s.d[1][i], s.d[2][i] }, v = { s.d[3][i], s.d[4][i], s.d[5][i] },
+       a = { s.d[6][i], s.d[7][i], s.d[8][i] };
+    plain_verlet(t, dt, s.up[i] != 0, p, v, a);
+    s.d[0][i] = p.x; s.d[1][i] = p.y; s.d[2][i] = p.z;
+    s.d[3][i] = v.x; s.d[4][i] = v.y; s.d[5][i] = v.z;
     s.d[6][i] = a.x; s.d[7][i] = a.y; s.d[8][i] = a.z;
 }
 
@@ -182,31 +145,15 @@ __global__ __launch_bounds__(kBlock) void k_spin_plain(TrapDev t, SpinParams sp,
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= *n_dev) return;
-    const double x0 = s.d[0][i], y0 = s.d[1][i], z0 = s.d[2][i];
-    double hx = 0.0, hy = 0.0, hz = 0.0;
-    if (sp.interp) {  // half-kicked velocity of the coming Verlet step
-        hx = s.d[3][i] + (0.5 * s.d[6][i]) * sp.dt;
-        hy = s.d[4][i] + (0.5 * s.d[7][i]) * sp.dt;
-        hz = s.d[5][i] + (0.5 * s.d[8][i]) * sp.dt;
+    const D3 p = { s.d[0][i], s.d[1][i], s.d[2][i] };
+    D3 v = { 0.0, 0.0, 0.0 }, a = v;
+    if (sp.interp) {
+        v = D3{ s.d[3][i], s.d[4][i], s.d[5][i] };
+        a = D3{ s.d[6][i], s.d[7][i], s.d[8][i] };
     }
-    double ur = s.psi[0][i], ui = s.psi[1][i], dr = s.psi[2][i], di = s.psi[3][i];
-    for (int m = 0; m < sp.substeps; ++m) {
-        double x = x0, y = y0, z = z0;
-        if (sp.interp) {
-            const double tau = (m + 0.5) * sp.dt_spin;
-            x = x0 + hx * tau; y = y0 + hy * tau; z = z0 + hz * tau;
-        }
-        D3 Bn;
-        const double B = field_dir(t, x, y, z, Bn);
-        const double theta = 0.5 * sp.gs * kMuB * B * sp.dt_spin / kHbar;
-        const double sn = sin(theta), cs = cos(theta);
-        const double nur = ur * cs + (Bn.x * di - Bn.y * dr + Bn.z * ui) * sn;
-        const double nui = ui * cs + ((-Bn.x) * dr - Bn.y * di - Bn.z * ur) * sn;
-        const double ndr = dr * cs + (Bn.x * ui + Bn.y * ur - Bn.z * di) * sn;
-        const double ndi = di * cs + ((-Bn.x) * ur + Bn.y * ui + Bn.z * dr) * sn;
-        ur = nur; ui = nui; dr = ndr; di = ndi;
-    }
-    s.psi[0][i] = ur; s.psi[1][i] = ui; s.psi[2][i] = dr; s.psi[3][i] = di;
+    Spinor q = { s.psi[0][i], s.psi[1][i], s.psi[2][i], s.psi[3][i] };
+    plain_spin(t, sp, p, v, a, q);
+    s.psi[0][i] = q.ur; s.psi[1][i] = q.ui; s.psi[2][i] = q.dr; s.psi[3][i] = q.di;
 }
 
 __global__ __launch_bounds__(kBlock) void k_normalise_plain(PlainPtrs s,
@@ -214,30 +161,12 @@ __global__ __launch_bounds__(kBlock) void k_normalise_plain(PlainPtrs s,
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= *n_dev) return;
-    const double ur = s.psi[0][i], ui = s.psi[1][i], dr = s.psi[2][i], di = s.psi[3][i];
-    const double N = sqrt(ur * ur + ui * ui + dr * dr + di * di);
-    s.psi[0][i] = ur / N; s.psi[1][i] = ui / N; s.psi[2][i] = dr / N; s.psi[3][i] = di / N;
+    Spinor q = { s.psi[0][i], s.psi[1][i], s.psi[2][i], s.psi[3][i] };
+    plain_normalise(q);
+    s.psi[0][i] = q.ur; s.psi[1][i] = q.ui; s.psi[2][i] = q.dr; s.psi[3][i] = q.di;
 }
 
-// ---------------------------------------------------------------------------
-// Majorana spin-flip model (wavefunction.cu:75-237): local populations before
-// the motion substeps of a collision step, flips and decoherence after them.
-// Populations are kept per atom label (the reference indexes them by atomID).
-// ---------------------------------------------------------------------------
-// projectLocalPopulations (wavefunction.cu:156-173): populations of the
-// spinor in the spin-up and spin-down states of the local field axis.
-__device__ __forceinline__ void local_pops(const TrapDev &t, double x, double y, double z,
-                                           double ur, double ui, double dr, double di,
-                                           double &pu, double &pd)
-{
-    D3 Bn;
-    (void)field_dir(t, x, y, z, Bn);
-    const double re = ur * dr + ui * di, im = ui * dr - ur * di;
-    const double w = 0.5 - ur * ur - ui * ui;
-    pu = 0.5 + Bn.x * re - Bn.y * im - Bn.z * w;
-    pd = 0.5 - Bn.x * re + Bn.y * im + Bn.z * w;
-}
-
+// Majorana spin-flip model, one call each (plain_device.hpp).
 __global__ __launch_bounds__(kBlock) void k_local_pops_plain(TrapDev t, PlainPtrs s,
                                                              double *__restrict__ pops,
                                                              const int *__restrict__ n_dev)
@@ -245,19 +174,13 @@ __global__ __launch_bounds__(kBlock) void k_local_pops_plain(TrapDev t, PlainPtr
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= *n_dev) return;
     double pu, pd;
-    local_pops(t, s.d[0][i], s.d[1][i], s.d[2][i], s.psi[0][i], s.psi[1][i], s.psi[2][i],
-               s.psi[3][i], pu, pd);
+    local_pops(t, D3{ s.d[0][i], s.d[1][i], s.d[2][i] },
+               Spinor{ s.psi[0][i], s.psi[1][i], s.psi[2][i], s.psi[3][i] }, pu, pd);
     const size_t id = (size_t)s.id[i];
     pops[2 * id] = pu;
     pops[2 * id + 1] = pd;
 }
 
-// flipAtoms (wavefunction.cu:99-154): an atom changes spin state with the
-// probability that its population moved into the other state since the
-// populations were taken, if its kinetic energy can pay the potential step
-// 2 mu |B| (gs muB |B| for the reference's mu); the speed then absorbs the
-// step along the old direction.  The uniform is Philox (label, step, 0,
-// purpose 3).
 __global__ __launch_bounds__(kBlock) void k_flip_plain(TrapDev t, FlipParams fp, PlainPtrs s,
                                                        const double *__restrict__ pops,
                                                        unsigned long long *__restrict__ flips,
@@ -266,36 +189,14 @@ __global__ __launch_bounds__(kBlock) void k_flip_plain(TrapDev t, FlipParams fp,
     const int i = blockIdx.x * kBlock + threadIdx.x;
     unsigned long long cnt = 0ull;
     if (i < *n_dev) {
-        const double x = s.d[0][i], y = s.d[1][i], z = s.d[2][i];
-        const double vx = s.d[3][i], vy = s.d[4][i], vz = s.d[5][i];
+        const D3 p = { s.d[0][i], s.d[1][i], s.d[2][i] };
+        D3 v = { s.d[3][i], s.d[4][i], s.d[5][i] };
         const uint32_t id = (uint32_t)s.id[i];
-        const bool up = s.up[i] != 0;
-        const double opu = pops[2 * (size_t)id], opd = pops[2 * (size_t)id + 1];
-        double npu, npd;
-        local_pops(t, x, y, z, s.psi[0][i], s.psi[1][i], s.psi[2][i], s.psi[3][i], npu, npd);
-        D3 Bn;
-        const double magB = field_dir(t, x, y, z, Bn);
-        double Pflip, dEp;
-        if (up) {
-            Pflip = (npd - opd) / opu;
-            dEp = fp.gap * magB;
-        } else {
-            Pflip = (npu - opu) / opd;
-            dEp = (-1.0 * fp.gap) * magB;
-        }
-        const double Ek = 0.5 * fp.mass * (vx * vx + vy * vy + vz * vz);
-        const U32x4 o = draw(fp.seed, t.stream, id, fp.step, 0u, kPurposeFlip, 0u);
-        if (Pflip > u01(o.x, o.y) && Ek + dEp > 0.0) {
-            s.up[i] = up ? 0 : 1;
-            const double magVel = sqrt(vx * vx + vy * vy + vz * vz);
-            const double speed = sqrt(2.0 * (Ek + dEp) / fp.mass);
-            if (magVel > 0.0) {
-                s.d[3][i] = speed * (vx / magVel);
-                s.d[4][i] = speed * (vy / magVel);
-                s.d[5][i] = speed * (vz / magVel);
-            } else {   // no direction to keep: along +z
-                s.d[3][i] = 0.0; s.d[4][i] = 0.0; s.d[5][i] = speed;
-            }
+        bool up = s.up[i] != 0;
+        if (plain_flip(t, fp, id, pops[2 * (size_t)id], pops[2 * (size_t)id + 1], p,
+                       Spinor{ s.psi[0][i], s.psi[1][i], s.psi[2][i], s.psi[3][i] }, v, up)) {
+            s.up[i] = up ? 1 : 0;
+            s.d[3][i] = v.x; s.d[4][i] = v.y; s.d[5][i] = v.z;
             cnt = 1ull;
         }
     }
@@ -303,37 +204,14 @@ __global__ __launch_bounds__(kBlock) void k_flip_plain(TrapDev t, FlipParams fp,
     if ((threadIdx.x & (kWave - 1)) == 0 && cnt) atomicAdd(flips, cnt);
 }
 
-// calculateTau (wavefunction.cu:206-219) with getAcc (:221-237), the spin-up
-// acceleration: the decoherence time from the position- and velocity-limited
-// times of an atom that the field gradient separates.
-__device__ __forceinline__ double decoherence_tau(const TrapDev &t, double sigma, double mass,
-                                                  double x, double y, double z)
-{
-    const D3 a = accel(t, x, y, z, true);
-    const double relAccel = 2.0 * sqrt(a.x * a.x + a.y * a.y + a.z * a.z);
-    const double tauPos = 1.163 * sqrt(sigma / relAccel);
-    const double tauVel = sqrt(2. / kPiRef) * kHbar / (mass * sigma * relAccel);
-    return pow(1 / (tauPos * tauPos * tauPos) + 1 / (tauVel * tauVel * tauVel), -1. / 3.);
-}
-
-// exponentialDecay (wavefunction.cu:175-204): psi <- P+ psi + e P- psi with
-// P+- = (1 +- B.sigma) / 2 and e = exp(-dt / tau), written out per component.
 __global__ __launch_bounds__(kBlock) void k_decay_plain(TrapDev t, DecayParams dp, PlainPtrs s,
                                                         const int *__restrict__ n_dev)
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= *n_dev) return;
-    const double x = s.d[0][i], y = s.d[1][i], z = s.d[2][i];
-    const double ur = s.psi[0][i], ui = s.psi[1][i], dr = s.psi[2][i], di = s.psi[3][i];
-    D3 Bn;
-    (void)field_dir(t, x, y, z, Bn);
-    const double tau = decoherence_tau(t, dp.sigma, dp.mass, x, y, z);
-    const double om = 1. - exp(-dp.dt / tau);
-    const double op = 1. + exp(-dp.dt / tau);
-    s.psi[0][i] = 0.5 * ((Bn.x * dr + Bn.y * di + Bn.z * ur) * om + ur * op);
-    s.psi[1][i] = 0.5 * ((Bn.x * di - Bn.y * dr + Bn.z * ui) * om + ui * op);
-    s.psi[2][i] = 0.5 * ((Bn.x * ur - Bn.y * ui - Bn.z * dr) * om + dr * op);
-    s.psi[3][i] = 0.5 * ((Bn.x * ui + Bn.y * ur - Bn.z * di) * om + di * op);
+    Spinor q = { s.psi[0][i], s.psi[1][i], s.psi[2][i], s.psi[3][i] };
+    plain_decay(t, dp, D3{ s.d[0][i], s.d[1][i], s.d[2][i] }, q);
+    s.psi[0][i] = q.ur; s.psi[1][i] = q.ui; s.psi[2][i] = q.dr; s.psi[3][i] = q.di;
 }
 
 // ---------------------------------------------------------------------------
@@ -349,26 +227,18 @@ __global__ __launch_bounds__(kBlock) void k_evap_tag_plain(TrapDev t, EvapParams
     const int i = blockIdx.x * kBlock + threadIdx.x;
     double e_lost = 0.0, n_lost = 0.0;
     if (i < *n_dev) {
-        const double x = s.d[0][i], y = s.d[1][i], z = s.d[2][i];
-        const double vx = s.d[3][i], vy = s.d[4][i], vz = s.d[5][i];
-        const double E = 0.5 * ep.mass * (vx * vx + vy * vy + vz * vz) + potential_energy(t, x, y, z);
-        bool lost = false;
-        if (ep.spin_loss) {
-            D3 Bn;
-            (void)field_dir(t, x, y, z, Bn);
-            const double ur = s.psi[0][i], ui = s.psi[1][i], dr = s.psi[2][i], di = s.psi[3][i];
-            const double proj = 2. * Bn.x * (ur * dr + ui * di) + 2. * Bn.y * (ur * di - ui * dr) +
-                                2. * Bn.z * (ur * ur + ui * ui - 0.5);
-            lost = proj < 0.0;
-        }
-        if (ep.e_cut > 0.0) lost = lost || E > ep.e_cut;
+        const D3 p = { s.d[0][i], s.d[1][i], s.d[2][i] }, v = { s.d[3][i], s.d[4][i], s.d[5][i] };
+        Spinor q = { 0.0, 0.0, 0.0, 0.0 };
+        if (ep.spin_loss) q = Spinor{ s.psi[0][i], s.psi[1][i], s.psi[2][i], s.psi[3][i] };
+        double E;
+        const bool lost = plain_lost(t, ep.mass, ep.spin_loss != 0, ep.e_cut, p, v, q, E);
         tag[i] = lost ? 1 : 0;
         if (lost) {
             const int id = s.id[i];
-            evap_pos[3 * (size_t)id + 0] = x; evap_pos[3 * (size_t)id + 1] = y;
-            evap_pos[3 * (size_t)id + 2] = z;
-            evap_vel[3 * (size_t)id + 0] = vx; evap_vel[3 * (size_t)id + 1] = vy;
-            evap_vel[3 * (size_t)id + 2] = vz;
+            evap_pos[3 * (size_t)id + 0] = p.x; evap_pos[3 * (size_t)id + 1] = p.y;
+            evap_pos[3 * (size_t)id + 2] = p.z;
+            evap_vel[3 * (size_t)id + 0] = v.x; evap_vel[3 * (size_t)id + 1] = v.y;
+            evap_vel[3 * (size_t)id + 2] = v.z;
             e_lost = E;
             n_lost = 1.0;
         }

@@ -14,11 +14,12 @@
  *
  * Two numerical forms share this interface:
  *   DSMC_FP64_PLAIN  -- the drop-in: FP64 structure-of-arrays state, one kernel
- *                       per reference call, single trap.
+ *                       per reference call, single trap; dsmc_step runs
+ *                       them fused, to the same bits.
  *   DSMC_FP32_KAHAN  -- FP32 state with Kahan-compensated position/velocity
  *                       updates, FP64 reductions, fused move/index/evaporate
- *                       kernel, any number of independent traps, optional
- *                       HIP-graph replay of the step loop.
+ *                       kernel, any number of independent traps.
+ * dsmc_step of both forms replays through a HIP graph when asked.
  */
 #ifndef DSMC_H
 #define DSMC_H
@@ -87,7 +88,7 @@ typedef struct dsmc_config {
     int    spin_interp;     /* 0: rotate at the pre-move position (reference);   */
                             /* 1: at substep midpoints along the drift            */
     int    lpc;             /* motion substeps per collision step (main.cu:168)   */
-    int    use_graph;       /* FP32 form: replay dsmc_step through a HIP graph    */
+    int    use_graph;       /* replay dsmc_step through a HIP graph               */
     double dt;              /* motion time step (s)                               */
     double mass;            /* kg (d_mRb)                                         */
     double sigma;           /* cross-section (8 pi a^2, collisions.cu:312)        */

@@ -140,8 +140,8 @@ struct dsmc_ctx {
     int srt_cur = 0;                // FP32: srt_*[srt_cur] holds the last sort's result
     int graph_srt = 0;              // srt_cur at graph capture
     int graph_ssel = 0, graph_tsel = 0, graph_cur = 0;   // other buffers' parities at graph capture
-    bool prepped = false;           // FP32: the last finalize ran the re-sort's first phase
-    bool prep_in_finalize = true;   // FP32: run it there (else in the re-sort itself)
+    bool bucketed = false;          // the last finalize ran the re-sort's first phase
+    bool counts_clear = true;       // the buckets' counts are zero (a collide clears them)
     bool split_step = true;         // FP32: dsmc_step runs collide and move as two kernels
     const uint32_t *sorted_key = nullptr, *perm = nullptr;
     SortScratch sort;
@@ -190,9 +190,8 @@ struct dsmc_ctx {
     // FP32 form
     FusedPtrs fs[2];
     uint32_t *cell_start = nullptr, *cell_end = nullptr;
-    uint32_t *blk_moved = nullptr, *blk_dead = nullptr;   // per move block, for the re-sort
+    uint32_t *blk_dead = nullptr;   // removed atoms per move block (FP32)
     uint64_t *mask_moved = nullptr, *mask_dead = nullptr; // per 64 slots, for the re-sort
-    uint32_t *key_samp = nullptr, *key_tsamp = nullptr;   // samples of the last sort's keys
     // trap ranges of the slot order, double-buffered: a sorted move's
     // finalize writes the next sort's ranges to ts_buf[tsel ^ 1]
     int *ts_buf[2] = { nullptr, nullptr };
@@ -353,9 +352,6 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
     x->T = n_traps;
     x->fp32 = c->precision == DSMC_FP32_KAHAN;
     x->block = c->block_size ? c->block_size : 256;
-    // DSMC_RESORT_PREP_IN_FINALIZE=0: the re-sort's first phase runs as a
-    // kernel of the re-sort instead of in the finalize (results are the same)
-    if (const char *e = std::getenv("DSMC_RESORT_PREP_IN_FINALIZE")) x->prep_in_finalize = std::atoi(e) != 0;
     // DSMC_STEP_FUSED=1: dsmc_step runs the collisions inside the move kernel
     // (the fused step) instead of the collide and move kernels one after the
     // other; the results are bitwise the same.  The fused step is slower on
@@ -408,16 +404,13 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
     x->coll_accum = x->alloc<unsigned long long>(n_traps);
     x->n_dev = x->alloc<int>(4);
     DSMC_HIP(hipHostMalloc((void **)&x->n_host, 4 * sizeof(int), hipHostMallocDefault));
-    // incremental re-sort
+    // incremental re-sort (its counts start cleared)
     resort_scratch_bind(x->res, N, x->alloc<char>(resort_scratch_bytes(N), false));
+    resort_clear_counts(x->res, x->stream, nullptr);
     // one entry per block of the smallest move block size, whole 2048-slot
     // tiles (never-written entries stay zero)
-    x->blk_moved = x->alloc<uint32_t>((size_t)div_up(N, 2048) * (2048 / 64) + 64);
     x->blk_dead = x->alloc<uint32_t>((size_t)div_up(N, 2048) * (2048 / 64) + 64);
     x->mask_moved = x->alloc<uint64_t>(resort_mask_words(N));
-    x->key_samp = x->alloc<uint32_t>(resort_mask_words(N));
-    // (+ 4: the locate reads the samples in 16-byte pieces)
-    x->key_tsamp = x->alloc<uint32_t>(resort_mask_words(N) / (kResortTile / 64) + 4);
 
     if (!x->fp32) {
         for (int b = 0; b < 2; ++b) {
@@ -663,7 +656,7 @@ static void plain_settle(dsmc_ctx *x)
     x->lazy_dead = false;
     x->sorted_ok = false;
     x->keys_ok = false;
-    x->prepped = false;
+    x->bucketed = false;
 }
 
 static void plain_need_acc(dsmc_ctx *x)
@@ -692,7 +685,17 @@ static void plain_enter(dsmc_ctx *x)
     x->ctl_live = false;
     x->sorted_ok = false;
     x->keys_ok = false;
-    x->prepped = false;
+    x->bucketed = false;
+}
+
+// The first phase of the re-sort that follows a move of n slots with the new
+// keys key (x->bucketed: wanted), for the finalize's launch.
+static ResortList resort_first_phase(dsmc_ctx *x, const uint32_t *key, const int *n, const uint64_t *mask_dead)
+{
+    if (!x->bucketed) return ResortList();
+    if (!x->counts_clear) resort_clear_counts(x->res, x->stream, &x->prof);
+    x->counts_clear = false;
+    return resort_list_args(x->res, key, n, x->mask_moved, mask_dead, x->cfg.evaporation != 0);
 }
 
 // Substeps of one launch: their log records are written by different blocks,
@@ -709,15 +712,15 @@ static void plain_substeps(dsmc_ctx *x, int L)
     const TrapDev &t = x->tdev[0];
     if (after) {
         uint32_t *ok = x->srt_k[x->srt_cur ^ 1], *ov = x->srt_v[x->srt_cur ^ 1];
-        if (x->sorted_ok && resort) {
-            resort_incremental(x->key_f, x->srt_k[x->srt_cur], &c->slots, x->dead_key, x->blk_moved,
-                               x->blk_dead, x->mask_moved, x->mask_d2[x->mpar], x->key_samp,
-                               x->key_tsamp, kStepBlock, x->prepped, x->res, ok, ov, x->stream, &x->prof);
+        if (x->sorted_ok && x->bucketed) {
+            resort_merge(resort_merge_args(x->res, x->srt_k[x->srt_cur], &c->slots, x->dead_key, x->mask_moved,
+                                           x->mask_d2[x->mpar], x->lazy_dead, ok, ov), x->stream, &x->prof);
         } else {
             if (!x->keys_ok)
                 launch_index_plain(t, x->ps[x->cur], x->key_f, &c->slots, x->n_cap, x->stream, &x->prof);
             radix_sort(x->key_f, nullptr, x->res.alt_k, x->res.alt_v, ok, ov, &c->slots, x->key_bits,
                        x->sort, x->stream, &x->prof);
+            resort_samples(x->res, ok, x->stream, &x->prof);
         }
         x->srt_cur ^= 1;
         x->sorted_key = ok;
@@ -725,7 +728,8 @@ static void plain_substeps(dsmc_ctx *x, int L)
         x->perm_mask = x->lazy_dead ? x->mpar : -1;
         x->mpar ^= 1;
         launch_collide_step(t, collide_params(x), x->ps[x->cur], ok, ov, c, x->n_cap, x->sigvrmax,
-                            x->cc_tagged, x->coll_accum, x->n_dev + 3, x->stream, &x->prof);
+                            x->cc_tagged, x->coll_accum, x->n_dev + 3, x->res.b, x->stream, &x->prof);
+        x->counts_clear = true;
     }
     PlainStepParams p;
     std::memset(&p, 0, sizeof p);
@@ -744,21 +748,16 @@ static void plain_substeps(dsmc_ctx *x, int L)
     p.dead_key = x->dead_key;
     const bool sorted = after || x->sorted_ok;
     p.key_prev = sorted ? x->srt_k[x->srt_cur] : nullptr;
-    p.blk_moved = x->blk_moved; p.blk_dead = x->blk_dead;
     p.mask_moved = x->mask_moved; p.mask_dead = x->mask_d2[x->mpar]; p.mask_last = x->mask_last;
-    p.key_samp = x->key_samp; p.key_tsamp = x->key_tsamp;
     launch_move_step(x->cfg.spin != 0, x->cfg.mcwf != 0, t, p, x->ps[x->cur],
                      x->ps[after ? x->cur ^ 1 : x->cur], after ? x->perm : nullptr,
                      !after && x->lazy_dead ? x->key_f : nullptr, after, c, x->key_f, x->pops,
                      x->evap_pos_d, x->evap_vel_d, x->rec64, step_rec_stride(x->n_cap), x->n_cap,
                      x->stream, &x->prof);
-    ResortPrepArgs prep;
-    x->prepped = sorted && resort && phase + L == lpc;
-    if (x->prepped)
-        prep = resort_prep_args(x->res, after ? &c->alive : &c->slots, kStepBlock, x->blk_moved, x->blk_dead,
-                                x->mask_moved, x->mask_d2[x->mpar]);
+    x->bucketed = sorted && resort && phase + L == lpc;
+    const ResortList list = resort_first_phase(x, x->key_f, after ? &c->alive : &c->slots, x->mask_d2[x->mpar]);
     launch_step_finalize(p, after, x->rec64, step_rec_stride(x->n_cap), c, x->ctl + (x->csel ^ 1),
-                         x->coll_accum, x->evap_accum, x->obs_log, x->obs_cap, prep, x->stream, &x->prof);
+                         x->coll_accum, x->evap_accum, x->obs_log, x->obs_cap, list, x->stream, &x->prof);
     x->csel ^= 1;
     if (after) {
         x->cur ^= 1;
@@ -793,12 +792,9 @@ static MoveParams move_params(const dsmc_ctx *x)
     mp.obs_cap = x->obs_cap;
     mp.dead_key = x->dead_key;
     mp.count_moved = 0;
-    mp.blk_moved = x->blk_moved;
     mp.blk_dead = x->blk_dead;
     mp.mask_moved = x->mask_moved;
     mp.mask_dead = x->mask_dead;
-    mp.key_samp = x->key_samp;
-    mp.key_tsamp = x->key_tsamp;
     return mp;
 }
 
@@ -817,15 +813,15 @@ static void fused_sort(dsmc_ctx *x)
 {
     const int *n = x->n_dev + x->cur;
     uint32_t *ok = x->srt_k[x->srt_cur ^ 1], *ov = x->srt_v[x->srt_cur ^ 1];
-    if (x->srt_valid && x->cfg.sort_mode == DSMC_SORT_INCREMENTAL && resort_supported(x->n_cap))
-        resort_incremental(x->key_a, x->srt_k[x->srt_cur], n, x->dead_key, x->blk_moved,
-                           x->blk_dead, x->mask_moved, x->mask_dead, x->key_samp, x->key_tsamp,
-                           x->block * x->apt, x->prepped, x->res,
-                           ok, ov, x->stream, &x->prof);
-    else
+    if (x->srt_valid && x->bucketed) {
+        resort_merge(resort_merge_args(x->res, x->srt_k[x->srt_cur], n, x->dead_key, x->mask_moved, x->mask_dead,
+                                       x->dead_in_state, ok, ov), x->stream, &x->prof);
+    } else {
         radix_sort(x->key_a, nullptr, x->res.alt_k, x->res.alt_v, ok, ov, n, x->key_bits,
                    x->sort, x->stream, &x->prof);
-    x->prepped = false;
+        resort_samples(x->res, ok, x->stream, &x->prof);
+    }
+    x->bucketed = false;
     x->srt_cur ^= 1;
     x->sorted_key = ok;
     x->perm = ov;
@@ -855,7 +851,8 @@ static void fused_collide(dsmc_ctx *x)
     fused_need_table(x);
     launch_collide_fused(x->d_traps, x->d_key_base, x->T, collide_params(x), x->sorted_key,
                          x->perm, x->n_dev + (x->cur ^ 1), x->fs[x->cur], x->sigvrmax_f,
-                         x->coll_accum, x->step_dev(), x->n_cap, x->stream, &x->prof);
+                         x->coll_accum, x->step_dev(), x->res.b, x->n_cap, x->stream, &x->prof);
+    x->counts_clear = true;
 }
 
 // coll: the fused step (the collisions of this step run inside the move
@@ -895,17 +892,13 @@ static void fused_move(dsmc_ctx *x, bool coll = false)
     // a sorted move's finalize also leaves the next sort's trap ranges and
     // alive count (the removed atoms go to the end), and runs the first phase
     // of the incremental re-sort that follows
-    ResortPrepArgs prep;
-    x->prepped = x->prep_in_finalize && x->have_sort &&
-                 x->cfg.sort_mode == DSMC_SORT_INCREMENTAL && resort_supported(x->n_cap);
-    if (x->prepped)
-        prep = resort_prep_args(x->res, n, x->block * x->apt, x->blk_moved, x->blk_dead,
-                                x->mask_moved, x->mask_dead);
+    x->bucketed = x->have_sort && x->cfg.sort_mode == DSMC_SORT_INCREMENTAL && resort_supported(x->n_cap);
+    const ResortList list = resort_first_phase(x, x->key_a, n, x->mask_dead);
     launch_obs_finalize(x->T, x->max_trap_atoms, x->block * x->apt, x->cfg.mass, x->trap_start(),
                         x->have_sort ? x->ts_buf[x->tsel ^ 1] : nullptr, x->blk_dead,
                         x->mask_dead, x->rec, x->coll_accum, x->step_dev(),
                         x->step_buf + (x->ssel ^ 1), x->obs_log, x->obs_cap,
-                        x->have_sort ? x->n_dev + x->cur : nullptr, prep, x->stream, &x->prof);
+                        x->have_sort ? x->n_dev + x->cur : nullptr, list, x->stream, &x->prof);
     x->ssel ^= 1;
     if (x->have_sort) x->tsel ^= 1;
     if (!x->have_sort)  // keep the count with the state it describes
@@ -1018,7 +1011,7 @@ static void do_steps(dsmc_ctx *x, int n)
         const bool resort = resort_supported(x->n_cap);
         while (n > 0) {
             const int phase = (int)(x->step % x->cfg.lpc), len = graph_len(x);
-            if (graph_ok(x) && phase == 0 && n >= len && ((x->sorted_ok && x->prepped) || !resort)) {
+            if (graph_ok(x) && phase == 0 && n >= len && ((x->sorted_ok && x->bucketed) || !resort)) {
                 const int times = n / len;
                 graph_steps(x, times);
                 n -= times * len;

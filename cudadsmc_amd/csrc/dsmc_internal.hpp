@@ -89,54 +89,69 @@ void radix_sort(const uint32_t *keys, const uint32_t *vals, uint32_t *keys_alt,
                 const int *n_dev, int key_bits, const SortScratch &s,
                 hipStream_t stream, Profiler *prof);
 
-// Incremental re-sort (see primitives.hip): the stable sort of key_new[0..n)
-// by (key, slot), for slots that are in stable sorted order of key_old, into
-// out (which must not alias key_old).  dead_key sorts last.  Slots are
-// grouped in tiles of kResortTile.
+// Incremental re-sort (see primitives.hip): the stable sort of a state's new
+// keys by (key, slot), for slots in stable sorted order of key_old, into out
+// (which must not alias key_old).  dead_key sorts last.  Slots are grouped in
+// tiles of kResortTile.
 constexpr int kResortTile = 2048;
+// What the first phase leaves for the merge: the movers in buckets and the
+// movers and removed atoms per tile.  tsamp: first key of every tile of the
+// order that the slots are in.
+struct ResortBuckets {
+    const uint32_t *tsamp = nullptr;
+    uint32_t *tile_moved = nullptr;
+    uint32_t *tile_dead = nullptr;
+    uint32_t *bcnt = nullptr;         // movers per bucket; cleared with n_over: n_counts words from here
+    uint32_t *n_over = nullptr;       // movers in the overflow list
+    uint64_t *room = nullptr;         // the buckets' fixed rooms (key << 32 | slot)
+    uint64_t *over = nullptr;
+    int n_counts = 0;
+};
+// One first phase: the n_dev slots' new keys and the move's masks of the atoms
+// whose key changed and of the removed ones.  blocks = 0: none.
+struct ResortList {
+    int blocks = 0;
+    int tiles = 0, may_remove = 1;
+    const int *n_dev = nullptr;
+    const uint32_t *key_new = nullptr;
+    const uint64_t *mask_m = nullptr, *mask_d = nullptr;
+    ResortBuckets b;
+};
 struct ResortScratch {
     int n_cap = 0, tiles = 0;
-    uint32_t *mov_k = nullptr, *mov_v = nullptr;
-    uint32_t *mov_q = nullptr, *mov_r = nullptr;
-    uint32_t *bk_k = nullptr, *bk_v = nullptr, *bk_q = nullptr;   // buckets' fixed rooms
-    uint32_t *srt_k = nullptr, *srt_v = nullptr, *srt_q = nullptr;
-    uint32_t *alt_k = nullptr, *alt_v = nullptr, *spare = nullptr;
-    uint32_t *tile_cnt = nullptr, *tile_dead = nullptr, *bcnt = nullptr;
-    int *counts = nullptr;       // [0] stays, [1] movers, [2] removed, [3] bucket overflow
+    ResortBuckets b;
+    uint32_t *tsamp = nullptr;        // b.tsamp, for its writers
+    uint64_t *big = nullptr, *big_alt = nullptr;        // buckets larger than the merge's LDS table
+    uint32_t *alt_k = nullptr, *alt_v = nullptr;        // the radix sort's alternates (share big_alt)
 };
-// Arguments of the re-sort's first phase when another kernel runs it (the
-// fused finalize); blocks = 0: not run there.
-struct ResortPrepArgs {
-    int blocks = 0;
-    int per_tile = 0;              // move blocks per tile
-    const int *n_dev = nullptr;    // slots the move wrote
-    const uint32_t *blk_moved = nullptr, *blk_dead = nullptr;
+// One merge: n_dev slots in sorted order of key_old, the move's masks of the
+// movers and removed atoms; may_remove = 0: no atom can have been removed.
+struct ResortMerge {
+    ResortBuckets b;
+    const uint32_t *key_old = nullptr;
     const uint64_t *mask_m = nullptr, *mask_d = nullptr;
-    uint32_t *pre_m = nullptr, *pre_d = nullptr, *mov_v = nullptr, *bcnt = nullptr;
-    int *counts = nullptr;
+    const int *n_dev = nullptr;
+    int n_cap = 0, tiles = 0, may_remove = 1;
+    uint32_t dead_key = 0;
+    uint64_t *big = nullptr, *big_alt = nullptr;
+    uint32_t *out_k = nullptr, *out_v = nullptr;
+    uint32_t *tsamp_out = nullptr;
 };
-// The first phase of an incremental re-sort of n_dev slots that follows a
-// move of move_block-slot blocks.
-ResortPrepArgs resort_prep_args(const ResortScratch &r, const int *n_dev, int move_block,
-                                const uint32_t *blk_moved, const uint32_t *blk_dead,
-                                const uint64_t *mask_m, const uint64_t *mask_d);
 size_t resort_scratch_bytes(int n_cap);
 void resort_scratch_bind(ResortScratch &r, int n_cap, void *mem);
 bool resort_supported(int n_cap);
 // 64-bit words of each of the mover and removal masks for n_cap slots.
 size_t resort_mask_words(int n_cap);
-// blk_moved / blk_dead: per block of move_block slots, the atoms whose key
-// changed (not removed) and the removed atoms; mask_m / mask_d: the same
-// atoms as one bit per slot; key_samp / key_tsamp: key_old[64 w] for every
-// 64-slot word w and key_old[kResortTile t] for every tile t below n (all
-// written by the fused move).  prepped: the first phase (resort_prep_block)
-// already ran on these masks (in the fused finalize).
-void resort_incremental(const uint32_t *key_new, const uint32_t *key_old, const int *n_dev,
-                        uint32_t dead_key, const uint32_t *blk_moved, const uint32_t *blk_dead,
-                        const uint64_t *mask_m, const uint64_t *mask_d, const uint32_t *key_samp,
-                        const uint32_t *key_tsamp, int move_block, bool prepped,
-                        const ResortScratch &r, uint32_t *out_k, uint32_t *out_v,
-                        hipStream_t stream, Profiler *prof);
+ResortList resort_list_args(const ResortScratch &r, const uint32_t *key_new, const int *n_dev,
+                            const uint64_t *mask_m, const uint64_t *mask_d, bool may_remove);
+ResortMerge resort_merge_args(const ResortScratch &r, const uint32_t *key_old, const int *n_dev,
+                              uint32_t dead_key, const uint64_t *mask_m, const uint64_t *mask_d,
+                              bool may_remove, uint32_t *out_k, uint32_t *out_v);
+void resort_merge(const ResortMerge &m, hipStream_t stream, Profiler *prof);
+// After a full sort: the first keys of the tiles of the sorted order.
+void resort_samples(const ResortScratch &r, const uint32_t *sorted, hipStream_t stream, Profiler *prof);
+// Clears the buckets' counts (a collide after the merge does it otherwise).
+void resort_clear_counts(const ResortScratch &r, hipStream_t stream, Profiler *prof);
 
 // Exclusive scan of n ints (n known on the host); partial holds div_up(n, tile).
 void exclusive_scan(const int *in, int *out, int n, int *partial, hipStream_t stream,

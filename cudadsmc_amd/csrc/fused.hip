@@ -10,7 +10,7 @@
 //
 // Step (one motion step, lpc = 1):
 //   sort(keys)           -> sorted keys + permutation: incrementally from the
-//                           last move's mover masks (k_ins_locate, k_ins_merge
+//                           last move's mover masks (k_ins_merge
 //                           in primitives.hip) or by a full radix sort, after
 //                           which k_table_fused finds the trap ranges and the
 //                           alive count
@@ -572,7 +572,7 @@ __global__ __launch_bounds__(CB, 5) void k_collide_fused(
     const uint32_t *__restrict__ key, const uint32_t *__restrict__ perm,
     const int *__restrict__ n_dev, int n_cap, FusedPtrs s, float *__restrict__ sigvrmax,
     unsigned long long *__restrict__ coll_accum, const long long *__restrict__ step_dev,
-    int wave_trials)
+    ResortBuckets rb, int wave_trials)
 {
     extern __shared__ int kb[];
     __shared__ WaveCells cells[CB / kWave];
@@ -593,6 +593,7 @@ __global__ __launch_bounds__(CB, 5) void k_collide_fused(
     chunk_load(key, n_cap, chunk0, ck);
     const int n = *n_dev;
     const uint32_t step = (uint32_t)*step_dev;
+    resort_clear(rb, blockIdx.x * CB + threadIdx.x, gridDim.x * CB);
     if (T > 1) {
         if (tb_j < T + 1) kb[tb_j] = tb0;
         if (tb_j + CB < T + 1) kb[tb_j + CB] = tb1;
@@ -1032,7 +1033,7 @@ void k_move_fused(
 {
     extern __shared__ int ts[];
     __shared__ double red[(BS / kWave) * 4];
-    __shared__ uint32_t wcnt[BS / kWave][2];
+    __shared__ uint32_t wcnt[BS / kWave];   // removed atoms per wave
     // (COLL) LDS of each wave's collisions
     __shared__ WaveColl<APT> wcl[COLL ? BS / kWave : 1];
     const int T = mp.n_traps;
@@ -1260,12 +1261,11 @@ void k_move_fused(
     // first slot can do that, so each accumulator receives at most one term
     // and the totals do not depend on the order of execution.
     bool any = false;
-    if (mp.count_moved) {   // per-wave masks and counts (published by the barrier below)
-        uint32_t cm = 0, cd = 0;
+    if (mp.count_moved) {   // per-wave masks and removal counts (published by the barrier below)
+        uint32_t cd = 0;
 #pragma unroll
         for (int k = 0; k < APT; ++k) {
             const uint64_t bm = __ballot(moved[k]), bd = __ballot(lost[k]);
-            cm += (uint32_t)__popcll(bm);
             cd += (uint32_t)__popcll(bd);
             if ((threadIdx.x & (kWave - 1)) == 0) {
                 // the 64-slot word of this wave's k-th atoms
@@ -1273,24 +1273,16 @@ void k_move_fused(
                                     : (b0 + k * BS) / kWave + (int)threadIdx.x / kWave;
                 mp.mask_moved[wd] = bm;
                 mp.mask_dead[wd] = bd;
-                if (at[k].t >= 0) {   // slot 64 wd is below n
-                    mp.key_samp[wd] = at[k].kold;
-                    if (wd % (kResortTile / kWave) == 0) mp.key_tsamp[wd / (kResortTile / kWave)] = at[k].kold;
-                }
             }
         }
-        if ((threadIdx.x & (kWave - 1)) == 0) {
-            wcnt[threadIdx.x / kWave][0] = cm;
-            wcnt[threadIdx.x / kWave][1] = cd;
-        }
+        if ((threadIdx.x & (kWave - 1)) == 0) wcnt[threadIdx.x / kWave] = cd;
     }
 #pragma unroll
     for (int k = 0; k < APT; ++k) any = any || lost[k];
     const bool any_lost = __syncthreads_or(any);
     if (mp.count_moved && threadIdx.x == 0) {
-        uint32_t nm = 0, nd = 0;
-        for (int w = 0; w < BS / kWave; ++w) { nm += wcnt[w][0]; nd += wcnt[w][1]; }
-        mp.blk_moved[blk] = nm;
+        uint32_t nd = 0;
+        for (int w = 0; w < BS / kWave; ++w) nd += wcnt[w];
         mp.blk_dead[blk] = nd;
     }
     if (b0 < n) {
@@ -1348,7 +1340,7 @@ __device__ __forceinline__ void stores_done()
 // finish (an atomic count) combines the others' partial sums, so no block
 // waits for another.  Block
 // (0, 0) writes the next step number to the other counter.  Blocks from P T
-// on run the next incremental re-sort's first phase (resort_prep_block).
+// on run the next incremental re-sort's first phase (resort_list_block).
 __global__ __launch_bounds__(256) void k_obs_finalize(
     int T, int P, int move_block, double half_mass, const int *__restrict__ trap_start,
     int *__restrict__ trap_next, const uint32_t *__restrict__ blk_dead,
@@ -1357,18 +1349,15 @@ __global__ __launch_bounds__(256) void k_obs_finalize(
     unsigned int *__restrict__ cnt, double *__restrict__ acc_over,
     unsigned long long *__restrict__ coll_accum, const long long *__restrict__ step_cur,
     long long *__restrict__ step_next, dsmc_observables *__restrict__ obs_log, int obs_cap,
-    int *__restrict__ n_next, ResortPrepArgs prep)
+    int *__restrict__ n_next, ResortList list)
 {
-    static_assert(kPrepWords == 256, "prep blocks are finalize blocks");
+    extern __shared__ __align__(16) uint32_t tile_first[];
+    __shared__ unsigned short list_slot[kListSlots];
     __shared__ double red[(256 / kWave) * kAccK];
-    __shared__ uint32_t ptmp[256 / kWave + 1];
-    __shared__ unsigned long long ptmp64[256 / kWave + 1];
     __shared__ bool fin;
     __shared__ double part[kMaxFinalizeP * kAccK];   // partial sums of a trap's P blocks
     if ((int)blockIdx.x >= P * T) {
-        resort_prep_block((int)blockIdx.x - P * T, *prep.n_dev, prep.blk_moved, prep.blk_dead,
-                          prep.per_tile, prep.mask_m, prep.mask_d, prep.pre_m, prep.pre_d,
-                          prep.counts, prep.mov_v, prep.bcnt, ptmp, ptmp64);
+        resort_list_block(list, (int)blockIdx.x - P * T, tile_first, list_slot);
         return;
     }
     const int p = (int)blockIdx.x % P, t = (int)blockIdx.x / P;
@@ -1663,8 +1652,8 @@ void launch_cell_range_fused(const uint32_t *key, const int *n_dev, uint32_t dea
 void launch_collide_fused(const TrapDev *traps, const int *key_base, int n_traps,
                           const CollideParams &cp, const uint32_t *key, const uint32_t *perm,
                           const int *n_dev, const FusedPtrs &s, float *sigvrmax,
-                          unsigned long long *coll_accum, const long long *step_dev, int n_cap,
-                          hipStream_t st, Profiler *prof)
+                          unsigned long long *coll_accum, const long long *step_dev,
+                          const ResortBuckets &rb, int n_cap, hipStream_t st, Profiler *prof)
 {
     const size_t lds = sizeof(int) * (size_t)(n_traps + 1);
     // DSMC_COLLIDE_WAVE_TRIALS: trial count above which a cell is run by a
@@ -1682,11 +1671,11 @@ void launch_collide_fused(const TrapDev *traps, const int *key_base, int n_traps
     if (n_traps > 1 && n_traps + 1 <= 512)
         hipLaunchKernelGGL(k_collide_fused<kWave>, dim3(fgrid(n_cap, kCollChunk)),
                            dim3(kWave), lds, st, traps, key_base, n_traps, cp, key, perm, n_dev,
-                           n_cap, s, sigvrmax, coll_accum, step_dev, wave_trials);
+                           n_cap, s, sigvrmax, coll_accum, step_dev, rb, wave_trials);
     else
         hipLaunchKernelGGL(k_collide_fused<kFBlock>, dim3(fgrid(n_cap, kFBlock * kCollItems)),
                            dim3(kFBlock), lds, st, traps, key_base, n_traps, cp, key, perm, n_dev,
-                           n_cap, s, sigvrmax, coll_accum, step_dev, wave_trials);
+                           n_cap, s, sigvrmax, coll_accum, step_dev, rb, wave_trials);
     DSMC_HIP(hipGetLastError());
     if (prof && prof->enabled) prof->end(st);
 }
@@ -1879,18 +1868,19 @@ void launch_obs_finalize(int n_traps, int max_trap_atoms, int move_block, double
                          const uint64_t *mask_dead, const ObsRecords &rec,
                          unsigned long long *coll_accum, const long long *step_cur,
                          long long *step_next, dsmc_observables *obs_log, int obs_cap,
-                         int *n_next, const ResortPrepArgs &prep, hipStream_t st,
-                         Profiler *prof)
+                         int *n_next, const ResortList &list, hipStream_t st, Profiler *prof)
 {
     // blocks per trap: about 256 move-block records each (a single block
     // summing thousands of records is a chain of dependent load rounds)
     const int blocks = div_up(max_trap_atoms > 0 ? max_trap_atoms : 1, move_block) + 1;
     const int P = std::min(kMaxFinalizeP, div_up(blocks, 256));
-    DSMC_LAUNCH(prof, "obs_finalize", (double)n_traps * 64.0, k_obs_finalize,
-                P * n_traps + prep.blocks, 256, st, n_traps, P, move_block, 0.5 * mass,
-                trap_start, trap_next, blk_dead, mask_dead, (const int *)rec.trap,
-                (const double *)rec.sum, rec.stride, rec.lvl2, rec.cnt, rec.acc_over, coll_accum,
-                step_cur, step_next, obs_log, obs_cap, n_next, prep);
+    if (prof && prof->enabled) prof->begin(st, "obs_finalize", (double)n_traps * 64.0);
+    hipLaunchKernelGGL(k_obs_finalize, dim3(P * n_traps + list.blocks), dim3(256), resort_list_lds(list), st,
+                       n_traps, P, move_block, 0.5 * mass, trap_start, trap_next, blk_dead, mask_dead,
+                       (const int *)rec.trap, (const double *)rec.sum, rec.stride, rec.lvl2, rec.cnt,
+                       rec.acc_over, coll_accum, step_cur, step_next, obs_log, obs_cap, n_next, list);
+    DSMC_HIP(hipGetLastError());
+    if (prof && prof->enabled) prof->end(st);
 }
 
 void launch_gather_fused(const FusedPtrs &dst, const FusedPtrs &src, const uint32_t *map,

@@ -115,20 +115,15 @@ struct MoveParams {
     int    n_traps;
     int    obs_cap;      // records in the observables ring (per trap)
     uint32_t dead_key;
-    // when count_moved is set: per move block, the atoms whose new key differs
-    // from their key before the move (key_prev: the last sort's sorted keys,
-    // indexed by output slot) and the removed atoms, and the same atoms as one
-    // bit per slot (64-slot words), for the incremental re-sort of the next step;
-    // key_samp / key_tsamp receive key_prev at every 64th and every
-    // kResortTile-th slot below n (the re-sort's search index)
+    // when count_moved is set: per move block the removed atoms, and as one bit
+    // per slot these and the atoms whose new key differs from their key before
+    // the move (key_prev: the last sort's sorted keys, indexed by output slot),
+    // in 64-slot words, for the incremental re-sort of the next step
     int count_moved;
     const uint32_t *key_prev;
-    uint32_t *blk_moved;
     uint32_t *blk_dead;
     uint64_t *mask_moved;
     uint64_t *mask_dead;
-    uint32_t *key_samp;
-    uint32_t *key_tsamp;
 };
 
 struct TableParams {
@@ -151,8 +146,8 @@ void launch_cell_range_fused(const uint32_t *key, const int *n_dev, uint32_t dea
 void launch_collide_fused(const TrapDev *traps, const int *key_base, int n_traps,
                           const CollideParams &cp, const uint32_t *key, const uint32_t *perm,
                           const int *n_dev, const FusedPtrs &s, float *sigvrmax,
-                          unsigned long long *coll_accum, const long long *step_dev, int n_cap,
-                          hipStream_t st, Profiler *prof);
+                          unsigned long long *coll_accum, const long long *step_dev,
+                          const ResortBuckets &rb, int n_cap, hipStream_t st, Profiler *prof);
 // Per-block observable records of the fused move (see k_move_fused).
 constexpr int kMaxFinalizeP = 64;
 struct ObsRecords {
@@ -196,16 +191,14 @@ void launch_collide_edges(const TrapDev *traps, const int *key_base, int n_traps
 // trap loses its atoms removed in this step, which the next sort puts last.
 // trap_next / n_next (when not null): the trap ranges and alive count after
 // the next sort, from the move's per-block removal counts and masks.  step
-// is read from step_cur; step + 1 is written to step_next.
-// prep.blocks > 0: the same launch also runs the next incremental re-sort's
-// first phase on the move's masks.
+// is read from step_cur; step + 1 is written to step_next.  list: the same
+// launch also runs the next incremental re-sort's first phase.
 void launch_obs_finalize(int n_traps, int max_trap_atoms, int move_block, double mass,
                          const int *trap_start, int *trap_next, const uint32_t *blk_dead,
                          const uint64_t *mask_dead, const ObsRecords &rec,
                          unsigned long long *coll_accum, const long long *step_cur,
                          long long *step_next, dsmc_observables *obs_log, int obs_cap,
-                         int *n_next, const ResortPrepArgs &prep, hipStream_t st,
-                         Profiler *prof);
+                         int *n_next, const ResortList &list, hipStream_t st, Profiler *prof);
 // Observables of the current state per trap into acc (kAccK doubles per
 // trap; kAccN = alive atoms), skipping slots with the dead key; a fixed-order
 // reduction.  first / last: n_traps ints of scratch each.

@@ -6,8 +6,8 @@
 // launches a step at lpc = 1 and 11 to 13 per motion step in the reference's
 // run.  At N = 1e4 that is launch latency (68 and 40 us a motion step), at 1e6
 // the state crosses memory some six times (188 us).  Here a collision step is
-// five launches whatever lpc is:
-//   k_ins_locate, k_ins_merge  the stable sort by (cell, slot) from the last
+// four launches whatever lpc is:
+//   k_ins_merge                the stable sort by (cell, slot) from the last
 //                              one (primitives.hip): the same permutation as
 //                              the radix sort's
 //   k_collide_step             cells of two or more atoms from the sorted keys,
@@ -48,7 +48,7 @@ __global__ __launch_bounds__(kCollBlock) void k_collide_step(
     TrapDev t, CollideParams cp, const uint32_t *__restrict__ key, const uint32_t *__restrict__ perm,
     const PlainCtl *__restrict__ ctl, int n_cap, double *__restrict__ vx, double *__restrict__ vy,
     double *__restrict__ vz, double *__restrict__ sigvrmax, unsigned long long *__restrict__ cc,
-    unsigned long long *__restrict__ coll_total, int *__restrict__ n_sorted)
+    unsigned long long *__restrict__ coll_total, int *__restrict__ n_sorted, ResortBuckets rb)
 {
     __shared__ WaveCells cells[kCollBlock / kWave];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
@@ -60,6 +60,7 @@ __global__ __launch_bounds__(kCollBlock) void k_collide_step(
     const uint32_t step = (uint32_t)ctl->step;
     const unsigned long long stamp = (unsigned long long)(ctl->coll + 1u) << 32;
     if (blockIdx.x == 0 && threadIdx.x == 0) *n_sorted = n;
+    resort_clear(rb, blockIdx.x * kCollBlock + threadIdx.x, gridDim.x * kCollBlock);
     uint32_t k_first, k_last;
     const int nm = wave_list_cells(key, n, chunk0, ck, L, k_first, k_last);
     unsigned long long mine = 0;
@@ -136,7 +137,6 @@ __global__ __launch_bounds__(kStepBlock) void k_move_step(
     constexpr int W = kStepBlock / kWave;
     __shared__ double red[kMaxSub][W][4];
     __shared__ double lred[kMaxSub][W][2];
-    __shared__ uint32_t wcnt[W][2];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int blk = blockIdx.x, i = blk * kStepBlock + threadIdx.x;
     const int n = *n_dev;
@@ -244,12 +244,6 @@ __global__ __launch_bounds__(kStepBlock) void k_move_step(
         sp.mask_moved[wd] = bm;
         sp.mask_dead[wd] = bd;
         sp.mask_last[wd] = bl;
-        if (in && sp.key_prev) {   // slot 64 wd is below n
-            sp.key_samp[wd] = kold;
-            if (wd % (kResortTile / kWave) == 0) sp.key_tsamp[wd / (kResortTile / kWave)] = kold;
-        }
-        wcnt[w][0] = (uint32_t)__popcll(bm);
-        wcnt[w][1] = (uint32_t)__popcll(bd);
     }
     __syncthreads();
     // block sums: waves in order; the atoms lost are counted up to each substep
@@ -270,33 +264,24 @@ __global__ __launch_bounds__(kStepBlock) void k_move_step(
             for (int ww = 0; ww < W; ++ww) c += lred[k][ww][1];
         rec[((size_t)l * kStepRec + 4) * stride + blk] = e;
         rec[((size_t)l * kStepRec + 5) * stride + blk] = c;
-    } else if (tid == 128) {
-        uint32_t nm = 0, nd = 0;
-#pragma unroll
-        for (int ww = 0; ww < W; ++ww) { nm += wcnt[ww][0]; nd += wcnt[ww][1]; }
-        sp.blk_moved[blk] = nm;
-        sp.blk_dead[blk] = nd;
     }
 }
 static_assert(kMaxSub * 4 <= 64, "the block sums' threads");
 
-// Grid: one block per substep, then prep.blocks blocks of the next re-sort's
+// Grid: one block per substep, then list.blocks blocks of the next re-sort's
 // first phase.  A block adds its substep's records over the move blocks (four
 // rounds of loads in flight per thread) in a fixed order.
 __global__ __launch_bounds__(256) void k_step_finalize(
     int L, double half_mass, const int *__restrict__ n_dev, const double *__restrict__ rec, int stride,
     const PlainCtl *__restrict__ ctl, PlainCtl *__restrict__ next, int collided,
     unsigned long long *__restrict__ coll_accum, double *__restrict__ evap_accum,
-    dsmc_observables *__restrict__ log, int obs_cap, ResortPrepArgs prep)
+    dsmc_observables *__restrict__ log, int obs_cap, ResortList list)
 {
-    static_assert(kPrepWords == 256, "prep blocks are finalize blocks");
+    extern __shared__ __align__(16) uint32_t tile_first[];
+    __shared__ unsigned short list_slot[kListSlots];
     __shared__ double red[(256 / kWave) * 8];
-    __shared__ uint32_t ptmp[256 / kWave + 1];
-    __shared__ unsigned long long ptmp64[256 / kWave + 1];
     if ((int)blockIdx.x >= L) {
-        resort_prep_block((int)blockIdx.x - L, *prep.n_dev, prep.blk_moved, prep.blk_dead, prep.per_tile,
-                          prep.mask_m, prep.mask_d, prep.pre_m, prep.pre_d, prep.counts, prep.mov_v,
-                          prep.bcnt, ptmp, ptmp64);
+        resort_list_block(list, (int)blockIdx.x - L, tile_first, list_slot);
         return;
     }
     const int l = (int)blockIdx.x;
@@ -392,11 +377,11 @@ __global__ __launch_bounds__(256) void k_untag_counts(const unsigned long long *
 void launch_collide_step(const TrapDev &t, const CollideParams &cp, const PlainPtrs &s, const uint32_t *key,
                          const uint32_t *perm, const PlainCtl *ctl, int n_cap, double *sigvrmax,
                          unsigned long long *cc, unsigned long long *coll_total, int *n_sorted,
-                         hipStream_t st, Profiler *prof)
+                         const ResortBuckets &rb, hipStream_t st, Profiler *prof)
 {
     DSMC_LAUNCH(prof, "collide_step", (double)n_cap * 4.0, k_collide_step,
                 div_up(n_cap > 0 ? n_cap : 1, kCollChunk * (kCollBlock / kWave)), kCollBlock, st, t, cp, key,
-                perm, ctl, n_cap, s.d[3], s.d[4], s.d[5], sigvrmax, cc, coll_total, n_sorted);
+                perm, ctl, n_cap, s.d[3], s.d[4], s.d[5], sigvrmax, cc, coll_total, n_sorted, rb);
 }
 
 void launch_move_step(bool spin, bool stored, const TrapDev &t, const PlainStepParams &p, const PlainPtrs &src,
@@ -418,12 +403,15 @@ void launch_move_step(bool spin, bool stored, const TrapDev &t, const PlainStepP
 
 void launch_step_finalize(const PlainStepParams &p, bool after_sort, const double *rec, int stride,
                           const PlainCtl *ctl, PlainCtl *next, unsigned long long *coll_accum,
-                          double *evap_accum, dsmc_observables *log, int obs_cap, const ResortPrepArgs &prep,
+                          double *evap_accum, dsmc_observables *log, int obs_cap, const ResortList &list,
                           hipStream_t st, Profiler *prof)
 {
-    DSMC_LAUNCH(prof, "step_finalize", (double)p.L * stride * kStepRec * 8.0, k_step_finalize,
-                p.L + prep.blocks, 256, st, p.L, 0.5 * p.mass, after_sort ? &ctl->alive : &ctl->slots, rec,
-                stride, ctl, next, after_sort ? 1 : 0, coll_accum, evap_accum, log, obs_cap, prep);
+    if (prof && prof->enabled) prof->begin(st, "step_finalize", (double)p.L * stride * kStepRec * 8.0);
+    hipLaunchKernelGGL(k_step_finalize, dim3(p.L + list.blocks), dim3(256), resort_list_lds(list), st, p.L,
+                       0.5 * p.mass, after_sort ? &ctl->alive : &ctl->slots, rec, stride, ctl, next,
+                       after_sort ? 1 : 0, coll_accum, evap_accum, log, obs_cap, list);
+    DSMC_HIP(hipGetLastError());
+    if (prof && prof->enabled) prof->end(st);
 }
 
 void launch_set_ctl(PlainCtl *ctl, long long step, unsigned coll, const int *n, hipStream_t st)

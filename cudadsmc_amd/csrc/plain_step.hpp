@@ -34,9 +34,7 @@ struct PlainStepParams {
     uint32_t dead_key;
     // incremental re-sort (key_prev null: the slots are in no sorted order)
     const uint32_t *key_prev;
-    uint32_t *blk_moved, *blk_dead;
     uint64_t *mask_moved, *mask_dead, *mask_last;   // mask_last: removed in the launch's last substep
-    uint32_t *key_samp, *key_tsamp;
 };
 
 // Collisions of the sorted slots (key, perm) on the state in its previous
@@ -45,7 +43,7 @@ struct PlainStepParams {
 void launch_collide_step(const TrapDev &t, const CollideParams &cp, const PlainPtrs &s, const uint32_t *key,
                          const uint32_t *perm, const PlainCtl *ctl, int n_cap, double *sigvrmax,
                          unsigned long long *cc, unsigned long long *coll_total, int *n_sorted,
-                         hipStream_t st, Profiler *prof);
+                         const ResortBuckets &rb, hipStream_t st, Profiler *prof);
 // Motion substeps of src (slot i taken from perm[i]; perm null: in place) into
 // dst.  after_sort: the launch covers ctl->alive slots, all alive; else
 // ctl->slots slots, of which key_in (when not null) marks the removed ones.
@@ -56,11 +54,11 @@ void launch_move_step(bool spin, bool stored, const TrapDev &t, const PlainStepP
                       const PlainCtl *ctl, uint32_t *key_out, double *pops, double *evap_pos, double *evap_vel,
                       double *rec, int stride, int n_cap, hipStream_t st, Profiler *prof);
 inline int step_rec_stride(int n_cap) { return div_up(n_cap > 0 ? n_cap : 1, kStepBlock); }
-// Log records of the launch's L substeps, the next counters, and (prep.blocks
+// Log records of the launch's L substeps, the next counters, and (list.blocks
 // > 0) the next re-sort's first phase.
 void launch_step_finalize(const PlainStepParams &p, bool after_sort, const double *rec, int stride,
                           const PlainCtl *ctl, PlainCtl *next, unsigned long long *coll_accum,
-                          double *evap_accum, dsmc_observables *log, int obs_cap, const ResortPrepArgs &prep,
+                          double *evap_accum, dsmc_observables *log, int obs_cap, const ResortList &list,
                           hipStream_t st, Profiler *prof);
 void launch_set_ctl(PlainCtl *ctl, long long step, unsigned coll, const int *n, hipStream_t st);
 // *n = the alive atoms of ctl.

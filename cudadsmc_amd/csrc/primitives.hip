@@ -198,463 +198,54 @@ void radix_sort(const uint32_t *keys, const uint32_t *vals, uint32_t *keys_alt,
 }
 
 // ---------------------------------------------------------------------------
-// Incremental re-sort.  Input: keys key_new[0..n) of slots that were in
-// stable sorted order of key_old[0..n) (the previous sort's keys), and the
-// move kernel's per-64-slot masks of the slots whose key changed ("movers")
-// and of removed atoms (dead key, which sorts last).  Output: the stable sort
-// of key_new by (key, slot) -- the same permutation a full radix sort gives
-// -- in a buffer other than key_old.  Between time steps only the atoms that
-// crossed a cell face change key (a few percent); the others ("stays") keep
-// their order, so nothing is sorted but the movers, and the stays are never
-// copied out of slot order:
-//   1-2. prep: movers and removed atoms before every 2048-slot tile (prefix
-//      sums of the move kernel's per-block counts) and the movers' slots in
-//      slot order (resort_prep_block; normally run by the fused finalize
-//      right after the move, alongside its per-trap sums);
-//   3. locate: each mover's insertion point q in slot space, the first slot
-//      j with (key_old[j], j) >= (key, slot) (binary search of key_old, whose
-//      stays equal key_new, through samples of it that the move kernel
-//      left): the mover goes after every stay below q and before every stay
-//      from q on.  Movers are bucketed by the tile of q: each takes the next
-//      place of its bucket's fixed room of kBucketCap entries (one atomic per
-//      bucket and wave), or, beyond the room, of an overflow list;
-//   4. merge: one block per tile adds up the bucket counts of the earlier
-//      tiles, ranks its bucket's movers by counting (buckets hold a few
-//      dozen; a bucket beyond the LDS table of kBucketLds movers is gathered
-//      from its room and the overflow list and sorted in scratch), and
-//      writes the tile's stays and movers to
-//      their final positions: with S = stays before the tile plus movers in
-//      earlier buckets, a stay goes to S + (stays of the tile before it) +
-//      (bucket movers with q <= its slot), a mover of rank r to S + (stays
-//      of the tile below q) + r.  The tile's removed atoms go to the end of
-//      the output, in slot order.
+// Incremental re-sort.  Input: slots that were in stable sorted order of
+// key_old[0..n) (the previous sort's keys), their new keys, and what the move
+// kernel left: per 64 slots a mask of the atoms whose key changed ("movers")
+// and one of the removed atoms (dead key, which sorts last).  Output: the
+// stable sort of the new keys by (key, slot) -- the same permutation a full
+// radix sort gives -- in a buffer other than key_old.  Between time steps only
+// the atoms that crossed a cell face change key (a few percent); the others
+// ("stays") keep their order, so nothing is sorted but the movers, and the
+// stays are never copied out of slot order:
+//   * first phase (resort_list_block, in the finalize's launch): the movers and
+//     removed atoms of every 2048-slot tile are counted, and every mover goes
+//     to the bucket of its tile, the last one whose first (key, slot) lies
+//     below its own: the next place of the bucket's fixed room of kBucketCap
+//     entries or, beyond it, of an overflow list;
+//   * merge (resort_merge_block): one block per tile adds up the counts of the
+//     earlier tiles, finds its bucket's insertion points by binary search of
+//     the tile's keys in LDS and ranks movers at the same point by counting
+//     (buckets hold a few dozen; one beyond the LDS table of kBucketLds movers
+//     is gathered and sorted in scratch), and writes the tile's stays and
+//     movers to their final positions: with S = stays before the tile plus
+//     movers in earlier buckets, a stay goes to S + (stays of the tile before
+//     it) + (bucket movers inserted up to it), a mover of rank r to S + (stays
+//     of the tile below its point) + r.  The tile's removed atoms go to the
+//     end of the output, in slot order.  It also leaves the first key of
+//     every tile of the new order, for the next move.
 // No kernel waits on another block.
 // ---------------------------------------------------------------------------
-constexpr int kBucketLds = 1024;               // movers a bucket ranks in LDS
-constexpr int kBucketCap = 1024;               // fixed room of a bucket (>= kBucketLds)
-constexpr int kBucketBits = 13;
-constexpr int kMaxBuckets = 1 << kBucketBits;  // tiles the locate's LDS sample table holds
-
-// Stand-alone first phase (when the fused finalize did not run it): see
-// resort_prep_block.
-__global__ __launch_bounds__(kPrepWords) void k_ins_prep(
-    const uint32_t *__restrict__ blk_moved, const uint32_t *__restrict__ blk_dead, int per_tile,
-    const uint64_t *__restrict__ mask_m, const uint64_t *__restrict__ mask_d,
-    const int *__restrict__ n_dev, uint32_t *__restrict__ pre_m, uint32_t *__restrict__ pre_d,
-    int *__restrict__ counts, uint32_t *__restrict__ mov_v, uint32_t *__restrict__ bcnt)
+__global__ __launch_bounds__(256) void k_ins_merge(ResortMerge m)
 {
-    __shared__ uint32_t tmp[kPrepWords / kWave + 1];
-    __shared__ unsigned long long tmp64[kPrepWords / kWave + 1];
-    resort_prep_block((int)blockIdx.x, *n_dev, blk_moved, blk_dead, per_tile, mask_m, mask_d, pre_m,
-                      pre_d, counts, mov_v, bcnt, tmp, tmp64);
+    __shared__ MergeLds lds;
+    resort_merge_block(m, (int)blockIdx.x, lds);
 }
 
-// (key, slot) order; slots are distinct.
-__device__ __forceinline__ bool kv_less(uint32_t ka, uint32_t va, uint32_t kb, uint32_t vb)
+__global__ __launch_bounds__(256) void k_tile_samples(const uint32_t *__restrict__ sorted, int tiles,
+                                                      uint32_t *__restrict__ tsamp)
 {
-    return ka < kb || (ka == kb && va < vb);
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t < tiles) tsamp[t] = sorted[(size_t)t * kStayTile];   // past the slots: never used
 }
 
-// Insertion point q of every mover in slot space: the first slot j with
-// (key_old[j], j) >= (key, slot) (key_old is sorted, so this is a prefix).
-// The move kernel sampled key_old at every tile start (tsamp, 2048 slots
-// apart) and every 64 slots (samp).  The search narrows q to one tile by a
-// binary search of the tile samples in LDS, to 64 slots by the 32 samples of
-// that tile (one 128-byte line, loaded at once), and then by a binary search
-// of those 64 slots of key_old (two lines): the same few steps wherever the
-// mover lands (a move along z crosses about Nc^2 cells' worth of atoms).
-// Each mover then takes the next place of q's bucket (the 2048-slot tile of
-// q): a bucket has a fixed room of kBucketCap movers, and the movers beyond
-// it go to an overflow list.
-__global__ __launch_bounds__(256) void k_ins_locate(
-    const uint32_t *__restrict__ key_new, const uint32_t *__restrict__ key_old,
-    const uint32_t *__restrict__ samp, const uint32_t *__restrict__ tsamp,
-    const uint32_t *__restrict__ mov_v, int n_cap, const int *__restrict__ n_dev,
-    int *__restrict__ counts, uint32_t *__restrict__ fb_k, uint32_t *__restrict__ fb_v,
-    uint32_t *__restrict__ fb_q, uint32_t *__restrict__ ov_k, uint32_t *__restrict__ ov_v,
-    uint32_t *__restrict__ ov_q, uint32_t *__restrict__ bcnt)
-{
-    __shared__ __align__(16) uint32_t lt[kMaxBuckets];
-    // the first round's mover slot and the tile samples are loaded with the
-    // counts (entries past them are never used); the samples four per
-    // 16-byte load, up to four loads per thread in flight
-    const int jf = blockIdx.x * 256 + threadIdx.x;
-    uint32_t vn = jf < n_cap ? mov_v[jf] : 0u;
-    const int ntc = (n_cap + kStayTile - 1) >> kStayShift;
-    {
-        const uint4 *t4 = (const uint4 *)tsamp;
-        uint4 *l4 = (uint4 *)lt;
-        const int nv = (ntc + 3) >> 2;
-        for (int v0 = threadIdx.x; v0 < nv; v0 += 4 * 256) {
-            uint4 c[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int v = v0 + u * 256;
-                c[u] = v < nv ? t4[v] : make_uint4(0u, 0u, 0u, 0u);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (v0 + u * 256 < nv) l4[v0 + u * 256] = c[u];
-        }
-    }
-    const int s = *n_dev, m = counts[1];
-    if (blockIdx.x * 256 >= m) return;   // whole block leaves together
-    const int nt = (s + kStayTile - 1) >> kStayShift;   // tiles (samples in tsamp)
-    const int nw = (s + 63) >> 6;                       // 64-slot samples in samp
-    uint32_t kn = jf < m ? key_new[vn] : 0u;
-    __syncthreads();
-    // the grid covers 1/16 of the slots; more movers take further rounds
-    for (int j0 = 0; j0 < m; j0 += (int)gridDim.x * 256) {
-        const int j = j0 + blockIdx.x * 256 + threadIdx.x;
-        const bool valid = j < m;
-        const uint32_t v = vn, k = kn;
-        if (j0 + (int)gridDim.x * 256 < m) {   // the next round's mover
-            const int jn = j + (int)gridDim.x * 256;
-            vn = jn < m ? mov_v[jn] : 0u;
-            kn = jn < m ? key_new[vn] : 0u;
-        }
-        int lo = 0;
-        if (valid) {
-            // tiles whose first slot lies below (k, v)
-            int hi = nt;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (kv_less(lt[mid], (uint32_t)mid << kStayShift, k, v)) lo = mid + 1; else hi = mid;
-            }
-            if (lo > 0) {
-                // the tile's 32 samples (one 128-byte line, loaded at once):
-                // those below (k, v) are a prefix, at least the first
-                const int w0 = (lo - 1) * kTileWords;
-                const uint4 *s4 = (const uint4 *)(samp + w0);
-                uint4 sw[kTileWords / 4];
-#pragma unroll
-                for (int u = 0; u < kTileWords / 4; ++u) sw[u] = s4[u];
-                int c = 0;
-#pragma unroll
-                for (int u = 0; u < kTileWords / 4; ++u) {
-                    const int w = w0 + 4 * u;
-                    c += (w + 0 < nw && kv_less(sw[u].x, (uint32_t)(w + 0) << 6, k, v));
-                    c += (w + 1 < nw && kv_less(sw[u].y, (uint32_t)(w + 1) << 6, k, v));
-                    c += (w + 2 < nw && kv_less(sw[u].z, (uint32_t)(w + 2) << 6, k, v));
-                    c += (w + 3 < nw && kv_less(sw[u].w, (uint32_t)(w + 3) << 6, k, v));
-                }
-                // q lies after the last such sample g and at or before g + 64
-                const int g = (w0 + c - 1) << 6;
-                lo = g + 1;
-                hi = min(g + 64, s);
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (kv_less(key_old[mid], (uint32_t)mid, k, v)) lo = mid + 1; else hi = mid;
-                }
-            }
-        }
-        // bucket slot: lanes of a wave with the same bucket share one atomic
-        // (nearby movers mostly share buckets)
-        const uint32_t bkt = (uint32_t)lo >> kStayShift;
-        const uint64_t peers = match_bits<kBucketBits>(bkt, __ballot(valid));
-        const int leader = __ffsll((unsigned long long)peers) - 1;
-        uint32_t base = 0;
-        if (valid && (int)(threadIdx.x & (kWave - 1)) == leader)
-            base = atomicAdd(&bcnt[bkt], (uint32_t)__popcll(peers));
-        base = __shfl(base, leader < 0 ? 0 : leader, kWave);
-        if (valid) {
-            const uint32_t r = base + (uint32_t)__popcll(peers & lanemask_lt());
-            if (r < (uint32_t)kBucketCap) {   // the bucket's fixed room
-                const size_t o = (size_t)bkt * kBucketCap + r;
-                fb_k[o] = k; fb_v[o] = v; fb_q[o] = (uint32_t)lo;
-            } else {   // beyond it: the overflow list
-                const int o = atomicAdd(&counts[kOverflowCount], 1);
-                ov_k[o] = k; ov_v[o] = v; ov_q[o] = (uint32_t)lo;
-            }
-        }
-    }
-}
-
-// Sort of one bucket that does not fit the LDS table, by one block, in
-// global scratch: chunks of kBucketLds sorted in LDS (bitonic network), then
-// pairwise merges of runs (merge path per thread).  Used only when a great
-// many atoms land between the same two stays (e.g. nearly all atoms change
-// cell in one step); O(b log b) work for one block.  Leaves the sorted bucket
-// in (k0, v0, q0) or (k1, v1, q1); returns the one that holds it.
-__device__ int big_bucket_sort(uint32_t *k0, uint32_t *v0, uint32_t *q0, uint32_t *k1, uint32_t *v1,
-                               uint32_t *q1, int b, uint32_t *lk, uint32_t *lv, uint32_t *lq)
-{
-    const int tid = threadIdx.x;
-    for (int c0 = 0; c0 < b; c0 += kBucketLds) {
-        const int c = min(kBucketLds, b - c0);
-        for (int e = tid; e < kBucketLds; e += 256) {
-            const bool in = e < c;
-            lk[e] = in ? k0[c0 + e] : 0xFFFFFFFFu;
-            lv[e] = in ? v0[c0 + e] : 0xFFFFFFFFu;
-            lq[e] = in ? q0[c0 + e] : 0xFFFFFFFFu;
-        }
-        __syncthreads();
-        for (int size = 2; size <= kBucketLds; size <<= 1) {
-            for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                for (int pr = tid; pr < kBucketLds / 2; pr += 256) {
-                    const int i = 2 * pr - (pr & (stride - 1));   // lower index of the pair
-                    const int j = i + stride;
-                    const bool up = (i & size) == 0;
-                    const bool gt = kv_less(lk[j], lv[j], lk[i], lv[i]);
-                    if (gt == up) {
-                        uint32_t t = lk[i]; lk[i] = lk[j]; lk[j] = t;
-                        t = lv[i]; lv[i] = lv[j]; lv[j] = t;
-                        t = lq[i]; lq[i] = lq[j]; lq[j] = t;
-                    }
-                }
-                __syncthreads();
-            }
-        }
-        for (int e = tid; e < c; e += 256) { k0[c0 + e] = lk[e]; v0[c0 + e] = lv[e]; q0[c0 + e] = lq[e]; }
-        __syncthreads();
-    }
-    int src = 0;
-    for (int wdt = kBucketLds; wdt < b; wdt <<= 1) {
-        const uint32_t *sk = src ? k1 : k0, *sv = src ? v1 : v0, *sq = src ? q1 : q0;
-        uint32_t *dk = src ? k0 : k1, *dv = src ? v0 : v1, *dq = src ? q0 : q1;
-        for (int lo = 0; lo < b; lo += 2 * wdt) {
-            const int na = min(wdt, b - lo), nb = max(0, min(wdt, b - lo - wdt));
-            const int len = na + nb;
-            const int per = (len + 255) / 256;
-            const int d0 = min(tid * per, len), d1 = min(d0 + per, len);
-            // merge path split of output d0 between run a = [lo, lo+na), b = [lo+na, ...)
-            int l = max(0, d0 - nb), h = min(d0, na);
-            while (l < h) {
-                const int mid = (l + h) >> 1;
-                const int jb = lo + na + d0 - 1 - mid;
-                if (kv_less(sk[lo + mid], sv[lo + mid], sk[jb], sv[jb])) l = mid + 1; else h = mid;
-            }
-            int ia = l, ib = d0 - l;
-            for (int d = d0; d < d1; ++d) {
-                const bool ta = ia < na && (ib >= nb || kv_less(sk[lo + ia], sv[lo + ia],
-                                                                 sk[lo + na + ib], sv[lo + na + ib]));
-                const int sidx = ta ? lo + ia : lo + na + ib;
-                dk[lo + d] = sk[sidx]; dv[lo + d] = sv[sidx]; dq[lo + d] = sq[sidx];
-                ia += ta; ib += !ta;
-            }
-        }
-        __syncthreads();   // this pass's writes are visible to the whole block
-        src ^= 1;
-    }
-    return src;
-}
-
-// One block per tile t (2048 slots).  The tile's output is a contiguous
-// window from w0: position p of the tile (slot g0 + p) is preceded there by
-// E(p) = the stays below p plus the bucket movers inserted below p, so a stay
-// at p goes to w0 + E(p) + h(p), h(p) = movers inserted at p, and a mover
-// inserted at p to w0 + E(p) + (its rank among the movers inserted at p).  E
-// is an exclusive scan of st(p) + h(p) over the tile, h a histogram of the
-// bucket in LDS.  Buckets larger than the LDS table are sorted in global
-// scratch by the block; their movers then go to w0 + (stays below p) + (rank
-// in the bucket).
-constexpr int kMergePer = kStayTile / 256;   // slots per thread
-
-__global__ __launch_bounds__(256) void k_ins_merge(
-    const uint32_t *__restrict__ key_new, const uint64_t *__restrict__ mask_m,
-    const uint64_t *__restrict__ mask_d, const int *__restrict__ n_dev, int n_cap,
-    const uint32_t *__restrict__ pre_m, const uint32_t *__restrict__ pre_d,
-    const uint32_t *__restrict__ fb_k, const uint32_t *__restrict__ fb_v,
-    const uint32_t *__restrict__ fb_q, const uint32_t *__restrict__ ov_k,
-    const uint32_t *__restrict__ ov_v, const uint32_t *__restrict__ ov_q,
-    const uint32_t *__restrict__ bcnt, const int *__restrict__ counts, uint32_t dead_key,
-    uint32_t *__restrict__ srt_k, uint32_t *__restrict__ srt_v,
-    uint32_t *__restrict__ srt_q, uint32_t *__restrict__ alt_k, uint32_t *__restrict__ alt_v,
-    uint32_t *__restrict__ alt_q, uint32_t *__restrict__ out_k, uint32_t *__restrict__ out_v)
-{
-    // the bucket's movers: (key << 32 | slot), the order they are ranked in,
-    // and insertion points
-    __shared__ __align__(16) uint64_t lkv[kBucketLds];
-    __shared__ __align__(16) uint32_t lq[kBucketLds];
-    __shared__ uint32_t H[kStayTile];      // histogram h, then the scan E
-    __shared__ uint64_t stw[kTileWords];   // stay bits of the tile's words
-    __shared__ uint32_t wst[kTileWords];   // stays of the tile before each word
-    __shared__ uint32_t tmp[256 / kWave + 1];
-    __shared__ int n_big;   // movers gathered for a big bucket
-    const int t = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int g0 = t * kStayTile;
-    const int p0 = tid * kMergePer;   // positions p0 .. p0 + 7 in the scan
-    // Every load that does not need the alive count is issued together with
-    // it, in one round: the tile's keys at positions tid + 256 u (coalesced;
-    // up to the capacity, those past the alive slots are never used), its
-    // mask words, counts and bucket size, the bucket counts of the earlier
-    // tiles, and this thread's first mover of the bucket's room (used when
-    // the bucket holds it).
-    uint32_t kk[kMergePer];
-#pragma unroll
-    for (int u = 0; u < kMergePer; ++u) {
-        const int p = tid + 256 * u;
-        kk[u] = g0 + p < n_cap ? key_new[g0 + p] : 0u;
-    }
-    const int n = *n_dev;
-    const uint32_t pm = pre_m[t], pd = pre_d[t];
-    const int b = (int)bcnt[t];
-    const int n_dead = counts[2];
-    uint64_t wm = 0ull, wd = 0ull;   // mask words of the tile (in bounds up to the last tile + 1)
-    if (tid < kTileWords) {
-        wm = mask_m[(g0 >> 6) + tid];
-        wd = mask_d[(g0 >> 6) + tid];
-    }
-    const size_t fb0 = (size_t)t * kBucketCap;   // the bucket's fixed room
-    const uint32_t mk = fb_k[fb0 + tid], mv = fb_v[fb0 + tid], mq = fb_q[fb0 + tid];
-    uint32_t bsum = 0;
-    {
-        const uint4 *c4 = (const uint4 *)bcnt;
-        const int nv = t >> 2;
-        for (int v0 = tid; v0 < nv; v0 += 4 * 256) {
-            uint4 c[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int v = v0 + u * 256;
-                c[u] = v < nv ? c4[v] : make_uint4(0u, 0u, 0u, 0u);
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) bsum += c[u].x + c[u].y + c[u].z + c[u].w;
-        }
-        if (tid < (t & 3)) bsum += bcnt[4 * nv + tid];
-    }
-    if (t > (n >> kStayShift)) return;   // whole block leaves together
-    const int ns = min(kStayTile, n - g0);   // slots of the tile (0 for the bucket at n)
-    if (tid < kTileWords) {
-        const int l0 = tid * 64;
-        uint64_t st = 0ull, dd = 0ull;
-        uint32_t od = 0u;
-        if (l0 < ns) {
-            const uint64_t in = ns - l0 >= 64 ? ~0ull : (1ull << (ns - l0)) - 1ull;
-            st = ~(wm | wd) & in;
-            dd = wd & in;
-            od = (uint32_t)(n - n_dead) + pd;
-        }
-        stw[tid] = st;
-        wst[tid] = halfwave_exclusive_scan((uint32_t)__popcll(st));
-        // removed atoms: to the end of the output, in slot order
-        od += halfwave_exclusive_scan((uint32_t)__popcll(dd));
-        for (uint64_t bb = dd; bb; bb &= bb - 1) {
-            out_k[od] = dead_key;
-            out_v[od++] = (uint32_t)(g0 + l0) + (uint32_t)(__ffsll((unsigned long long)bb) - 1);
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < kMergePer; ++u) H[tid + 256 * u] = 0u;
-    const bool small = b <= kBucketLds;
-    // movers in earlier buckets
-    uint32_t before;
-    (void)block_exclusive_scan<256>(bsum, tmp, &before);   // syncs: H cleared, stay words in place
-    // first output slot of the tile: stays of earlier tiles + earlier movers
-    const uint32_t w0 = (uint32_t)g0 - pm - pd + before;
-    const uint32_t *gk = nullptr, *gv = nullptr, *gq = nullptr;   // sorted big bucket
-    if (small) {
-        if (tid < b) {
-            lkv[tid] = (uint64_t)mk << 32 | mv;
-            lq[tid] = mq;
-            atomicAdd(&H[mq - (uint32_t)g0], 1u);
-        }
-        for (int e = tid + 256; e < b; e += 256) {
-            const uint32_t q = fb_q[fb0 + e];
-            lkv[e] = (uint64_t)fb_k[fb0 + e] << 32 | fb_v[fb0 + e];
-            lq[e] = q;
-            atomicAdd(&H[q - (uint32_t)g0], 1u);
-        }
-    } else {
-        // gather the bucket (its room, then its movers in the overflow list)
-        // in scratch and sort it there
-        uint32_t *ak = srt_k + before, *av = srt_v + before, *aq = srt_q + before;
-        uint32_t *ck = alt_k + before, *cv = alt_v + before, *cq = alt_q + before;
-        const int nr = min(b, kBucketCap);   // movers in the room
-        for (int e = tid; e < nr; e += 256) {
-            ak[e] = fb_k[fb0 + e]; av[e] = fb_v[fb0 + e]; aq[e] = fb_q[fb0 + e];
-        }
-        if (tid == 0) n_big = nr;
-        __syncthreads();
-        const int no = counts[kOverflowCount];
-        for (int e = tid; e < no; e += 256) {
-            const uint32_t q = ov_q[e];
-            if ((q >> kStayShift) == (uint32_t)t) {
-                const int o = atomicAdd(&n_big, 1);
-                ak[o] = ov_k[e]; av[o] = ov_v[e]; aq[o] = q;
-            }
-        }
-        __syncthreads();
-        uint32_t *lk = (uint32_t *)lkv, *lv = lk + kBucketLds;   // scratch of the sort
-        const int which = big_bucket_sort(ak, av, aq, ck, cv, cq, b, lk, lv, lq);
-        gk = which ? ck : ak; gv = which ? cv : av; gq = which ? cq : aq;
-        for (int r = tid; r < b; r += 256) atomicAdd(&H[gq[r] - (uint32_t)g0], 1u);
-    }
-    __syncthreads();
-    // E: exclusive scan of st(p) + h(p) over the tile, 8 consecutive
-    // positions per thread
-    const uint32_t st8 = (uint32_t)(stw[p0 >> 6] >> (p0 & 63)) & 0xFFu;
-    uint32_t e[kMergePer], run = 0;
-#pragma unroll
-    for (int u = 0; u < kMergePer; ++u) {
-        e[u] = run;
-        run += ((st8 >> u) & 1u) + H[p0 + u];
-    }
-    uint32_t total;
-    const uint32_t base = block_exclusive_scan<256>(run, tmp, &total);   // syncs: H read
-#pragma unroll
-    for (int u = 0; u < kMergePer; ++u) H[p0 + u] = base + e[u];
-    __syncthreads();   // E complete
-    // stays, at positions tid + 256 u (coalesced stores): E(p) + h(p) =
-    // E(p + 1) - st(p) = E(p + 1) - 1
-#pragma unroll
-    for (int u = 0; u < kMergePer; ++u) {
-        const int p = tid + 256 * u;
-        if (p >= ns || !((stw[p >> 6] >> (p & 63)) & 1ull)) continue;
-        const uint32_t o = w0 + (p + 1 < kStayTile ? H[p + 1] : total) - 1u;
-        out_k[o] = kk[u];
-        out_v[o] = (uint32_t)(g0 + p);
-    }
-    if (small) {
-        for (int x = tid; x < b; x += 256) {
-            const uint32_t q = lq[x], p = q - (uint32_t)g0;
-            const uint32_t ep = H[p];
-            const uint32_t stp = (uint32_t)(stw[p >> 6] >> (p & 63)) & 1u;
-            const uint32_t hp = (p + 1 < (uint32_t)kStayTile ? H[p + 1] : total) - ep - stp;
-            uint32_t r = 0;   // rank among the movers inserted at the same point
-            const uint64_t kx = lkv[x];
-            if (hp > 1) {
-                // four movers per step, without branches: (key, slot) order is
-                // the order of key << 32 | slot
-                const uint4 *lq4 = (const uint4 *)lq;
-                const ulonglong2 *k2 = (const ulonglong2 *)lkv;
-#pragma unroll 2
-                for (int f = 0; f < b; f += 4) {
-                    const uint4 qq = lq4[f >> 2];
-                    const ulonglong2 ka = k2[f >> 1], kb = k2[(f >> 1) + 1];
-                    r += (uint32_t)((qq.x == q) & (ka.x < kx));
-                    r += (uint32_t)((qq.y == q) & (ka.y < kx) & (f + 1 < b));
-                    r += (uint32_t)((qq.z == q) & (kb.x < kx) & (f + 2 < b));
-                    r += (uint32_t)((qq.w == q) & (kb.y < kx) & (f + 3 < b));
-                }
-            }
-            const uint32_t o = w0 + ep + r;
-            out_k[o] = (uint32_t)(kx >> 32);
-            out_v[o] = (uint32_t)kx;
-        }
-    } else {
-        for (int r = tid; r < b; r += 256) {
-            const int p = (int)(gq[r] - (uint32_t)g0);
-            const uint64_t below = (p & 63) ? stw[p >> 6] & (~0ull >> (64 - (p & 63))) : 0ull;
-            const uint32_t o = w0 + wst[p >> 6] + (uint32_t)__popcll(below) + (uint32_t)r;
-            out_k[o] = gk[r];
-            out_v[o] = gv[r];
-        }
-    }
-}
-
-// Per-slot arrays (movers, big-bucket scratch, radix alternates), the
-// buckets' fixed rooms (kBucketCap movers for each of the tiles + 1 buckets),
-// and per-tile counts.
-static size_t resort_room(size_t tiles) { return (tiles + 1) * (size_t)kBucketCap; }
-
+// The buckets' fixed rooms (kBucketCap movers for each of the tiles), the
+// overflow list, scratch for large buckets, and the counts.
 size_t resort_scratch_bytes(int n_cap)
 {
     const size_t n = (size_t)(n_cap > 0 ? n_cap : 1);
     const size_t tiles = (size_t)div_up((long long)n, kStayTile);
-    return 10 * n * sizeof(uint32_t) + 3 * resort_room(tiles) * sizeof(uint32_t) +
-           4 * (tiles + 2) * sizeof(uint32_t) + 8 * sizeof(int) + 24 * 256;
+    return (3 * n + tiles * (size_t)kBucketCap) * sizeof(uint64_t) + (4 * (tiles + 8) + 4) * sizeof(uint32_t) +
+           16 * 256;
 }
 
 void resort_scratch_bind(ResortScratch &r, int n_cap, void *mem)
@@ -663,66 +254,76 @@ void resort_scratch_bind(ResortScratch &r, int n_cap, void *mem)
     const size_t n = (size_t)(n_cap > 0 ? n_cap : 1);
     r.n_cap = (int)n;
     r.tiles = div_up((long long)n, kStayTile);
+    const size_t row = ((size_t)r.tiles + 1 + 3) & ~(size_t)3;   // rows 16-byte aligned, an even number of tiles
     char *p = align((char *)mem);
-    uint32_t **arrays[10] = {&r.mov_k, &r.mov_v, &r.mov_q, &r.mov_r, &r.srt_k,
-                             &r.srt_v, &r.srt_q, &r.alt_k, &r.alt_v, &r.spare};
-    for (auto a : arrays) { *a = (uint32_t *)p; p = align(p + n * sizeof(uint32_t)); }
-    uint32_t **rooms[3] = {&r.bk_k, &r.bk_v, &r.bk_q};
-    for (auto a : rooms) { *a = (uint32_t *)p; p = align(p + resort_room(r.tiles) * sizeof(uint32_t)); }
-    r.tile_cnt = (uint32_t *)p; p = align(p + (size_t)(r.tiles + 2) * sizeof(uint32_t));
-    r.tile_dead = (uint32_t *)p; p = align(p + (size_t)(r.tiles + 2) * sizeof(uint32_t));
-    r.bcnt = (uint32_t *)p; p = align(p + (size_t)(r.tiles + 2) * sizeof(uint32_t));
-    r.counts = (int *)p;
+    r.b.room = (uint64_t *)p; p = align(p + (size_t)r.tiles * kBucketCap * sizeof(uint64_t));
+    r.b.over = (uint64_t *)p; p = align(p + n * sizeof(uint64_t));
+    r.big = (uint64_t *)p; p = align(p + n * sizeof(uint64_t));
+    r.big_alt = (uint64_t *)p; p = align(p + n * sizeof(uint64_t));
+    r.alt_k = (uint32_t *)r.big_alt;
+    r.alt_v = r.alt_k + n;
+    r.tsamp = (uint32_t *)p; p = align(p + row * sizeof(uint32_t));
+    r.b.tile_moved = (uint32_t *)p;
+    r.b.tile_dead = r.b.tile_moved + row;
+    r.b.bcnt = r.b.tile_dead + row;
+    r.b.n_over = r.b.bcnt + row;
+    r.b.n_counts = (int)row + 1;
+    r.b.tsamp = r.tsamp;
 }
 
-bool resort_supported(int n_cap)
-{
-    // the locate keeps one LDS sample per tile (n / 2048 + 1 buckets)
-    return (n_cap > 0 ? n_cap : 1) / kStayTile + 1 <= kMaxBuckets;
-}
+bool resort_supported(int n_cap) { return (n_cap > 0 ? n_cap : 1) / kStayTile + 1 <= kMaxTiles; }
 
 size_t resort_mask_words(int n_cap)
 {
-    // whole tiles, so that every word of a move grid of blocks up to 2048
-    // slots is inside
-    return (size_t)div_up(n_cap > 0 ? n_cap : 1, kStayTile) * kTileWords + kTileWords;
+    // whole tiles and whole first-phase blocks, so that every word of a move
+    // grid of blocks up to 2048 slots is inside
+    return (size_t)resort_list_blocks(n_cap) * kListWords + kTileWords;
 }
 
-ResortPrepArgs resort_prep_args(const ResortScratch &r, const int *n_dev, int move_block,
-                                const uint32_t *blk_moved, const uint32_t *blk_dead,
-                                const uint64_t *mask_m, const uint64_t *mask_d)
+ResortList resort_list_args(const ResortScratch &r, const uint32_t *key_new, const int *n_dev,
+                            const uint64_t *mask_m, const uint64_t *mask_d, bool may_remove)
 {
-    ResortPrepArgs a;
-    a.blocks = resort_prep_blocks(r.n_cap);
-    a.per_tile = kStayTile / move_block;
-    a.n_dev = n_dev;
-    a.blk_moved = blk_moved; a.blk_dead = blk_dead;
-    a.mask_m = mask_m; a.mask_d = mask_d;
-    a.pre_m = r.tile_cnt; a.pre_d = r.tile_dead; a.mov_v = r.mov_v; a.bcnt = r.bcnt;
-    a.counts = r.counts;
-    return a;
+    ResortList l;
+    l.blocks = resort_list_blocks(r.n_cap);
+    l.tiles = r.tiles; l.may_remove = may_remove ? 1 : 0;
+    l.n_dev = n_dev;
+    l.key_new = key_new;
+    l.mask_m = mask_m; l.mask_d = mask_d;
+    l.b = r.b;
+    return l;
 }
 
-void resort_incremental(const uint32_t *key_new, const uint32_t *key_old, const int *n_dev,
-                        uint32_t dead_key, const uint32_t *blk_moved, const uint32_t *blk_dead,
-                        const uint64_t *mask_m, const uint64_t *mask_d,
-                        const uint32_t *key_samp, const uint32_t *key_tsamp, int move_block,
-                        bool prepped, const ResortScratch &r, uint32_t *out_k, uint32_t *out_v,
-                        hipStream_t stream, Profiler *prof)
+ResortMerge resort_merge_args(const ResortScratch &r, const uint32_t *key_old, const int *n_dev,
+                              uint32_t dead_key, const uint64_t *mask_m, const uint64_t *mask_d,
+                              bool may_remove, uint32_t *out_k, uint32_t *out_v)
 {
-    const double n = (double)r.n_cap;
-    if (!prepped)
-        DSMC_LAUNCH(prof, "resort_prep", 0.0, k_ins_prep, resort_prep_blocks(r.n_cap), kPrepWords,
-                    stream, blk_moved, blk_dead, kStayTile / move_block, mask_m, mask_d, n_dev,
-                    r.tile_cnt, r.tile_dead, r.counts, r.mov_v, r.bcnt);
-    // the overflow list reuses the mover arrays that the locate does not read
-    DSMC_LAUNCH(prof, "resort_locate", 0.0, k_ins_locate, div_up(div_up(r.n_cap, 16), 256), 256,
-                stream, key_new, key_old, key_samp, key_tsamp, r.mov_v, r.n_cap, n_dev, r.counts,
-                r.bk_k, r.bk_v, r.bk_q, r.mov_k, r.mov_r, r.mov_q, r.bcnt);
-    DSMC_LAUNCH(prof, "resort_merge", n * 12.0, k_ins_merge, div_up(r.n_cap, kStayTile) + 1, 256,
-                stream, key_new, mask_m, mask_d, n_dev, r.n_cap, r.tile_cnt, r.tile_dead, r.bk_k, r.bk_v,
-                r.bk_q, r.mov_k, r.mov_r, r.mov_q, r.bcnt, r.counts, dead_key, r.srt_k, r.srt_v,
-                r.srt_q, r.alt_k, r.alt_v, r.spare, out_k, out_v);
+    ResortMerge m;
+    m.b = r.b;
+    m.key_old = key_old;
+    m.mask_m = mask_m; m.mask_d = mask_d;
+    m.n_dev = n_dev;
+    m.n_cap = r.n_cap; m.tiles = r.tiles; m.may_remove = may_remove ? 1 : 0;
+    m.dead_key = dead_key;
+    m.big = r.big; m.big_alt = r.big_alt;
+    m.out_k = out_k; m.out_v = out_v;
+    m.tsamp_out = r.tsamp;
+    return m;
+}
+
+void resort_merge(const ResortMerge &m, hipStream_t stream, Profiler *prof)
+{
+    DSMC_LAUNCH(prof, "resort_merge", (double)m.n_cap * 12.0, k_ins_merge, m.tiles, 256, stream, m);
+}
+
+void resort_samples(const ResortScratch &r, const uint32_t *sorted, hipStream_t stream, Profiler *prof)
+{
+    DSMC_LAUNCH(prof, "resort_samples", (double)r.tiles * 8.0, k_tile_samples, div_up(r.tiles, 256), 256, stream,
+                sorted, r.tiles, r.tsamp);
+}
+
+void resort_clear_counts(const ResortScratch &r, hipStream_t stream, Profiler *prof)
+{
+    fill_u32(r.b.bcnt, 0u, r.b.n_counts, stream, prof);
 }
 
 // ---------------------------------------------------------------------------

@@ -1,6 +1,6 @@
-// resort_device.hpp -- device side of the incremental re-sort shared by its
-// own kernels (primitives.hip) and the fused finalize (fused.hip), which runs
-// the re-sort's first phase alongside its per-trap reductions.
+// resort_device.hpp -- device side of the incremental re-sort: its first phase
+// (run by the finalize kernels of both forms beside their sums) and the merge
+// of one tile.  The scheme is described in primitives.hip.
 #pragma once
 
 #include "dsmc_device.hpp"
@@ -11,11 +11,10 @@ namespace dsmc {
 constexpr int kStayTile = kResortTile;         // slots per tile (and bucket)
 constexpr int kStayShift = 11;
 constexpr int kTileWords = kStayTile / 64;     // mask words per tile
-constexpr int kPrepWords = 256;                // mask words per prep block (8 tiles)
-constexpr int kOverflowCount = 3;              // counts[]: movers in the buckets' overflow list
+constexpr int kBucketLds = 512;                // movers a bucket ranks in LDS
+constexpr int kBucketCap = 1024;               // fixed room of a bucket (>= kBucketLds)
 static_assert((1 << kStayShift) == kStayTile, "stay tile");
 static_assert(kTileWords == 32, "a tile's mask words are half a wave");
-static_assert(kPrepWords % kTileWords == 0, "prep blocks hold whole tiles");
 
 // Exclusive prefix of v over the 32 lanes of this lane's half-wave.
 __device__ __forceinline__ uint32_t halfwave_exclusive_scan(uint32_t v)
@@ -30,92 +29,431 @@ __device__ __forceinline__ uint32_t halfwave_exclusive_scan(uint32_t v)
     return s - v;
 }
 
-// Prep blocks needed for n_cap slots (at least one, for n = 0).
-__host__ __device__ inline int resort_prep_blocks(int n_cap)
+// (key, slot) order; slots are distinct.
+__device__ __forceinline__ bool kv_less(uint32_t ka, uint32_t va, uint32_t kb, uint32_t vb)
 {
-    const int words = (n_cap + 63) / 64;
-    return words > 0 ? (words + kPrepWords - 1) / kPrepWords : 1;
+    return ka < kb || (ka == kb && va < vb);
 }
 
-// Block k (kPrepWords threads) of the re-sort's first phase, over mask words
-// [256 k, 256 k + 256) of the move's mover and removal masks (n slots):
-//   * the movers and removed atoms before the block are the sums of the
-//     move's per-block counts below it (every block adds them up itself, so
-//     no block waits for another), those before each word a block scan;
-//   * pre_m / pre_d: movers and removed atoms before each tile, entry
-//     `tiles` the totals; counts = {stays, movers, removed, 0 overflow}
-//     (last block);
-//   * mov_v: the movers' slots in slot order;
-//   * the bucket counts are cleared.
-// per_tile = move blocks per tile (kStayTile / move block size).
-__device__ __forceinline__ void resort_prep_block(
-    int k, int n, const uint32_t *__restrict__ blk_moved, const uint32_t *__restrict__ blk_dead,
-    int per_tile, const uint64_t *__restrict__ mask_m, const uint64_t *__restrict__ mask_d,
-    uint32_t *__restrict__ pre_m, uint32_t *__restrict__ pre_d, int *__restrict__ counts,
-    uint32_t *__restrict__ mov_v, uint32_t *__restrict__ bcnt, uint32_t *tmp,
-    unsigned long long *tmp64)
+// Block j (256 threads) of the re-sort's first phase, on the move's masks of
+// mask words [64 j, 64 j + 64) (two tiles of the n slots): the tiles' movers
+// and removed atoms counted, and every mover (new key k, slot v) put into the
+// bucket of its tile, the last one whose first (key, slot) lies below (k, v),
+// or the first tile.  The tiles' first keys (left by the merge) are searched
+// in LDS; lanes of a wave with the same bucket share one atomic (nearby
+// movers mostly do): 30000 movers' own returning atomics took the move that
+// issued them from 26 to 98 us at N = 1e6, and to 44 us with every counter in
+// a line of its own.  A bucket has a fixed room of kBucketCap movers; those
+// beyond it go to an overflow list.  Bound by its chain of dependent loads
+// (masks, keys, atomic), which runs beside the finalize's sums: the step lost
+// the launch that located every mover's exact slot (six more dependent loads;
+// the merge now finds it in LDS), N = 2e4 30.5 -> 26.5 us, N = 1e6 61.3 ->
+// 55.5 us, 256 traps in two groups 155 -> 150 us.
+constexpr int kListWords = 64;               // mask words per block
+constexpr int kListSlots = kListWords * 64;
+constexpr int kBucketBits = 13;
+constexpr int kMaxTiles = 1 << kBucketBits;  // tiles the LDS sample table holds
+static_assert(kListSlots == 2 * kStayTile, "two tiles per block");
+
+__host__ __device__ inline int resort_list_blocks(int n_cap)
 {
-    const int tid = (int)threadIdx.x;
-    const int words = (n + 63) >> 6;
-    const int tiles = n > 0 ? (n - 1) / kStayTile + 1 : 1;
-    const int nblk = words > 0 ? (words + kPrepWords - 1) / kPrepWords : 1;
-    if (k >= nblk) return;   // whole block leaves together
-    const int g = k * kPrepWords + tid;   // this thread's word
-    if (g <= (n >> kStayShift)) bcnt[g] = 0u;   // buckets 0 .. n / 2048
-    uint64_t mm = 0ull, md = 0ull;
-    if (g < words) { mm = mask_m[g]; md = mask_d[g]; }
-    // move blocks before this block: 8 k tiles of per_tile each, a multiple
-    // of 8 entries, read as 16-byte vectors, eight of each array per thread
-    // in flight
-    uint32_t bm = 0, bd = 0;
+    return n_cap > 0 ? (n_cap + kListSlots - 1) / kListSlots : 1;
+}
+
+// LDS of the tiles' first keys (dynamic).
+inline size_t resort_list_lds(const ResortList &rl)
+{
+    return rl.blocks > 0 ? (((size_t)rl.tiles + 3) & ~(size_t)3) * sizeof(uint32_t) : 0;
+}
+
+// first: the dynamic LDS above; slot: the block's movers, from its first slot.
+__device__ __forceinline__ void resort_list_block(const ResortList &rl, int j, uint32_t *first,
+                                                  unsigned short *slot)
+{
+    const ResortBuckets &rb = rl.b;
+    const int tid = (int)threadIdx.x, lane = tid & (kWave - 1);
+    const int w = j * kListWords + lane;   // every wave reads the block's 64 words
+    const uint64_t mm = rl.mask_m[w];
+    const uint64_t md = rl.may_remove ? rl.mask_d[w] : 0ull;
     {
-        const uint4 *vm = (const uint4 *)blk_moved, *vd = (const uint4 *)blk_dead;
-        const int nv = k * (kPrepWords / kTileWords) * per_tile / 4;
-        for (int v0 = tid; v0 < nv; v0 += 8 * kPrepWords) {
-            uint4 a[8], d[8];
+        const uint4 *t4 = (const uint4 *)rb.tsamp;
+        uint4 *l4 = (uint4 *)first;
+        const int nv = (rl.tiles + 3) >> 2;
+        for (int v0 = tid; v0 < nv; v0 += 4 * 256) {
+            uint4 c[4];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int v = v0 + u * kPrepWords;
-                a[u] = v < nv ? vm[v] : make_uint4(0, 0, 0, 0);
-                d[u] = v < nv ? vd[v] : make_uint4(0, 0, 0, 0);
-            }
+            for (int u = 0; u < 4; ++u) c[u] = v0 + u * 256 < nv ? t4[v0 + u * 256] : make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                bm += a[u].x + a[u].y + a[u].z + a[u].w;
-                bd += d[u].x + d[u].y + d[u].z + d[u].w;
-            }
+            for (int u = 0; u < 4; ++u)
+                if (v0 + u * 256 < nv) l4[v0 + u * 256] = c[u];
         }
     }
-    // two block scans: the earlier blocks' totals packed as (movers, removed)
-    // in 64 bits, and the words' counts as (movers, removed) in 16-bit halves
-    // (a block holds at most 16384 slots)
-    static_assert(kPrepWords * 64 < 65536, "16-bit halves");
-    unsigned long long tot64;
-    (void)block_exclusive_scan<kPrepWords>(((unsigned long long)bm << 32) | bd, tmp64, &tot64);
-    bm = (uint32_t)(tot64 >> 32);
-    bd = (uint32_t)tot64;
-    uint32_t tot;
-    const uint32_t ex = block_exclusive_scan<kPrepWords>(
-        ((uint32_t)__popcll(mm) << 16) | (uint32_t)__popcll(md), tmp, &tot);
-    const uint32_t tm = tot >> 16, td = tot & 0xFFFFu;
-    const uint32_t om = bm + (ex >> 16);
-    const uint32_t od = bd + (ex & 0xFFFFu);
-    if ((g & (kTileWords - 1)) == 0 && (g >> 5) < tiles) {
-        pre_m[g >> 5] = om;
-        pre_d[g >> 5] = od;
+    const int n = *rl.n_dev;
+    if (j > 0 && j * kListSlots >= n) return;   // whole block leaves together
+    // the words' movers and removed atoms (bits past the slots are zero)
+    const uint32_t cnt = (uint32_t)__popcll(mm) << 16 | (uint32_t)__popcll(md);
+    const uint32_t inc = wave_inclusive_scan(cnt);
+    const uint32_t half = __shfl(inc, kTileWords - 1, kWave);   // the first tile's: words 0 .. 31
+    if (tid == kTileWords - 1 || tid == kWave - 1) {
+        const uint32_t c = tid == kWave - 1 ? inc - half : inc;
+        const int t = 2 * j + (tid == kWave - 1);
+        rb.tile_moved[t] = c >> 16;
+        rb.tile_dead[t] = c & 0xFFFFu;
     }
-    if (k == nblk - 1 && tid == 0) {
-        const uint32_t M = bm + tm, D = bd + td;
-        pre_m[tiles] = M;
-        pre_d[tiles] = D;
-        counts[0] = n - (int)M - (int)D;
-        counts[1] = (int)M;
-        counts[2] = (int)D;
-        counts[kOverflowCount] = 0;
+    const int m = (int)(__builtin_amdgcn_readlane(inc, kWave - 1) >> 16);
+    if (m == 0) return;
+    // list the movers: wave q lists the words 16 q .. 16 q + 15, four lanes a
+    // word, a quarter of its bits each
+    {
+        const int q = tid / kWave, wl = 16 * q + (lane >> 2), part = lane & 3;
+        const uint64_t word = __shfl(mm, wl, kWave);
+        const uint32_t excl = __shfl((inc >> 16) - (uint32_t)__popcll(mm), wl, kWave);
+        const uint64_t below = part ? word & (~0ull >> (64 - 16 * part)) : 0ull;
+        int o = (int)excl + __popcll(below);
+        for (uint32_t bits = (uint32_t)(word >> (16 * part)) & 0xFFFFu; bits; bits &= bits - 1)
+            slot[o++] = (unsigned short)(wl * 64 + 16 * part + __ffs((int)bits) - 1);
     }
-    uint32_t o = om;
-    for (uint64_t b = mm; b; b &= b - 1)
-        mov_v[o++] = (uint32_t)g * 64u + (uint32_t)(__ffsll((unsigned long long)b) - 1);
+    __syncthreads();   // (m is the same in every wave)
+    const int nt = (n + kStayTile - 1) >> kStayShift;
+    for (int e0 = 0; e0 < m; e0 += 256) {
+        const int e = e0 + tid;
+        const bool valid = e < m;
+        const uint32_t v = valid ? (uint32_t)(j * kListSlots) + slot[e] : 0u;
+        const uint32_t k = valid ? rl.key_new[v] : 0u;
+        int lo = 0;   // tiles after the first that lie below (k, v): a prefix
+        if (valid) {
+            int hi = nt - 1;
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) >> 1;
+                if (kv_less(first[mid], (uint32_t)mid << kStayShift, k, v)) lo = mid; else hi = mid - 1;
+            }
+        }
+        const uint64_t peers = match_bits<kBucketBits>((uint32_t)lo, __ballot(valid));
+        const int leader = __ffsll((unsigned long long)peers) - 1;
+        uint32_t base = 0;
+        if (valid && lane == leader) base = atomicAdd(&rb.bcnt[lo], (uint32_t)__popcll(peers));
+        base = __shfl(base, leader < 0 ? 0 : leader, kWave);
+        if (valid) {
+            const uint32_t r = base + (uint32_t)__popcll(peers & lanemask_lt());
+            const uint64_t kv = (uint64_t)k << 32 | v;
+            if (r < (uint32_t)kBucketCap) rb.room[(size_t)lo * kBucketCap + r] = kv;
+            else rb.over[atomicAdd(rb.n_over, 1u)] = kv;
+        }
+    }
+}
+
+// Clears the buckets' counts (by the collide, which runs between the merge
+// that reads them and the next first phase): thread g of `threads`.
+__device__ __forceinline__ void resort_clear(const ResortBuckets &rb, int g, int threads)
+{
+    for (int i = g; i < rb.n_counts; i += threads) rb.bcnt[i] = 0u;
+}
+
+// LDS of a merge block (256 threads): 17.4 KB, so that eight blocks fit a CU.
+struct MergeLds {
+    __align__(16) uint64_t kv[kBucketLds];      // the bucket's movers: key << 32 | slot
+    __align__(16) unsigned short q[kBucketLds]; // their insertion points in the tile
+    uint32_t K[kStayTile];                      // the tile's keys of the last sort
+    // movers inserted at each slot, then the scan E (below 2048 + kBucketLds)
+    __align__(16) unsigned short H[kStayTile];
+    uint64_t stay[kTileWords];                  // stay bits of the tile's words
+    uint32_t wst[kTileWords];                   // stays of the tile before each word
+    uint32_t sum[3][256 / kWave];
+    uint32_t at_end;                            // movers inserted after the tile's last slot
+    int n_big;                                  // movers gathered for a big bucket
+};
+
+// Insertion point in the tile: the first p in [0, ns] with (K[p], g0 + p) >= (k, v).
+__device__ __forceinline__ uint32_t merge_point(const uint32_t *K, int ns, uint32_t g0, uint32_t k, uint32_t v)
+{
+    int lo = 0, hi = ns;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (kv_less(K[mid], g0 + (uint32_t)mid, k, v)) lo = mid + 1; else hi = mid;
+    }
+    return (uint32_t)lo;
+}
+
+// Sort of one bucket that does not fit the LDS table, by one block, in
+// global scratch: chunks of kBucketLds sorted in LDS (bitonic network), then
+// pairwise merges of runs (merge path per thread).  Used only when a great
+// many atoms land in the same tile (e.g. nearly all atoms change cell in one
+// step); O(b log b) work for one block.  Leaves the sorted bucket in a0 or
+// a1; returns the one that holds it.
+__device__ inline uint64_t *big_bucket_sort(uint64_t *a0, uint64_t *a1, int b, uint64_t *lds)
+{
+    const int tid = threadIdx.x;
+    for (int c0 = 0; c0 < b; c0 += kBucketLds) {
+        const int c = min(kBucketLds, b - c0);
+        for (int e = tid; e < kBucketLds; e += 256) lds[e] = e < c ? a0[c0 + e] : ~0ull;
+        __syncthreads();
+        for (int size = 2; size <= kBucketLds; size <<= 1) {
+            for (int stride = size >> 1; stride > 0; stride >>= 1) {
+                for (int pr = tid; pr < kBucketLds / 2; pr += 256) {
+                    const int i = 2 * pr - (pr & (stride - 1));   // lower index of the pair
+                    const int j = i + stride;
+                    const uint64_t x = lds[i], y = lds[j];
+                    if ((y < x) == ((i & size) == 0)) { lds[i] = y; lds[j] = x; }
+                }
+                __syncthreads();
+            }
+        }
+        for (int e = tid; e < c; e += 256) a0[c0 + e] = lds[e];
+        __syncthreads();
+    }
+    uint64_t *s = a0, *d = a1;
+    for (int wdt = kBucketLds; wdt < b; wdt <<= 1) {
+        for (int lo = 0; lo < b; lo += 2 * wdt) {
+            const int na = min(wdt, b - lo), nb = max(0, min(wdt, b - lo - wdt));
+            const int len = na + nb;
+            const int per = (len + 255) / 256;
+            const int d0 = min(tid * per, len), d1 = min(d0 + per, len);
+            // merge path split of output d0 between run a = [lo, lo+na), b = [lo+na, ...)
+            int l = max(0, d0 - nb), h = min(d0, na);
+            while (l < h) {
+                const int mid = (l + h) >> 1;
+                if (s[lo + mid] < s[lo + na + d0 - 1 - mid]) l = mid + 1; else h = mid;
+            }
+            int ia = l, ib = d0 - l;
+            for (int o = d0; o < d1; ++o) {
+                const bool ta = ia < na && (ib >= nb || s[lo + ia] < s[lo + na + ib]);
+                d[lo + o] = ta ? s[lo + ia] : s[lo + na + ib];
+                ia += ta; ib += !ta;
+            }
+        }
+        __syncthreads();   // this pass's writes are visible to the whole block
+        uint64_t *x = s; s = d; d = x;
+    }
+    return s;
+}
+
+// Sum of v[0 .. n), this thread's share (256 threads; v is 16-byte aligned).
+__device__ __forceinline__ uint32_t sum_share(const uint32_t *__restrict__ v, int n)
+{
+    const int tid = threadIdx.x;
+    const uint4 *v4 = (const uint4 *)v;
+    const int nv = n >> 2;
+    uint32_t s = 0;
+    for (int v0 = tid; v0 < nv; v0 += 4 * 256) {
+        uint4 c[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c[u] = v0 + u * 256 < nv ? v4[v0 + u * 256] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s += c[u].x + c[u].y + c[u].z + c[u].w;
+    }
+    if (tid < (n & 3)) s += v[4 * nv + tid];
+    return s;
+}
+
+// Block of 256 threads for tile t (2048 slots).  The tile's output is a
+// contiguous window from w0: position p of the tile (slot g0 + p) is preceded
+// there by E(p) = the stays below p plus the bucket movers inserted below p,
+// so a stay at p goes to w0 + E(p) + h(p), h(p) = movers inserted at p, and a
+// mover inserted at p to w0 + E(p) + (its rank among the movers inserted at
+// p).  E is an exclusive scan of st(p) + h(p) over the tile, h a histogram of
+// the bucket in LDS; p may also be the tile's end.  A stay's key is its key of
+// the last sort and a mover's comes with it, so the new keys are not read.
+// Buckets larger than the LDS table are sorted in global scratch by the
+// block; movers then go to w0 + (stays below p) + (rank in the bucket), stays
+// after the movers below them.
+constexpr int kMergePer = kStayTile / 256;   // slots per thread
+
+__device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t, MergeLds &L)
+{
+    const ResortBuckets &rb = ra.b;
+    const int tid = threadIdx.x;
+    const int g0 = t * kStayTile;
+    const int p0 = tid * kMergePer;   // positions p0 .. p0 + 7 in the scan
+    // Every load that does not need the slot count is issued together with
+    // it, in one round: the tile's keys at positions tid + 256 u (coalesced;
+    // up to the capacity, those past the slots are never used), its mask
+    // words, the counts of the earlier tiles, its bucket's size, and this
+    // thread's first mover of the bucket's room (used when the bucket holds it).
+    uint32_t kk[kMergePer];
+#pragma unroll
+    for (int u = 0; u < kMergePer; ++u) {
+        const int p = tid + 256 * u;
+        kk[u] = g0 + p < ra.n_cap ? ra.key_old[g0 + p] : 0u;
+    }
+    const int n = *ra.n_dev;
+    const int b = (int)rb.bcnt[t];
+    uint64_t wm = 0ull, wd = 0ull;   // mask words of the tile (in bounds up to the last tile + 1)
+    if (tid < kTileWords) {
+        wm = ra.mask_m[(g0 >> 6) + tid];
+        wd = ra.mask_d[(g0 >> 6) + tid];
+    }
+    const size_t fb0 = (size_t)t * kBucketCap;   // the bucket's fixed room
+    constexpr int kFirst = 128;                  // movers loaded before the count is known
+    const uint64_t mkv = tid < kFirst ? rb.room[fb0 + tid] : 0ull;
+    // movers inserted before the tile less the movers and removed atoms that
+    // left its earlier slots; removed atoms before it, and all
+    uint32_t part[3] = { sum_share(rb.bcnt, t) - sum_share(rb.tile_moved, t), 0u, 0u };
+    if (ra.may_remove) {
+        part[1] = sum_share(rb.tile_dead, t);
+        part[2] = sum_share(rb.tile_dead, (n + kStayTile - 1) >> kStayShift);
+        part[0] -= part[1];
+    }
+    if (t > 0 && g0 >= n) return;   // whole block leaves together
+    const int ns = min(kStayTile, n - g0);   // slots of the tile
+#pragma unroll
+    for (int u = 0; u < kMergePer; ++u) L.K[tid + 256 * u] = kk[u];
+    ((uint4 *)L.H)[tid] = make_uint4(0u, 0u, 0u, 0u);
+    if (tid == 0) L.at_end = 0u;
+    uint64_t dd = 0ull;
+    if (tid < kTileWords) {
+        const int l0 = tid * 64;
+        uint64_t st = 0ull;
+        if (l0 < ns) {
+            const uint64_t in = ns - l0 >= 64 ? ~0ull : (1ull << (ns - l0)) - 1ull;
+            st = ~(wm | wd) & in;
+            dd = wd & in;
+        }
+        L.stay[tid] = st;
+        L.wst[tid] = halfwave_exclusive_scan((uint32_t)__popcll(st));
+    }
+    const int lane = tid & (kWave - 1), w = tid / kWave;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        if (k > 0 && !ra.may_remove) break;
+        part[k] = wave_sum(part[k]);
+        if (lane == 0) L.sum[k][w] = part[k];
+    }
+    __syncthreads();   // H cleared, keys, stay words and sums in place
+    auto total_of = [&](int k) { return L.sum[k][0] + L.sum[k][1] + L.sum[k][2] + L.sum[k][3]; };
+    const uint32_t w0 = (uint32_t)g0 + total_of(0);   // first output slot of the tile
+    if (ra.may_remove && tid < kTileWords) {
+        // removed atoms: to the end of the output, in slot order
+        uint32_t od = (uint32_t)n - total_of(2) + total_of(1) + halfwave_exclusive_scan((uint32_t)__popcll(dd));
+        for (uint64_t bb = dd; bb; bb &= bb - 1) {
+            ra.out_k[od] = ra.dead_key;
+            ra.out_v[od++] = (uint32_t)(g0 + tid * 64) + (uint32_t)(__ffsll((unsigned long long)bb) - 1);
+        }
+    }
+    auto put = [&](uint32_t o, uint32_t k, uint32_t v) {
+        ra.out_k[o] = k;
+        ra.out_v[o] = v;
+        if ((o & (kStayTile - 1)) == 0) ra.tsamp_out[o >> kStayShift] = k;
+    };
+    auto stays_below = [&](uint32_t p) {
+        if (p >= (uint32_t)kStayTile) return L.wst[kTileWords - 1] + (uint32_t)__popcll(L.stay[kTileWords - 1]);
+        const uint64_t m = (p & 63) ? L.stay[p >> 6] & (~0ull >> (64 - (p & 63))) : 0ull;
+        return L.wst[p >> 6] + (uint32_t)__popcll(m);
+    };
+    if (b > kBucketLds) {
+        // gather the bucket (its room, then its movers in the overflow list)
+        // in scratch, at the earlier buckets' movers, and sort it there
+        __syncthreads();   // the sums are read
+        uint32_t fs = wave_sum(sum_share(rb.bcnt, t));
+        if (lane == 0) L.sum[0][w] = fs;
+        if (tid == 0) L.n_big = min(b, kBucketCap);
+        __syncthreads();
+        const uint32_t at = total_of(0);
+        uint64_t *a = ra.big + at, *c = ra.big_alt + at;
+        for (int e = tid; e < min(b, kBucketCap); e += 256) a[e] = rb.room[fb0 + e];
+        if (b > kBucketCap) {
+            const int no = (int)*rb.n_over;
+            const bool has1 = g0 + kStayTile < n;   // (tsamp is being replaced by the merge)
+            const uint32_t f1 = has1 ? ra.key_old[g0 + kStayTile] : 0u;
+            for (int e = tid; e < no; e += 256) {
+                // of this bucket: above the tile's first (or the first tile)
+                // and not above the next tile's first
+                const uint64_t kv = rb.over[e];
+                const uint32_t k = (uint32_t)(kv >> 32), v = (uint32_t)kv;
+                const bool ge = t == 0 || kv_less(L.K[0], (uint32_t)g0, k, v);
+                const bool lt = !has1 || !kv_less(f1, (uint32_t)(g0 + kStayTile), k, v);
+                if (ge && lt) a[atomicAdd(&L.n_big, 1)] = kv;
+            }
+        }
+        __syncthreads();
+        const uint64_t *g = big_bucket_sort(a, c, b, L.kv);
+        // a stay goes after the movers below it, found in the sorted bucket
+        for (int u = 0; u < kMergePer; ++u) {
+            const int p = tid + 256 * u;
+            if (p >= ns || !((L.stay[p >> 6] >> (p & 63)) & 1ull)) continue;
+            const uint64_t key = (uint64_t)kk[u] << 32 | (uint32_t)(g0 + p);
+            int lo = 0, hi = b;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (g[mid] < key) lo = mid + 1; else hi = mid;
+            }
+            put(w0 + stays_below((uint32_t)p) + (uint32_t)lo, kk[u], (uint32_t)(g0 + p));
+        }
+        for (int r = tid; r < b; r += 256) {
+            const uint32_t k = (uint32_t)(g[r] >> 32), v = (uint32_t)g[r];
+            put(w0 + stays_below(merge_point(L.K, ns, (uint32_t)g0, k, v)) + (uint32_t)r, k, v);
+        }
+        return;
+    }
+    for (int e = tid; e < b; e += 256) {
+        const uint64_t kv = e < kFirst ? mkv : rb.room[fb0 + e];
+        const uint32_t q = merge_point(L.K, ns, (uint32_t)g0, (uint32_t)(kv >> 32), (uint32_t)kv);
+        L.kv[e] = kv;
+        L.q[e] = (unsigned short)q;
+        if (q < (uint32_t)kStayTile) atomicAdd((uint32_t *)L.H + (q >> 1), 1u << (16 * (q & 1)));
+        else atomicAdd(&L.at_end, 1u);
+    }
+    __syncthreads();
+    // E: exclusive scan of st(p) + h(p) over the tile, 8 consecutive
+    // positions per thread (16 bytes of H)
+    {
+        const uint4 h4 = ((const uint4 *)L.H)[tid];
+        const uint32_t h[4] = { h4.x, h4.y, h4.z, h4.w };
+        const uint32_t st8 = (uint32_t)(L.stay[p0 >> 6] >> (p0 & 63)) & 0xFFu;
+        uint32_t e[kMergePer], run = 0;
+#pragma unroll
+        for (int u = 0; u < kMergePer; ++u) {
+            e[u] = run;
+            run += ((st8 >> u) & 1u) + ((h[u >> 1] >> (16 * (u & 1))) & 0xFFFFu);
+        }
+        const uint32_t inc = wave_inclusive_scan(run);
+        if (lane == kWave - 1) L.sum[1][w] = inc;
+        __syncthreads();
+        uint32_t base = inc - run;
+        for (int ww = 0; ww < w; ++ww) base += L.sum[1][ww];
+        uint4 o;
+        o.x = (base + e[0]) | (base + e[1]) << 16;
+        o.y = (base + e[2]) | (base + e[3]) << 16;
+        o.z = (base + e[4]) | (base + e[5]) << 16;
+        o.w = (base + e[6]) | (base + e[7]) << 16;
+        ((uint4 *)L.H)[tid] = o;
+    }
+    __syncthreads();   // E complete
+    const uint32_t total = total_of(1), at_end = L.at_end;
+    // stays, at positions tid + 256 u (coalesced stores): E(p) + h(p) =
+    // E(p + 1) - st(p) = E(p + 1) - 1
+#pragma unroll
+    for (int u = 0; u < kMergePer; ++u) {
+        const int p = tid + 256 * u;
+        if (p >= ns || !((L.stay[p >> 6] >> (p & 63)) & 1ull)) continue;
+        put(w0 + (p + 1 < kStayTile ? L.H[p + 1] : total) - 1u, kk[u], (uint32_t)(g0 + p));
+    }
+    for (int x = tid; x < b; x += 256) {
+        const uint32_t p = L.q[x];
+        uint32_t ep = total, hp = at_end;
+        if (p < (uint32_t)kStayTile) {
+            ep = L.H[p];
+            hp = (p + 1 < (uint32_t)kStayTile ? L.H[p + 1] : total) - ep -
+                 ((uint32_t)(L.stay[p >> 6] >> (p & 63)) & 1u);
+        }
+        uint32_t r = 0;   // rank among the movers inserted at the same point
+        const uint64_t kx = L.kv[x];
+        if (hp > 1) {
+            // four movers per step, without branches: (key, slot) order is
+            // the order of key << 32 | slot
+            const ushort4 *lq4 = (const ushort4 *)L.q;
+            const ulonglong2 *k2 = (const ulonglong2 *)L.kv;
+#pragma unroll 2
+            for (int f = 0; f < b; f += 4) {
+                const ushort4 qq = lq4[f >> 2];
+                const ulonglong2 ka = k2[f >> 1], kb = k2[(f >> 1) + 1];
+                r += (uint32_t)((qq.x == p) & (ka.x < kx));
+                r += (uint32_t)((qq.y == p) & (ka.y < kx) & (f + 1 < b));
+                r += (uint32_t)((qq.z == p) & (kb.x < kx) & (f + 2 < b));
+                r += (uint32_t)((qq.w == p) & (kb.y < kx) & (f + 3 < b));
+            }
+        }
+        put(w0 + ep + r, (uint32_t)(kx >> 32), (uint32_t)kx);
+    }
 }
 
 }  // namespace dsmc

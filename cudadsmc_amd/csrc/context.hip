@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -103,6 +104,8 @@ Profiler::~Profiler()
 // ---------------------------------------------------------------------------
 // Context
 // ---------------------------------------------------------------------------
+
+static void free_kept();   // scratch kept between the primitives' calls
 
 struct dsmc_ctx {
     dsmc_config cfg{};
@@ -211,7 +214,11 @@ struct dsmc_ctx {
     {
         void *p = nullptr;
         const size_t bytes = std::max<size_t>(count_ * sizeof(T_), 16);
-        DSMC_HIP(hipMalloc(&p, bytes));
+        if (hipMalloc(&p, bytes) != hipSuccess) {   // without the scratch kept for the primitives
+            (void)hipGetLastError();
+            free_kept();
+            DSMC_HIP(hipMalloc(&p, bytes));
+        }
         allocs.push_back(p);
         if (zero) DSMC_HIP(hipMemsetAsync(p, 0, bytes, stream));
         return (T_ *)p;
@@ -510,8 +517,11 @@ static void run_sort(dsmc_ctx *x, const int *n_dev)
 {
     const bool odd = (x->passes % 2) == 1;
     uint32_t *ok = odd ? x->key_b : x->key_a, *ov = odd ? x->val_b : x->val_a;
-    uint32_t *ak = odd ? x->key_a : x->key_b, *av = odd ? x->val_a : x->val_b;
-    radix_sort(x->key_a, nullptr, ak, av, ok, ov, n_dev, x->key_bits, x->sort, x->stream, &x->prof);
+    // sorting in place takes an even number of passes
+    RadixPlan plan = radix_plan(x->n_cap, x->key_bits);
+    if (!odd && plan.passes % 2) plan = radix_plan(x->n_cap, x->key_bits, kRadixBits);
+    uint32_t *ak = odd ? x->res.alt_k : x->key_b, *av = odd ? x->res.alt_v : x->val_b;
+    radix_sort(x->key_a, nullptr, ak, av, ok, ov, n_dev, plan, x->sort, x->stream, &x->prof);
     x->sorted_key = ok;
     x->perm = ov;
     x->perm_mask = -1;
@@ -718,8 +728,8 @@ static void plain_substeps(dsmc_ctx *x, int L)
         } else {
             if (!x->keys_ok)
                 launch_index_plain(t, x->ps[x->cur], x->key_f, &c->slots, x->n_cap, x->stream, &x->prof);
-            radix_sort(x->key_f, nullptr, x->res.alt_k, x->res.alt_v, ok, ov, &c->slots, x->key_bits,
-                       x->sort, x->stream, &x->prof);
+            radix_sort(x->key_f, nullptr, x->res.alt_k, x->res.alt_v, ok, ov, &c->slots,
+                       radix_plan(x->n_cap, x->key_bits), x->sort, x->stream, &x->prof);
             resort_samples(x->res, ok, x->stream, &x->prof);
         }
         x->srt_cur ^= 1;
@@ -817,8 +827,8 @@ static void fused_sort(dsmc_ctx *x)
         resort_merge(resort_merge_args(x->res, x->srt_k[x->srt_cur], n, x->dead_key, x->mask_moved, x->mask_dead,
                                        x->dead_in_state, ok, ov), x->stream, &x->prof);
     } else {
-        radix_sort(x->key_a, nullptr, x->res.alt_k, x->res.alt_v, ok, ov, n, x->key_bits,
-                   x->sort, x->stream, &x->prof);
+        radix_sort(x->key_a, nullptr, x->res.alt_k, x->res.alt_v, ok, ov, n,
+                   radix_plan(x->n_cap, x->key_bits), x->sort, x->stream, &x->prof);
         resort_samples(x->res, ok, x->stream, &x->prof);
     }
     x->bucketed = false;
@@ -1395,12 +1405,99 @@ static void copy_field(dsmc_ctx *x, int field, void *host, size_t bytes)
     catch (const Error &e) { g_create_error = e.what(); return (dsmc_status)e.status; } \
     catch (const std::exception &e) { g_create_error = e.what(); return DSMC_EHIP; }
 
-// Temporary device buffer owned by one primitive call.
-struct DevBuf {
-    void *p = nullptr;
-    explicit DevBuf(size_t bytes) { DSMC_HIP(hipMalloc(&p, std::max<size_t>(bytes, 16))); }
-    ~DevBuf() { if (p) (void)hipFree(p); }
-    template <typename T_> T_ *as() const { return (T_ *)p; }
+// Device scratch of one primitive call.  A call allocated its scratch and
+// freed it (which waits for the device): some 70 us a sort, of 95 at n = 1000
+// and 195 at n = 1e6.  A few idle blocks are kept for the next call instead:
+// at most kKeptBlocks, of at most kKeptBytes together, per process; one that
+// kKeptUnused calls did not use is freed, and all are when an allocation
+// fails.  A block belongs to one call at a time and the calls wait for their
+// stream before they return, so threads and streams never share one (a call
+// that fails does not keep its block).
+constexpr int kKeptBlocks = 8;
+constexpr size_t kKeptBytes = (size_t)512 << 20;
+constexpr int kKeptUnused = 64;
+
+struct KeptBlock {
+    void *p;
+    int *host;      // 64 bytes of pinned host memory, for a result
+    size_t bytes;
+    int device;
+    int unused;
+};
+static std::mutex g_kept_mu;
+static std::vector<KeptBlock> *const g_kept = new std::vector<KeptBlock>();   // outlives static destructors
+
+static void free_kept()
+{
+    std::lock_guard<std::mutex> lock(g_kept_mu);
+    for (const KeptBlock &b : *g_kept) { (void)hipFree(b.p); (void)hipHostFree(b.host); }
+    g_kept->clear();
+}
+
+struct Workspace {
+    KeptBlock b{ nullptr, nullptr, 0, 0, 0 };
+    explicit Workspace(size_t bytes)
+    {
+        bytes = (std::max<size_t>(bytes, 16) + 65535) & ~(size_t)65535;
+        DSMC_HIP(hipGetDevice(&b.device));
+        {
+            std::lock_guard<std::mutex> lock(g_kept_mu);
+            int best = -1;
+            for (size_t i = 0; i < g_kept->size(); ++i) {
+                KeptBlock &k = (*g_kept)[i];
+                ++k.unused;
+                if (k.device == b.device && k.bytes >= bytes && (best < 0 || k.bytes < (*g_kept)[best].bytes))
+                    best = (int)i;
+            }
+            if (best >= 0) {
+                b = (*g_kept)[best];
+                g_kept->erase(g_kept->begin() + best);
+                return;
+            }
+        }
+        b.bytes = bytes;
+        if (hipMalloc(&b.p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            free_kept();
+            DSMC_HIP(hipMalloc(&b.p, bytes));
+        }
+        if (hipHostMalloc((void **)&b.host, 64, hipHostMallocDefault) != hipSuccess) {
+            (void)hipFree(b.p);
+            fail(DSMC_ENOMEM, "no pinned host memory for a primitive's result");
+        }
+    }
+    ~Workspace()
+    {
+        if (!b.p) return;
+        if (std::uncaught_exceptions() > 0) {   // the stream may still use it: hipFree waits
+            (void)hipFree(b.p);
+            (void)hipHostFree(b.host);
+            return;
+        }
+        b.unused = 0;
+        std::vector<KeptBlock> gone;
+        {
+            std::lock_guard<std::mutex> lock(g_kept_mu);
+            g_kept->push_back(b);
+            size_t total = 0;
+            for (const KeptBlock &k : *g_kept) total += k.bytes;
+            // the longest unused first
+            for (size_t i = 0; i < g_kept->size();) {
+                size_t old = 0;
+                for (size_t j = 1; j < g_kept->size(); ++j)
+                    if ((*g_kept)[j].unused > (*g_kept)[old].unused) old = j;
+                const KeptBlock k = (*g_kept)[old];
+                if (total <= kKeptBytes && g_kept->size() <= (size_t)kKeptBlocks && k.unused < kKeptUnused) break;
+                total -= k.bytes;
+                gone.push_back(k);
+                g_kept->erase(g_kept->begin() + old);
+            }
+        }
+        for (const KeptBlock &k : gone) { (void)hipFree(k.p); (void)hipHostFree(k.host); }
+    }
+    Workspace(const Workspace &) = delete;
+    Workspace &operator=(const Workspace &) = delete;
+    template <typename T_> T_ *as() const { return (T_ *)b.p; }
 };
 
 // ---------------------------------------------------------------------------
@@ -1441,8 +1538,6 @@ static char *noalloc_scratch()
     }
     return (char *)g_noalloc_ptr[dev];
 }
-
-__global__ void k_store_i32(int *p, int v) { *p = v; }
 
 __global__ __launch_bounds__(256) void k_copy_pairs(uint32_t *__restrict__ dk, uint32_t *__restrict__ dv,
                                                     const uint32_t *__restrict__ sk,
@@ -1993,20 +2088,19 @@ dsmc_status dsmc_sort_by_key(unsigned int *d_keys, unsigned int *d_values, int n
         fail(DSMC_EINVAL, "bad sort arguments");
     if (n == 0) return DSMC_OK;
     hipStream_t st = (hipStream_t)stream;
-    const int passes = key_bits <= kRadixBits ? 1 : div_up(key_bits, kRadixBits);
-    DevBuf tk(sizeof(uint32_t) * n), tv(sizeof(uint32_t) * n), nd(sizeof(int)),
-        scratch(sort_scratch_bytes(n));
+    const RadixPlan plan = radix_plan(n, key_bits);
+    const size_t row = ((size_t)n + 63) & ~(size_t)63;
+    Workspace ws(2 * row * sizeof(uint32_t) + sort_scratch_bytes(n));
+    uint32_t *tk = ws.as<uint32_t>(), *tv = tk + row;
     SortScratch s;
-    sort_scratch_bind(s, n, scratch.p);
-    DSMC_HIP(hipMemcpyAsync(nd.p, &n, sizeof(int), hipMemcpyHostToDevice, st));
-    if (passes % 2 == 0) {
-        radix_sort(d_keys, d_values, tk.as<uint32_t>(), tv.as<uint32_t>(), d_keys, d_values,
-                   nd.as<int>(), key_bits, s, st, nullptr);
+    sort_scratch_bind(s, n, tv + row);
+    if (plan.passes % 2 == 0) {
+        radix_sort(d_keys, d_values, tk, tv, d_keys, d_values, nullptr, plan, s, st, nullptr);
     } else {
-        radix_sort(d_keys, d_values, d_keys, d_values, tk.as<uint32_t>(), tv.as<uint32_t>(),
-                   nd.as<int>(), key_bits, s, st, nullptr);
-        DSMC_HIP(hipMemcpyAsync(d_keys, tk.p, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st));
-        DSMC_HIP(hipMemcpyAsync(d_values, tv.p, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, st));
+        radix_sort(d_keys, d_values, d_keys, d_values, tk, tv, nullptr, plan, s, st, nullptr);
+        hipLaunchKernelGGL(k_copy_pairs, dim3(std::min(div_up(n, 256), 2048)), dim3(256), 0, st, d_keys,
+                           d_values, tk, tv, n);
+        DSMC_HIP(hipGetLastError());
     }
     DSMC_HIP(hipStreamSynchronize(st));
     PRIM_END
@@ -2023,18 +2117,15 @@ dsmc_status dsmc_sort_by_key_noalloc(unsigned int *d_keys, unsigned int *d_value
     char *base = noalloc_scratch();
     if (n == 0) return DSMC_OK;
     hipStream_t st = (hipStream_t)stream;
-    int *nd = (int *)base;
     SortScratch s;
-    sort_scratch_bind(s, n, base + kNoAllocHdr);
+    sort_scratch_bind(s, n, base + kNoAllocHdr, kRadix);
     uint32_t *tk = (uint32_t *)(base + kNoAllocHdr + kNoAllocSortBytes);
     uint32_t *tv = tk + kNoAllocMaxPairs;
-    hipLaunchKernelGGL(k_store_i32, dim3(1), dim3(1), 0, st, nd, n);
-    DSMC_HIP(hipGetLastError());
-    const int passes = key_bits <= kRadixBits ? 1 : div_up(key_bits, kRadixBits);
-    if (passes % 2 == 0) {
-        radix_sort(d_keys, d_values, tk, tv, d_keys, d_values, nd, key_bits, s, st, nullptr);
+    const RadixPlan plan = radix_plan(n, key_bits, kRadixBits);   // its fixed scratch holds 256 digits
+    if (plan.passes % 2 == 0) {
+        radix_sort(d_keys, d_values, tk, tv, d_keys, d_values, nullptr, plan, s, st, nullptr);
     } else {
-        radix_sort(d_keys, d_values, d_keys, d_values, tk, tv, nd, key_bits, s, st, nullptr);
+        radix_sort(d_keys, d_values, d_keys, d_values, tk, tv, nullptr, plan, s, st, nullptr);
         hipLaunchKernelGGL(k_copy_pairs, dim3(std::min(div_up(n, 256), 2048)), dim3(256), 0, st,
                            d_keys, d_values, tk, tv, n);
         DSMC_HIP(hipGetLastError());
@@ -2048,7 +2139,7 @@ dsmc_status dsmc_exclusive_scan(const int *d_in, int *d_out, int n, void *stream
     if (n < 0 || (n > 0 && (!d_in || !d_out))) fail(DSMC_EINVAL, "bad scan arguments");
     if (n == 0) return DSMC_OK;
     hipStream_t st = (hipStream_t)stream;
-    DevBuf part(sizeof(int) * (scan_partials(n) + 8));
+    Workspace part(sizeof(int) * (scan_partials(n) + 8));
     exclusive_scan(d_in, d_out, n, part.as<int>(), st, nullptr);
     DSMC_HIP(hipStreamSynchronize(st));
     PRIM_END
@@ -2060,17 +2151,11 @@ dsmc_status dsmc_remove_if(int *d_values, const int *d_stencil, int n, int *n_ou
     if (n < 0 || (n > 0 && (!d_values || !d_stencil))) fail(DSMC_EINVAL, "bad remove_if arguments");
     if (n == 0) { if (n_out) *n_out = 0; return DSMC_OK; }
     hipStream_t st = (hipStream_t)stream;
-    DevBuf map(sizeof(uint32_t) * n), nd(sizeof(int) * 2), part(sizeof(int) * (scan_partials(n) + 8)),
-        tmp(sizeof(int) * n);
-    DSMC_HIP(hipMemcpyAsync(nd.p, &n, sizeof(int), hipMemcpyHostToDevice, st));
-    compaction_map(d_stencil, nd.as<int>(), n, map.as<uint32_t>(), nd.as<int>() + 1, part.as<int>(),
-                   st, nullptr);
-    DSMC_HIP(hipMemcpyAsync(tmp.p, d_values, sizeof(int) * n, hipMemcpyDeviceToDevice, st));
-    gather_u32((uint32_t *)d_values, tmp.as<uint32_t>(), map.as<uint32_t>(), nd.as<int>() + 1, n, st,
-               nullptr);
-    int kept = 0;
-    DSMC_HIP(hipMemcpyAsync(&kept, nd.as<int>() + 1, sizeof(int), hipMemcpyDeviceToHost, st));
+    Workspace ws(sizeof(int) * ((size_t)n + remove_if_blocks(n)));
+    int *tmp = ws.as<int>();
+    remove_if(d_values, d_stencil, n, tmp, tmp + n, ws.b.host, st);
     DSMC_HIP(hipStreamSynchronize(st));
+    const int kept = *ws.b.host;
     if (n_out) *n_out = kept;
     PRIM_END
 }

@@ -70,23 +70,30 @@ constexpr int kScanTile = kScanBlock * kScanItems;
 
 inline int div_up(long long a, long long b) { return (int)((a + b - 1) / b); }
 
-// Scratch for a radix sort of up to n_cap pairs.
+// How a radix sort goes over its keys: `passes` passes over digits of `bits`
+// bits, in tiles of block * kSortItems pairs.
+struct RadixPlan { int bits, passes, block; };
+constexpr int kRadixMax = 1 << 10;
+// The plan for n pairs with keys in [0, 2^key_bits); digits of at most
+// `widest` bits.
+RadixPlan radix_plan(int n, int key_bits, int widest = 10);
+
+// Scratch for a radix sort of up to n_cap pairs with at most `digits` digits.
 struct SortScratch {
     int n_cap = 0;
-    int nb = 0;                   // blocks per pass
-    uint32_t *hist = nullptr;     // kRadix * nb
-    uint32_t *totals = nullptr;   // kRadix
+    uint32_t *totals = nullptr;   // digits
+    uint32_t *hist = nullptr;     // digits * tiles
 };
 size_t sort_scratch_bytes(int n_cap);
-void sort_scratch_bind(SortScratch &s, int n_cap, void *mem);
+void sort_scratch_bind(SortScratch &s, int n_cap, void *mem, int digits = kRadixMax);
 
 // Stable LSD radix sort of keys[0..n) with values (identity slot indices when
-// vals == nullptr).  n is read from device memory.  The sorted result lands in
-// (keys_out, vals_out); ping-pong through (keys_alt, vals_alt) for the
-// intermediate passes.  key_bits selects the number of 8-bit passes.
+// vals == nullptr).  n is read from device memory (n_dev null: s.n_cap).  The
+// sorted result lands in (keys_out, vals_out); ping-pong through (keys_alt,
+// vals_alt) for the intermediate passes.
 void radix_sort(const uint32_t *keys, const uint32_t *vals, uint32_t *keys_alt,
                 uint32_t *vals_alt, uint32_t *keys_out, uint32_t *vals_out,
-                const int *n_dev, int key_bits, const SortScratch &s,
+                const int *n_dev, const RadixPlan &plan, const SortScratch &s,
                 hipStream_t stream, Profiler *prof);
 
 // Incremental re-sort (see primitives.hip): the stable sort of a state's new
@@ -163,6 +170,12 @@ inline int scan_partials(int n) { return div_up(n > 0 ? n : 1, kScanTile) + 1; }
 // n_cap bounds the grid.  partial holds div_up(n_cap, tile) + 1 ints.
 void compaction_map(const int *stencil, const int *n_dev, int n_cap, uint32_t *map,
                     int *n_out_dev, int *partial, hipStream_t stream, Profiler *prof);
+
+// Stable in-place removal of the values with a non-zero stencil; *kept (device
+// or pinned host memory) receives how many stay.  tmp holds n ints, partial
+// remove_if_blocks(n).
+int remove_if_blocks(int n);
+void remove_if(int *values, const int *stencil, int n, int *tmp, int *partial, int *kept, hipStream_t stream);
 
 // dst[i] = src[map[i]] for i < *n_dev (i < n_cap when n_dev is null).
 void gather_u32(uint32_t *dst, const uint32_t *src, const uint32_t *map, const int *n_dev,

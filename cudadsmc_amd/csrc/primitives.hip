@@ -1,9 +1,9 @@
 // primitives.hip -- data-movement primitives of the DSMC step written for
 // wave64 / LDS on gfx950:
-//   * stable LSD radix sort of (uint32 key, uint32 value) pairs, 8-bit digits,
-//     reduce-then-scan per pass (upsweep histogram, per-digit scan, downsweep
+//   * stable LSD radix sort of (uint32 key, uint32 value) pairs, digits of 8 or
+//     10 bits, reduce-then-scan per pass (upsweep histogram, per-digit scan, downsweep
 //     scatter).  Within a tile the rank of each key among equal digits comes
-//     from 8 wave ballots (lanes whose digit matches) plus a per-wave running
+//     from one wave ballot per bit (lanes whose digit matches) plus a per-wave running
 //     count in LDS, so the order of equal keys is the input order (stable);
 //     the scatter is staged through LDS so global writes are digit runs.
 //     Replaces thrust::sort_by_key (collisions.cu:282-284).
@@ -16,50 +16,50 @@
 #include "dsmc_internal.hpp"
 #include "resort_device.hpp"
 
-namespace dsmc {
+#include <algorithm>
 
-static_assert(kSortBlock == kRadix, "downsweep assigns one digit per thread");
+namespace dsmc {
 
 // ---------------------------------------------------------------------------
 // Radix sort
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kSortBlock) void k_radix_upsweep(
-    const uint32_t *__restrict__ keys, const int *__restrict__ n_dev, int shift,
-    uint32_t *__restrict__ hist, int nb)
+// One pass over digits of B bits: BLOCK threads take a tile of BLOCK * ITEMS
+// pairs.  n_dev: the pair count on the device, or null (then n).
+template <int B, int BLOCK, int ITEMS>
+__global__ __launch_bounds__(BLOCK) void k_radix_upsweep(const uint32_t *__restrict__ keys,
+                                                         const int *__restrict__ n_dev, int n_host, int shift,
+                                                         uint32_t *__restrict__ hist, int nb)
 {
-    __shared__ uint32_t h[kRadix];
+    constexpr int R = 1 << B, TILE = BLOCK * ITEMS;
+    __shared__ uint32_t h[R];
     const int tid = threadIdx.x;
-    for (int i = tid; i < kRadix; i += kSortBlock) h[i] = 0;
+    for (int i = tid; i < R; i += BLOCK) h[i] = 0;
     __syncthreads();
-    const int n = *n_dev;
-    const int tile0 = blockIdx.x * kSortTile;
+    const int n = n_dev ? *n_dev : n_host;
+    const long long tile0 = (long long)blockIdx.x * TILE;
     if (tile0 < n) {
         const int lane = tid & (kWave - 1), w = tid / kWave;
-        const int base = tile0 + w * (kWave * kSortItems);
-        const uint64_t lt = lanemask_lt();
+        const long long base = tile0 + w * (kWave * ITEMS) + lane;
+        uint32_t k[ITEMS];
 #pragma unroll
-        for (int k = 0; k < kSortItems; ++k) {
-            const int idx = base + k * kWave + lane;
-            const bool valid = idx < n;
-            const uint32_t d = valid ? (keys[idx] >> shift) & (kRadix - 1) : 0u;
-            const uint64_t peers = match_digit8(d, __ballot(valid));
-            if (valid && (peers & lt) == 0) atomicAdd(&h[d], (uint32_t)__popcll(peers));
-        }
+        for (int u = 0; u < ITEMS; ++u) k[u] = base + u * kWave < n ? keys[base + u * kWave] : 0u;
+#pragma unroll
+        for (int u = 0; u < ITEMS; ++u)
+            if (base + u * kWave < n) atomicAdd(&h[(k[u] >> shift) & (R - 1)], 1u);
     }
     // tiles past the end are not scanned (block 0 always writes: n may be 0)
     if (tile0 >= n && blockIdx.x > 0) return;
     __syncthreads();
-    for (int d = tid; d < kRadix; d += kSortBlock) hist[(size_t)d * nb + blockIdx.x] = h[d];
+    for (int d = tid; d < R; d += BLOCK) hist[(size_t)d * nb + blockIdx.x] = h[d];
 }
 
 // One block per digit: exclusive scan of that digit's per-block counts.
-__global__ __launch_bounds__(256) void k_radix_scan(uint32_t *__restrict__ hist,
-                                                    uint32_t *__restrict__ totals,
-                                                    const int *__restrict__ n_dev, int nb)
+__global__ __launch_bounds__(256) void k_radix_scan(uint32_t *__restrict__ hist, uint32_t *__restrict__ totals,
+                                                    const int *__restrict__ n_dev, int n_host, int tile, int nb)
 {
     __shared__ uint32_t tmp[256 / kWave + 1];
-    const int n = *n_dev;
-    const int nb_used = min(nb, ((n > 0 ? n : 1) + kSortTile - 1) / kSortTile);  // tiles with data
+    const int n = n_dev ? *n_dev : n_host;
+    const int nb_used = min(nb, ((n > 0 ? n : 1) + tile - 1) / tile);  // tiles with data
     uint32_t *row = hist + (size_t)blockIdx.x * nb;
     const int per = (nb_used + 255) / 256;
     const int b0 = threadIdx.x * per;
@@ -77,39 +77,52 @@ __global__ __launch_bounds__(256) void k_radix_scan(uint32_t *__restrict__ hist,
     if (threadIdx.x == 0) totals[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(kSortBlock) void k_radix_downsweep(
+template <int B, int BLOCK, int ITEMS>
+__global__ __launch_bounds__(BLOCK) void k_radix_downsweep(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ vals_in,
     uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
-    const int *__restrict__ n_dev, int shift, const uint32_t *__restrict__ hist,
+    const int *__restrict__ n_dev, int n_host, int shift, const uint32_t *__restrict__ hist,
     const uint32_t *__restrict__ totals, int nb)
 {
-    constexpr int W = kSortBlock / kWave;
-    __shared__ uint32_t wcnt[W][kRadix];
-    __shared__ uint32_t lstart[kRadix];
-    __shared__ int delta[kRadix];
-    __shared__ uint32_t skey[kSortTile];
-    __shared__ uint32_t sval[kSortTile];
+    constexpr int R = 1 << B, TILE = BLOCK * ITEMS, W = BLOCK / kWave, D = (R + BLOCK - 1) / BLOCK;
+    __shared__ uint32_t wcnt[W][R];
+    __shared__ uint32_t lstart[R];
+    __shared__ int delta[R];
+    __shared__ uint32_t skey[TILE];
+    __shared__ uint32_t sval[TILE];
     __shared__ uint32_t tmp[W + 1];
 
-    const int n = *n_dev;
-    const int tile0 = blockIdx.x * kSortTile;
+    const int n = n_dev ? *n_dev : n_host;
+    const long long tile0 = (long long)blockIdx.x * TILE;
     if (tile0 >= n) return;  // whole block leaves together
 
     const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
-    for (int i = tid; i < W * kRadix; i += kSortBlock) (&wcnt[0][0])[i] = 0;
-    __syncthreads();
+    // the digits' places are loaded with the keys: thread t holds digits t D ..
+    uint32_t tot[D], before[D];
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+        const int d = tid * D + u;
+        tot[u] = d < R ? totals[d] : 0u;
+        before[u] = d < R ? hist[(size_t)d * nb + blockIdx.x] : 0u;
+    }
+    for (int i = tid; i < W * R; i += BLOCK) (&wcnt[0][0])[i] = 0;
 
-    uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
-    const int base = tile0 + w * (kWave * kSortItems);
+    uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
+    const long long base = tile0 + w * (kWave * ITEMS) + lane;
     const uint64_t lt = lanemask_lt();
 #pragma unroll
-    for (int k = 0; k < kSortItems; ++k) {
-        const int idx = base + k * kWave + lane;
+    for (int k = 0; k < ITEMS; ++k) {
+        const long long idx = base + k * kWave;
         const bool valid = idx < n;
         key[k] = valid ? keys_in[idx] : 0xFFFFFFFFu;
         val[k] = valid ? (vals_in ? vals_in[idx] : (uint32_t)idx) : 0u;
-        const uint32_t d = (key[k] >> shift) & (kRadix - 1);
-        const uint64_t peers = match_digit8(d, __ballot(valid));
+    }
+    __syncthreads();   // counts cleared
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        const bool valid = base + k * kWave < n;
+        const uint32_t d = (key[k] >> shift) & (R - 1);
+        const uint64_t peers = match_bits<B>(d, __ballot(valid));
         const uint32_t prev = wcnt[w][d];
         // Lanes of one wave issue the read above before the leader's write below
         // (in-order LDS per wave; the write depends on the read).
@@ -118,80 +131,114 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_downsweep(
     }
     __syncthreads();
 
-    {   // exclusive offsets across waves, per digit; block count of the digit
-        const int d = tid;
+    // exclusive offsets across waves, per digit; the digits' first places in
+    // the tile and in the output
+    uint32_t cnt[D], csum = 0, tsum = 0;
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+        const int d = tid * D + u;
         uint32_t run = 0;
+        if (d < R) {
 #pragma unroll
-        for (int ww = 0; ww < W; ++ww) { const uint32_t c = wcnt[ww][d]; wcnt[ww][d] = run; run += c; }
-        lstart[d] = run;
+            for (int ww = 0; ww < W; ++ww) { const uint32_t c = wcnt[ww][d]; wcnt[ww][d] = run; run += c; }
+        }
+        cnt[u] = run;
+        csum += run;
+        tsum += tot[u];
+    }
+    uint32_t all;
+    uint32_t lex = block_exclusive_scan<BLOCK>(csum, tmp, &all);
+    uint32_t gex = block_exclusive_scan<BLOCK>(tsum, tmp, &all);
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+        const int d = tid * D + u;
+        if (d < R) {
+            lstart[d] = lex;
+            delta[d] = (int)(gex + before[u] - lex);
+        }
+        lex += cnt[u];
+        gex += tot[u];
     }
     __syncthreads();
-    {
-        const int d = tid;
-        const uint32_t cnt = lstart[d];
-        uint32_t tot;
-        const uint32_t lex = block_exclusive_scan<kSortBlock>(cnt, tmp, &tot);
-        const uint32_t gex = block_exclusive_scan<kSortBlock>(totals[d], tmp, &tot);
-        const uint32_t g = gex + hist[(size_t)d * nb + blockIdx.x];
-        lstart[d] = lex;
-        delta[d] = (int)(g - lex);
-    }
-    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < kSortItems; ++k) {
-        const int idx = base + k * kWave + lane;
-        if (idx < n) {
-            const uint32_t d = (key[k] >> shift) & (kRadix - 1);
+    for (int k = 0; k < ITEMS; ++k) {
+        if (base + k * kWave < n) {
+            const uint32_t d = (key[k] >> shift) & (R - 1);
             const uint32_t p = lstart[d] + wcnt[w][d] + rank[k];
             skey[p] = key[k];
             sval[p] = val[k];
         }
     }
     __syncthreads();
-    const int cnt = min(kSortTile, n - tile0);
-    for (int p = tid; p < cnt; p += kSortBlock) {
+    const int m = (int)min((long long)TILE, n - tile0);
+    for (int p = tid; p < m; p += BLOCK) {
         const uint32_t k = skey[p];
-        const uint32_t d = (k >> shift) & (kRadix - 1);
-        const uint32_t g = (uint32_t)(p + delta[d]);
+        const uint32_t g = (uint32_t)(p + delta[(k >> shift) & (R - 1)]);
         keys_out[g] = k;
         vals_out[g] = sval[p];
     }
 }
 
+// Digits of 10 bits where they save a pass and the pairs are few enough: a
+// tile's runs of equal digits, which its writes are made of, are four times
+// shorter than with 8 bits (2^20 keys of 20 bits 63 us against 72, of 26 bits
+// 90 against 83; 4e6 of 24 bits 198 against 125; 1e5 of 20 bits 48 against 53).
+// Tiles of 4096 pairs from 2^18 pairs on: runs twice as long (1.6e7 pairs of
+// 31 bits 474 us against 644 with 2048), below that too few blocks.
+constexpr int kWideBits = 10;
+RadixPlan radix_plan(int n, int key_bits, int widest)
+{
+    RadixPlan p;
+    const int p8 = std::max(1, div_up(key_bits, kRadixBits)), p10 = std::max(1, div_up(key_bits, kWideBits));
+    const bool wide = widest >= kWideBits && p10 < p8 && n <= (p10 == 2 ? 3 << 19 : 1 << 18);
+    p.bits = wide ? kWideBits : kRadixBits;
+    p.passes = wide ? p10 : p8;
+    p.block = wide || n >= 1 << 18 ? 512 : 256;
+    return p;
+}
+
 size_t sort_scratch_bytes(int n_cap)
 {
-    const int nb = div_up(n_cap > 0 ? n_cap : 1, kSortTile);
-    return (size_t)kRadix * nb * sizeof(uint32_t) + (size_t)kRadix * sizeof(uint32_t) + 256;
+    const int n = n_cap > 0 ? n_cap : 1;
+    const size_t wide = (size_t)kRadixMax * div_up(n, 512 * kSortItems), narrow = (size_t)kRadix * div_up(n, kSortTile);
+    return (std::max(wide, narrow) + kRadixMax) * sizeof(uint32_t) + 256;
 }
 
-void sort_scratch_bind(SortScratch &s, int n_cap, void *mem)
+void sort_scratch_bind(SortScratch &s, int n_cap, void *mem, int digits)
 {
     s.n_cap = n_cap;
-    s.nb = div_up(n_cap > 0 ? n_cap : 1, kSortTile);
-    s.hist = (uint32_t *)mem;
-    s.totals = s.hist + (size_t)kRadix * s.nb;
+    s.totals = (uint32_t *)mem;
+    s.hist = s.totals + digits;
 }
 
-void radix_sort(const uint32_t *keys, const uint32_t *vals, uint32_t *keys_alt,
-                uint32_t *vals_alt, uint32_t *keys_out, uint32_t *vals_out,
-                const int *n_dev, int key_bits, const SortScratch &s,
-                hipStream_t stream, Profiler *prof)
+template <int B, int BLOCK, int ITEMS>
+static void radix_pass(const uint32_t *sk, const uint32_t *sv, uint32_t *dk, uint32_t *dv, const int *n_dev, int n,
+                       int shift, const SortScratch &s, hipStream_t stream, Profiler *prof)
 {
-    const int passes = key_bits <= kRadixBits ? 1 : div_up(key_bits, kRadixBits);
+    const int nb = div_up(n > 0 ? n : 1, BLOCK * ITEMS), digits = 1 << B;
+    DSMC_LAUNCH(prof, "radix_upsweep", (double)n * 4.0, (k_radix_upsweep<B, BLOCK, ITEMS>), nb, BLOCK, stream, sk,
+                n_dev, n, shift, s.hist, nb);
+    DSMC_LAUNCH(prof, "radix_scan", (double)digits * nb * 8.0, k_radix_scan, digits, 256, stream, s.hist, s.totals,
+                n_dev, n, BLOCK * ITEMS, nb);
+    DSMC_LAUNCH(prof, "radix_downsweep", (double)n * 16.0, (k_radix_downsweep<B, BLOCK, ITEMS>), nb, BLOCK, stream,
+                sk, sv, dk, dv, n_dev, n, shift, s.hist, s.totals, nb);
+}
+
+void radix_sort(const uint32_t *keys, const uint32_t *vals, uint32_t *keys_alt, uint32_t *vals_alt,
+                uint32_t *keys_out, uint32_t *vals_out, const int *n_dev, const RadixPlan &plan,
+                const SortScratch &s, hipStream_t stream, Profiler *prof)
+{
     const uint32_t *sk = keys;
     const uint32_t *sv = vals;
-    const double bytes_pass = (double)s.n_cap * 16.0;
-    for (int p = 0; p < passes; ++p) {
-        const int q = passes - 1 - p;  // passes still to go after this one
+    for (int p = 0; p < plan.passes; ++p) {
+        const int q = plan.passes - 1 - p;  // passes still to go after this one
         uint32_t *dk = (q % 2 == 0) ? keys_out : keys_alt;
         uint32_t *dv = (q % 2 == 0) ? vals_out : vals_alt;
-        const int shift = p * kRadixBits;
-        DSMC_LAUNCH(prof, "radix_upsweep", (double)s.n_cap * 4.0, k_radix_upsweep, s.nb,
-                    kSortBlock, stream, sk, n_dev, shift, s.hist, s.nb);
-        DSMC_LAUNCH(prof, "radix_scan", (double)kRadix * s.nb * 8.0, k_radix_scan, kRadix, 256,
-                    stream, s.hist, s.totals, n_dev, s.nb);
-        DSMC_LAUNCH(prof, "radix_downsweep", bytes_pass, k_radix_downsweep, s.nb, kSortBlock,
-                    stream, sk, sv, dk, dv, n_dev, shift, s.hist, s.totals, s.nb);
+        const int shift = p * plan.bits;
+        auto pass = plan.bits == kWideBits ? radix_pass<kWideBits, 512, kSortItems>
+                    : plan.block == 512    ? radix_pass<kRadixBits, 512, kSortItems>
+                                           : radix_pass<kRadixBits, 256, kSortItems>;
+        pass(sk, sv, dk, dv, n_dev, s.n_cap, shift, s, stream, prof);
         sk = dk;
         sv = dv;
     }
@@ -361,6 +408,24 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_partials(int *__restrict__ 
     if (threadIdx.x == 0) partial[nb] = carry;
 }
 
+// Sum of partial[0 .. b) over the block's threads (every thread returns it).
+__device__ __forceinline__ int sum_below(const int *__restrict__ partial, int b, int *tmp)
+{
+    int s = 0;
+    for (int i0 = threadIdx.x; i0 < b; i0 += 4 * kScanBlock) {
+        int c[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) c[u] = i0 + u * kScanBlock < b ? partial[i0 + u * kScanBlock] : 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s += c[u];
+    }
+    int total;
+    (void)block_exclusive_scan<kScanBlock>(s, tmp, &total);
+    return total;
+}
+
+// Every block adds up the tiles' sums before its own itself: one launch fewer
+// than a scan of the partials, and for a million elements 489 words a block.
 __global__ __launch_bounds__(kScanBlock) void k_scan_final(const int *__restrict__ in,
                                                            int *__restrict__ out, int n,
                                                            const int *__restrict__ partial)
@@ -374,8 +439,9 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_final(const int *__restrict
         v[k] = (t0 + k < n) ? in[t0 + k] : 0;
         s += v[k];
     }
+    const int before = sum_below(partial, (int)blockIdx.x, tmp);
     int total;
-    int run = block_exclusive_scan<kScanBlock>(s, tmp, &total) + partial[blockIdx.x];
+    int run = block_exclusive_scan<kScanBlock>(s, tmp, &total) + before;
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
         if (t0 + k < n) out[t0 + k] = run;
@@ -390,10 +456,78 @@ void exclusive_scan(const int *in, int *out, int n, int *partial, hipStream_t st
     const int nb = div_up(n, kScanTile);
     DSMC_LAUNCH(prof, "scan_reduce", (double)n * 4.0, k_scan_reduce, nb, kScanBlock, stream,
                 in, n, partial);
-    DSMC_LAUNCH(prof, "scan_partials", (double)nb * 8.0, k_scan_partials, 1, kScanBlock,
-                stream, partial, nb);
     DSMC_LAUNCH(prof, "scan_final", (double)n * 8.0, k_scan_final, nb, kScanBlock, stream, in,
                 out, n, (const int *)partial);
+}
+
+// ---------------------------------------------------------------------------
+// Removal in place (thrust::remove_if): every block compacts its tile's kept
+// values into tmp, then moves them to their place behind the earlier tiles'.
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(kScanBlock) void k_remove_tile(const int *__restrict__ values,
+                                                            const int *__restrict__ stencil, int n,
+                                                            int *__restrict__ tmp_out, int *__restrict__ partial)
+{
+    constexpr int W = kScanBlock / kWave;
+    __shared__ int wtot[W];
+    __shared__ int kept[kScanTile];
+    const int tile0 = blockIdx.x * kScanTile;
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const int base = tile0 + w * (kWave * kScanItems) + lane;
+    const uint64_t lt = lanemask_lt();
+    int v[kScanItems], rank[kScanItems];
+    bool keep[kScanItems];
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        const int i = base + k * kWave;
+        v[k] = i < n ? values[i] : 0;
+        keep[k] = i < n && stencil[i] == 0;
+    }
+    int run = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        const uint64_t b = __ballot(keep[k]);
+        rank[k] = run + __popcll(b & lt);
+        run += __popcll(b);
+    }
+    if (lane == 0) wtot[w] = run;
+    __syncthreads();
+    int off = 0, all = 0;
+#pragma unroll
+    for (int ww = 0; ww < W; ++ww) {
+        if (ww < w) off += wtot[ww];
+        all += wtot[ww];
+    }
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k)
+        if (keep[k]) kept[off + rank[k]] = v[k];
+    __syncthreads();
+    for (int i = threadIdx.x; i < all; i += kScanBlock) tmp_out[tile0 + i] = kept[i];
+    if (threadIdx.x == 0) partial[blockIdx.x] = all;
+}
+
+__global__ __launch_bounds__(kScanBlock) void k_remove_place(const int *__restrict__ tmp_in,
+                                                             const int *__restrict__ partial, int nb,
+                                                             int *__restrict__ values, int *__restrict__ kept)
+{
+    __shared__ int tmp[kScanBlock / kWave + 1];
+    const int m = partial[blockIdx.x];
+    const int before = sum_below(partial, (int)blockIdx.x, tmp);
+    const int *src = tmp_in + (size_t)blockIdx.x * kScanTile;
+    for (int i = threadIdx.x; i < m; i += kScanBlock) values[before + i] = src[i];
+    if ((int)blockIdx.x == nb - 1 && threadIdx.x == 0) *kept = before + m;
+}
+
+int remove_if_blocks(int n) { return div_up(n > 0 ? n : 1, kScanTile); }
+
+void remove_if(int *values, const int *stencil, int n, int *tmp, int *partial, int *kept, hipStream_t stream)
+{
+    const int nb = remove_if_blocks(n);
+    hipLaunchKernelGGL(k_remove_tile, dim3(nb), dim3(kScanBlock), 0, stream, values, stencil, n, tmp, partial);
+    DSMC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_remove_place, dim3(nb), dim3(kScanBlock), 0, stream, tmp, partial, nb, values,
+                       kept);
+    DSMC_HIP(hipGetLastError());
 }
 
 // ---------------------------------------------------------------------------

@@ -280,8 +280,9 @@ dsmc_status dsmc_profile_read(dsmc_ctx *ctx, dsmc_kernel_stat *stats, int max_st
 dsmc_status dsmc_autotune(dsmc_ctx *ctx, int *block_size_out);
 
 /* ---- device primitives on caller-owned device memory ------------------ */
-/* stream may be NULL (default stream).  Temporary storage is allocated and
- * freed inside the call. */
+/* stream may be NULL (default stream).  Each call takes its temporary storage
+ * for itself and waits for the stream before it returns; a little of it (at
+ * most 512 MB) is kept idle for later calls. */
 
 /* thrust::sort_by_key(int keys, int values) (collisions.cu:282-284): stable
  * LSD radix sort of n (key, value) pairs, keys in [0, 2^key_bits). */

@@ -161,6 +161,7 @@ struct dsmc_ctx {
     unsigned long long *coll_accum = nullptr;
     int *n_dev = nullptr;           // [0], [1]: alive counts; [2]: scratch
     int *n_host = nullptr;          // pinned copy of n_dev for host reads
+    dsmc_observables *obs_host = nullptr;   // pinned record (FP64 form)
     int *scan_partial = nullptr;    // partials of scans and compactions
     // FP64 form
     PlainPtrs ps[2];
@@ -232,6 +233,7 @@ struct dsmc_ctx {
         if (graph) (void)hipGraphDestroy(graph);
         for (void *p : allocs) (void)hipFree(p);
         if (n_host) (void)hipHostFree(n_host);
+        if (obs_host) (void)hipHostFree(obs_host);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -411,6 +413,8 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
     x->coll_accum = x->alloc<unsigned long long>(n_traps);
     x->n_dev = x->alloc<int>(4);
     DSMC_HIP(hipHostMalloc((void **)&x->n_host, 4 * sizeof(int), hipHostMallocDefault));
+    if (!x->fp32)
+        DSMC_HIP(hipHostMalloc((void **)&x->obs_host, sizeof(dsmc_observables), hipHostMallocDefault));
     // incremental re-sort (its counts start cleared)
     resort_scratch_bind(x->res, N, x->alloc<char>(resort_scratch_bytes(N), false));
     resort_clear_counts(x->res, x->stream, nullptr);
@@ -538,7 +542,7 @@ static void plain_sort(dsmc_ctx *x)
 static void plain_table(dsmc_ctx *x)
 {
     launch_cell_table_plain(x->sorted_key, x->n_dev, x->n_cap, x->start_end, x->count, x->prefix,
-                            x->scan_partial, x->ncells, x->stream, &x->prof);
+                            x->ncells, x->stream, &x->prof);
 }
 
 static void plain_collide(dsmc_ctx *x)
@@ -631,16 +635,15 @@ static void plain_compact(dsmc_ctx *x)
     compaction_map(x->tag, x->n_dev, x->n_cap, x->cmap, x->n_dev + 2, x->scan_partial, x->stream,
                    &x->prof);
     launch_gather_plain(x->ps[x->cur ^ 1], x->ps[x->cur], x->cmap, x->n_dev + 2, x->n_cap,
-                        x->cfg.spin, x->stream, &x->prof);
+                        x->cfg.spin, x->stream, &x->prof, x->n_dev, x->n_host);
     x->cur ^= 1;
-    DSMC_HIP(hipMemcpyAsync(x->n_dev, x->n_dev + 2, sizeof(int), hipMemcpyDeviceToDevice,
-                            x->stream));
 }
 
-static void plain_observe(dsmc_ctx *x, dsmc_observables *slot, long long step)
+// The record of the sums that a move or launch_observe_plain left.
+static void plain_record(dsmc_ctx *x, dsmc_observables *slot, long long step)
 {
-    launch_observe_plain(x->tdev[0], x->cfg.mass, x->ps[x->cur], x->n_dev, x->n_cap, x->partials,
-                         slot, x->coll_accum, x->evap_accum, step, x->stream, &x->prof);
+    launch_observe_finalize_plain(x->n_dev, x->n_cap, x->partials, slot, x->coll_accum, x->evap_accum, step,
+                                  x->stream, &x->prof);
 }
 
 // ---------------------------------------------------------------------------
@@ -680,7 +683,7 @@ static void plain_need_tables(dsmc_ctx *x)
 {
     if (!x->tables_stale) return;
     launch_cell_table_plain(x->sorted_key, x->n_dev + 3, x->n_cap, x->start_end, x->count, x->prefix,
-                            x->scan_partial, x->ncells, x->stream, nullptr);
+                            x->ncells, x->stream, nullptr);
     launch_untag_counts(x->cc_tagged, (unsigned)x->coll_steps, x->ncells, x->coll_count, x->stream);
     x->tables_stale = false;
 }
@@ -1105,10 +1108,12 @@ static void observe_now(dsmc_ctx *x, std::vector<dsmc_observables> &out)
     out.assign(x->T, dsmc_observables{});
     if (!x->fp32) {
         plain_settle(x);
-        plain_observe(x, x->obs_log + x->obs_cap, x->step);
+        // the record comes back through pinned memory
+        launch_observe_plain(x->tdev[0], x->cfg.mass, x->ps[x->cur], x->n_dev, x->n_cap, x->partials, x->stream,
+                             &x->prof);
+        plain_record(x, x->obs_host, x->step);
         DSMC_HIP(hipStreamSynchronize(x->stream));
-        DSMC_HIP(hipMemcpy(out.data(), x->obs_log + x->obs_cap, sizeof(dsmc_observables),
-                           hipMemcpyDeviceToHost));
+        out[0] = *x->obs_host;
         return;
     }
     launch_observe_fused(x->d_traps, x->d_key_base, x->T, x->cfg.mass, x->fs[x->cur], x->key_a,
@@ -1732,9 +1737,9 @@ dsmc_status dsmc_move_atoms(dsmc_ctx *ctx)
         fused_move(ctx);
     } else {
         plain_enter(ctx);
-        launch_move_plain(ctx->tdev[0], ctx->cfg.dt, ctx->ps[ctx->cur], ctx->n_dev, ctx->n_cap,
-                          ctx->stream, &ctx->prof);
-        plain_observe(ctx, ctx->obs_log + (ctx->step % ctx->obs_cap), ctx->step);
+        launch_move_plain(ctx->tdev[0], ctx->cfg.dt, ctx->cfg.mass, ctx->ps[ctx->cur], ctx->n_dev, ctx->n_cap,
+                          ctx->partials, ctx->stream, &ctx->prof);
+        plain_record(ctx, ctx->obs_log + (ctx->step % ctx->obs_cap), ctx->step);
     }
     ctx->step++;
     DSMC_API_END(ctx)
@@ -1801,7 +1806,10 @@ dsmc_status dsmc_compact(dsmc_ctx *ctx, int *n_alive)
     if (ctx->fp32) fail(DSMC_ENOTSUP, "the FP32 form compacts inside the sort");
     plain_enter(ctx);
     plain_compact(ctx);
-    if (n_alive) *n_alive = host_alive(ctx);
+    if (n_alive) {   // the gather left the count in n_host
+        DSMC_HIP(hipStreamSynchronize(ctx->stream));
+        *n_alive = ctx->n_host[0];
+    }
     DSMC_API_END(ctx)
 }
 

@@ -28,13 +28,20 @@ __global__ __launch_bounds__(kBlock) void k_index_plain(TrapDev t, const double 
     if (i < *n_dev) key[i] = (uint32_t)(t.key_base + cell_of(t, x[i], y[i], z[i]));
 }
 
-// Gather every state array through `map` (dst[i] = src[map[i]]).
+// Gather every state array through `map` (dst[i] = src[map[i]]).  n_out,
+// n_host (pinned; when not null) receive the count.
 __global__ __launch_bounds__(kBlock) void k_gather_plain(PlainPtrs dst, PlainPtrs src,
                                                          const uint32_t *__restrict__ map,
-                                                         const int *__restrict__ n_dev, int spin)
+                                                         const int *__restrict__ n_dev, int spin,
+                                                         int *__restrict__ n_out, int *__restrict__ n_host)
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= *n_dev) return;
+    const int n = *n_dev;
+    if (i == 0) {
+        if (n_out) *n_out = n;
+        if (n_host) *n_host = n;
+    }
+    if (i >= n) return;
     const uint32_t j = map[i];
 #pragma unroll
     for (int c = 0; c < 9; ++c) dst.d[c][i] = src.d[c][j];
@@ -49,25 +56,68 @@ __global__ __launch_bounds__(kBlock) void k_gather_plain(PlainPtrs dst, PlainPtr
 // ---------------------------------------------------------------------------
 // Cell table (main.cu:426-442; collisions.cu:228-271).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void k_cell_start_end(const uint32_t *__restrict__ key,
-                                                           const int *__restrict__ n_dev,
-                                                           int2 *__restrict__ se)
+// First slot with a key of at least c, of n slots with ascending keys: the wave
+// probes 64 places at a time (four rounds of loads for 2^24 slots).
+__device__ __forceinline__ int wave_lower_bound(const uint32_t *__restrict__ key, int n, uint32_t c)
 {
-    const int n = *n_dev;
-    const int s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= n) return;
-    const uint32_t c = key[s];
-    if (s == 0 || key[s - 1] != c) se[c].x = s;
-    if (s == n - 1 || key[s + 1] != c) se[c].y = s;
+    const int lane = threadIdx.x & (kWave - 1);
+    int lo = 0, hi = n;   // the answer is in [lo, hi]
+    while (hi > lo) {
+        const int s = (hi - lo + kWave - 1) / kWave;   // probes at lo + (lane + 1) s - 1
+        const long long p = (long long)lo + (long long)(lane + 1) * s - 1;
+        const bool below = p < hi && key[p] < c;
+        const int k = __popcll(__ballot(below));   // a prefix of the lanes
+        const int first = lo + k * s;
+        hi = (int)min((long long)hi, (long long)lo + (long long)(k + 1) * s - 1);
+        lo = first;
+        if (hi < lo) hi = lo;
+    }
+    return lo;
 }
 
-__global__ __launch_bounds__(kBlock) void k_cell_count(const int2 *__restrict__ se,
-                                                       int *__restrict__ count, int n)
+// The whole table in one launch: a block finds where the keys of its 256 cells
+// lie (two searches by waves), takes them into LDS when they fit, and every
+// cell finds its first slot there.  Bound by that chain of loads; it replaces a
+// fill, a pass over the keys, a pass over the cells and a scan, five launches
+// (the loop of single calls at N = 3e4 in 41^3 cells, with the move leaving its
+// own sums and the compaction in three launches: 145 -> 111 us).
+constexpr int kTableKeys = 4096;
+
+__global__ __launch_bounds__(kBlock) void k_cell_table(const uint32_t *__restrict__ key,
+                                                       const int *__restrict__ n_dev, int cells,
+                                                       int2 *__restrict__ se, int *__restrict__ count,
+                                                       int *__restrict__ prefix)
 {
-    const int c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= n) return;
-    const int2 v = se[c];
-    count[c] = v.x == -1 ? 0 : v.y - v.x + 1;
+    __shared__ uint32_t k[kTableKeys];
+    __shared__ int bound[2];
+    __shared__ int first[kBlock + 1];
+    const int n = *n_dev;
+    const int c0 = blockIdx.x * kBlock, tid = threadIdx.x;
+    const int w = tid / kWave;
+    if (w < 2) {
+        const int b = wave_lower_bound(key, n, (uint32_t)(c0 + w * kBlock));
+        if ((tid & (kWave - 1)) == 0) bound[w] = b;
+    }
+    __syncthreads();
+    const int a = bound[0], m = bound[1] - a;
+    const bool in_lds = m <= kTableKeys;
+    if (in_lds)
+        for (int i = tid; i < m; i += kBlock) k[i] = key[a + i];
+    __syncthreads();
+    int lo = 0, hi = m;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if ((in_lds ? k[mid] : key[a + mid]) < (uint32_t)(c0 + tid)) lo = mid + 1; else hi = mid;
+    }
+    first[tid] = a + lo;
+    if (tid == 0) first[kBlock] = a + m;
+    __syncthreads();
+    const int c = c0 + tid;
+    if (c >= cells) return;
+    const int f = first[tid], cnt = first[tid + 1] - f;
+    prefix[c] = f;
+    count[c] = cnt;
+    se[c] = cnt > 0 ? make_int2(f, f + cnt - 1) : make_int2(-1, -1);
 }
 
 // ---------------------------------------------------------------------------
@@ -124,17 +174,56 @@ __global__ __launch_bounds__(kBlock) void k_collide_plain(
 // ---------------------------------------------------------------------------
 // moveAtoms (moveAtoms.cu:23-91): velocity Verlet with stored acceleration.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void k_move_plain(TrapDev t, double dt, PlainPtrs s,
-                                                       const int *__restrict__ n_dev)
+__device__ __forceinline__ void move_atom(const TrapDev &t, double dt, const PlainPtrs &s, int i, D3 &p, D3 &v,
+                                          bool &up)
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= *n_dev) return;
-    D3 p = { s.d[0][i], s.d[1][i], s.d[2][i] }, v = { s.d[3][i], s.d[4][i], s.d[5][i] },
-       a = { s.d[6][i], s.d[7][i], s.d[8][i] };
-    plain_verlet(t, dt, s.up[i] != 0, p, v, a);
+    p = D3{ s.d[0][i], s.d[1][i], s.d[2][i] };
+    v = D3{ s.d[3][i], s.d[4][i], s.d[5][i] };
+    D3 a = { s.d[6][i], s.d[7][i], s.d[8][i] };
+    up = s.up[i] != 0;
+    plain_verlet(t, dt, up, p, v, a);
     s.d[0][i] = p.x; s.d[1][i] = p.y; s.d[2][i] = p.z;
     s.d[3][i] = v.x; s.d[4][i] = v.y; s.d[5][i] = v.z;
     s.d[6][i] = a.x; s.d[7][i] = a.y; s.d[8][i] = a.z;
+}
+
+// The observables of the moved state (calculateTemp, evaporation.cu:108-189,
+// and the energy of energyChecker.py:117-122): a block's sums, in a fixed
+// order (reproducible); k_observe_finalize_plain adds the blocks.
+constexpr int kObsK = 5;  // ek, ep, vx^2, vy^2, vz^2
+
+__device__ __forceinline__ void observe_block(const TrapDev &t, double mass, bool in, bool up, const D3 &p,
+                                              const D3 &w, double *__restrict__ partials)
+{
+    __shared__ double tmp[(kBlock / kWave) * kObsK];
+    double v[kObsK] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
+    if (in) {
+        v[0] = 0.5 * mass * (w.x * w.x + w.y * w.y + w.z * w.z);
+        // U_up = mu (|B| - B0); a spin-down atom (after a flip) has
+        // U_down = -mu (|B| + B0), so that a flip conserves E_k + U
+        const double u = potential_energy(t, p.x, p.y, p.z);
+        v[1] = up ? u : -u - 2.0 * t.mu * t.B0;
+        v[2] = w.x * w.x; v[3] = w.y * w.y; v[4] = w.z * w.z;
+    }
+    block_sum<kBlock, kObsK>(v, tmp);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < kObsK; ++k) partials[(size_t)blockIdx.x * kObsK + k] = v[k];
+    }
+}
+
+// The move leaves the block sums of the moved state as it goes (the state was
+// read a second time for them).
+__global__ __launch_bounds__(kBlock) void k_move_plain(TrapDev t, double dt, double mass, PlainPtrs s,
+                                                       const int *__restrict__ n_dev,
+                                                       double *__restrict__ partials)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const bool in = i < *n_dev;
+    D3 p = { 0.0, 0.0, 0.0 }, v = p;
+    bool up = true;
+    if (in) move_atom(t, dt, s, i, p, v, up);
+    observe_block(t, mass, in, up, p, v, partials);
 }
 
 // ---------------------------------------------------------------------------
@@ -252,35 +341,22 @@ __global__ __launch_bounds__(kBlock) void k_evap_tag_plain(TrapDev t, EvapParams
 }
 
 // ---------------------------------------------------------------------------
-// FP64 observables (calculateTemp, evaporation.cu:108-189, and the energy of
-// energyChecker.py:117-122).  Per-block partials; the last block to finish
-// adds them in a fixed order (reproducible) and appends one log record.
+// FP64 observables of the current state.
 // ---------------------------------------------------------------------------
-constexpr int kObsK = 5;  // ek, ep, vx^2, vy^2, vz^2
-
 __global__ __launch_bounds__(kBlock) void k_observe_plain(TrapDev t, double mass, PlainPtrs s,
                                                           const int *__restrict__ n_dev,
                                                           double *__restrict__ partials)
 {
-    __shared__ double tmp[(kBlock / kWave) * kObsK];
-    const int n = *n_dev;
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    double v[kObsK] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
-    if (i < n) {
-        const double x = s.d[0][i], y = s.d[1][i], z = s.d[2][i];
-        const double vx = s.d[3][i], vy = s.d[4][i], vz = s.d[5][i];
-        v[0] = 0.5 * mass * (vx * vx + vy * vy + vz * vz);
-        // U_up = mu (|B| - B0); a spin-down atom (after a flip) has
-        // U_down = -mu (|B| + B0), so that a flip conserves E_k + U
-        const double u = potential_energy(t, x, y, z);
-        v[1] = s.up[i] ? u : -u - 2.0 * t.mu * t.B0;
-        v[2] = vx * vx; v[3] = vy * vy; v[4] = vz * vz;
+    const bool in = i < *n_dev;
+    D3 p = { 0.0, 0.0, 0.0 }, v = p;
+    bool up = true;
+    if (in) {
+        p = D3{ s.d[0][i], s.d[1][i], s.d[2][i] };
+        v = D3{ s.d[3][i], s.d[4][i], s.d[5][i] };
+        up = s.up[i] != 0;
     }
-    block_sum<kBlock, kObsK>(v, tmp);
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int k = 0; k < kObsK; ++k) partials[(size_t)blockIdx.x * kObsK + k] = v[k];
-    }
+    observe_block(t, mass, in, up, p, v, partials);
 }
 
 // One block adds the block partials in a fixed order (reproducible) and
@@ -364,23 +440,19 @@ void launch_index_plain(const TrapDev &t, const PlainPtrs &s, uint32_t *key, con
 }
 
 void launch_gather_plain(const PlainPtrs &dst, const PlainPtrs &src, const uint32_t *map,
-                         const int *n_dev, int n_cap, int spin, hipStream_t st, Profiler *prof)
+                         const int *n_dev, int n_cap, int spin, hipStream_t st, Profiler *prof,
+                         int *n_out, int *n_host)
 {
     const double per = 4.0 + 2.0 * (9 * 8 + 4 + 1 + (spin ? 32 : 0));
     DSMC_LAUNCH(prof, "gather_plain", (double)n_cap * per, k_gather_plain, grid_for(n_cap), kBlock,
-                st, dst, src, map, n_dev, spin);
+                st, dst, src, map, n_dev, spin, n_out, n_host);
 }
 
 void launch_cell_table_plain(const uint32_t *key, const int *n_dev, int n_cap, int2 *se,
-                             int *count, int *prefix, int *partial, int ncells,
-                             hipStream_t st, Profiler *prof)
+                             int *count, int *prefix, int ncells, hipStream_t st, Profiler *prof)
 {
-    fill_u32((uint32_t *)se, 0xFFFFFFFFu, 2LL * (ncells + 1), st, prof);
-    DSMC_LAUNCH(prof, "cell_start_end", (double)n_cap * 4.0, k_cell_start_end, grid_for(n_cap),
-                kBlock, st, key, n_dev, se);
-    DSMC_LAUNCH(prof, "cell_count", (double)(ncells + 1) * 12.0, k_cell_count,
-                grid_for(ncells + 1), kBlock, st, (const int2 *)se, count, ncells + 1);
-    exclusive_scan(count, prefix, ncells + 1, partial, st, prof);
+    DSMC_LAUNCH(prof, "cell_table", (double)n_cap * 4.0 + (ncells + 1) * 16.0, k_cell_table,
+                grid_for(ncells + 1), kBlock, st, key, n_dev, ncells + 1, se, count, prefix);
 }
 
 void launch_collide_plain(const TrapDev &t, const CollideParams &cp, const PlainPtrs &s,
@@ -394,11 +466,11 @@ void launch_collide_plain(const TrapDev &t, const CollideParams &cp, const Plain
                 step);
 }
 
-void launch_move_plain(const TrapDev &t, double dt, const PlainPtrs &s, const int *n_dev,
-                       int n_cap, hipStream_t st, Profiler *prof)
+void launch_move_plain(const TrapDev &t, double dt, double mass, const PlainPtrs &s, const int *n_dev,
+                       int n_cap, double *partials, hipStream_t st, Profiler *prof)
 {
     DSMC_LAUNCH(prof, "move_plain", (double)n_cap * 145.0, k_move_plain, grid_for(n_cap), kBlock,
-                st, t, dt, s, n_dev);
+                st, t, dt, mass, s, n_dev, partials);
 }
 
 void launch_spin_plain(const TrapDev &t, const SpinParams &sp, const PlainPtrs &s,
@@ -448,15 +520,18 @@ void launch_decay_plain(const TrapDev &t, const DecayParams &dp, const PlainPtrs
 int observe_plain_blocks(int n_cap) { return grid_for(n_cap); }
 
 void launch_observe_plain(const TrapDev &t, double mass, const PlainPtrs &s, const int *n_dev,
-                          int n_cap, double *partials, dsmc_observables *out,
-                          unsigned long long *coll_accum, double *evap_accum, long long step,
-                          hipStream_t st, Profiler *prof)
+                          int n_cap, double *partials, hipStream_t st, Profiler *prof)
 {
     DSMC_LAUNCH(prof, "observe_plain", (double)n_cap * 48.0, k_observe_plain, grid_for(n_cap),
                 kBlock, st, t, mass, s, n_dev, partials);
+}
+
+void launch_observe_finalize_plain(const int *n_dev, int n_cap, const double *partials, dsmc_observables *out,
+                                   unsigned long long *coll_accum, double *evap_accum, long long step,
+                                   hipStream_t st, Profiler *prof)
+{
     DSMC_LAUNCH(prof, "observe_finalize", (double)grid_for(n_cap) * 40.0, k_observe_finalize_plain,
-                1, kBlock, st, n_dev, (const double *)partials, grid_for(n_cap), out, coll_accum,
-                evap_accum, step);
+                1, kBlock, st, n_dev, partials, grid_for(n_cap), out, coll_accum, evap_accum, step);
 }
 
 void launch_init_plain(const TrapDev &t, const InitParams &ip, const PlainPtrs &s, int n,

@@ -57,16 +57,17 @@ struct EvapParams {
 void launch_index_plain(const TrapDev &t, const PlainPtrs &s, uint32_t *key, const int *n_dev,
                         int n_cap, hipStream_t st, Profiler *prof);
 void launch_gather_plain(const PlainPtrs &dst, const PlainPtrs &src, const uint32_t *map,
-                         const int *n_dev, int n_cap, int spin, hipStream_t st, Profiler *prof);
+                         const int *n_dev, int n_cap, int spin, hipStream_t st, Profiler *prof,
+                         int *n_out = nullptr, int *n_host = nullptr);
 void launch_cell_table_plain(const uint32_t *key, const int *n_dev, int n_cap, int2 *se,
-                             int *count, int *prefix, int *partial, int ncells,
-                             hipStream_t st, Profiler *prof);
+                             int *count, int *prefix, int ncells, hipStream_t st, Profiler *prof);
 void launch_collide_plain(const TrapDev &t, const CollideParams &cp, const PlainPtrs &s,
                           double *sigvrmax, const int *prefix, int *coll_count,
                           unsigned long long *coll_total, int ncells, uint32_t step,
                           hipStream_t st, Profiler *prof);
-void launch_move_plain(const TrapDev &t, double dt, const PlainPtrs &s, const int *n_dev,
-                       int n_cap, hipStream_t st, Profiler *prof);
+// partials: observe_plain_blocks(n_cap) * 5 doubles, the observables' block sums.
+void launch_move_plain(const TrapDev &t, double dt, double mass, const PlainPtrs &s, const int *n_dev,
+                       int n_cap, double *partials, hipStream_t st, Profiler *prof);
 void launch_spin_plain(const TrapDev &t, const SpinParams &sp, const PlainPtrs &s,
                        const int *n_dev, int n_cap, hipStream_t st, Profiler *prof);
 void launch_normalise_plain(const PlainPtrs &s, const int *n_dev, int n_cap, hipStream_t st,
@@ -83,9 +84,12 @@ void launch_evap_tag_plain(const TrapDev &t, const EvapParams &ep, const PlainPt
                            const int *n_dev, int n_cap, hipStream_t st, Profiler *prof);
 int  observe_plain_blocks(int n_cap);
 void launch_observe_plain(const TrapDev &t, double mass, const PlainPtrs &s, const int *n_dev,
-                          int n_cap, double *partials, dsmc_observables *out,
-                          unsigned long long *coll_accum, double *evap_accum, long long step,
-                          hipStream_t st, Profiler *prof);
+                          int n_cap, double *partials, hipStream_t st, Profiler *prof);
+// The record of the sums in partials to *out (device or pinned host memory);
+// clears the accumulators.
+void launch_observe_finalize_plain(const int *n_dev, int n_cap, const double *partials, dsmc_observables *out,
+                                   unsigned long long *coll_accum, double *evap_accum, long long step,
+                                   hipStream_t st, Profiler *prof);
 void launch_init_plain(const TrapDev &t, const InitParams &ip, const PlainPtrs &s, int n,
                        hipStream_t st, Profiler *prof);
 void launch_accel_plain(const TrapDev &t, const PlainPtrs &s, int n, hipStream_t st,

@@ -392,22 +392,6 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const int *__restric
     if (threadIdx.x == 0) partial[blockIdx.x] = total;
 }
 
-// Single block: exclusive scan of partial[0..nb) in place; partial[nb] = total.
-__global__ __launch_bounds__(kScanBlock) void k_scan_partials(int *__restrict__ partial, int nb)
-{
-    __shared__ int tmp[kScanBlock / kWave + 1];
-    int carry = 0;
-    for (int c0 = 0; c0 < nb; c0 += kScanBlock) {
-        const int i = c0 + threadIdx.x;
-        const int v = i < nb ? partial[i] : 0;
-        int total;
-        const int ex = block_exclusive_scan<kScanBlock>(v, tmp, &total);
-        if (i < nb) partial[i] = ex + carry;
-        carry += total;
-    }
-    if (threadIdx.x == 0) partial[nb] = carry;
-}
-
 // Sum of partial[0 .. b) over the block's threads (every thread returns it).
 __device__ __forceinline__ int sum_below(const int *__restrict__ partial, int b, int *tmp)
 {
@@ -557,9 +541,14 @@ __global__ __launch_bounds__(kScanBlock) void k_compact_scatter(
 {
     constexpr int W = kScanBlock / kWave;
     __shared__ int wtot[W];
+    __shared__ int tmp[W + 1];
     const int n = *n_dev;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *n_out = partial[nb];
     const int tile0 = blockIdx.x * kScanTile;
+    const bool last = (int)blockIdx.x == nb - 1;
+    if (tile0 >= n && !last) return;
+    // every block adds up the kept ones of the tiles before its own
+    const int before = sum_below(partial, (int)blockIdx.x, tmp);
+    if (last && threadIdx.x == 0) *n_out = before + partial[blockIdx.x];
     if (tile0 >= n) return;
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int base = tile0 + w * (kWave * kScanItems);
@@ -577,7 +566,7 @@ __global__ __launch_bounds__(kScanBlock) void k_compact_scatter(
     }
     if (lane == 0) wtot[w] = run;
     __syncthreads();
-    int off = partial[blockIdx.x];
+    int off = before;
     for (int ww = 0; ww < w; ++ww) off += wtot[ww];
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k)
@@ -590,8 +579,6 @@ void compaction_map(const int *stencil, const int *n_dev, int n_cap, uint32_t *m
     const int nb = div_up(n_cap > 0 ? n_cap : 1, kScanTile);
     DSMC_LAUNCH(prof, "compact_count", (double)n_cap * 4.0, k_compact_count, nb, kScanBlock,
                 stream, stencil, n_dev, partial);
-    DSMC_LAUNCH(prof, "scan_partials", (double)nb * 8.0, k_scan_partials, 1, kScanBlock, stream,
-                partial, nb);
     DSMC_LAUNCH(prof, "compact_scatter", (double)n_cap * 8.0, k_compact_scatter, nb, kScanBlock,
                 stream, stencil, n_dev, (const int *)partial, map, n_out_dev, nb);
 }

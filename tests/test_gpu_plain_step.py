@@ -69,3 +69,25 @@ def test_step_equals_calls(n, lpc, kind, cut):
         if n > 2000:
             assert not cut or ia.n_alive < n
             assert kind == "ip" or a.obs_log()["collisions"].sum() > 0
+
+
+@pytest.mark.parametrize("n", [1, 63, 255, 257, 4096, 4097, 20000])
+@pytest.mark.parametrize("nc", [1, 4, 7, 20])
+def test_cell_table(n, nc):
+    """start/end, count and prefix of every cell from the sorted keys: blocks of
+    256 cells with more or fewer keys than fit LDS, empty cells, the last block."""
+    run = configs.Run(traps=[configs.quadrupole_trap(n, nc)])
+    with Simulation(run) as sim:
+        sim.init_distribution()
+        sim.index_atoms()
+        sim.sort_arrays()
+        sim.build_cell_table()
+        key = sim.copy_out(_abi.FIELD_CELL_ID)
+        se, count, prefix = (sim.copy_out(f) for f in (_abi.FIELD_CELL_START_END, _abi.FIELD_CELL_COUNT,
+                                                       _abi.FIELD_CELL_PREFIX))
+    want = np.bincount(key, minlength=nc ** 3 + 1)
+    first = np.concatenate([[0], np.cumsum(want)[:-1]])
+    np.testing.assert_array_equal(count, want)
+    np.testing.assert_array_equal(prefix, first)
+    np.testing.assert_array_equal(se[:, 0], np.where(want > 0, first, -1))
+    np.testing.assert_array_equal(se[:, 1], np.where(want > 0, first + want - 1, -1))

@@ -206,6 +206,7 @@ struct dsmc_ctx {
     int *obs_first = nullptr, *obs_last = nullptr;   // on-demand observables scratch
     int max_trap_atoms = 0;
     float *evap_pos_f = nullptr, *evap_vel_f = nullptr;
+    float *spin_tau = nullptr;   // (spin) the substeps' times in a step
     // graph of two FP32 steps (parity 0 then 1)
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -464,6 +465,17 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
         for (int b = 0; b < 2; ++b) {
             x->fs[b].r = x->alloc<f4>(rec_elems(N));
             for (int k = 0; k < 3; ++k) x->fs[b].s[k] = c->spin ? x->alloc<float>(N) : nullptr;
+        }
+        if (c->spin) {
+            const int S = std::max(1, c->spin_substeps);
+            const float dts = (float)(c->dt / S);
+            std::vector<float> tau((size_t)S + 1, 0.0f);   // (the kernel reads one ahead)
+            if (c->spin_interp)
+                for (int k = 0; k < S; ++k) tau[k] = ((float)k + 0.5f) * dts;
+            x->spin_tau = x->alloc<float>(tau.size(), false);
+            DSMC_HIP(hipMemcpyAsync(x->spin_tau, tau.data(), tau.size() * sizeof(float),
+                                    hipMemcpyHostToDevice, x->stream));
+            DSMC_HIP(hipStreamSynchronize(x->stream));   // (tau goes)
         }
         x->mask_dead = x->alloc<uint64_t>(resort_mask_words(N));
         x->srt_k[0] = x->key_b; x->srt_v[0] = x->val_b;
@@ -795,10 +807,11 @@ static MoveParams move_params(const dsmc_ctx *x)
     mp.f_dt = (float)x->cfg.dt;
     mp.mass = x->cfg.mass;
     mp.f_half_mass = (float)(0.5 * x->cfg.mass);
-    mp.gs = x->cfg.gs;
     mp.spin = x->cfg.spin;
     mp.substeps = std::max(1, x->cfg.spin_substeps);
-    mp.interp = x->cfg.spin_interp;
+    const double dts = mp.dt / mp.substeps;
+    mp.f_spin_w = (float)(x->cfg.gs * kMuB * dts / kHbar);
+    mp.spin_tau = x->spin_tau;
     mp.spin_loss = (x->cfg.evaporation & DSMC_EVAP_SPIN) ? 1 : 0;
     mp.energy_cut = (x->cfg.evaporation & DSMC_EVAP_ENERGY) ? 1 : 0;
     mp.n_traps = x->T;

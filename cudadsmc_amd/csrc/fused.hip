@@ -694,13 +694,14 @@ __device__ __forceinline__ void move_load(const MoveParams &mp, const FusedPtrs 
     m.kold = 0;
 }
 
+// Uniform reads of a constant table, as scalar loads.
+typedef const __attribute__((address_space(4))) float *ConstFloats;
+
 // The Bloch vector s rotated by the angle phi about the unit axis n
 // (Rodrigues): s cos phi + (n x s) sin phi + n (n . s)(1 - cos phi); the
 // precession of one spin substep, phi = gs muB |B| dt / hbar.
-__device__ __forceinline__ void rotate_about(const F3 &n, float phi, float &sx, float &sy, float &sz)
+__device__ __forceinline__ void rotate_by(const F3 &n, float sn, float cs, float &sx, float &sy, float &sz)
 {
-    float sn, cs;
-    sincos_f32(phi, &sn, &cs);
     const float nd = fmaf(n.x, sx, fmaf(n.y, sy, n.z * sz));
     const float kx = fmaf(n.y, sz, -(n.z * sy));
     const float ky = fmaf(n.z, sx, -(n.x * sz));
@@ -709,6 +710,45 @@ __device__ __forceinline__ void rotate_about(const F3 &n, float phi, float &sx, 
     sx = fmaf(sx, cs, fmaf(kx, sn, n.x * om));
     sy = fmaf(sy, cs, fmaf(ky, sn, n.y * om));
     sz = fmaf(sz, cs, fmaf(kz, sn, n.z * om));
+}
+
+// a / b with r = 1 / b: the quotient's remainder brings it to the rounded one.
+__device__ __forceinline__ double div_by(double a, double b, double r)
+{
+    const double q = a * r;
+    return fma(fma(-q, b, a), r, q);
+}
+
+// The spin substeps in a quadrupole, B ~ (x, y, -2 z), |B| = B' rho, with z
+// carried as -2 z (its square is the 4 z^2 of rho^2, to the same bits).  They
+// bound the move together with its memory traffic (N = 4e6: 93 us at 1 substep,
+// 123 to 139 at 20 by the clock the card holds, where it was 147 on the same
+// cards): 58 vector instructions a substep; with the range and zero tests, the
+// substep's time and compares for the quadrant in the loop it was 71.  Two
+// substeps per iteration save the copies of s; four are no faster.
+// GUARD: with the tests for the field's zero (or a NaN position), where the
+// spin is left as it is, and for angles beyond the reduction.
+template <bool GUARD>
+__device__ __forceinline__ void spin_quad(const MoveParams &mp, float dBdz, const FState &f, float &sx,
+                                          float &sy, float &sz)
+{
+    const ConstFloats taus = (ConstFloats)mp.spin_tau;
+    const float w = mp.f_spin_w;
+    const float pm2z = -2.0f * f.pz, vm2z = -2.0f * f.vz;
+#pragma unroll GUARD ? 1 : 2
+    for (int k = 0; k < mp.substeps; ++k) {
+        const float tau = taus[k];
+        const float x = fmaf(f.vx, tau, f.px), y = fmaf(f.vy, tau, f.py), m2z = fmaf(vm2z, tau, pm2z);
+        const float r2 = fmaf(x, x, fmaf(y, y, m2z * m2z));
+        const bool zero = GUARD && !(r2 > 0.0f);
+        const float inv = zero ? 0.0f : rsqrt_f(r2);
+        const F3 Bn = { x * inv, y * inv, zero ? 1.0f : m2z * inv };
+        const float phi = zero ? 0.0f : w * (dBdz * (r2 * inv));
+        float sn, cs;
+        if (GUARD) sincos_f32(phi, &sn, &cs);
+        else sincos_reduced(phi, &sn, &cs);
+        rotate_by(Bn, sn, cs, sx, sy, sz);
+    }
 }
 
 // Half a velocity kick, v += a dt / 2 (Kahan), with the trap's acceleration
@@ -746,35 +786,36 @@ __device__ __forceinline__ void move_update(const MoveParams &mp, const TrapDev 
     half_kick(tr, m.f, hdt);
 
     if (SPIN) {
-        const double dts = mp.dt / mp.substeps;
-        const float w = (float)(mp.gs * kMuB * dts / kHbar);
-        const float fdts = (float)dts;
         float sx = m.sx, sy = m.sy, sz = m.sz;
         if (tr.kind == kTrapQuad) {
-            // the quadrupole field inline: B ~ (x, y, -2 z), |B| = B' rho
-            const float dBdz = tr.f_dBdz;
-            for (int k = 0; k < mp.substeps; ++k) {
-                const float tau = mp.interp ? ((float)k + 0.5f) * fdts : 0.0f;
-                const float x = fmaf(m.f.vx, tau, m.f.px), y = fmaf(m.f.vy, tau, m.f.py),
-                            z = fmaf(m.f.vz, tau, m.f.pz);
-                const float r2 = fmaf(x, x, fmaf(y, y, 4.0f * (z * z)));
-                // at the field's zero (or a NaN position) no rotation, as field_dir_f
-                const bool zero = !(r2 > 0.0f);
-                const float inv = zero ? 0.0f : rsqrt_f(r2);
-                const F3 Bn = { x * inv, y * inv, zero ? 1.0f : (-2.0f * z) * inv };
-                rotate_about(Bn, zero ? 0.0f : w * (dBdz * (r2 * inv)), sx, sy, sz);
+            // every angle of the step is below w B' (|x| + |y| + 2 |z|) of the
+            // path's far end; a NaN afterwards is the field's zero (or a NaN
+            // that was there): both rare, and a wave with either runs the
+            // substeps with the tests in them
+            const float far = fmaf(fabsf(m.f.vx), dt, fabsf(m.f.px)) + fmaf(fabsf(m.f.vy), dt, fabsf(m.f.py)) +
+                              2.0f * fmaf(fabsf(m.f.vz), dt, fabsf(m.f.pz));
+            bool guard = __any(!(fabsf(mp.f_spin_w * tr.f_dBdz) * far * 1.0001f <= kSinCosReduceMax));
+            if (!guard) {
+                spin_quad<false>(mp, tr.f_dBdz, m.f, sx, sy, sz);
+                guard = __any(!(sx + sy + sz == sx + sy + sz));
+                if (guard) { sx = m.sx; sy = m.sy; sz = m.sz; }
             }
+            if (guard) spin_quad<true>(mp, tr.f_dBdz, m.f, sx, sy, sz);
         } else {
+            const ConstFloats taus = (ConstFloats)mp.spin_tau;
             for (int k = 0; k < mp.substeps; ++k) {
-                const float tau = mp.interp ? ((float)k + 0.5f) * fdts : 0.0f;
+                const float tau = taus[k];
                 F3 Bn;
                 const float Bm = field_dir_f(tr, fmaf(m.f.vx, tau, m.f.px), fmaf(m.f.vy, tau, m.f.py),
                                              fmaf(m.f.vz, tau, m.f.pz), Bn);
-                rotate_about(Bn, w * Bm, sx, sy, sz);
+                float sn, cs;
+                sincos_f32(mp.f_spin_w * Bm, &sn, &cs);
+                rotate_by(Bn, sn, cs, sx, sy, sz);
             }
         }
         const double L = sqrt((double)sx * sx + (double)sy * sy + (double)sz * sz);
-        m.sx = (float)((double)sx / L); m.sy = (float)((double)sy / L); m.sz = (float)((double)sz / L);
+        const double rL = 1.0 / L;
+        m.sx = (float)div_by(sx, L, rL); m.sy = (float)div_by(sy, L, rL); m.sz = (float)div_by(sz, L, rL);
     }
 
     kahan_fma(m.f.px, m.f.rpx, m.f.vx, dt);
@@ -1021,8 +1062,12 @@ __device__ __forceinline__ void wave_collide(const TrapDev *__restrict__ traps, 
 // updates, the block runs the collisions of its cells on an LDS copy of the
 // velocities (block_collide).
 // Without spin, two atoms per thread fit 80 registers: six waves per SIMD.
+// With spin, one atom per thread (the default) fits 64, eight waves: its
+// arithmetic and its memory traffic are about equal at 20 substeps and overlap
+// the better the more waves there are.
 template <int BS, int APT, bool SPIN, bool COLL>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(APT == 2 && !SPIN && !COLL ? 6 : 1)))
+__global__ __launch_bounds__(BS)
+    __attribute__((amdgpu_waves_per_eu(COLL ? 1 : SPIN ? (APT == 1 ? 8 : 1) : APT == 2 ? 6 : 1)))
 void k_move_fused(
     const TrapDev *__restrict__ traps, MoveParams mp, FusedPtrs A, FusedPtrs B,
     const uint32_t *__restrict__ perm, const int *__restrict__ trap_start,

@@ -104,12 +104,15 @@ constexpr int kAccDead = kAccN;
 struct MoveParams {
     double dt;
     double mass;
-    double gs;
     float  f_dt;
     float  f_half_mass;
+    // spin substeps: gs muB dt_s / hbar (the precession angle is this times
+    // |B|), and at spin_tau[k], k = 0 .. substeps, the time of substep k in the
+    // step, (k + 1/2) dt_s, or zero without interpolation
+    float  f_spin_w;
+    const float *spin_tau;
     int    spin;
     int    substeps;
-    int    interp;
     int    spin_loss;
     int    energy_cut;
     int    n_traps;

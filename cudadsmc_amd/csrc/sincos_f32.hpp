@@ -12,6 +12,7 @@
 #pragma once
 
 #include <cmath>
+#include <cstdint>
 
 #ifndef DSMC_HOST_DEVICE
 #if defined(__HIPCC__)
@@ -25,13 +26,13 @@ namespace dsmc {
 
 constexpr float kSinCosReduceMax = 8192.0f;
 
-DSMC_HOST_DEVICE inline void sincos_f32(float x, float *sp, float *cp)
+// For |x| <= kSinCosReduceMax.
+DSMC_HOST_DEVICE inline void sincos_reduced(float x, float *sp, float *cp)
 {
-    if (!(fabsf(x) <= kSinCosReduceMax)) {
-        sincosf(x, sp, cp);
-        return;
-    }
-    const float kf = rintf(x * 0.636619772f);            // nearest multiple of pi/2
+    // k = the multiple of pi/2 nearest to x: adding 3 2^22 rounds to a whole
+    // number and leaves k in the sum's low bits, which saves the conversion
+    const float big = x * 0.636619772f + 12582912.0f;
+    const float kf = big - 12582912.0f;
     float r = fmaf(-kf, 1.57079637e+00f, x);              // pi/2 = hi
     r = fmaf(-kf, -4.37113883e-08f, r);                   //      + mid
     r = fmaf(-kf, -1.71512451e-15f, r);                   //      + lo
@@ -46,12 +47,20 @@ DSMC_HOST_DEVICE inline void sincos_f32(float x, float *sp, float *cp)
                           -0.5f);
     const float c = fmaf(r2, pc, 1.0f);
     // quadrant k mod 4: odd k swaps sine and cosine; the sine changes sign
-    // for k = 2, 3 and the cosine for k = 1, 2 (mod 4)
-    const int q = (int)kf;
-    const bool swap = (q & 1) != 0;
-    const float sv = swap ? c : s, cv = swap ? s : c;
-    *sp = (q & 2) ? -sv : sv;
-    *cp = ((q + 1) & 2) ? -cv : cv;
+    // for k = 2, 3 and the cosine for k = 1, 2 (mod 4): bit 1 of k and of
+    // k + 1, moved to the sign bit
+    const uint32_t q30 = __builtin_bit_cast(uint32_t, big) << 30;
+    const uint32_t odd = (uint32_t)((int32_t)(q30 << 1) >> 31);
+    const uint32_t us = __builtin_bit_cast(uint32_t, s), uc = __builtin_bit_cast(uint32_t, c);
+    const uint32_t d = (us ^ uc) & odd, sv = us ^ d, cv = uc ^ d;
+    *sp = __builtin_bit_cast(float, sv ^ (q30 & 0x80000000u));
+    *cp = __builtin_bit_cast(float, cv ^ ((q30 + 0x40000000u) & 0x80000000u));
+}
+
+DSMC_HOST_DEVICE inline void sincos_f32(float x, float *sp, float *cp)
+{
+    if (fabsf(x) <= kSinCosReduceMax) sincos_reduced(x, sp, cp);
+    else sincosf(x, sp, cp);
 }
 
 }  // namespace dsmc

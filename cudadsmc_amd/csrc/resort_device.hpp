@@ -89,14 +89,17 @@ __device__ __forceinline__ void resort_list_block(const ResortList &rl, int j, u
         }
     }
     const int n = *rl.n_dev;
-    if (j > 0 && j * kListSlots >= n) return;   // whole block leaves together
+    if (j > 0 && j * kListSlots >= n) {         // whole block leaves together
+        if (tid < 2) rb.tile_moved[2 * j + tid] = rb.tile_dead[2 * j + tid] = 0u;   // (all tiles are summed)
+        return;
+    }
     // the words' movers and removed atoms (bits past the slots are zero)
     const uint32_t cnt = (uint32_t)__popcll(mm) << 16 | (uint32_t)__popcll(md);
     const uint32_t inc = wave_inclusive_scan(cnt);
     const uint32_t half = __shfl(inc, kTileWords - 1, kWave);   // the first tile's: words 0 .. 31
     if (tid == kTileWords - 1 || tid == kWave - 1) {
-        const uint32_t c = tid == kWave - 1 ? inc - half : inc;
         const int t = 2 * j + (tid == kWave - 1);
+        const uint32_t c = t > 0 && t * kStayTile >= n ? 0u : tid == kWave - 1 ? inc - half : inc;
         rb.tile_moved[t] = c >> 16;
         rb.tile_dead[t] = c & 0xFFFFu;
     }
@@ -149,10 +152,9 @@ __device__ __forceinline__ void resort_clear(const ResortBuckets &rb, int g, int
     for (int i = g; i < rb.n_counts; i += threads) rb.bcnt[i] = 0u;
 }
 
-// LDS of a merge block (256 threads): 17.4 KB, so that eight blocks fit a CU.
+// LDS of a merge block (256 threads): 16.3 KB, so that nine blocks fit a CU.
 struct MergeLds {
-    __align__(16) uint64_t kv[kBucketLds];      // the bucket's movers: key << 32 | slot
-    __align__(16) unsigned short q[kBucketLds]; // their insertion points in the tile
+    __align__(16) uint64_t kv[kBucketLds];      // the bucket's movers, key << 32 | slot, by insertion point
     uint32_t K[kStayTile];                      // the tile's keys of the last sort
     // movers inserted at each slot, then the scan E (below 2048 + kBucketLds)
     __align__(16) unsigned short H[kStayTile];
@@ -227,22 +229,52 @@ __device__ inline uint64_t *big_bucket_sort(uint64_t *a0, uint64_t *a1, int b, u
     return s;
 }
 
-// Sum of v[0 .. n), this thread's share (256 threads; v is 16-byte aligned).
+// The sum of the elements of c, elements i0 .. i0 + 3 of an array, below n.
+__device__ __forceinline__ uint32_t sum_below_n(uint4 c, int i0, int n)
+{
+    return (i0 < n ? c.x : 0u) + (i0 + 1 < n ? c.y : 0u) + (i0 + 2 < n ? c.z : 0u) + (i0 + 3 < n ? c.w : 0u);
+}
+
+// Sum of v[0 .. n), this thread's share (256 threads; v is 16-byte aligned
+// and ends on a multiple of four elements).
 __device__ __forceinline__ uint32_t sum_share(const uint32_t *__restrict__ v, int n)
 {
-    const int tid = threadIdx.x;
     const uint4 *v4 = (const uint4 *)v;
-    const int nv = n >> 2;
     uint32_t s = 0;
-    for (int v0 = tid; v0 < nv; v0 += 4 * 256) {
-        uint4 c[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) c[u] = v0 + u * 256 < nv ? v4[v0 + u * 256] : make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) s += c[u].x + c[u].y + c[u].z + c[u].w;
-    }
-    if (tid < (n & 3)) s += v[4 * nv + tid];
+    for (int i = (int)threadIdx.x; 4 * i < n; i += 256) s += sum_below_n(v4[i], 4 * i, n);
     return s;
+}
+
+// This thread's shares of the sums over the tiles (256 threads): movers
+// inserted before tile t less the movers and removed atoms that left its
+// earlier slots; removed atoms before it; and all.  The three arrays'
+// loads go out together, two words of each: one round of latency up to 4 M
+// slots (a loop per array, each waiting for its own, took four).
+__device__ __forceinline__ void tile_sums(const ResortBuckets &rb, bool may_remove, int t, int tiles,
+                                          uint32_t (&part)[3])
+{
+    const uint4 *ins = (const uint4 *)rb.bcnt, *mv = (const uint4 *)rb.tile_moved, *dd = (const uint4 *)rb.tile_dead;
+    const uint4 zero = make_uint4(0u, 0u, 0u, 0u);
+    part[0] = part[1] = part[2] = 0u;
+    const int end = may_remove ? tiles : t;
+    for (int i = (int)threadIdx.x; 4 * i < end; i += 2 * 256) {
+        uint4 a[2], b[2], c[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = 4 * (i + 256 * u);
+            a[u] = e < t ? ins[i + 256 * u] : zero;
+            b[u] = e < t ? mv[i + 256 * u] : zero;
+            c[u] = may_remove && e < end ? dd[i + 256 * u] : zero;
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = 4 * (i + 256 * u);
+            const uint32_t d = sum_below_n(c[u], e, t);
+            part[0] += sum_below_n(a[u], e, t) - sum_below_n(b[u], e, t) - d;
+            part[1] += d;
+            part[2] += sum_below_n(c[u], e, end);
+        }
+    }
 }
 
 // Block of 256 threads for tile t (2048 slots).  The tile's output is a
@@ -255,7 +287,11 @@ __device__ __forceinline__ uint32_t sum_share(const uint32_t *__restrict__ v, in
 // the last sort and a mover's comes with it, so the new keys are not read.
 // Buckets larger than the LDS table are sorted in global scratch by the
 // block; movers then go to w0 + (stays below p) + (rank in the bucket), stays
-// after the movers below them.
+// after the movers below them.  Bound by its chain of loads and barriers at
+// small N and by the O(b) work of the movers at large: the histogram's atomics
+// number the movers of a point, so that each is ranked among those alone
+// (comparing it with all b of the bucket, and the sums one after the other:
+// 11.2 us at N = 1e6, 7.8 at 2e4; now 8.3 and 6.8).
 constexpr int kMergePer = kStayTile / 256;   // slots per thread
 
 __device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t, MergeLds &L)
@@ -285,14 +321,8 @@ __device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t,
     const size_t fb0 = (size_t)t * kBucketCap;   // the bucket's fixed room
     constexpr int kFirst = 128;                  // movers loaded before the count is known
     const uint64_t mkv = tid < kFirst ? rb.room[fb0 + tid] : 0ull;
-    // movers inserted before the tile less the movers and removed atoms that
-    // left its earlier slots; removed atoms before it, and all
-    uint32_t part[3] = { sum_share(rb.bcnt, t) - sum_share(rb.tile_moved, t), 0u, 0u };
-    if (ra.may_remove) {
-        part[1] = sum_share(rb.tile_dead, t);
-        part[2] = sum_share(rb.tile_dead, (n + kStayTile - 1) >> kStayShift);
-        part[0] -= part[1];
-    }
+    uint32_t part[3];
+    tile_sums(rb, ra.may_remove, t, ra.tiles, part);
     if (t > 0 && g0 >= n) return;   // whole block leaves together
     const int ns = min(kStayTile, n - g0);   // slots of the tile
 #pragma unroll
@@ -384,13 +414,23 @@ __device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t,
         }
         return;
     }
-    for (int e = tid; e < b; e += 256) {
-        const uint64_t kv = e < kFirst ? mkv : rb.room[fb0 + e];
-        const uint32_t q = merge_point(L.K, ns, (uint32_t)g0, (uint32_t)(kv >> 32), (uint32_t)kv);
-        L.kv[e] = kv;
-        L.q[e] = (unsigned short)q;
-        if (q < (uint32_t)kStayTile) atomicAdd((uint32_t *)L.H + (q >> 1), 1u << (16 * (q & 1)));
-        else atomicAdd(&L.at_end, 1u);
+    // the movers stay in registers until their points' windows are known;
+    // `claim` numbers the movers of one point
+    constexpr int kMv = kBucketLds / 256;
+    uint64_t kv[kMv];
+    uint32_t q[kMv], claim[kMv];
+#pragma unroll
+    for (int u = 0; u < kMv; ++u) {
+        const int e = tid + 256 * u;
+        if (e >= b) continue;
+        kv[u] = e < kFirst ? mkv : rb.room[fb0 + e];
+        q[u] = merge_point(L.K, ns, (uint32_t)g0, (uint32_t)(kv[u] >> 32), (uint32_t)kv[u]);
+        if (q[u] < (uint32_t)kStayTile) {
+            const int sh = 16 * (q[u] & 1);
+            claim[u] = (atomicAdd((uint32_t *)L.H + (q[u] >> 1), 1u << sh) >> sh) & 0xFFFFu;
+        } else {
+            claim[u] = atomicAdd(&L.at_end, 1u);
+        }
     }
     __syncthreads();
     // E: exclusive scan of st(p) + h(p) over the tile, 8 consecutive
@@ -427,32 +467,29 @@ __device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t,
         if (p >= ns || !((L.stay[p >> 6] >> (p & 63)) & 1ull)) continue;
         put(w0 + (p + 1 < kStayTile ? L.H[p + 1] : total) - 1u, kk[u], (uint32_t)(g0 + p));
     }
-    for (int x = tid; x < b; x += 256) {
-        const uint32_t p = L.q[x];
-        uint32_t ep = total, hp = at_end;
+    // movers: those of one point beside each other in LDS, then each one's
+    // rank among them
+    uint32_t ep[kMv], at[kMv], hp[kMv];
+#pragma unroll
+    for (int u = 0; u < kMv; ++u) {
+        if (tid + 256 * u >= b) continue;
+        const uint32_t p = q[u];
+        ep[u] = total; hp[u] = at_end;
         if (p < (uint32_t)kStayTile) {
-            ep = L.H[p];
-            hp = (p + 1 < (uint32_t)kStayTile ? L.H[p + 1] : total) - ep -
-                 ((uint32_t)(L.stay[p >> 6] >> (p & 63)) & 1u);
+            ep[u] = L.H[p];
+            hp[u] = (p + 1 < (uint32_t)kStayTile ? L.H[p + 1] : total) - ep[u] -
+                    ((uint32_t)(L.stay[p >> 6] >> (p & 63)) & 1u);
         }
-        uint32_t r = 0;   // rank among the movers inserted at the same point
-        const uint64_t kx = L.kv[x];
-        if (hp > 1) {
-            // four movers per step, without branches: (key, slot) order is
-            // the order of key << 32 | slot
-            const ushort4 *lq4 = (const ushort4 *)L.q;
-            const ulonglong2 *k2 = (const ulonglong2 *)L.kv;
-#pragma unroll 2
-            for (int f = 0; f < b; f += 4) {
-                const ushort4 qq = lq4[f >> 2];
-                const ulonglong2 ka = k2[f >> 1], kb = k2[(f >> 1) + 1];
-                r += (uint32_t)((qq.x == p) & (ka.x < kx));
-                r += (uint32_t)((qq.y == p) & (ka.y < kx) & (f + 1 < b));
-                r += (uint32_t)((qq.z == p) & (kb.x < kx) & (f + 2 < b));
-                r += (uint32_t)((qq.w == p) & (kb.y < kx) & (f + 3 < b));
-            }
-        }
-        put(w0 + ep + r, (uint32_t)(kx >> 32), (uint32_t)kx);
+        at[u] = ep[u] - stays_below(p);   // movers inserted below p
+        L.kv[at[u] + claim[u]] = kv[u];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kMv; ++u) {
+        if (tid + 256 * u >= b) continue;
+        uint32_t r = 0;   // (key, slot) order is the order of key << 32 | slot
+        for (uint32_t f = 0; hp[u] > 1 && f < hp[u]; ++f) r += (uint32_t)(L.kv[at[u] + f] < kv[u]);
+        put(w0 + ep[u] + r, (uint32_t)(kv[u] >> 32), (uint32_t)kv[u]);
     }
 }
 

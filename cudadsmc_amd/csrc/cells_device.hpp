@@ -6,24 +6,25 @@
 
 namespace dsmc {
 
-constexpr int kCollItems = 8;                        // consecutive slots per lane
-constexpr int kCollChunk = kWave * kCollItems;       // slots per wave
-constexpr int kMaxCells = kCollChunk / 2;            // cells of >= 2 atoms that start in a chunk
 constexpr uint32_t kNoKey = 0xFFFFFFFFu;             // no slot there (keys are below 2^31)
-static_assert(kCollItems == 8, "a lane's keys are two 16-byte loads");
 
-// Cells of two or more atoms that start in a wave's chunk, in slot order.
+// Cells of two or more atoms that start in a wave's chunk of 64 ITEMS slots,
+// in slot order.
+template <int ITEMS>
 struct WaveCells {
-    uint32_t key[kMaxCells];
-    int      end[kMaxCells];     // slot after the cell's last
-    short    start[kMaxCells];   // first slot, from the chunk's
-    short    heavy[kMaxCells];   // (the collide's) cells run by the whole wave
+    static constexpr int kMax = kWave * ITEMS / 2;
+    uint32_t key[kMax];
+    int      end[kMax];     // slot after the cell's last
+    short    start[kMax];   // first slot, from the chunk's
+    short    heavy[kMax];   // (the collide's) cells run by the whole wave
 };
 
-// A chunk's keys: lane l holds slots chunk0 + 8 l .. + 7; the key before the
-// chunk, and slot chunk0 + kCollChunk + l (for the end of the last cell).
+// A chunk's keys: lane l holds slots chunk0 + ITEMS l .. + ITEMS - 1; the key
+// before the chunk, and the l-th slot after it (for the end of the last cell).
+template <int ITEMS>
 struct ChunkKeys {
-    uint32_t k[kCollItems];
+    static_assert(ITEMS == 2 || ITEMS == 4 || ITEMS == 8, "a lane's keys are whole loads");
+    uint32_t k[ITEMS];
     uint32_t before, after;
 };
 
@@ -36,20 +37,29 @@ __device__ __forceinline__ void wave_lds_fence()
 
 // Issues the chunk's loads (those below the capacity n_cap; the buffer is
 // 16-byte aligned).  Which slots are alive is not needed yet.
+template <int ITEMS>
 __device__ __forceinline__ void chunk_load(const uint32_t *__restrict__ key, int n_cap, int chunk0,
-                                           ChunkKeys &c)
+                                           ChunkKeys<ITEMS> &c)
 {
     const int lane = threadIdx.x & (kWave - 1);
-    const int b = chunk0 + lane * kCollItems;
-    if (b + kCollItems <= n_cap) {
-        const uint4 x = *(const uint4 *)(key + b), y = *(const uint4 *)(key + b + 4);
-        c.k[0] = x.x; c.k[1] = x.y; c.k[2] = x.z; c.k[3] = x.w;
-        c.k[4] = y.x; c.k[5] = y.y; c.k[6] = y.z; c.k[7] = y.w;
+    const int b = chunk0 + lane * ITEMS;
+    if (b + ITEMS <= n_cap) {
+        if constexpr (ITEMS == 8) {
+            const uint4 x = *(const uint4 *)(key + b), y = *(const uint4 *)(key + b + 4);
+            c.k[0] = x.x; c.k[1] = x.y; c.k[2] = x.z; c.k[3] = x.w;
+            c.k[4] = y.x; c.k[5] = y.y; c.k[6] = y.z; c.k[7] = y.w;
+        } else if constexpr (ITEMS == 4) {
+            const uint4 x = *(const uint4 *)(key + b);
+            c.k[0] = x.x; c.k[1] = x.y; c.k[2] = x.z; c.k[3] = x.w;
+        } else {
+            const uint2 x = *(const uint2 *)(key + b);
+            c.k[0] = x.x; c.k[1] = x.y;
+        }
     } else {
 #pragma unroll
-        for (int j = 0; j < kCollItems; ++j) c.k[j] = b + j < n_cap ? key[b + j] : kNoKey;
+        for (int j = 0; j < ITEMS; ++j) c.k[j] = b + j < n_cap ? key[b + j] : kNoKey;
     }
-    const int a = chunk0 + kCollChunk + lane;
+    const int a = chunk0 + kWave * ITEMS + lane;
     c.after = a < n_cap ? key[a] : kNoKey;
     c.before = chunk0 > 0 && chunk0 <= n_cap ? key[chunk0 - 1] : kNoKey;
 }
@@ -57,32 +67,33 @@ __device__ __forceinline__ void chunk_load(const uint32_t *__restrict__ key, int
 // Lists the cells of two or more atoms that start in the chunk (n alive
 // slots); returns their number.  k_first: key of the chunk's first slot,
 // k_last: of the last cell that starts in it.  Every lane of the wave calls
-// it.  A lane's eight slots are consecutive, so a cell's head, and mostly its
+// it.  A lane's slots are consecutive, so a cell's head, and mostly its
 // end, are found in the lane's own registers: five exchanges per wave where
 // slots dealt out 64 apart needed five for every eighth of the chunk.  That
 // was 40 % of a wave's time in the collide (N = 1e6 in one trap: collide
 // 16.3 -> 14.4 us, a group of 128 traps: 21.2 -> 19.6 us).
+template <int ITEMS>
 __device__ __forceinline__ int wave_list_cells(const uint32_t *__restrict__ key, int n, int chunk0,
-                                               ChunkKeys &c, WaveCells &L, uint32_t &k_first,
+                                               ChunkKeys<ITEMS> &c, WaveCells<ITEMS> &L, uint32_t &k_first,
                                                uint32_t &k_last)
 {
     const int lane = threadIdx.x & (kWave - 1);
-    const int b = chunk0 + lane * kCollItems;
-    const int chunk1 = min(n, chunk0 + kCollChunk);
+    const int b = chunk0 + lane * ITEMS;
+    const int chunk1 = min(n, chunk0 + kWave * ITEMS);
 #pragma unroll
-    for (int j = 0; j < kCollItems; ++j)
+    for (int j = 0; j < ITEMS; ++j)
         if (b + j >= n) c.k[j] = kNoKey;
-    if (chunk0 + kCollChunk + lane >= n) c.after = kNoKey;
-    uint32_t kp = __shfl_up(c.k[kCollItems - 1], 1, kWave), kn = __shfl_down(c.k[0], 1, kWave);
+    if (chunk0 + kWave * ITEMS + lane >= n) c.after = kNoKey;
+    uint32_t kp = __shfl_up(c.k[ITEMS - 1], 1, kWave), kn = __shfl_down(c.k[0], 1, kWave);
     const uint32_t k_after = __builtin_amdgcn_readfirstlane(c.after);
     if (lane == 0) kp = chunk0 <= n ? c.before : kNoKey;
     if (lane == kWave - 1) kn = k_after;
     // heads of all cells, and of those of two or more atoms, one bit per slot
     uint32_t hm = 0, mm = 0, kl = 0;
 #pragma unroll
-    for (int j = 0; j < kCollItems; ++j) {
+    for (int j = 0; j < ITEMS; ++j) {
         const uint32_t k = c.k[j], p = j > 0 ? c.k[j > 0 ? j - 1 : 0] : kp,
-                       x = j + 1 < kCollItems ? c.k[j + 1 < kCollItems ? j + 1 : j] : kn;
+                       x = j + 1 < ITEMS ? c.k[j + 1 < ITEMS ? j + 1 : j] : kn;
         const bool head = k != kNoKey && (k != p || b + j == 0);
         hm |= (uint32_t)head << j;
         mm |= (uint32_t)(head && x == k) << j;
@@ -97,7 +108,7 @@ __device__ __forceinline__ int wave_list_cells(const uint32_t *__restrict__ key,
     // outside the grid) is searched by galloping.
     int end;
     {
-        const uint64_t bd = __ballot(chunk1 == chunk0 + kCollChunk && c.after != kNoKey && c.after != k_last);
+        const uint64_t bd = __ballot(chunk1 == chunk0 + kWave * ITEMS && c.after != kNoKey && c.after != k_last);
         end = chunk1 + kWave;
         if (bd) end = chunk1 + __ffsll((unsigned long long)bd) - 1;
         if (chunk1 + kWave >= n) end = min(end, n);
@@ -120,16 +131,17 @@ __device__ __forceinline__ int wave_list_cells(const uint32_t *__restrict__ key,
     // places in the list: lanes list up to four cells each, counted bit by bit
     const uint32_t cnt = (uint32_t)__popc(mm);
     const uint64_t lt = lanemask_lt();
-    const uint64_t c0 = __ballot(cnt & 1u), c1 = __ballot(cnt & 2u), c2 = __ballot(cnt & 4u);
+    const uint64_t c0 = __ballot(cnt & 1u), c1 = ITEMS > 2 ? __ballot(cnt & 2u) : 0ull,
+                   c2 = ITEMS > 4 ? __ballot(cnt & 4u) : 0ull;
     int pos = __popcll(c0 & lt) + 2 * __popcll(c1 & lt) + 4 * __popcll(c2 & lt);
     const int nm = __popcll(c0) + 2 * __popcll(c1) + 4 * __popcll(c2);
 #pragma unroll
-    for (int j = 0; j < kCollItems; ++j) {
+    for (int j = 0; j < ITEMS; ++j) {
         if ((mm >> j) & 1u) {
             const uint32_t rest = hm >> (j + 1);
             L.key[pos] = c.k[j];
             L.end[pos] = rest ? b + j + __ffs((int)rest) : end;
-            L.start[pos] = (short)(lane * kCollItems + j);
+            L.start[pos] = (short)(lane * ITEMS + j);
             ++pos;
         }
     }

@@ -14,7 +14,7 @@
 //                           in primitives.hip) or by a full radix sort, after
 //                           which k_table_fused finds the trap ranges and the
 //                           alive count
-//   k_collide_fused      -> each wave scans 512 sorted slots for cells of two
+//   k_collide_fused      -> each wave scans 128 to 512 sorted slots for cells of two
 //                           or more atoms and runs their trials, velocities
 //                           read through the permutation (no reorder pass)
 //   k_move_fused         -> gathers state through the permutation into the
@@ -558,7 +558,7 @@ __device__ __forceinline__ int run_cell(const CollideParams &cp, const CellJob &
     return cnt;
 }
 
-// Each wave takes kWave * kCollItems consecutive sorted slots and runs the
+// Each wave takes kWave * ITEMS consecutive sorted slots and runs the
 // cells that start there (wave_list_cells), one cell of two or more atoms per
 // lane; cells with more than `wave_trials` trials are then run by the whole
 // wave.  When the chunk lies in one trap, its parameters are wave-uniform
@@ -566,7 +566,7 @@ __device__ __forceinline__ int run_cell(const CollideParams &cp, const CellJob &
 // its dependent loads (key, sigma v_r,max, permutation, velocities).  CB
 // threads per block (one or four waves); the waves share nothing but the
 // trap table, which a single trap does without (no block barrier then).
-template <int CB>
+template <int CB, int ITEMS>
 __global__ __launch_bounds__(CB, 5) void k_collide_fused(
     const TrapDev *__restrict__ traps, const int *__restrict__ key_base, int T, CollideParams cp,
     const uint32_t *__restrict__ key, const uint32_t *__restrict__ perm,
@@ -575,12 +575,12 @@ __global__ __launch_bounds__(CB, 5) void k_collide_fused(
     ResortBuckets rb, int wave_trials)
 {
     extern __shared__ int kb[];
-    __shared__ WaveCells cells[CB / kWave];
+    __shared__ WaveCells<ITEMS> cells[CB / kWave];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    const int chunk0 = (blockIdx.x * (CB / kWave) + w) * kCollChunk;
+    const int chunk0 = (blockIdx.x * (CB / kWave) + w) * kWave * ITEMS;
     const VelGlobal vg = { s.r, perm };
     const uint64_t lt = lanemask_lt();
-    WaveCells &L = cells[w];
+    WaveCells<ITEMS> &L = cells[w];
     // the keys are loaded with the alive count, the step and the trap table's
     // first 2 CB entries
     const int tb_j = (int)threadIdx.x;
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(CB, 5) void k_collide_fused(
         tb0 = tb_j < T + 1 ? key_base[tb_j] : 0;
         tb1 = tb_j + CB < T + 1 ? key_base[tb_j + CB] : 0;
     }
-    ChunkKeys ck;
+    ChunkKeys<ITEMS> ck;
     chunk_load(key, n_cap, chunk0, ck);
     const int n = *n_dev;
     const uint32_t step = (uint32_t)*step_dev;
@@ -1694,6 +1694,9 @@ void launch_cell_range_fused(const uint32_t *key, const int *n_dev, uint32_t dea
     DSMC_HIP(hipGetLastError());
 }
 
+// largest capacities for which a lane of the collide takes two and four slots
+constexpr int kCollTwo = 1 << 17, kCollFour = 3 << 17;
+
 void launch_collide_fused(const TrapDev *traps, const int *key_base, int n_traps,
                           const CollideParams &cp, const uint32_t *key, const uint32_t *perm,
                           const int *n_dev, const FusedPtrs &s, float *sigvrmax,
@@ -1706,21 +1709,28 @@ void launch_collide_fused(const TrapDev *traps, const int *key_base, int n_traps
     const char *env = std::getenv("DSMC_COLLIDE_WAVE_TRIALS");
     const int wave_trials = env ? std::atoi(env) : kWaveTrialsDefault;
     if (prof && prof->enabled) prof->begin(st, "collide_fused", (double)n_cap * 4.0);
-    // One wave per block when the context holds several traps: with trap
-    // groups stepped on two streams, one-wave blocks find room beside the
-    // other group's move blocks (batched step of two groups 157 -> 154 us on
-    // MI355X, bitwise the same results); a single trap's collide runs about
-    // 1 us faster in blocks of four waves.  Every block holds the trap table
-    // in LDS, so beyond 511 traps (a 2 KB table) one-wave blocks would put
-    // fewer than five waves on a SIMD, and four-wave blocks are used.
-    if (n_traps > 1 && n_traps + 1 <= 512)
-        hipLaunchKernelGGL(k_collide_fused<kWave>, dim3(fgrid(n_cap, kCollChunk)),
-                           dim3(kWave), lds, st, traps, key_base, n_traps, cp, key, perm, n_dev,
-                           n_cap, s, sigvrmax, coll_accum, step_dev, rb, wave_trials);
-    else
-        hipLaunchKernelGGL(k_collide_fused<kFBlock>, dim3(fgrid(n_cap, kFBlock * kCollItems)),
-                           dim3(kFBlock), lds, st, traps, key_base, n_traps, cp, key, perm, n_dev,
-                           n_cap, s, sigvrmax, coll_accum, step_dev, rb, wave_trials);
+    auto launch = [&](auto kernel, int block, int items) {
+        hipLaunchKernelGGL(kernel, dim3(fgrid(n_cap, block * items)), dim3(block), lds, st, traps, key_base, n_traps,
+                           cp, key, perm, n_dev, n_cap, s, sigvrmax, coll_accum, step_dev, rb, wave_trials);
+    };
+    // Slots per lane: a wave runs the cells of its slots 64 at a time, each
+    // round a chain of dependent loads, so with few slots the chip would sit
+    // idle while each wave goes through several rounds.  Two slots per lane
+    // make it one round, eight spread the cost of listing the cells (step in
+    // us, eight / four / two: N = 2e4 25.9 / 24.6 / 23.9, 5e4 27.0 / 25.2 /
+    // 24.4, 2e5 31.7 / 29.4 / 31.1, 1e6 53.2 / 53.8 / 55.7).
+    // Waves per block: one, beside the move blocks of another group of traps
+    // on its own stream (batched step of two groups 157 -> 154 us), and with
+    // four slots per lane (2e5 30.2 -> 29.4 us); a single trap's collide is
+    // faster in blocks of four waves with two slots (5e4 25.2 -> 24.4) and
+    // with eight (1e6 54.5 -> 53.2).  Every block holds the trap table in LDS,
+    // so beyond 511 traps (2 KB) one-wave blocks would put fewer than five
+    // waves on a SIMD.
+    const bool small_table = n_traps + 1 <= 512;
+    if (n_cap <= kCollTwo) launch(k_collide_fused<kFBlock, 2>, kFBlock, 2);
+    else if (n_cap <= kCollFour && small_table) launch(k_collide_fused<kWave, 4>, kWave, 4);
+    else if (n_traps > 1 && small_table) launch(k_collide_fused<kWave, 8>, kWave, 8);
+    else launch(k_collide_fused<kFBlock, 8>, kFBlock, 8);
     DSMC_HIP(hipGetLastError());
     if (prof && prof->enabled) prof->end(st);
 }

@@ -39,22 +39,23 @@ constexpr int kCollBlock = 256;
 
 // ---------------------------------------------------------------------------
 // collide (collisions.cu:291-445): the cells of two or more atoms of a wave's
-// 512 sorted slots, one per lane, trials in sequence.  Bound by its chain of
-// dependent loads (keys; sigma v_r,max and permutation; velocities): the
-// first trial's pair is loaded beside sigma v_r,max, before the trial count
-// that needs it.
+// 128 or 512 sorted slots, one per lane, trials in sequence.  Bound by its
+// chain of dependent loads (keys; sigma v_r,max and permutation; velocities):
+// the first trial's pair is loaded beside sigma v_r,max, before the trial
+// count that needs it.
 // ---------------------------------------------------------------------------
+template <int ITEMS>
 __global__ __launch_bounds__(kCollBlock) void k_collide_step(
     TrapDev t, CollideParams cp, const uint32_t *__restrict__ key, const uint32_t *__restrict__ perm,
     const PlainCtl *__restrict__ ctl, int n_cap, double *__restrict__ vx, double *__restrict__ vy,
     double *__restrict__ vz, double *__restrict__ sigvrmax, unsigned long long *__restrict__ cc,
     unsigned long long *__restrict__ coll_total, int *__restrict__ n_sorted, ResortBuckets rb)
 {
-    __shared__ WaveCells cells[kCollBlock / kWave];
+    __shared__ WaveCells<ITEMS> cells[kCollBlock / kWave];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    const int chunk0 = (blockIdx.x * (kCollBlock / kWave) + w) * kCollChunk;
-    WaveCells &L = cells[w];
-    ChunkKeys ck;
+    const int chunk0 = (blockIdx.x * (kCollBlock / kWave) + w) * kWave * ITEMS;
+    WaveCells<ITEMS> &L = cells[w];
+    ChunkKeys<ITEMS> ck;
     chunk_load(key, n_cap, chunk0, ck);
     const int n = ctl->alive;
     const uint32_t step = (uint32_t)ctl->step;
@@ -374,14 +375,23 @@ __global__ __launch_bounds__(256) void k_untag_counts(const unsigned long long *
 // ---------------------------------------------------------------------------
 // Host launchers.
 // ---------------------------------------------------------------------------
+constexpr int kCollTwo = 1 << 19;   // largest capacity for which a lane of the collide takes two slots
+
 void launch_collide_step(const TrapDev &t, const CollideParams &cp, const PlainPtrs &s, const uint32_t *key,
                          const uint32_t *perm, const PlainCtl *ctl, int n_cap, double *sigvrmax,
                          unsigned long long *cc, unsigned long long *coll_total, int *n_sorted,
                          const ResortBuckets &rb, hipStream_t st, Profiler *prof)
 {
-    DSMC_LAUNCH(prof, "collide_step", (double)n_cap * 4.0, k_collide_step,
-                div_up(n_cap > 0 ? n_cap : 1, kCollChunk * (kCollBlock / kWave)), kCollBlock, st, t, cp, key,
-                perm, ctl, n_cap, s.d[3], s.d[4], s.d[5], sigvrmax, cc, coll_total, n_sorted, rb);
+    auto launch = [&](auto kernel, int items) {
+        DSMC_LAUNCH(prof, "collide_step", (double)n_cap * 4.0, kernel,
+                    div_up(n_cap > 0 ? n_cap : 1, kCollBlock * items), kCollBlock, st, t, cp, key, perm, ctl,
+                    n_cap, s.d[3], s.d[4], s.d[5], sigvrmax, cc, coll_total, n_sorted, rb);
+    };
+    // two slots per lane while the chip has room for the waves (one round of
+    // cells each), eight beyond (step in us, eight / two: N = 1e4 23.5 / 21.2,
+    // 1e5 28.6 / 25.5, 4e5 38.9 / 37.4, 1e6 55.4 / 56.7)
+    if (n_cap <= kCollTwo) launch(k_collide_step<2>, 2);
+    else launch(k_collide_step<8>, 8);
 }
 
 void launch_move_step(bool spin, bool stored, const TrapDev &t, const PlainStepParams &p, const PlainPtrs &src,

@@ -21,6 +21,7 @@
 #include "../../include/dsmc.h"
 #include "dsmc_internal.hpp"
 #include "fused.hpp"
+#include "host_copy.hpp"
 #include "plain.hpp"
 #include "plain_step.hpp"
 #include "readout.hpp"
@@ -210,6 +211,7 @@ struct dsmc_ctx {
     // graph of two FP32 steps (parity 0 then 1)
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
+    HostCopy host_copy;
 
     template <typename T_>
     T_ *alloc(size_t count_, bool zero = true)
@@ -1210,9 +1212,7 @@ static void *stage(dsmc_ctx *x)
 
 static void to_host(dsmc_ctx *x, void *host, const void *dev, size_t bytes)
 {
-    if (!bytes) return;
-    DSMC_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, x->stream));
-    DSMC_HIP(hipStreamSynchronize(x->stream));
+    if (bytes) x->host_copy.to_host(host, dev, bytes, x->device, x->stream);
 }
 
 static size_t field_size(dsmc_ctx *x, int field, int n)

@@ -715,14 +715,27 @@ static void plain_enter(dsmc_ctx *x)
     x->bucketed = false;
 }
 
+// Small contexts re-sort in the finalize's launch; the next sort finds its
+// keys and permutation in the other sort buffer.
+static bool resort_early(const dsmc_ctx *x) { return x->n_cap <= kScanSlots; }
+
 // The first phase of the re-sort that follows a move of n slots with the new
-// keys key (x->bucketed: wanted), for the finalize's launch.
-static ResortList resort_first_phase(dsmc_ctx *x, const uint32_t *key, const int *n, const uint64_t *mask_dead)
+// keys key (x->bucketed: wanted), or the whole of it, for the finalize's launch.
+static ResortWork resort_work(dsmc_ctx *x, const uint32_t *key, const int *n, const uint64_t *mask_dead)
 {
-    if (!x->bucketed) return ResortList();
+    ResortWork w;
+    if (!x->bucketed) return w;
+    const bool may_remove = x->cfg.evaporation != 0;
+    if (resort_early(x)) {
+        w.merge = resort_merge_args(x->res, x->srt_k[x->srt_cur], n, x->dead_key, x->mask_moved, mask_dead,
+                                    may_remove, x->srt_k[x->srt_cur ^ 1], x->srt_v[x->srt_cur ^ 1]);
+        w.merge.key_new = key;
+        return w;
+    }
     if (!x->counts_clear) resort_clear_counts(x->res, x->stream, &x->prof);
     x->counts_clear = false;
-    return resort_list_args(x->res, key, n, x->mask_moved, mask_dead, x->cfg.evaporation != 0);
+    w.list = resort_list_args(x->res, key, n, x->mask_moved, mask_dead, may_remove);
+    return w;
 }
 
 // Substeps of one launch: their log records are written by different blocks,
@@ -740,7 +753,7 @@ static void plain_substeps(dsmc_ctx *x, int L)
     if (after) {
         uint32_t *ok = x->srt_k[x->srt_cur ^ 1], *ov = x->srt_v[x->srt_cur ^ 1];
         if (x->sorted_ok && x->bucketed) {
-            resort_merge(resort_merge_args(x->res, x->srt_k[x->srt_cur], &c->slots, x->dead_key, x->mask_moved,
+            if (!resort_early(x)) resort_merge(resort_merge_args(x->res, x->srt_k[x->srt_cur], &c->slots, x->dead_key, x->mask_moved,
                                            x->mask_d2[x->mpar], x->lazy_dead, ok, ov), x->stream, &x->prof);
         } else {
             if (!x->keys_ok)
@@ -782,9 +795,9 @@ static void plain_substeps(dsmc_ctx *x, int L)
                      x->evap_pos_d, x->evap_vel_d, x->rec64, step_rec_stride(x->n_cap), x->n_cap,
                      x->stream, &x->prof);
     x->bucketed = sorted && resort && phase + L == lpc;
-    const ResortList list = resort_first_phase(x, x->key_f, after ? &c->alive : &c->slots, x->mask_d2[x->mpar]);
+    const ResortWork work = resort_work(x, x->key_f, after ? &c->alive : &c->slots, x->mask_d2[x->mpar]);
     launch_step_finalize(p, after, x->rec64, step_rec_stride(x->n_cap), c, x->ctl + (x->csel ^ 1),
-                         x->coll_accum, x->evap_accum, x->obs_log, x->obs_cap, list, x->stream, &x->prof);
+                         x->coll_accum, x->evap_accum, x->obs_log, x->obs_cap, work, x->stream, &x->prof);
     x->csel ^= 1;
     if (after) {
         x->cur ^= 1;
@@ -842,7 +855,7 @@ static void fused_sort(dsmc_ctx *x)
     const int *n = x->n_dev + x->cur;
     uint32_t *ok = x->srt_k[x->srt_cur ^ 1], *ov = x->srt_v[x->srt_cur ^ 1];
     if (x->srt_valid && x->bucketed) {
-        resort_merge(resort_merge_args(x->res, x->srt_k[x->srt_cur], n, x->dead_key, x->mask_moved, x->mask_dead,
+        if (!resort_early(x)) resort_merge(resort_merge_args(x->res, x->srt_k[x->srt_cur], n, x->dead_key, x->mask_moved, x->mask_dead,
                                        x->dead_in_state, ok, ov), x->stream, &x->prof);
     } else {
         radix_sort(x->key_a, nullptr, x->res.alt_k, x->res.alt_v, ok, ov, n,
@@ -921,12 +934,12 @@ static void fused_move(dsmc_ctx *x, bool coll = false)
     // alive count (the removed atoms go to the end), and runs the first phase
     // of the incremental re-sort that follows
     x->bucketed = x->have_sort && x->cfg.sort_mode == DSMC_SORT_INCREMENTAL && resort_supported(x->n_cap);
-    const ResortList list = resort_first_phase(x, x->key_a, n, x->mask_dead);
+    const ResortWork work = resort_work(x, x->key_a, n, x->mask_dead);
     launch_obs_finalize(x->T, x->max_trap_atoms, x->block * x->apt, x->cfg.mass, x->trap_start(),
                         x->have_sort ? x->ts_buf[x->tsel ^ 1] : nullptr, x->blk_dead,
                         x->mask_dead, x->rec, x->coll_accum, x->step_dev(),
                         x->step_buf + (x->ssel ^ 1), x->obs_log, x->obs_cap,
-                        x->have_sort ? x->n_dev + x->cur : nullptr, list, x->stream, &x->prof);
+                        x->have_sort ? x->n_dev + x->cur : nullptr, work, x->stream, &x->prof);
     x->ssel ^= 1;
     if (x->have_sort) x->tsel ^= 1;
     if (!x->have_sort)  // keep the count with the state it describes

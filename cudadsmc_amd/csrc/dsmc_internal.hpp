@@ -140,6 +140,7 @@ struct ResortMerge {
     const int *n_dev = nullptr;
     int n_cap = 0, tiles = 0, may_remove = 1;
     uint32_t dead_key = 0;
+    const uint32_t *key_new = nullptr;   // (without a first phase) the new keys
     uint64_t *big = nullptr, *big_alt = nullptr;
     uint32_t *out_k = nullptr, *out_v = nullptr;
     uint32_t *tsamp_out = nullptr;
@@ -155,6 +156,19 @@ ResortMerge resort_merge_args(const ResortScratch &r, const uint32_t *key_old, c
                               uint32_t dead_key, const uint64_t *mask_m, const uint64_t *mask_d,
                               bool may_remove, uint32_t *out_k, uint32_t *out_v);
 void resort_merge(const ResortMerge &m, hipStream_t stream, Profiler *prof);
+// Largest capacity whose merge needs no first phase (its blocks read all the
+// masks and all the movers' new keys) and runs in the finalize's launch: three
+// launches a step instead of four, N = 2e3 21.1 -> 19.2 us, 1e4 23.2 -> 20.8,
+// 2e4 24.0 -> 22.1 (FP64 21.9 -> 20.2).  The gain shrinks with the movers that
+// every block reads, and two mask words per thread end here.
+constexpr int kScanSlots = 32768;
+// What a finalize launch runs beside its sums: the first phase of a re-sort,
+// a whole one (merge.tiles > 0), or neither.
+struct ResortWork {
+    ResortList list;
+    ResortMerge merge;
+    int blocks() const { return merge.tiles > 0 ? merge.tiles : list.blocks; }
+};
 // After a full sort: the first keys of the tiles of the sorted order.
 void resort_samples(const ResortScratch &r, const uint32_t *sorted, hipStream_t stream, Profiler *prof);
 // Clears the buckets' counts (a collide after the merge does it otherwise).

@@ -23,7 +23,8 @@
 //                           next cell key, FP64 observables per block
 //   k_obs_finalize       -> per-trap sums in fixed order and the log record,
 //                           the next trap ranges and alive count, and the
-//                           incremental re-sort's first phase
+//                           incremental re-sort's first phase, or for a
+//                           small context the whole re-sort
 // Every kernel reads the alive count and the step number from device memory,
 // so the loop can be captured once and replayed as a HIP graph.
 #include "cells_device.hpp"
@@ -1386,6 +1387,7 @@ __device__ __forceinline__ void stores_done()
 // waits for another.  Block
 // (0, 0) writes the next step number to the other counter.  Blocks from P T
 // on run the next incremental re-sort's first phase (resort_list_block).
+template <bool MERGE>
 __global__ __launch_bounds__(256) void k_obs_finalize(
     int T, int P, int move_block, double half_mass, const int *__restrict__ trap_start,
     int *__restrict__ trap_next, const uint32_t *__restrict__ blk_dead,
@@ -1394,15 +1396,18 @@ __global__ __launch_bounds__(256) void k_obs_finalize(
     unsigned int *__restrict__ cnt, double *__restrict__ acc_over,
     unsigned long long *__restrict__ coll_accum, const long long *__restrict__ step_cur,
     long long *__restrict__ step_next, dsmc_observables *__restrict__ obs_log, int obs_cap,
-    int *__restrict__ n_next, ResortList list)
+    int *__restrict__ n_next, ResortWork work)
 {
-    extern __shared__ __align__(16) uint32_t tile_first[];
+    extern __shared__ __align__(16) uint32_t lds[];   // first phase: tiles' first keys; merge: movers' slots
     __shared__ unsigned short list_slot[kListSlots];
+    __shared__ MergeLds merge_lds;
     __shared__ double red[(256 / kWave) * kAccK];
     __shared__ bool fin;
     __shared__ double part[kMaxFinalizeP * kAccK];   // partial sums of a trap's P blocks
     if ((int)blockIdx.x >= P * T) {
-        resort_list_block(list, (int)blockIdx.x - P * T, tile_first, list_slot);
+        const int j = (int)blockIdx.x - P * T;
+        if constexpr (MERGE) resort_scan_merge_block(work.merge, j, merge_lds, (unsigned short *)lds);
+        else resort_list_block(work.list, j, lds, list_slot);
         return;
     }
     const int p = (int)blockIdx.x % P, t = (int)blockIdx.x / P;
@@ -1923,17 +1928,17 @@ void launch_obs_finalize(int n_traps, int max_trap_atoms, int move_block, double
                          const uint64_t *mask_dead, const ObsRecords &rec,
                          unsigned long long *coll_accum, const long long *step_cur,
                          long long *step_next, dsmc_observables *obs_log, int obs_cap,
-                         int *n_next, const ResortList &list, hipStream_t st, Profiler *prof)
+                         int *n_next, const ResortWork &work, hipStream_t st, Profiler *prof)
 {
     // blocks per trap: about 256 move-block records each (a single block
     // summing thousands of records is a chain of dependent load rounds)
     const int blocks = div_up(max_trap_atoms > 0 ? max_trap_atoms : 1, move_block) + 1;
     const int P = std::min(kMaxFinalizeP, div_up(blocks, 256));
     if (prof && prof->enabled) prof->begin(st, "obs_finalize", (double)n_traps * 64.0);
-    hipLaunchKernelGGL(k_obs_finalize, dim3(P * n_traps + list.blocks), dim3(256), resort_list_lds(list), st,
-                       n_traps, P, move_block, 0.5 * mass, trap_start, trap_next, blk_dead, mask_dead,
+    hipLaunchKernelGGL(work.merge.tiles > 0 ? k_obs_finalize<true> : k_obs_finalize<false>,
+                       dim3(P * n_traps + work.blocks()), dim3(256), resort_work_lds(work), st, n_traps, P, move_block, 0.5 * mass, trap_start, trap_next, blk_dead, mask_dead,
                        (const int *)rec.trap, (const double *)rec.sum, rec.stride, rec.lvl2, rec.cnt,
-                       rec.acc_over, coll_accum, step_cur, step_next, obs_log, obs_cap, n_next, list);
+                       rec.acc_over, coll_accum, step_cur, step_next, obs_log, obs_cap, n_next, work);
     DSMC_HIP(hipGetLastError());
     if (prof && prof->enabled) prof->end(st);
 }

@@ -201,7 +201,7 @@ void launch_obs_finalize(int n_traps, int max_trap_atoms, int move_block, double
                          const uint64_t *mask_dead, const ObsRecords &rec,
                          unsigned long long *coll_accum, const long long *step_cur,
                          long long *step_next, dsmc_observables *obs_log, int obs_cap,
-                         int *n_next, const ResortList &list, hipStream_t st, Profiler *prof);
+                         int *n_next, const ResortWork &work, hipStream_t st, Profiler *prof);
 // Observables of the current state per trap into acc (kAccK doubles per
 // trap; kAccN = alive atoms), skipping slots with the dead key; a fixed-order
 // reduction.  first / last: n_traps ints of scratch each.

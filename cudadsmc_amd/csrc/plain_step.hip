@@ -272,17 +272,21 @@ static_assert(kMaxSub * 4 <= 64, "the block sums' threads");
 // Grid: one block per substep, then list.blocks blocks of the next re-sort's
 // first phase.  A block adds its substep's records over the move blocks (four
 // rounds of loads in flight per thread) in a fixed order.
+template <bool MERGE>
 __global__ __launch_bounds__(256) void k_step_finalize(
     int L, double half_mass, const int *__restrict__ n_dev, const double *__restrict__ rec, int stride,
     const PlainCtl *__restrict__ ctl, PlainCtl *__restrict__ next, int collided,
     unsigned long long *__restrict__ coll_accum, double *__restrict__ evap_accum,
-    dsmc_observables *__restrict__ log, int obs_cap, ResortList list)
+    dsmc_observables *__restrict__ log, int obs_cap, ResortWork work)
 {
-    extern __shared__ __align__(16) uint32_t tile_first[];
+    extern __shared__ __align__(16) uint32_t lds[];   // first phase: tiles' first keys; merge: movers' slots
     __shared__ unsigned short list_slot[kListSlots];
+    __shared__ MergeLds merge_lds;
     __shared__ double red[(256 / kWave) * 8];
     if ((int)blockIdx.x >= L) {
-        resort_list_block(list, (int)blockIdx.x - L, tile_first, list_slot);
+        const int j = (int)blockIdx.x - L;
+        if constexpr (MERGE) resort_scan_merge_block(work.merge, j, merge_lds, (unsigned short *)lds);
+        else resort_list_block(work.list, j, lds, list_slot);
         return;
     }
     const int l = (int)blockIdx.x;
@@ -413,13 +417,14 @@ void launch_move_step(bool spin, bool stored, const TrapDev &t, const PlainStepP
 
 void launch_step_finalize(const PlainStepParams &p, bool after_sort, const double *rec, int stride,
                           const PlainCtl *ctl, PlainCtl *next, unsigned long long *coll_accum,
-                          double *evap_accum, dsmc_observables *log, int obs_cap, const ResortList &list,
+                          double *evap_accum, dsmc_observables *log, int obs_cap, const ResortWork &work,
                           hipStream_t st, Profiler *prof)
 {
     if (prof && prof->enabled) prof->begin(st, "step_finalize", (double)p.L * stride * kStepRec * 8.0);
-    hipLaunchKernelGGL(k_step_finalize, dim3(p.L + list.blocks), dim3(256), resort_list_lds(list), st, p.L,
+    hipLaunchKernelGGL(work.merge.tiles > 0 ? k_step_finalize<true> : k_step_finalize<false>,
+                       dim3(p.L + work.blocks()), dim3(256), resort_work_lds(work), st, p.L,
                        0.5 * p.mass, after_sort ? &ctl->alive : &ctl->slots, rec, stride, ctl, next,
-                       after_sort ? 1 : 0, coll_accum, evap_accum, log, obs_cap, list);
+                       after_sort ? 1 : 0, coll_accum, evap_accum, log, obs_cap, work);
     DSMC_HIP(hipGetLastError());
     if (prof && prof->enabled) prof->end(st);
 }

@@ -58,7 +58,7 @@ inline int step_rec_stride(int n_cap) { return div_up(n_cap > 0 ? n_cap : 1, kSt
 // > 0) the next re-sort's first phase.
 void launch_step_finalize(const PlainStepParams &p, bool after_sort, const double *rec, int stride,
                           const PlainCtl *ctl, PlainCtl *next, unsigned long long *coll_accum,
-                          double *evap_accum, dsmc_observables *log, int obs_cap, const ResortList &list,
+                          double *evap_accum, dsmc_observables *log, int obs_cap, const ResortWork &work,
                           hipStream_t st, Profiler *prof);
 void launch_set_ctl(PlainCtl *ctl, long long step, unsigned coll, const int *n, hipStream_t st);
 // *n = the alive atoms of ctl.

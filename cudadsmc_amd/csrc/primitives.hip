@@ -270,6 +270,10 @@ void radix_sort(const uint32_t *keys, const uint32_t *vals, uint32_t *keys_alt, 
 //     of the tile below its point) + r.  The tile's removed atoms go to the
 //     end of the output, in slot order.  It also leaves the first key of
 //     every tile of the new order, for the next move.
+// Up to kScanSlots slots both run in the finalize's launch
+// (resort_scan_merge_block): a tile's block reads the masks and the movers'
+// new keys of all slots and keeps those of its bucket, so that nothing has to
+// be finished by other blocks first.
 // No kernel waits on another block.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_ins_merge(ResortMerge m)

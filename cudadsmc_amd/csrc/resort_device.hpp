@@ -66,6 +66,13 @@ inline size_t resort_list_lds(const ResortList &rl)
     return rl.blocks > 0 ? (((size_t)rl.tiles + 3) & ~(size_t)3) * sizeof(uint32_t) : 0;
 }
 
+// Dynamic LDS of a finalize with that work.
+inline size_t resort_work_lds(const ResortWork &w)
+{
+    return w.merge.tiles > 0 ? (((size_t)w.merge.n_cap + 7) & ~(size_t)7) * sizeof(unsigned short)
+                             : resort_list_lds(w.list);
+}
+
 // first: the dynamic LDS above; slot: the block's movers, from its first slot.
 __device__ __forceinline__ void resort_list_block(const ResortList &rl, int j, uint32_t *first,
                                                   unsigned short *slot)
@@ -277,6 +284,27 @@ __device__ __forceinline__ void tile_sums(const ResortBuckets &rb, bool may_remo
     }
 }
 
+// Of tile t's bucket: above the tile's first (key, slot) (or the first tile)
+// and not above the next tile's (if it has one).
+__device__ __forceinline__ bool in_bucket(int t, uint32_t f0, bool has1, uint32_t f1, uint64_t kv)
+{
+    const uint32_t k = (uint32_t)(kv >> 32), v = (uint32_t)kv;
+    const bool ge = t == 0 || kv_less(f0, (uint32_t)(t * kStayTile), k, v);
+    const bool lt = !has1 || !kv_less(f1, (uint32_t)((t + 1) * kStayTile), k, v);
+    return ge && lt;
+}
+
+constexpr int kMergePer = kStayTile / 256;   // slots per thread
+
+// What a merge block starts from.
+struct MergeTile {
+    uint32_t kk[kMergePer];   // keys of the last sort at positions tid + 256 u
+    uint64_t wm, wd;          // mask words (threads 0 .. 31)
+    uint32_t part[3];         // this thread's shares: movers inserted before the tile less the movers and
+                              // removed atoms that left its earlier slots; removed atoms before it; all
+    int n, b;                 // slots, and movers of the bucket
+};
+
 // Block of 256 threads for tile t (2048 slots).  The tile's output is a
 // contiguous window from w0: position p of the tile (slot g0 + p) is preceded
 // there by E(p) = the stays below p plus the bucket movers inserted below p,
@@ -292,38 +320,19 @@ __device__ __forceinline__ void tile_sums(const ResortBuckets &rb, bool may_remo
 // number the movers of a point, so that each is ranked among those alone
 // (comparing it with all b of the bucket, and the sums one after the other:
 // 11.2 us at N = 1e6, 7.8 at 2e4; now 8.3 and 6.8).
-constexpr int kMergePer = kStayTile / 256;   // slots per thread
-
-__device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t, MergeLds &L)
+// mover(e): the bucket's e-th mover, for e = tid, tid + 256 below kBucketLds;
+// gather(): all of a larger bucket's movers, in ra.big.
+template <class Mover, class Gather>
+__device__ __forceinline__ void merge_window(const ResortMerge &ra, int t, MergeLds &L, const MergeTile &mt,
+                                             Mover mover, Gather gather)
 {
-    const ResortBuckets &rb = ra.b;
     const int tid = threadIdx.x;
     const int g0 = t * kStayTile;
     const int p0 = tid * kMergePer;   // positions p0 .. p0 + 7 in the scan
-    // Every load that does not need the slot count is issued together with
-    // it, in one round: the tile's keys at positions tid + 256 u (coalesced;
-    // up to the capacity, those past the slots are never used), its mask
-    // words, the counts of the earlier tiles, its bucket's size, and this
-    // thread's first mover of the bucket's room (used when the bucket holds it).
-    uint32_t kk[kMergePer];
-#pragma unroll
-    for (int u = 0; u < kMergePer; ++u) {
-        const int p = tid + 256 * u;
-        kk[u] = g0 + p < ra.n_cap ? ra.key_old[g0 + p] : 0u;
-    }
-    const int n = *ra.n_dev;
-    const int b = (int)rb.bcnt[t];
-    uint64_t wm = 0ull, wd = 0ull;   // mask words of the tile (in bounds up to the last tile + 1)
-    if (tid < kTileWords) {
-        wm = ra.mask_m[(g0 >> 6) + tid];
-        wd = ra.mask_d[(g0 >> 6) + tid];
-    }
-    const size_t fb0 = (size_t)t * kBucketCap;   // the bucket's fixed room
-    constexpr int kFirst = 128;                  // movers loaded before the count is known
-    const uint64_t mkv = tid < kFirst ? rb.room[fb0 + tid] : 0ull;
-    uint32_t part[3];
-    tile_sums(rb, ra.may_remove, t, ra.tiles, part);
-    if (t > 0 && g0 >= n) return;   // whole block leaves together
+    const int n = mt.n, b = mt.b;
+    const uint32_t(&kk)[kMergePer] = mt.kk;
+    const uint64_t wm = mt.wm, wd = mt.wd;
+    uint32_t part[3] = { mt.part[0], mt.part[1], mt.part[2] };
     const int ns = min(kStayTile, n - g0);   // slots of the tile
 #pragma unroll
     for (int u = 0; u < kMergePer; ++u) L.K[tid + 256 * u] = kk[u];
@@ -370,30 +379,10 @@ __device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t,
         return L.wst[p >> 6] + (uint32_t)__popcll(m);
     };
     if (b > kBucketLds) {
-        // gather the bucket (its room, then its movers in the overflow list)
-        // in scratch, at the earlier buckets' movers, and sort it there
+        // the bucket gathered in scratch, at the earlier buckets' movers, and
+        // sorted there
         __syncthreads();   // the sums are read
-        uint32_t fs = wave_sum(sum_share(rb.bcnt, t));
-        if (lane == 0) L.sum[0][w] = fs;
-        if (tid == 0) L.n_big = min(b, kBucketCap);
-        __syncthreads();
-        const uint32_t at = total_of(0);
-        uint64_t *a = ra.big + at, *c = ra.big_alt + at;
-        for (int e = tid; e < min(b, kBucketCap); e += 256) a[e] = rb.room[fb0 + e];
-        if (b > kBucketCap) {
-            const int no = (int)*rb.n_over;
-            const bool has1 = g0 + kStayTile < n;   // (tsamp is being replaced by the merge)
-            const uint32_t f1 = has1 ? ra.key_old[g0 + kStayTile] : 0u;
-            for (int e = tid; e < no; e += 256) {
-                // of this bucket: above the tile's first (or the first tile)
-                // and not above the next tile's first
-                const uint64_t kv = rb.over[e];
-                const uint32_t k = (uint32_t)(kv >> 32), v = (uint32_t)kv;
-                const bool ge = t == 0 || kv_less(L.K[0], (uint32_t)g0, k, v);
-                const bool lt = !has1 || !kv_less(f1, (uint32_t)(g0 + kStayTile), k, v);
-                if (ge && lt) a[atomicAdd(&L.n_big, 1)] = kv;
-            }
-        }
+        uint64_t *const a = gather(), *const c = ra.big_alt + (a - ra.big);
         __syncthreads();
         const uint64_t *g = big_bucket_sort(a, c, b, L.kv);
         // a stay goes after the movers below it, found in the sorted bucket
@@ -423,7 +412,7 @@ __device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t,
     for (int u = 0; u < kMv; ++u) {
         const int e = tid + 256 * u;
         if (e >= b) continue;
-        kv[u] = e < kFirst ? mkv : rb.room[fb0 + e];
+        kv[u] = mover(e);
         q[u] = merge_point(L.K, ns, (uint32_t)g0, (uint32_t)(kv[u] >> 32), (uint32_t)kv[u]);
         if (q[u] < (uint32_t)kStayTile) {
             const int sh = 16 * (q[u] & 1);
@@ -491,6 +480,151 @@ __device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t,
         for (uint32_t f = 0; hp[u] > 1 && f < hp[u]; ++f) r += (uint32_t)(L.kv[at[u] + f] < kv[u]);
         put(w0 + ep[u] + r, (uint32_t)(kv[u] >> 32), (uint32_t)kv[u]);
     }
+}
+
+// After the first phase.
+__device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t, MergeLds &L)
+{
+    const ResortBuckets &rb = ra.b;
+    const int tid = threadIdx.x;
+    const int g0 = t * kStayTile;
+    // Every load that does not need the slot count is issued together with
+    // it, in one round: the tile's keys at positions tid + 256 u (coalesced;
+    // up to the capacity, those past the slots are never used), its mask
+    // words, the counts of the earlier tiles, its bucket's size, and this
+    // thread's first mover of the bucket's room (used when the bucket holds it).
+    MergeTile mt;
+#pragma unroll
+    for (int u = 0; u < kMergePer; ++u) {
+        const int p = tid + 256 * u;
+        mt.kk[u] = g0 + p < ra.n_cap ? ra.key_old[g0 + p] : 0u;
+    }
+    mt.n = *ra.n_dev;
+    mt.b = (int)rb.bcnt[t];
+    mt.wm = mt.wd = 0ull;   // (in bounds up to the last tile + 1)
+    if (tid < kTileWords) {
+        mt.wm = ra.mask_m[(g0 >> 6) + tid];
+        mt.wd = ra.mask_d[(g0 >> 6) + tid];
+    }
+    const size_t fb0 = (size_t)t * kBucketCap;   // the bucket's fixed room
+    constexpr int kFirst = 128;                  // movers loaded before the count is known
+    const uint64_t mkv = tid < kFirst ? rb.room[fb0 + tid] : 0ull;
+    tile_sums(rb, ra.may_remove, t, ra.tiles, mt.part);
+    if (t > 0 && g0 >= mt.n) return;   // whole block leaves together
+    auto mover = [&](int e) { return e < kFirst ? mkv : rb.room[fb0 + e]; };
+    // the bucket's room, then its movers in the overflow list
+    auto gather = [&]() {
+        const int lane = tid & (kWave - 1), w = tid / kWave;
+        const uint32_t fs = wave_sum(sum_share(rb.bcnt, t));
+        if (lane == 0) L.sum[0][w] = fs;
+        if (tid == 0) L.n_big = min(mt.b, kBucketCap);
+        __syncthreads();
+        uint64_t *const a = ra.big + (L.sum[0][0] + L.sum[0][1] + L.sum[0][2] + L.sum[0][3]);
+        for (int e = tid; e < min(mt.b, kBucketCap); e += 256) a[e] = rb.room[fb0 + e];
+        if (mt.b > kBucketCap) {
+            const int no = (int)*rb.n_over;
+            const bool has1 = g0 + kStayTile < mt.n;   // (tsamp is being replaced by the merge)
+            const uint32_t f1 = has1 ? ra.key_old[g0 + kStayTile] : 0u;
+            for (int e = tid; e < no; e += 256) {
+                const uint64_t kv = rb.over[e];
+                if (in_bucket(t, L.K[0], has1, f1, kv)) a[atomicAdd(&L.n_big, 1)] = kv;
+            }
+        }
+        return a;
+    };
+    merge_window(ra, t, L, mt, mover, gather);
+}
+
+// Without a first phase, for up to kScanSlots slots: every tile's block reads
+// the masks and the movers' new keys of all slots and keeps those of its
+// bucket.  list: the movers' slots (n_cap of them at most).
+__device__ __forceinline__ void resort_scan_merge_block(const ResortMerge &ra, int t, MergeLds &L,
+                                                        unsigned short *list)
+{
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+    const int g0 = t * kStayTile, g1 = g0 + kStayTile;
+    MergeTile mt;
+#pragma unroll
+    for (int u = 0; u < kMergePer; ++u) {
+        const int p = tid + 256 * u;
+        mt.kk[u] = g0 + p < ra.n_cap ? ra.key_old[g0 + p] : 0u;
+    }
+    const int n = *ra.n_dev;
+    const uint32_t f0 = g0 < ra.n_cap ? ra.key_old[g0] : 0u, f1 = g1 < ra.n_cap ? ra.key_old[g1] : 0u;
+    mt.wm = mt.wd = 0ull;
+    if (tid < kTileWords) {
+        mt.wm = ra.mask_m[(g0 >> 6) + tid];
+        mt.wd = ra.mask_d[(g0 >> 6) + tid];
+    }
+    // two words of the masks per thread
+    static_assert(kScanSlots == 2 * 256 * 64, "two words per thread");
+    uint64_t m[2], d[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int wl = 2 * tid + u;
+        m[u] = 64 * wl < ra.n_cap ? ra.mask_m[wl] : 0ull;
+        d[u] = 64 * wl < ra.n_cap && ra.may_remove ? ra.mask_d[wl] : 0ull;
+    }
+    if (t > 0 && g0 >= n) return;   // whole block leaves together
+    mt.n = n;
+    uint32_t moved = 0, gone_before = 0, gone = 0, moved_before = 0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int s0 = 64 * (2 * tid + u);
+        const uint64_t in = n - s0 >= 64 ? ~0ull : n > s0 ? (1ull << (n - s0)) - 1ull : 0ull;
+        m[u] &= in; d[u] &= in;
+        const uint32_t cm = (uint32_t)__popcll(m[u]), cd = (uint32_t)__popcll(d[u]);
+        moved += cm; gone += cd;
+        if (s0 < g0) { moved_before += cm; gone_before += cd; }
+    }
+    const uint32_t inc = wave_inclusive_scan(moved);
+    if (lane == kWave - 1) L.sum[0][w] = inc;
+    if (tid == 0) L.n_big = 0;
+    __syncthreads();
+    uint32_t at = inc - moved;
+    for (int ww = 0; ww < w; ++ww) at += L.sum[0][ww];
+    const int total = (int)(L.sum[0][0] + L.sum[0][1] + L.sum[0][2] + L.sum[0][3]);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        for (uint64_t bits = m[u]; bits; bits &= bits - 1)
+            list[at++] = (unsigned short)(64 * (2 * tid + u) + __ffsll((unsigned long long)bits) - 1);
+    __syncthreads();
+    const bool has1 = g1 < n;
+    uint32_t below = 0;   // movers inserted before the tile (this thread's)
+#pragma unroll 4
+    for (int e = tid; e < total; e += 256) {
+        const uint32_t v = list[e], k = ra.key_new[v];
+        const uint64_t kv = (uint64_t)k << 32 | v;
+        if (in_bucket(t, f0, has1, f1, kv)) {
+            const int x = atomicAdd(&L.n_big, 1);
+            if (x < kBucketLds) L.kv[x] = kv;
+        } else if (t > 0 && !kv_less(f0, (uint32_t)g0, k, v)) {
+            ++below;
+        }
+    }
+    mt.part[0] = below - moved_before - gone_before;
+    mt.part[1] = gone_before;
+    mt.part[2] = gone;
+    __syncthreads();
+    mt.b = L.n_big;
+    uint64_t mine[kBucketLds / 256];
+#pragma unroll
+    for (int u = 0; u < kBucketLds / 256; ++u) mine[u] = tid + 256 * u < mt.b ? L.kv[tid + 256 * u] : 0ull;
+    auto mover = [&](int e) { return e < 256 ? mine[0] : mine[1]; };
+    auto gather = [&]() {
+        const uint32_t s = wave_sum(below);
+        if (lane == 0) L.sum[0][w] = s;
+        if (tid == 0) L.n_big = 0;
+        __syncthreads();
+        uint64_t *const a = ra.big + (L.sum[0][0] + L.sum[0][1] + L.sum[0][2] + L.sum[0][3]);
+        for (int e = tid; e < total; e += 256) {
+            const uint32_t v = list[e];
+            const uint64_t kv = (uint64_t)ra.key_new[v] << 32 | v;
+            if (in_bucket(t, f0, has1, f1, kv)) a[atomicAdd(&L.n_big, 1)] = kv;
+        }
+        return a;
+    };
+    merge_window(ra, t, L, mt, mover, gather);
 }
 
 }  // namespace dsmc

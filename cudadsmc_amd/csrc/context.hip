@@ -108,6 +108,19 @@ Profiler::~Profiler()
 
 static void free_kept();   // scratch kept between the primitives' calls
 
+// A captured run of steps.
+struct StepGraph {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    void destroy()
+    {
+        if (exec) (void)hipGraphExecDestroy(exec);
+        if (graph) (void)hipGraphDestroy(graph);
+        exec = nullptr;
+        graph = nullptr;
+    }
+};
+
 struct dsmc_ctx {
     dsmc_config cfg{};
     std::vector<dsmc_trap> traps;
@@ -208,9 +221,9 @@ struct dsmc_ctx {
     int max_trap_atoms = 0;
     float *evap_pos_f = nullptr, *evap_vel_f = nullptr;
     float *spin_tau = nullptr;   // (spin) the substeps' times in a step
-    // graph of two FP32 steps (parity 0 then 1)
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
+    // captured steps (FP32: parity 0 then 1)
+    StepGraph graphs[2];            // of one pair of steps and of kLongPairs
+    int pairs_run = 0;              // pairs of steps replayed since they were captured (up to kLongFrom)
     HostCopy host_copy;
 
     template <typename T_>
@@ -232,8 +245,7 @@ struct dsmc_ctx {
     {
         // drain the stream before destroying a graph it may still be running
         if (stream) (void)hipStreamSynchronize(stream);
-        if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-        if (graph) (void)hipGraphDestroy(graph);
+        for (StepGraph &g : graphs) g.destroy();
         for (void *p : allocs) (void)hipFree(p);
         if (n_host) (void)hipHostFree(n_host);
         if (obs_host) (void)hipHostFree(obs_host);
@@ -976,15 +988,13 @@ static bool graph_ok(const dsmc_ctx *x) { return x->cfg.use_graph && !x->prof.en
 // destroyed while the device may still run it.
 static void drop_graph(dsmc_ctx *x)
 {
-    if (!x->graph_exec && !x->graph) return;
+    x->pairs_run = 0;
+    if (!x->graphs[0].graph && !x->graphs[1].graph) return;
     DSMC_HIP(hipStreamSynchronize(x->stream));
-    if (x->graph_exec) (void)hipGraphExecDestroy(x->graph_exec);
-    if (x->graph) (void)hipGraphDestroy(x->graph);
-    x->graph_exec = nullptr;
-    x->graph = nullptr;
+    for (StepGraph &g : x->graphs) g.destroy();
 }
 
-// The steps of one graph: two FP32 steps, or two collision steps of the FP64
+// The steps of one pair: two FP32 steps, or two collision steps of the FP64
 // form.  Every double buffer is back where it was after them.
 static int graph_len(const dsmc_ctx *x) { return x->fp32 ? 2 : 2 * x->cfg.lpc; }
 
@@ -1003,33 +1013,53 @@ static void graph_body(dsmc_ctx *x)
         }
 }
 
+// One graph launch leaves the device idle for some 5 us, so a long graph of
+// kLongPairs pairs replays them 2.2 us a step faster than pair by pair (N = 2e4
+// 22.0 -> 19.8 us a step, 1e6 53.7 -> 51.4; four pairs 20.2 and 51.9).  Its
+// capture costs 145 us more, what kLongFrom pairs gain: it is captured once a
+// context has replayed so many (those of the present call counted), so that no
+// run loses more by it than it would have without.
+constexpr int kLongPairs = 8, kLongFrom = 32;
+
+// Captures `pairs` pairs of steps, unless there already.
+static void capture_steps(dsmc_ctx *x, StepGraph &g, int pairs)
+{
+    if (g.exec) return;
+    g.destroy();   // (what a failed instantiation left)
+    DSMC_HIP(hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
+    try {
+        for (int k = 0; k < pairs; ++k) graph_body(x);
+    } catch (...) {
+        hipGraph_t broken = nullptr;
+        (void)hipStreamEndCapture(x->stream, &broken);
+        if (broken) (void)hipGraphDestroy(broken);
+        throw;
+    }
+    DSMC_HIP(hipStreamEndCapture(x->stream, &g.graph));
+    DSMC_HIP(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
+}
+
+// `times` pairs of steps.
 static void graph_steps(dsmc_ctx *x, int times)
 {
     const int ssel = x->fp32 ? x->ssel : x->csel, tsel = x->fp32 ? x->tsel : x->mpar;
-    if (x->graph_exec && (x->graph_srt != x->srt_cur || x->graph_ssel != ssel ||
-                          x->graph_tsel != tsel || x->graph_cur != x->cur)) {
+    if ((x->graphs[0].graph || x->graphs[1].graph) &&
+        (x->graph_srt != x->srt_cur || x->graph_ssel != ssel || x->graph_tsel != tsel || x->graph_cur != x->cur)) {
         // captured with the other sort (step, trap-range) buffer current
         drop_graph(x);
     }
     const long long step0 = x->step, cs0 = x->coll_steps;
-    if (!x->graph_exec) {
-        x->graph_srt = x->srt_cur;
-        x->graph_ssel = ssel;
-        x->graph_tsel = tsel;
-        x->graph_cur = x->cur;
-        DSMC_HIP(hipStreamBeginCapture(x->stream, hipStreamCaptureModeThreadLocal));
-        try {
-            graph_body(x);
-        } catch (...) {
-            hipGraph_t g;
-            (void)hipStreamEndCapture(x->stream, &g);
-            if (g) (void)hipGraphDestroy(g);
-            throw;
-        }
-        DSMC_HIP(hipStreamEndCapture(x->stream, &x->graph));
-        DSMC_HIP(hipGraphInstantiate(&x->graph_exec, x->graph, nullptr, nullptr, 0));
-    }
-    for (int k = 0; k < times; ++k) DSMC_HIP(hipGraphLaunch(x->graph_exec, x->stream));
+    x->graph_srt = x->srt_cur;
+    x->graph_ssel = ssel;
+    x->graph_tsel = tsel;
+    x->graph_cur = x->cur;
+    x->pairs_run = (int)std::min<long long>(kLongFrom, (long long)x->pairs_run + times);
+    const int longs = x->pairs_run >= kLongFrom || x->graphs[1].exec ? times / kLongPairs : 0;
+    const int singles = times - longs * kLongPairs;
+    if (longs > 0) capture_steps(x, x->graphs[1], kLongPairs);
+    if (singles > 0) capture_steps(x, x->graphs[0], 1);
+    for (int k = 0; k < longs; ++k) DSMC_HIP(hipGraphLaunch(x->graphs[1].exec, x->stream));
+    for (int k = 0; k < singles; ++k) DSMC_HIP(hipGraphLaunch(x->graphs[0].exec, x->stream));
     x->step = step0 + (long long)graph_len(x) * times;
     x->coll_steps = cs0 + 2LL * times;
     if (!x->fp32) {

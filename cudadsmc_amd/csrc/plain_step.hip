@@ -6,7 +6,8 @@
 // launches a step at lpc = 1 and 11 to 13 per motion step in the reference's
 // run.  At N = 1e4 that is launch latency (68 and 40 us a motion step), at 1e6
 // the state crosses memory some six times (188 us).  Here a collision step is
-// four launches whatever lpc is:
+// four launches whatever lpc is (three where the finalize's launch holds the
+// whole sort, up to kScanSlots atoms):
 //   k_ins_merge                the stable sort by (cell, slot) from the last
 //                              one (primitives.hip): the same permutation as
 //                              the radix sort's

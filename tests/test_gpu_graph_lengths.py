@@ -1,0 +1,42 @@
+"""Steps replayed from the captured pair of steps, from the long graph of eight
+pairs and from both, against the same steps launched one by one, bitwise after
+every call: calls below, at and above one pair, eight pairs and the number of
+pairs from which the long graph is used, odd ones (which leave the buffers the
+other way round), reads and single steps in between, and a re-initialised
+context; with and without removed atoms, with the re-sort in the finalize's
+launch and outside it."""
+import numpy as np
+import pytest
+
+from cudadsmc_amd import Simulation, _abi, configs
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = [_abi.FIELD_ATOM_ID, _abi.FIELD_POS, _abi.FIELD_VEL, _abi.FIELD_CELL_ID, _abi.FIELD_PERM,
+          _abi.FIELD_SIGVRMAX]
+CALLS = [1, 2, 14, 16, 15, 17, 64, 1, 33, 130, 3, 62, 16]
+
+
+@pytest.mark.parametrize("n", [500, 40000])
+@pytest.mark.parametrize("precision,lpc,cut", [("fp32", 1, False), ("fp32", 1, True), ("fp64", 1, True),
+                                               ("fp64", 3, False), ("fp64", 17, True)])
+def test_replayed_steps_equal_launched_steps(n, precision, lpc, cut):
+    trap = configs.quadrupole_trap(n, 9, n_real=1e9)
+    if cut:
+        trap.eta_start, trap.eta_end, trap.T_cut, trap.eta_steps = 7.0, 4.0, trap.T, 300
+    run = configs.Run(traps=[trap], precision=precision, energy_cut=cut, lpc=lpc, dt=1e-6, seed=11)
+    with Simulation(run.with_(use_graph=True)) as a, Simulation(run.with_(use_graph=False)) as b:
+        for again in range(2):
+            a.init_distribution()
+            b.init_distribution()
+            for k, steps in enumerate(CALLS if again == 0 else [200, 40]):
+                steps *= lpc
+                a.step(steps)
+                b.step(steps)
+                if k % 3 == 1:
+                    continue
+                for f in FIELDS:
+                    np.testing.assert_array_equal(a.copy_out(f), b.copy_out(f), err_msg=f"field {f}, call {k}")
+                la, lb = a.obs_log(), b.obs_log()
+                for f in la.dtype.names:
+                    np.testing.assert_array_equal(la[f], lb[f], err_msg=f)

@@ -121,6 +121,24 @@ struct StepGraph {
     }
 };
 
+// The captured runs of steps for one state of the double buffers: of one pair
+// of steps, and of kLongPairs pairs.
+struct StepGraphs {
+    int srt = 0, ssel = 0, tsel = 0, cur = 0;   // the buffers current at the capture
+    StepGraph one, many;
+    int pairs_run = 0;   // pairs replayed (up to kLongFrom)
+    bool same(const StepGraphs &o) const
+    {
+        return srt == o.srt && ssel == o.ssel && tsel == o.tsel && cur == o.cur;
+    }
+    void destroy()
+    {
+        one.destroy();
+        many.destroy();
+        pairs_run = 0;
+    }
+};
+
 struct dsmc_ctx {
     dsmc_config cfg{};
     std::vector<dsmc_trap> traps;
@@ -155,8 +173,6 @@ struct dsmc_ctx {
     uint32_t *key_a = nullptr, *key_b = nullptr, *val_a = nullptr, *val_b = nullptr;
     uint32_t *srt_k[2] = {nullptr, nullptr}, *srt_v[2] = {nullptr, nullptr};  // FP32 sort outputs
     int srt_cur = 0;                // FP32: srt_*[srt_cur] holds the last sort's result
-    int graph_srt = 0;              // srt_cur at graph capture
-    int graph_ssel = 0, graph_tsel = 0, graph_cur = 0;   // other buffers' parities at graph capture
     bool bucketed = false;          // the last finalize ran the re-sort's first phase
     bool counts_clear = true;       // the buckets' counts are zero (a collide clears them)
     bool split_step = true;         // FP32: dsmc_step runs collide and move as two kernels
@@ -221,9 +237,10 @@ struct dsmc_ctx {
     int max_trap_atoms = 0;
     float *evap_pos_f = nullptr, *evap_vel_f = nullptr;
     float *spin_tau = nullptr;   // (spin) the substeps' times in a step
-    // captured steps (FP32: parity 0 then 1)
-    StepGraph graphs[2];            // of one pair of steps and of kLongPairs
-    int pairs_run = 0;              // pairs of steps replayed since they were captured (up to kLongFrom)
+    // captured steps (FP32: parity 0 then 1), the last used first.  Two: reads
+    // of a run with losses swap the FP64 state's buffers, so runs with a read
+    // after each come by two states in turn
+    StepGraphs graphs[2];
     HostCopy host_copy;
 
     template <typename T_>
@@ -245,7 +262,7 @@ struct dsmc_ctx {
     {
         // drain the stream before destroying a graph it may still be running
         if (stream) (void)hipStreamSynchronize(stream);
-        for (StepGraph &g : graphs) g.destroy();
+        for (StepGraphs &g : graphs) g.destroy();
         for (void *p : allocs) (void)hipFree(p);
         if (n_host) (void)hipHostFree(n_host);
         if (obs_host) (void)hipHostFree(obs_host);
@@ -983,15 +1000,13 @@ static void fused_step(dsmc_ctx *x)
 
 static bool graph_ok(const dsmc_ctx *x) { return x->cfg.use_graph && !x->prof.enabled; }
 
-// Destroy the captured graph.  Its earlier launches may still be in flight on
-// the stream, so the stream is drained first: an executable graph is not
+// Destroy the captured graphs.  Their earlier launches may still be in flight
+// on the stream, so the stream is drained first: an executable graph is not
 // destroyed while the device may still run it.
-static void drop_graph(dsmc_ctx *x)
+static void drop_graphs(dsmc_ctx *x)
 {
-    x->pairs_run = 0;
-    if (!x->graphs[0].graph && !x->graphs[1].graph) return;
     DSMC_HIP(hipStreamSynchronize(x->stream));
-    for (StepGraph &g : x->graphs) g.destroy();
+    for (StepGraphs &g : x->graphs) g.destroy();
 }
 
 // The steps of one pair: two FP32 steps, or two collision steps of the FP64
@@ -1042,24 +1057,28 @@ static void capture_steps(dsmc_ctx *x, StepGraph &g, int pairs)
 // `times` pairs of steps.
 static void graph_steps(dsmc_ctx *x, int times)
 {
-    const int ssel = x->fp32 ? x->ssel : x->csel, tsel = x->fp32 ? x->tsel : x->mpar;
-    if ((x->graphs[0].graph || x->graphs[1].graph) &&
-        (x->graph_srt != x->srt_cur || x->graph_ssel != ssel || x->graph_tsel != tsel || x->graph_cur != x->cur)) {
-        // captured with the other sort (step, trap-range) buffer current
-        drop_graph(x);
+    StepGraphs now;
+    now.srt = x->srt_cur;
+    now.ssel = x->fp32 ? x->ssel : x->csel;
+    now.tsel = x->fp32 ? x->tsel : x->mpar;
+    now.cur = x->cur;
+    if (!x->graphs[0].same(now)) {
+        std::swap(x->graphs[0], x->graphs[1]);
+        if (!x->graphs[0].same(now)) {   // captured with other buffers current than these
+            DSMC_HIP(hipStreamSynchronize(x->stream));
+            x->graphs[0].destroy();
+            x->graphs[0] = now;
+        }
     }
+    StepGraphs &g = x->graphs[0];
     const long long step0 = x->step, cs0 = x->coll_steps;
-    x->graph_srt = x->srt_cur;
-    x->graph_ssel = ssel;
-    x->graph_tsel = tsel;
-    x->graph_cur = x->cur;
-    x->pairs_run = (int)std::min<long long>(kLongFrom, (long long)x->pairs_run + times);
-    const int longs = x->pairs_run >= kLongFrom || x->graphs[1].exec ? times / kLongPairs : 0;
+    g.pairs_run = (int)std::min<long long>(kLongFrom, (long long)g.pairs_run + times);
+    const int longs = g.pairs_run >= kLongFrom ? times / kLongPairs : 0;
     const int singles = times - longs * kLongPairs;
-    if (longs > 0) capture_steps(x, x->graphs[1], kLongPairs);
-    if (singles > 0) capture_steps(x, x->graphs[0], 1);
-    for (int k = 0; k < longs; ++k) DSMC_HIP(hipGraphLaunch(x->graphs[1].exec, x->stream));
-    for (int k = 0; k < singles; ++k) DSMC_HIP(hipGraphLaunch(x->graphs[0].exec, x->stream));
+    if (longs > 0) capture_steps(x, g.many, kLongPairs);
+    if (singles > 0) capture_steps(x, g.one, 1);
+    for (int k = 0; k < longs; ++k) DSMC_HIP(hipGraphLaunch(g.many.exec, x->stream));
+    for (int k = 0; k < singles; ++k) DSMC_HIP(hipGraphLaunch(g.one.exec, x->stream));
     x->step = step0 + (long long)graph_len(x) * times;
     x->coll_steps = cs0 + 2LL * times;
     if (!x->fp32) {
@@ -2132,7 +2151,7 @@ dsmc_status dsmc_autotune(dsmc_ctx *ctx, int *block_size_out)
     DSMC_HIP(hipStreamSynchronize(ctx->stream));
     if (mp.count_moved) ctx->srt_valid = false;
     if (ctx->block != best_bs || ctx->apt != best_apt) {
-        drop_graph(ctx);
+        drop_graphs(ctx);
         // the per-block counts of the last move are for the old block size
         ctx->srt_valid = false;
     }

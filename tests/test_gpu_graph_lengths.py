@@ -40,3 +40,20 @@ def test_replayed_steps_equal_launched_steps(n, precision, lpc, cut):
                 la, lb = a.obs_log(), b.obs_log()
                 for f in la.dtype.names:
                     np.testing.assert_array_equal(la[f], lb[f], err_msg=f)
+
+
+def test_runs_with_reads_between():
+    """Reads of a run with losses swap the state's buffers: two captured states
+    in turn, and a third (an odd number of steps) in place of the older."""
+    trap = configs.quadrupole_trap(3000, 9, n_real=1e9)
+    trap.eta_start, trap.eta_end, trap.T_cut, trap.eta_steps = 6.0, 3.0, trap.T, 2000
+    run = configs.Run(traps=[trap], precision="fp64", energy_cut=True, dt=1e-6, seed=5)
+    with Simulation(run.with_(use_graph=True)) as a, Simulation(run.with_(use_graph=False)) as b:
+        a.init_distribution()
+        b.init_distribution()
+        for steps in [40, 40, 40, 80, 80, 41, 40, 40, 43, 90, 90, 90, 90]:
+            a.step(steps)
+            b.step(steps)
+            for f in FIELDS:
+                np.testing.assert_array_equal(a.copy_out(f), b.copy_out(f))
+        assert a.info().n_alive == b.info().n_alive < 3000

@@ -24,8 +24,9 @@ namespace dsmc {
 // Radix sort
 // ---------------------------------------------------------------------------
 // One pass over digits of B bits: BLOCK threads take a tile of BLOCK * ITEMS
-// pairs.  n_dev: the pair count on the device, or null (then n).
-template <int B, int BLOCK, int ITEMS>
+// pairs.  n_dev: the pair count on the device, or null (then n).  FEW: the
+// counts go out tile by tile, for a downsweep that adds them up itself.
+template <int B, int BLOCK, int ITEMS, bool FEW>
 __global__ __launch_bounds__(BLOCK) void k_radix_upsweep(const uint32_t *__restrict__ keys,
                                                          const int *__restrict__ n_dev, int n_host, int shift,
                                                          uint32_t *__restrict__ hist, int nb)
@@ -50,7 +51,10 @@ __global__ __launch_bounds__(BLOCK) void k_radix_upsweep(const uint32_t *__restr
     // tiles past the end are not scanned (block 0 always writes: n may be 0)
     if (tile0 >= n && blockIdx.x > 0) return;
     __syncthreads();
-    for (int d = tid; d < R; d += BLOCK) hist[(size_t)d * nb + blockIdx.x] = h[d];
+    for (int d = tid; d < R; d += BLOCK) {
+        if constexpr (FEW) hist[(size_t)blockIdx.x * R + d] = h[d];
+        else hist[(size_t)d * nb + blockIdx.x] = h[d];
+    }
 }
 
 // One block per digit: exclusive scan of that digit's per-block counts.
@@ -77,7 +81,7 @@ __global__ __launch_bounds__(256) void k_radix_scan(uint32_t *__restrict__ hist,
     if (threadIdx.x == 0) totals[blockIdx.x] = total;
 }
 
-template <int B, int BLOCK, int ITEMS>
+template <int B, int BLOCK, int ITEMS, bool FEW>
 __global__ __launch_bounds__(BLOCK) void k_radix_downsweep(
     const uint32_t *__restrict__ keys_in, const uint32_t *__restrict__ vals_in,
     uint32_t *__restrict__ keys_out, uint32_t *__restrict__ vals_out,
@@ -102,8 +106,32 @@ __global__ __launch_bounds__(BLOCK) void k_radix_downsweep(
 #pragma unroll
     for (int u = 0; u < D; ++u) {
         const int d = tid * D + u;
+        if constexpr (FEW) {
+            tot[u] = before[u] = 0u;
+            continue;
+        }
         tot[u] = d < R ? totals[d] : 0u;
         before[u] = d < R ? hist[(size_t)d * nb + blockIdx.x] : 0u;
+    }
+    if constexpr (FEW) {   // every tile's counts of this thread's digits
+        const int used = (int)((n + (long long)TILE - 1) / TILE);   // tiles with data
+        for (int b0 = 0; b0 < used; b0 += 8) {
+            uint32_t c[8][D];
+#pragma unroll
+            for (int x = 0; x < 8; ++x)
+#pragma unroll
+                for (int u = 0; u < D; ++u) {
+                    const int d = tid * D + u;
+                    c[x][u] = b0 + x < used && d < R ? hist[(size_t)(b0 + x) * R + d] : 0u;
+                }
+#pragma unroll
+            for (int x = 0; x < 8; ++x)
+#pragma unroll
+                for (int u = 0; u < D; ++u) {
+                    tot[u] += c[x][u];
+                    before[u] += b0 + x < (int)blockIdx.x ? c[x][u] : 0u;
+                }
+        }
     }
     for (int i = tid; i < W * R; i += BLOCK) (&wcnt[0][0])[i] = 0;
 
@@ -211,16 +239,28 @@ void sort_scratch_bind(SortScratch &s, int n_cap, void *mem, int digits)
     s.hist = s.totals + digits;
 }
 
+// Up to kFewTiles tiles a pass is two launches: every block of the downsweep
+// adds up the tiles' counts itself (two passes: 1e3 pairs 60 -> 36 us, 3e4
+// 60 -> 44, 1e5 62 -> 52; 2e5, 49 tiles, 60 to 64 either way).
+constexpr int kFewTiles = 32;
+
 template <int B, int BLOCK, int ITEMS>
 static void radix_pass(const uint32_t *sk, const uint32_t *sv, uint32_t *dk, uint32_t *dv, const int *n_dev, int n,
                        int shift, const SortScratch &s, hipStream_t stream, Profiler *prof)
 {
     const int nb = div_up(n > 0 ? n : 1, BLOCK * ITEMS), digits = 1 << B;
-    DSMC_LAUNCH(prof, "radix_upsweep", (double)n * 4.0, (k_radix_upsweep<B, BLOCK, ITEMS>), nb, BLOCK, stream, sk,
-                n_dev, n, shift, s.hist, nb);
+    if (nb <= kFewTiles) {
+        DSMC_LAUNCH(prof, "radix_upsweep", (double)n * 4.0, (k_radix_upsweep<B, BLOCK, ITEMS, true>), nb, BLOCK,
+                    stream, sk, n_dev, n, shift, s.hist, nb);
+        DSMC_LAUNCH(prof, "radix_downsweep", (double)n * 16.0, (k_radix_downsweep<B, BLOCK, ITEMS, true>), nb, BLOCK,
+                    stream, sk, sv, dk, dv, n_dev, n, shift, s.hist, s.totals, nb);
+        return;
+    }
+    DSMC_LAUNCH(prof, "radix_upsweep", (double)n * 4.0, (k_radix_upsweep<B, BLOCK, ITEMS, false>), nb, BLOCK, stream,
+                sk, n_dev, n, shift, s.hist, nb);
     DSMC_LAUNCH(prof, "radix_scan", (double)digits * nb * 8.0, k_radix_scan, digits, 256, stream, s.hist, s.totals,
                 n_dev, n, BLOCK * ITEMS, nb);
-    DSMC_LAUNCH(prof, "radix_downsweep", (double)n * 16.0, (k_radix_downsweep<B, BLOCK, ITEMS>), nb, BLOCK, stream,
+    DSMC_LAUNCH(prof, "radix_downsweep", (double)n * 16.0, (k_radix_downsweep<B, BLOCK, ITEMS, false>), nb, BLOCK, stream,
                 sk, sv, dk, dv, n_dev, n, shift, s.hist, s.totals, nb);
 }
 
@@ -613,25 +653,12 @@ __global__ void k_fill_u32(uint32_t *p, uint32_t v, long long n)
         p[i] = v;
 }
 
-__global__ void k_fill_f64(double *p, double v, long long n)
-{
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n;
-         i += (long long)gridDim.x * blockDim.x)
-        p[i] = v;
-}
-
 static int fill_grid(long long n) { return (int)std::min<long long>(4096, (n + 255) / 256 + 1); }
 
 void fill_u32(uint32_t *p, uint32_t v, long long n, hipStream_t stream, Profiler *prof)
 {
     if (n <= 0) return;
     DSMC_LAUNCH(prof, "fill", (double)n * 4.0, k_fill_u32, fill_grid(n), 256, stream, p, v, n);
-}
-
-void fill_f64(double *p, double v, long long n, hipStream_t stream, Profiler *prof)
-{
-    if (n <= 0) return;
-    DSMC_LAUNCH(prof, "fill", (double)n * 8.0, k_fill_f64, fill_grid(n), 256, stream, p, v, n);
 }
 
 // Streaming copy for counter calibration: four 16-byte vectors per thread

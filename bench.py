@@ -293,7 +293,7 @@ def pmc_traffic(steps=10, timeout_s=150):
     out = dict(scales={k: round(v, 4) for k, v in scales.items()}, steps=steps, kernels={})
     # profiler names -> kernel names
     names = {"move_fused": "move_fused", "collide_fused": "collide_fused",
-             "resort_merge": "ins_merge", "resort_locate": "ins_locate",
+             "resort_merge": "ins_merge",
              "obs_finalize": "obs_finalize", "collide_edges": "collide_edges"}
     for key, kname in names.items():
         f, w = pick(F, kname), pick(W, kname)

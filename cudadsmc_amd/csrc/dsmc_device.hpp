@@ -555,16 +555,4 @@ __device__ __forceinline__ uint64_t match_bits(uint32_t v, uint64_t active)
     return m;
 }
 
-__device__ __forceinline__ uint64_t match_digit8(uint32_t d, uint64_t active)
-{
-    uint64_t m = active;
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
-        const bool bit = (d >> b) & 1u;
-        const uint64_t bal = __ballot(bit);
-        m &= bit ? bal : ~bal;
-    }
-    return m;
-}
-
 }  // namespace dsmc

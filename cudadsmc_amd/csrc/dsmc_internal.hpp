@@ -196,7 +196,6 @@ void gather_u32(uint32_t *dst, const uint32_t *src, const uint32_t *map, const i
                 int n_cap, hipStream_t stream, Profiler *prof);
 
 void fill_u32(uint32_t *p, uint32_t v, long long n, hipStream_t stream, Profiler *prof);
-void fill_f64(double *p, double v, long long n, hipStream_t stream, Profiler *prof);
 
 // Streaming device-to-device copy of bytes (multiple of 16) for counter
 // calibration.

@@ -590,16 +590,26 @@ __device__ __forceinline__ void resort_scan_merge_block(const ResortMerge &ra, i
             list[at++] = (unsigned short)(64 * (2 * tid + u) + __ffsll((unsigned long long)bits) - 1);
     __syncthreads();
     const bool has1 = g1 < n;
-    uint32_t below = 0;   // movers inserted before the tile (this thread's)
-#pragma unroll 4
-    for (int e = tid; e < total; e += 256) {
-        const uint32_t v = list[e], k = ra.key_new[v];
-        const uint64_t kv = (uint64_t)k << 32 | v;
-        if (in_bucket(t, f0, has1, f1, kv)) {
-            const int x = atomicAdd(&L.n_big, 1);
-            if (x < kBucketLds) L.kv[x] = kv;
-        } else if (t > 0 && !kv_less(f0, (uint32_t)g0, k, v)) {
-            ++below;
+    constexpr int kAhead = 8;   // movers whose keys a thread loads together
+    uint32_t below = 0;         // movers inserted before the tile (this thread's)
+    for (int e0 = tid; e0 < total; e0 += kAhead * 256) {
+        uint32_t v[kAhead], k[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int e = e0 + 256 * u;
+            v[u] = e < total ? list[e] : 0u;
+            k[u] = e < total ? ra.key_new[v[u]] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (e0 + 256 * u >= total) continue;
+            const uint64_t kv = (uint64_t)k[u] << 32 | v[u];
+            if (in_bucket(t, f0, has1, f1, kv)) {
+                const int x = atomicAdd(&L.n_big, 1);
+                if (x < kBucketLds) L.kv[x] = kv;
+            } else if (t > 0 && !kv_less(f0, (uint32_t)g0, k[u], v[u])) {
+                ++below;
+            }
         }
     }
     mt.part[0] = below - moved_before - gone_before;

@@ -418,6 +418,34 @@ __device__ __forceinline__ T wave_inclusive_scan(T v)
 // Exclusive scan over a block of BLOCK threads (one value per thread).  Uses
 // `tmp` (>= BLOCK/64 + 1 entries of LDS).  Returns the exclusive prefix and
 // writes the block total to *total.
+// 32-bit integers: the exchanges as DPP operands of the additions (row shifts
+// of 1, 2, 4 and 8 scan each row of 16 lanes, the last lane of rows 0 and 2
+// goes to rows 1 and 3, then lane 31 to the upper half) instead of LDS
+// permutes: some 10 cycles a step where a permute takes about 100.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t add_dpp(uint32_t v)
+{
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, true);
+}
+// Inclusive scan over the 32 lanes of each half-wave.
+__device__ __forceinline__ uint32_t halfwave_inclusive_scan(uint32_t v)
+{
+    v = add_dpp<0x111, 0xF>(v);
+    v = add_dpp<0x112, 0xF>(v);
+    v = add_dpp<0x114, 0xF>(v);
+    v = add_dpp<0x118, 0xF>(v);
+    return add_dpp<0x142, 0xA>(v);
+}
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v)
+{
+    return add_dpp<0x143, 0xC>(halfwave_inclusive_scan(v));
+}
+__device__ __forceinline__ int wave_inclusive_scan(int v) { return (int)wave_inclusive_scan((uint32_t)v); }
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_scan(v), kWave - 1);
+}
+
 template <int BLOCK, typename T>
 __device__ __forceinline__ T block_exclusive_scan(T v, T *tmp, T *total)
 {
@@ -427,14 +455,14 @@ __device__ __forceinline__ T block_exclusive_scan(T v, T *tmp, T *total)
     T inc = wave_inclusive_scan(v);
     if (lane == kWave - 1) tmp[w] = inc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        T run = 0;
-        for (int i = 0; i < W; ++i) { T c = tmp[i]; tmp[i] = run; run += c; }
-        tmp[W] = run;
+    T res = inc - v, all = 0;
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        const T c = tmp[i];
+        if (i < w) res += c;
+        all += c;
     }
-    __syncthreads();
-    T res = inc - v + tmp[w];
-    *total = tmp[W];
+    *total = all;
     __syncthreads();
     return res;
 }

@@ -19,14 +19,7 @@ static_assert(kTileWords == 32, "a tile's mask words are half a wave");
 // Exclusive prefix of v over the 32 lanes of this lane's half-wave.
 __device__ __forceinline__ uint32_t halfwave_exclusive_scan(uint32_t v)
 {
-    const int hl = threadIdx.x & 31;
-    uint32_t s = v;
-#pragma unroll
-    for (int d = 1; d < 32; d <<= 1) {
-        const uint32_t u = __shfl_up(s, d, 32);
-        if (hl >= d) s += u;
-    }
-    return s - v;
+    return halfwave_inclusive_scan(v) - v;
 }
 
 // (key, slot) order; slots are distinct.

@@ -394,6 +394,41 @@ __device__ __forceinline__ uint64_t lanemask_lt()
     return lane ? (~0ull >> (64 - lane)) : 0ull;
 }
 
+// x of lane ^ O, as register exchanges (the lane swaps of 32 and 16 lanes, row
+// rotations and shifts, quad permutes) instead of an LDS permute.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_of(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);
+}
+template <int O>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t x)
+{
+    static_assert(O == 32 || O == 16 || O == 8 || O == 4 || O == 2 || O == 1, "one bit");
+    if constexpr (O >= 16) {
+        // both results hold x: of the lower lanes (rows) twice, and of the upper
+        const auto r = [&] {
+            if constexpr (O == 32) return __builtin_amdgcn_permlane32_swap(x, x, false, false);
+            else return __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        }();
+        return (threadIdx.x & O) ? r[0] : r[1];
+    } else if constexpr (O == 8) {
+        return dpp_of<0x128>(x);   // row rotation by 8
+    } else if constexpr (O == 4) {   // from 4 lanes above, and in the upper quads from 4 below
+        return (uint32_t)__builtin_amdgcn_update_dpp((int)dpp_of<0x104>(x), (int)x, 0x114, 0xF, 0xA, false);
+    } else if constexpr (O == 2) {
+        return dpp_of<0x4E>(x);
+    } else {
+        return dpp_of<0xB1>(x);
+    }
+}
+template <int O>
+__device__ __forceinline__ double lane_xor(double x)
+{
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    return __builtin_bit_cast(double, (uint64_t)lane_xor<O>((uint32_t)(b >> 32)) << 32 | lane_xor<O>((uint32_t)b));
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v)
 {
@@ -510,12 +545,14 @@ __device__ __forceinline__ void block_sum4(double (&v)[4], double *tmp)
     const bool b5 = (lane & 32) != 0, b4 = (lane & 16) != 0;
     double k0 = b5 ? v[2] : v[0], k1 = b5 ? v[3] : v[1];
     const double s0 = b5 ? v[0] : v[2], s1 = b5 ? v[1] : v[3];
-    k0 += __shfl_xor(s0, 32, kWave);
-    k1 += __shfl_xor(s1, 32, kWave);
+    k0 += lane_xor<32>(s0);
+    k1 += lane_xor<32>(s1);
     double k = b4 ? k1 : k0;
-    k += __shfl_xor(b4 ? k0 : k1, 16, kWave);
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) k += __shfl_xor(k, o, kWave);
+    k += lane_xor<16>(b4 ? k0 : k1);
+    k += lane_xor<8>(k);
+    k += lane_xor<4>(k);
+    k += lane_xor<2>(k);
+    k += lane_xor<1>(k);
     if ((lane & 15) == 0) tmp[w * 4 + (b5 ? 2 : 0) + (b4 ? 1 : 0)] = k;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -544,17 +581,18 @@ __device__ __forceinline__ void block_sum8(double (&v)[8], double *tmp)
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const double keep = b5 ? v[4 + q] : v[q], send = b5 ? v[q] : v[4 + q];
-        a[q] = keep + __shfl_xor(send, 32, kWave);
+        a[q] = keep + lane_xor<32>(send);
     }
     double c[2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         const double keep = b4 ? a[2 + q] : a[q], send = b4 ? a[q] : a[2 + q];
-        c[q] = keep + __shfl_xor(send, 16, kWave);
+        c[q] = keep + lane_xor<16>(send);
     }
-    double k = (b3 ? c[1] : c[0]) + __shfl_xor(b3 ? c[0] : c[1], 8, kWave);
-#pragma unroll
-    for (int o = 4; o > 0; o >>= 1) k += __shfl_xor(k, o, kWave);
+    double k = (b3 ? c[1] : c[0]) + lane_xor<8>(b3 ? c[0] : c[1]);
+    k += lane_xor<4>(k);
+    k += lane_xor<2>(k);
+    k += lane_xor<1>(k);
     if ((lane & 7) == 0) tmp[w * 8 + (b5 ? 4 : 0) + (b4 ? 2 : 0) + (b3 ? 1 : 0)] = k;
     __syncthreads();
     if (threadIdx.x == 0) {

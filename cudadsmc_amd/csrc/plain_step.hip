@@ -120,12 +120,14 @@ __device__ __forceinline__ double wave_sum4(const double (&v)[4])
     const bool b5 = (lane & 32) != 0, b4 = (lane & 16) != 0;
     double k0 = b5 ? v[2] : v[0], k1 = b5 ? v[3] : v[1];
     const double s0 = b5 ? v[0] : v[2], s1 = b5 ? v[1] : v[3];
-    k0 += __shfl_xor(s0, 32, kWave);
-    k1 += __shfl_xor(s1, 32, kWave);
+    k0 += lane_xor<32>(s0);
+    k1 += lane_xor<32>(s1);
     double k = b4 ? k1 : k0;
-    k += __shfl_xor(b4 ? k0 : k1, 16, kWave);
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) k += __shfl_xor(k, o, kWave);
+    k += lane_xor<16>(b4 ? k0 : k1);
+    k += lane_xor<8>(k);
+    k += lane_xor<4>(k);
+    k += lane_xor<2>(k);
+    k += lane_xor<1>(k);
     return k;
 }
 

@@ -265,7 +265,6 @@ struct dsmc_ctx {
         for (StepGraphs &g : graphs) g.destroy();
         for (void *p : allocs) (void)hipFree(p);
         if (n_host) (void)hipHostFree(n_host);
-        if (obs_host) (void)hipHostFree(obs_host);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -444,9 +443,9 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
     x->step_save = x->alloc<long long>(1);
     x->coll_accum = x->alloc<unsigned long long>(n_traps);
     x->n_dev = x->alloc<int>(4);
-    DSMC_HIP(hipHostMalloc((void **)&x->n_host, 4 * sizeof(int), hipHostMallocDefault));
-    if (!x->fp32)
-        DSMC_HIP(hipHostMalloc((void **)&x->obs_host, sizeof(dsmc_observables), hipHostMallocDefault));
+    // one pinned block: the counts, and behind them the FP64 form's record
+    DSMC_HIP(hipHostMalloc((void **)&x->n_host, 64 + sizeof(dsmc_observables), hipHostMallocDefault));
+    if (!x->fp32) x->obs_host = (dsmc_observables *)((char *)x->n_host + 64);
     // incremental re-sort (its counts start cleared)
     resort_scratch_bind(x->res, N, x->alloc<char>(resort_scratch_bytes(N), false));
     resort_clear_counts(x->res, x->stream, nullptr);

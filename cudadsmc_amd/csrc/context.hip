@@ -1080,14 +1080,25 @@ static void graph_steps(dsmc_ctx *x, int times)
     for (int k = 0; k < singles; ++k) DSMC_HIP(hipGraphLaunch(g.one.exec, x->stream));
     x->step = step0 + (long long)graph_len(x) * times;
     x->coll_steps = cs0 + 2LL * times;
-    if (!x->fp32) {
-        // as the captured steps leave it
-        x->sorted_key = x->srt_k[x->srt_cur];
-        x->perm = x->srt_v[x->srt_cur];
-        x->perm_mask = x->cfg.evaporation ? x->mpar ^ 1 : -1;
-        x->tables_stale = true;
-        x->acc_stale = !x->cfg.mcwf;
+    // as the captured steps leave it (a graph of an earlier run may have been
+    // replayed without a step of this one before it)
+    x->sorted_key = x->srt_k[x->srt_cur];
+    x->perm = x->srt_v[x->srt_cur];
+    if (x->fp32) {
+        x->have_sort = false;
+        x->srt_valid = true;
+        x->tbl_valid = true;
+        x->dead_in_state = x->cfg.evaporation != 0;
+        x->bucketed = x->cfg.sort_mode == DSMC_SORT_INCREMENTAL && resort_supported(x->n_cap);
+        return;
     }
+    x->perm_mask = x->cfg.evaporation ? x->mpar ^ 1 : -1;
+    x->tables_stale = true;
+    x->acc_stale = !x->cfg.mcwf;
+    x->sorted_ok = true;
+    x->keys_ok = true;
+    x->lazy_dead = x->cfg.evaporation != 0;
+    x->bucketed = resort_supported(x->n_cap);
 }
 
 static void do_steps(dsmc_ctx *x, int n)

@@ -1111,7 +1111,11 @@ static void do_steps(dsmc_ctx *x, int n)
         const bool resort = resort_supported(x->n_cap);
         while (n > 0) {
             const int phase = (int)(x->step % x->cfg.lpc), len = graph_len(x);
-            if (graph_ok(x) && phase == 0 && n >= len && ((x->sorted_ok && x->bucketed) || !resort)) {
+            // a graph holds the sort that follows a step (from its buckets or
+            // its keys), so the state must be as one left it, at the capture
+            // and at every replay: after anything else a launched step is first
+            const bool as_left = resort ? x->sorted_ok && x->bucketed : x->keys_ok;
+            if (graph_ok(x) && phase == 0 && n >= len && as_left) {
                 const int times = n / len;
                 graph_steps(x, times);
                 n -= times * len;

@@ -181,6 +181,7 @@ struct dsmc_ctx {
     ResortScratch res;              // FP32: incremental re-sort
     double *sigvrmax = nullptr;     // FP64 form
     float *sigvrmax_f = nullptr;    // FP32 form: sigma v_r,max in float (half the bytes)
+    uint64_t *edge_sm = nullptr;    // FP32 form, fused step: its scratch
     dsmc_observables *obs_log = nullptr;  // (obs_cap + 1) * T records
     // device step counter, double-buffered: the kernels of a step read
     // step_buf[ssel] and its finalize writes the next value to the other one
@@ -526,6 +527,7 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
         for (int t = 0; t < n_traps; ++t) x->max_trap_atoms = std::max(x->max_trap_atoms, traps[t].n_atoms);
         x->acc2 = x->alloc<double>((size_t)n_traps * kAccK);
         x->scan_partial = x->alloc<int>(scan_partials(N) + 8);
+        if (!x->split_step) x->edge_sm = x->alloc<uint64_t>((size_t)edge_sm_spans(N));
         x->obs_first = x->alloc<int>((size_t)n_traps);
         x->obs_last = x->alloc<int>((size_t)n_traps);
         x->evap_pos_f = x->alloc<float>(3 * (size_t)N);
@@ -948,6 +950,7 @@ static void fused_move(dsmc_ctx *x, bool coll = false)
         if (!x->have_sort) fail(DSMC_ESTATE, "the fused step needs a sorted state");
         sc.cp = collide_params(x);
         sc.sigvrmax = x->sigvrmax_f;
+        sc.edge_sm = x->edge_sm;
         sc.coll_accum = x->coll_accum;
         sc.dry = 0;
         launch_collide_edges(x->d_traps, x->d_key_base, x->T, sc.cp, x->sorted_key, x->perm, n,
@@ -2133,6 +2136,7 @@ dsmc_status dsmc_autotune(dsmc_ctx *ctx, int *block_size_out)
     StepCollide sc;
     sc.cp = collide_params(ctx);
     sc.sigvrmax = ctx->sigvrmax_f;
+    sc.edge_sm = ctx->edge_sm;
     sc.coll_accum = ctx->coll_accum;
     sc.dry = 1;
     const StepCollide *coll = (ctx->srt_valid && !ctx->split_step) ? &sc : nullptr;

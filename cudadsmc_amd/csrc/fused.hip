@@ -544,18 +544,22 @@ __device__ __forceinline__ int cell_trials_wave(const CollideParams &cp, const C
 constexpr int kWaveTrialsDefault = 16;
 
 // Trials of one cell (serial by one lane, or by the whole wave when heavy);
-// sigma v_r,max is stored when it grew (unless `dry`).  Returns the accepted
-// collisions.
+// sigma v_r,max is stored when it grew (unless `dry`), in `edge` with its key
+// where that is given.  Returns the accepted collisions.
 template <class V>
 __device__ __forceinline__ int run_cell(const CollideParams &cp, const CellJob &c, uint32_t stream,
                                         uint32_t step, const V &vs, float *__restrict__ sigvrmax,
-                                        bool wave, const Trial0 &t0, bool dry = false)
+                                        bool wave, const Trial0 &t0, bool dry = false,
+                                        uint64_t *edge = nullptr)
 {
     double smax = c.smax;
     const int cnt = wave ? cell_trials_wave(cp, c, stream, step, vs, smax)
                          : cell_trials_serial(cp, c, stream, step, vs, smax, t0);
     const bool writer = !wave || (threadIdx.x & (kWave - 1)) == 0;
-    if (writer && smax != c.smax && !dry) sigvrmax[c.k] = (float)smax;
+    if (writer && smax != c.smax && !dry) {
+        if (edge) *edge = (uint64_t)c.k << 32 | __float_as_uint((float)smax);
+        else sigvrmax[c.k] = (float)smax;
+    }
     return cnt;
 }
 
@@ -907,6 +911,7 @@ __device__ __forceinline__ void move_update(const MoveParams &mp, const TrapDev 
 struct CollArgs {
     CollideParams cp;
     float *sigvrmax;
+    uint64_t *edge_sm;   // per span: what k_edge_sigvrmax stores
     unsigned long long *coll_accum;
     int wave_trials;
     int dry;
@@ -916,10 +921,13 @@ struct CollArgs {
 // consecutive sorted slots (its "span") and, next to them, kExt slots of the
 // neighbouring spans on each side.  A cell across a span boundary with at
 // most kExt slots on either side of it is run by both waves (the same
-// trials, so the same velocities; the wave holding its first slot stores
-// sigma v_r,max and counts its collisions).  Larger cells across a boundary
-// ("oversized") are run before the step kernel by k_collide_edges.
+// trials, so the same velocities; the wave holding its first slot counts its
+// collisions and leaves its raised sigma v_r,max for k_edge_sigvrmax, after
+// the launch: the other wave may still have to read the old one).  Larger
+// cells across a boundary ("oversized") are run before the step kernel by
+// k_collide_edges.
 constexpr int kExt = 16;
+constexpr uint64_t kNoEdge = ~0ull;
 
 // Oversized: the cell across boundary B (slots B - 1 and B hold key k) has
 // more than kExt slots on one side of it.  kb = key of slot B - kExt - 1
@@ -938,6 +946,7 @@ struct WaveColl {
     static constexpr int W = kWave * APT;
     f4 v[W + 2 * kExt];
     f2 w[W + 2 * kExt];
+    uint64_t edge;   // key << 32 | raised sigma v_r,max of the cell across the last boundary
     uint32_t k[W + 2 * kExt + 2];
     float sm[W];
     short mh[W / 2 + 1], me[W / 2 + 1], hv[W / 2 + 1];
@@ -945,7 +954,7 @@ struct WaveColl {
 
 // The collisions of one wave's span [ws, ws + len) (len <= W).  pre_h /
 // pre_e, post_h / post_e: the cells across its first and last boundary that
-// it runs (-1: none).  Each lane runs one cell (those with more than
+// it runs (-1: none).  L.edge holds kNoEdge.  Each lane runs one cell (those with more than
 // wave_trials trials are run by the whole wave); the same trial sequence per
 // cell as k_collide_fused, so the velocities are bitwise the same.
 template <int APT>
@@ -1023,7 +1032,8 @@ __device__ __forceinline__ void wave_collide(const TrapDev *__restrict__ traps, 
         if (is_heavy) L.hv[nheavy + __popcll(hb & lt)] = (short)mi;
         nheavy += __popcll(hb);
         if (ok && !is_heavy) {
-            const int cnt = run_cell(ca.cp, c, stream, step, vl, ca.sigvrmax, false, t0, ca.dry != 0 || !own);
+            const int cnt = run_cell(ca.cp, c, stream, step, vl, ca.sigvrmax, false, t0, ca.dry != 0 || !own,
+                                     c.i == post_h ? &L.edge : nullptr);
             if (own) {
                 if (one) wave_cnt += (unsigned long long)cnt;
                 else if (cnt && !ca.dry) atomicAdd(&ca.coll_accum[c.t], (unsigned long long)cnt);
@@ -1042,7 +1052,7 @@ __device__ __forceinline__ void wave_collide(const TrapDev *__restrict__ traps, 
         (void)cell_setup(traps[t], t, k, ca.cp, (double)(own ? L.sm[h - ws] : ca.sigvrmax[k]), h, e, c);
         const Trial0 none = { 0u, 0u, 0.0f, 0.0f };
         const int cnt = run_cell(ca.cp, c, traps[t].stream, step, vl, ca.sigvrmax, true, none,
-                                 ca.dry != 0 || !own);
+                                 ca.dry != 0 || !own, c.i == post_h ? &L.edge : nullptr);
         if (lane == 0 && own) {
             if (one) wave_cnt += (unsigned long long)cnt;
             else if (cnt && !ca.dry) atomicAdd(&ca.coll_accum[t], (unsigned long long)cnt);
@@ -1191,6 +1201,7 @@ void k_move_fused(
                 rpz[k] = v2.y;
             }
         }
+        if (lane == 0) L.edge = kNoEdge;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
         // the cells across the span's first and last boundary that it runs
@@ -1227,6 +1238,7 @@ void k_move_fused(
         if (len > 0)
             wave_collide<APT>(traps, ts, T, one, t_first, ca, (uint32_t)step, ws, len, L, pre_h, pre_e,
                               post_h);
+        if (lane == 0 && !ca.dry) ca.edge_sm[ws / W] = L.edge;
 #pragma unroll
         for (int k = 0; k < APT; ++k) {
             const int l = k * kWave + lane;
@@ -1748,6 +1760,18 @@ double move_fused_bytes_per_atom(int spin)
     return 4.0 + state + 4.0 + state + 4.0;
 }
 
+// After the fused step: the raised sigma v_r,max of the cells across the
+// boundaries between spans.
+__global__ __launch_bounds__(kFBlock) void k_edge_sigvrmax(const uint64_t *__restrict__ edge, int spans,
+                                                           float *__restrict__ sigvrmax)
+{
+    const int i = blockIdx.x * kFBlock + threadIdx.x;
+    if (i >= spans || edge[i] == kNoEdge) return;
+    sigvrmax[edge[i] >> 32] = __uint_as_float((uint32_t)edge[i]);
+}
+
+int edge_sm_spans(int n_cap) { return fgrid(n_cap, 1024) * (1024 / kWave); }
+
 template <int BS, int APT, bool COLL>
 static void move_fused_bs(const TrapDev *traps, const MoveParams &mp, const FusedPtrs &src,
                           const FusedPtrs &dst, const uint32_t *perm, const int *trap_start,
@@ -1790,6 +1814,7 @@ void launch_move_fused(int block, int apt, const TrapDev *traps, const MoveParam
     if (coll) {
         ca.cp = coll->cp;
         ca.sigvrmax = coll->sigvrmax;
+        ca.edge_sm = coll->edge_sm;
         ca.coll_accum = coll->coll_accum;
         ca.wave_trials = wave_trials_setting();
         ca.dry = coll->dry;
@@ -1824,6 +1849,11 @@ void launch_move_fused(int block, int apt, const TrapDev *traps, const MoveParam
 #undef DSMC_MOVE_CASE
     DSMC_HIP(hipGetLastError());
     if (prof && prof->enabled) prof->end(st);
+    if (coll && !coll->dry) {
+        const int spans = fgrid(n_cap, block * apt) * (block / kWave);
+        DSMC_LAUNCH(prof, "edge_sigvrmax", (double)spans * 8.0, k_edge_sigvrmax, fgrid(spans, kFBlock), kFBlock,
+                    st, coll->edge_sm, spans, coll->sigvrmax);
+    }
 }
 
 // ---------------------------------------------------------------------------

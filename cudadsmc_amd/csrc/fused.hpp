@@ -166,9 +166,11 @@ int  obs_record_stride(int n_cap);
 struct StepCollide {
     CollideParams cp;
     float *sigvrmax;
+    uint64_t *edge_sm;   // edge_sm_spans() words of scratch
     unsigned long long *coll_accum;
     int dry;   // compute but write neither sigma v_r,max nor counts (autotuner trials)
 };
+int  edge_sm_spans(int n_cap);
 // block: threads per block (64 .. 1024); apt: atoms per thread (1 or 2).  A
 // block moves block * apt consecutive slots and leaves one observables record
 // and one pair of re-sort counts.  With coll (the fused step; needs the

@@ -471,7 +471,7 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
         x->count = x->alloc<int>(C1);
         x->prefix = x->alloc<int>(C1);
         x->coll_count = x->alloc<int>(C1);
-        x->scan_partial = x->alloc<int>(scan_partials(std::max(C1, N)) + 8);
+        x->scan_partial = x->alloc<int>(scan_partials(N));
         x->tag = x->alloc<int>(N);
         x->cmap = x->alloc<uint32_t>(N);
         x->evap_pos_d = x->alloc<double>(3 * (size_t)N);
@@ -526,7 +526,7 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
         x->rec.cnt = x->alloc<unsigned int>((size_t)n_traps);
         for (int t = 0; t < n_traps; ++t) x->max_trap_atoms = std::max(x->max_trap_atoms, traps[t].n_atoms);
         x->acc2 = x->alloc<double>((size_t)n_traps * kAccK);
-        x->scan_partial = x->alloc<int>(scan_partials(N) + 8);
+        x->scan_partial = x->alloc<int>(scan_partials(N));
         if (!x->split_step) x->edge_sm = x->alloc<uint64_t>((size_t)edge_sm_spans(N));
         x->obs_first = x->alloc<int>((size_t)n_traps);
         x->obs_last = x->alloc<int>((size_t)n_traps);
@@ -2240,7 +2240,7 @@ dsmc_status dsmc_exclusive_scan(const int *d_in, int *d_out, int n, void *stream
     if (n < 0 || (n > 0 && (!d_in || !d_out))) fail(DSMC_EINVAL, "bad scan arguments");
     if (n == 0) return DSMC_OK;
     hipStream_t st = (hipStream_t)stream;
-    Workspace part(sizeof(int) * (scan_partials(n) + 8));
+    Workspace part(sizeof(int) * (scan_partials(n)));
     exclusive_scan(d_in, d_out, n, part.as<int>(), st, nullptr);
     DSMC_HIP(hipStreamSynchronize(st));
     PRIM_END
@@ -2252,7 +2252,7 @@ dsmc_status dsmc_remove_if(int *d_values, const int *d_stencil, int n, int *n_ou
     if (n < 0 || (n > 0 && (!d_values || !d_stencil))) fail(DSMC_EINVAL, "bad remove_if arguments");
     if (n == 0) { if (n_out) *n_out = 0; return DSMC_OK; }
     hipStream_t st = (hipStream_t)stream;
-    Workspace ws(sizeof(int) * ((size_t)n + remove_if_blocks(n)));
+    Workspace ws(sizeof(int) * ((size_t)n + scan_partials(n)));
     int *tmp = ws.as<int>();
     remove_if(d_values, d_stencil, n, tmp, tmp + n, ws.b.host, st);
     DSMC_HIP(hipStreamSynchronize(st));

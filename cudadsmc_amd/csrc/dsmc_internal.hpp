@@ -175,21 +175,28 @@ void resort_samples(const ResortScratch &r, const uint32_t *sorted, hipStream_t 
 // Clears the buckets' counts (a collide after the merge does it otherwise).
 void resort_clear_counts(const ResortScratch &r, hipStream_t stream, Profiler *prof);
 
-// Exclusive scan of n ints (n known on the host); partial holds div_up(n, tile).
+// Exclusive scan of n ints (n known on the host; in and out may be the same);
+// partial holds scan_partials(n).
 void exclusive_scan(const int *in, int *out, int n, int *partial, hipStream_t stream,
                     Profiler *prof);
-inline int scan_partials(int n) { return div_up(n > 0 ? n : 1, kScanTile) + 1; }
+// Up to kSumTiles tiles every block of a scan, a removal or a compaction map
+// adds up the tiles before its own itself; beyond, where that grows with the
+// square of the tiles, their sums are scanned first, in two more launches
+// (added up / scanned first, us: scan of 1e6 elements 20 / 24, 1.6e7 87 / 93,
+// 3.2e7 163 / 162, 6.4e7 384 / 323, 2.56e8 2230 / 1190, 1e9 18500 / 4500;
+// removal of 1.6e7 58 / 60, 3.2e7 123 / 114, 2.56e8 2350 / 1160).
+constexpr int kSumTiles = 12288;
+int scan_partials(int n);
 
 // Stable compaction map: for stencil[i] == 0 (kept), map[j] = i for the j-th
 // kept element; *n_out (device) = number kept.  n read from device memory;
-// n_cap bounds the grid.  partial holds div_up(n_cap, tile) + 1 ints.
+// n_cap bounds the grid.  partial holds scan_partials(n_cap).
 void compaction_map(const int *stencil, const int *n_dev, int n_cap, uint32_t *map,
                     int *n_out_dev, int *partial, hipStream_t stream, Profiler *prof);
 
 // Stable in-place removal of the values with a non-zero stencil; *kept (device
 // or pinned host memory) receives how many stay.  tmp holds n ints, partial
-// remove_if_blocks(n).
-int remove_if_blocks(int n);
+// scan_partials(n).
 void remove_if(int *values, const int *stencil, int n, int *tmp, int *partial, int *kept, hipStream_t stream);
 
 // dst[i] = src[map[i]] for i < *n_dev (i < n_cap when n_dev is null).

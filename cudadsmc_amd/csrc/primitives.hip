@@ -452,11 +452,16 @@ __device__ __forceinline__ int sum_below(const int *__restrict__ partial, int b,
     return total;
 }
 
-// Every block adds up the tiles' sums before its own itself: one launch fewer
-// than a scan of the partials, and for a million elements 489 words a block.
-__global__ __launch_bounds__(kScanBlock) void k_scan_final(const int *__restrict__ in,
-                                                           int *__restrict__ out, int n,
-                                                           const int *__restrict__ partial)
+// Sum of the tiles before tile b: partial holds the tiles' own sums, or
+// (scanned) the sums before them.
+__device__ __forceinline__ int tiles_before(const int *__restrict__ partial, int b, bool scanned, int *tmp)
+{
+    return scanned ? partial[b] : sum_below(partial, b, tmp);
+}
+
+// in and out may be the same array.
+__global__ __launch_bounds__(kScanBlock) void k_scan_final(const int *in, int *out, int n,
+                                                           const int *__restrict__ partial, bool scanned)
 {
     __shared__ int tmp[kScanBlock / kWave + 1];
     const int t0 = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
@@ -467,7 +472,7 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_final(const int *__restrict
         v[k] = (t0 + k < n) ? in[t0 + k] : 0;
         s += v[k];
     }
-    const int before = sum_below(partial, (int)blockIdx.x, tmp);
+    const int before = tiles_before(partial, (int)blockIdx.x, scanned, tmp);
     int total;
     int run = block_exclusive_scan<kScanBlock>(s, tmp, &total) + before;
 #pragma unroll
@@ -477,6 +482,16 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_final(const int *__restrict
     }
 }
 
+// Scans the sums of more than kSumTiles tiles in place (partial's nb words and
+// `extra` behind them); returns whether it did.
+static bool scan_tiles(int *partial, int nb, int extra, hipStream_t stream, Profiler *prof);
+
+int scan_partials(int n)
+{
+    const int nb = div_up(n > 0 ? n : 1, kScanTile);
+    return nb + 1 + (nb > kSumTiles ? scan_partials(nb + 1) : 0);
+}
+
 void exclusive_scan(const int *in, int *out, int n, int *partial, hipStream_t stream,
                     Profiler *prof)
 {
@@ -484,8 +499,16 @@ void exclusive_scan(const int *in, int *out, int n, int *partial, hipStream_t st
     const int nb = div_up(n, kScanTile);
     DSMC_LAUNCH(prof, "scan_reduce", (double)n * 4.0, k_scan_reduce, nb, kScanBlock, stream,
                 in, n, partial);
+    const bool scanned = scan_tiles(partial, nb, 0, stream, prof);
     DSMC_LAUNCH(prof, "scan_final", (double)n * 8.0, k_scan_final, nb, kScanBlock, stream, in,
-                out, n, (const int *)partial);
+                out, n, (const int *)partial, scanned);
+}
+
+static bool scan_tiles(int *partial, int nb, int extra, hipStream_t stream, Profiler *prof)
+{
+    if (nb <= kSumTiles) return false;
+    exclusive_scan(partial, partial, nb + extra, partial + nb + 1, stream, prof);
+    return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -532,29 +555,29 @@ __global__ __launch_bounds__(kScanBlock) void k_remove_tile(const int *__restric
     __syncthreads();
     for (int i = threadIdx.x; i < all; i += kScanBlock) tmp_out[tile0 + i] = kept[i];
     if (threadIdx.x == 0) partial[blockIdx.x] = all;
+    if (threadIdx.x == 0 && blockIdx.x == 0) partial[gridDim.x] = 0;   // (scanned, the total)
 }
 
 __global__ __launch_bounds__(kScanBlock) void k_remove_place(const int *__restrict__ tmp_in,
-                                                             const int *__restrict__ partial, int nb,
+                                                             const int *__restrict__ partial, int nb, bool scanned,
                                                              int *__restrict__ values, int *__restrict__ kept)
 {
     __shared__ int tmp[kScanBlock / kWave + 1];
-    const int m = partial[blockIdx.x];
-    const int before = sum_below(partial, (int)blockIdx.x, tmp);
+    const int before = tiles_before(partial, (int)blockIdx.x, scanned, tmp);
+    const int m = scanned ? partial[blockIdx.x + 1] - before : partial[blockIdx.x];
     const int *src = tmp_in + (size_t)blockIdx.x * kScanTile;
     for (int i = threadIdx.x; i < m; i += kScanBlock) values[before + i] = src[i];
     if ((int)blockIdx.x == nb - 1 && threadIdx.x == 0) *kept = before + m;
 }
 
-int remove_if_blocks(int n) { return div_up(n > 0 ? n : 1, kScanTile); }
-
 void remove_if(int *values, const int *stencil, int n, int *tmp, int *partial, int *kept, hipStream_t stream)
 {
-    const int nb = remove_if_blocks(n);
+    const int nb = div_up(n > 0 ? n : 1, kScanTile);
     hipLaunchKernelGGL(k_remove_tile, dim3(nb), dim3(kScanBlock), 0, stream, values, stencil, n, tmp, partial);
     DSMC_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_remove_place, dim3(nb), dim3(kScanBlock), 0, stream, tmp, partial, nb, values,
-                       kept);
+    const bool scanned = scan_tiles(partial, nb, 1, stream, nullptr);
+    hipLaunchKernelGGL(k_remove_place, dim3(nb), dim3(kScanBlock), 0, stream, tmp, partial, nb, scanned,
+                       values, kept);
     DSMC_HIP(hipGetLastError());
 }
 
@@ -577,11 +600,13 @@ __global__ __launch_bounds__(kScanBlock) void k_compact_count(const int *__restr
     int total;
     (void)block_exclusive_scan<kScanBlock>(s, tmp, &total);
     if (threadIdx.x == 0) partial[blockIdx.x] = total;
+    if (threadIdx.x == 0 && blockIdx.x == 0) partial[gridDim.x] = 0;   // (scanned, the total)
 }
 
 __global__ __launch_bounds__(kScanBlock) void k_compact_scatter(
     const int *__restrict__ stencil, const int *__restrict__ n_dev,
-    const int *__restrict__ partial, uint32_t *__restrict__ map, int *__restrict__ n_out, int nb)
+    const int *__restrict__ partial, bool scanned, uint32_t *__restrict__ map, int *__restrict__ n_out,
+    int nb)
 {
     constexpr int W = kScanBlock / kWave;
     __shared__ int wtot[W];
@@ -590,9 +615,8 @@ __global__ __launch_bounds__(kScanBlock) void k_compact_scatter(
     const int tile0 = blockIdx.x * kScanTile;
     const bool last = (int)blockIdx.x == nb - 1;
     if (tile0 >= n && !last) return;
-    // every block adds up the kept ones of the tiles before its own
-    const int before = sum_below(partial, (int)blockIdx.x, tmp);
-    if (last && threadIdx.x == 0) *n_out = before + partial[blockIdx.x];
+    const int before = tiles_before(partial, (int)blockIdx.x, scanned, tmp);
+    if (last && threadIdx.x == 0) *n_out = scanned ? partial[nb] : before + partial[blockIdx.x];
     if (tile0 >= n) return;
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const int base = tile0 + w * (kWave * kScanItems);
@@ -623,8 +647,9 @@ void compaction_map(const int *stencil, const int *n_dev, int n_cap, uint32_t *m
     const int nb = div_up(n_cap > 0 ? n_cap : 1, kScanTile);
     DSMC_LAUNCH(prof, "compact_count", (double)n_cap * 4.0, k_compact_count, nb, kScanBlock,
                 stream, stencil, n_dev, partial);
+    const bool scanned = scan_tiles(partial, nb, 1, stream, prof);
     DSMC_LAUNCH(prof, "compact_scatter", (double)n_cap * 8.0, k_compact_scatter, nb, kScanBlock,
-                stream, stencil, n_dev, (const int *)partial, map, n_out_dev, nb);
+                stream, stencil, n_dev, (const int *)partial, scanned, map, n_out_dev, nb);
 }
 
 __global__ __launch_bounds__(256) void k_gather_u32(uint32_t *__restrict__ dst,

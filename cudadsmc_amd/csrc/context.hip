@@ -108,6 +108,18 @@ Profiler::~Profiler()
 
 static void free_kept();   // scratch kept between the primitives' calls
 
+// Device memory, if need be without that scratch.
+static void *device_alloc(size_t bytes)
+{
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        free_kept();
+        DSMC_HIP(hipMalloc(&p, bytes));
+    }
+    return p;
+}
+
 // A captured run of steps.
 struct StepGraph {
     hipGraph_t graph = nullptr;
@@ -247,13 +259,8 @@ struct dsmc_ctx {
     template <typename T_>
     T_ *alloc(size_t count_, bool zero = true)
     {
-        void *p = nullptr;
         const size_t bytes = std::max<size_t>(count_ * sizeof(T_), 16);
-        if (hipMalloc(&p, bytes) != hipSuccess) {   // without the scratch kept for the primitives
-            (void)hipGetLastError();
-            free_kept();
-            DSMC_HIP(hipMalloc(&p, bytes));
-        }
+        void *p = device_alloc(bytes);
         allocs.push_back(p);
         if (zero) DSMC_HIP(hipMemsetAsync(p, 0, bytes, stream));
         return (T_ *)p;
@@ -1506,8 +1513,8 @@ static void copy_field(dsmc_ctx *x, int field, void *host, size_t bytes)
 // freed it (which waits for the device): some 70 us a sort, of 95 at n = 1000
 // and 195 at n = 1e6.  A few idle blocks are kept for the next call instead:
 // at most kKeptBlocks, of at most kKeptBytes together, per process; one that
-// kKeptUnused calls did not use is freed, and all are when an allocation
-// fails.  A block belongs to one call at a time and the calls wait for their
+// kKeptUnused calls did not use is freed, and all are when an allocation of
+// this library fails.  A block belongs to one call at a time and the calls wait for their
 // stream before they return, so threads and streams never share one (a call
 // that fails does not keep its block).
 constexpr int kKeptBlocks = 8;
@@ -1553,11 +1560,7 @@ struct Workspace {
             }
         }
         b.bytes = bytes;
-        if (hipMalloc(&b.p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            free_kept();
-            DSMC_HIP(hipMalloc(&b.p, bytes));
-        }
+        b.p = device_alloc(bytes);
         if (hipHostMalloc((void **)&b.host, 64, hipHostMallocDefault) != hipSuccess) {
             (void)hipFree(b.p);
             fail(DSMC_ENOMEM, "no pinned host memory for a primitive's result");
@@ -2318,7 +2321,7 @@ dsmc_status dsmc_device_alloc(void **d_ptr, size_t bytes)
 {
     PRIM_BEGIN
     if (!d_ptr) fail(DSMC_EINVAL, "null output");
-    DSMC_HIP(hipMalloc(d_ptr, std::max<size_t>(bytes, 16)));
+    *d_ptr = device_alloc(std::max<size_t>(bytes, 16));
     PRIM_END
 }
 

@@ -282,7 +282,8 @@ dsmc_status dsmc_autotune(dsmc_ctx *ctx, int *block_size_out);
 /* ---- device primitives on caller-owned device memory ------------------ */
 /* stream may be NULL (default stream).  Each call takes its temporary storage
  * for itself and waits for the stream before it returns; a little of it (at
- * most 512 MB) is kept idle for later calls. */
+ * most 512 MB) is kept idle for later calls, until an allocation of this
+ * library (dsmc_device_alloc too) needs it. */
 
 /* thrust::sort_by_key(int keys, int values) (collisions.cu:282-284): stable
  * LSD radix sort of n (key, value) pairs, keys in [0, 2^key_bits). */

@@ -15,12 +15,10 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
-#include <thread>
-#include <vector>
 
 #include "dsmc_device.hpp"
 #include "dsmc_internal.hpp"
+#include "host_threads.hpp"
 
 namespace dsmc {
 
@@ -71,14 +69,7 @@ public:
             int none = (int)hipSuccess;
             if (e != hipSuccess) error.compare_exchange_strong(none, (int)e);
         };
-        std::vector<std::thread> pool;
-        pool.reserve((size_t)T);
-        try {
-            for (int k = 1; k < T; ++k) pool.emplace_back(work, k);
-        } catch (const std::system_error &) {   // no more threads: with those there are
-        }
-        work(0);
-        for (std::thread &t : pool) t.join();
+        run_threads(T, work);
         DSMC_HIP((hipError_t)error.load());
     }
 

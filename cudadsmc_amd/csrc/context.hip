@@ -233,6 +233,7 @@ struct dsmc_ctx {
     bool lazy_dead = false;         // removed atoms may still hold slots
     bool acc_stale = false;         // the accelerations in memory are not the state's
     bool tables_stale = false;      // cell table and counts are those of an earlier sort
+    bool index_stale = false;       // key_a is not as the last step's index and sort leave it
     int perm_mask = -1;             // perm's slots count the removed atoms of mask_d2[perm_mask]
     // FP32 form
     FusedPtrs fs[2];
@@ -564,6 +565,7 @@ static void plain_index(dsmc_ctx *x)
     // an even number of radix passes sorts in place: the sorted keys are then
     // the array that the index overwrites
     if (x->sorted_key && x->passes % 2 == 0) x->sorted_key = x->key_a;
+    x->index_stale = false;
     launch_index_plain(x->tdev[0], x->ps[x->cur], x->key_a, x->n_dev, x->n_cap, x->stream, &x->prof);
 }
 
@@ -739,6 +741,26 @@ static void plain_need_tables(dsmc_ctx *x)
     x->tables_stale = false;
 }
 
+// Before a single sort: key_a as the index and the sort of the last step's
+// calls leave it, in place sorted (an even number of passes) or the keys of the
+// slots as they were before the sort.
+static void plain_need_index(dsmc_ctx *x)
+{
+    if (!x->index_stale) return;
+    const bool in_place = x->passes % 2 == 0, gaps = x->perm_mask >= 0;
+    const int *sorted = x->n_dev + 3;
+    uint32_t *dst = !in_place && gaps ? x->key_f : x->key_a;
+    if (!in_place && gaps) fill_u32(dst, kNoSlot, x->n_cap, x->stream, nullptr);
+    launch_keys_by_slot(x->sorted_key, in_place ? nullptr : x->perm, sorted, x->n_cap, dst, x->stream);
+    if (!in_place && gaps) {   // the slots were counted without the removed atoms (n_dev[1]: the capacity)
+        int *stencil = (int *)x->res.alt_k;
+        launch_dead_stencil(dst, x->n_dev + 1, x->n_cap, kNoSlot, stencil, x->stream);
+        compaction_map(stencil, x->n_dev + 1, x->n_cap, x->cmap, x->n_dev + 2, x->scan_partial, x->stream, nullptr);
+        gather_u32(x->key_a, dst, x->cmap, x->n_dev + 2, x->n_cap, x->stream, nullptr);
+    }
+    x->index_stale = false;
+}
+
 // Before a single call of the FP64 form: everything in memory as the calls
 // leave it.  What the call changes is not in the order of the last step's sort.
 static void plain_enter(dsmc_ctx *x)
@@ -840,6 +862,7 @@ static void plain_substeps(dsmc_ctx *x, int L)
         x->cur ^= 1;
         x->sorted_ok = true;
         x->tables_stale = true;
+        x->index_stale = true;
         x->coll_steps++;
     }
     x->keys_ok = true;
@@ -1104,6 +1127,7 @@ static void graph_steps(dsmc_ctx *x, int times)
     }
     x->perm_mask = x->cfg.evaporation ? x->mpar ^ 1 : -1;
     x->tables_stale = true;
+    x->index_stale = true;
     x->acc_stale = !x->cfg.mcwf;
     x->sorted_ok = true;
     x->keys_ok = true;
@@ -1781,6 +1805,7 @@ dsmc_status dsmc_sort_arrays(dsmc_ctx *ctx)
         fused_sort(ctx);
     } else {
         plain_enter(ctx);
+        plain_need_index(ctx);
         plain_sort(ctx);
     }
     DSMC_API_END(ctx)

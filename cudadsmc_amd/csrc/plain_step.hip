@@ -379,6 +379,14 @@ __global__ __launch_bounds__(256) void k_untag_counts(const unsigned long long *
     count[c] = (unsigned)(v >> 32) == coll ? (int)(uint32_t)v : 0;
 }
 
+__global__ __launch_bounds__(256) void k_keys_by_slot(const uint32_t *__restrict__ key,
+                                                      const uint32_t *__restrict__ perm,
+                                                      const int *__restrict__ n, uint32_t *__restrict__ out)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < *n) out[perm ? perm[i] : (uint32_t)i] = key[i];
+}
+
 // ---------------------------------------------------------------------------
 // Host launchers.
 // ---------------------------------------------------------------------------
@@ -456,6 +464,13 @@ void launch_last_tags(const uint32_t *map, const uint64_t *mask_last, const int 
                       hipStream_t st)
 {
     hipLaunchKernelGGL(k_last_tags, dim3(div_up(n_cap, 256)), dim3(256), 0, st, map, mask_last, n, tag);
+    DSMC_HIP(hipGetLastError());
+}
+
+void launch_keys_by_slot(const uint32_t *key, const uint32_t *perm, const int *n, int n_cap, uint32_t *out,
+                         hipStream_t st)
+{
+    hipLaunchKernelGGL(k_keys_by_slot, dim3(div_up(n_cap, 256)), dim3(256), 0, st, key, perm, n, out);
     DSMC_HIP(hipGetLastError());
 }
 

@@ -63,6 +63,10 @@ void launch_step_finalize(const PlainStepParams &p, bool after_sort, const doubl
 void launch_set_ctl(PlainCtl *ctl, long long step, unsigned coll, const int *n, hipStream_t st);
 // *n = the alive atoms of ctl.
 void launch_ctl_alive(const PlainCtl *ctl, int *n, hipStream_t st);
+// out[perm[i]] (perm null: out[i]) = key[i], i < *n.
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;   // no key: no such slot
+void launch_keys_by_slot(const uint32_t *key, const uint32_t *perm, const int *n, int n_cap, uint32_t *out,
+                         hipStream_t st);
 // stencil = 1 for slots whose atom was removed before the launch's last substep.
 void launch_prev_dead_stencil(const uint32_t *key, const uint64_t *mask_last, const PlainCtl *ctl, int n_cap,
                               uint32_t dead_key, int *stencil, hipStream_t st);

@@ -901,8 +901,8 @@ static MoveParams move_params(const dsmc_ctx *x)
 
 static void fused_index(dsmc_ctx *x)
 {
-    launch_index_fused(x->d_traps, x->trap_start(), x->T, x->fs[x->cur], x->key_a, x->n_dev + x->cur,
-                       x->n_cap, x->dead_key, x->dead_in_state, x->stream, &x->prof);
+    launch_index_fused(x->d_traps, x->dead_in_state ? x->d_key_base : x->trap_start(), x->T, x->fs[x->cur],
+                       x->key_a, x->n_dev + x->cur, x->n_cap, x->dead_key, x->dead_in_state, x->stream, &x->prof);
     x->tbl_valid = false;   // the new keys decide the trap ranges of the next sort
 }
 

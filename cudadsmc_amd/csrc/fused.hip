@@ -122,22 +122,25 @@ __global__ __launch_bounds__(kFBlock) void k_init_fused(const TrapDev *__restric
     }
 }
 
-// indexAtoms for the FP32 state: the FP64 index of p + cp.  With keep_dead, a
-// slot that already holds the dead key (an atom removed by the last move,
-// which stays in place until the next sort drops it) keeps it.
+// indexAtoms for the FP32 state: the FP64 index of p + cp.  starts: the traps'
+// first slots.  With keep_dead (after a move that may have removed atoms) a
+// slot that holds the dead key (a removed atom, which stays in place until the
+// next sort drops it) keeps it, and a slot's trap is that of its present key,
+// starts the traps' first keys: the removed atoms still hold slots that the
+// trap ranges, those of the next sort, no longer count.
 __global__ __launch_bounds__(kFBlock) void k_index_fused(const TrapDev *__restrict__ traps,
-                                                         const int *__restrict__ trap_start,
+                                                         const int *__restrict__ starts,
                                                          int T, FusedPtrs s,
                                                          uint32_t *__restrict__ key,
                                                          const int *__restrict__ n_dev,
                                                          uint32_t dead_key, int keep_dead)
 {
     extern __shared__ int ts[];
-    load_table(ts, trap_start, T + 1);
+    load_table(ts, starts, T + 1);
     const int i = blockIdx.x * kFBlock + threadIdx.x;
     if (i >= *n_dev) return;
     if (keep_dead && key[i] == dead_key) return;
-    const int t = last_le(ts, T, i);
+    const int t = last_le(ts, T, keep_dead ? (int)key[i] : i);
     const TrapDev &tr = traps[t];
     const f4 *q = s.r + rec_index((uint32_t)i);
     const f4 p0 = q[0], p2 = q[2 * kRecTile];
@@ -1678,14 +1681,14 @@ void launch_init_fused(const TrapDev *traps, const int *trap_start, int n_traps,
     if (p_ && p_->enabled) p_->end(st);
 }
 
-void launch_index_fused(const TrapDev *traps, const int *trap_start, int n_traps,
+void launch_index_fused(const TrapDev *traps, const int *starts, int n_traps,
                         const FusedPtrs &s, uint32_t *key, const int *n_dev, int n_cap,
                         uint32_t dead_key, bool keep_dead, hipStream_t st, Profiler *prof)
 {
     const size_t lds = sizeof(int) * (size_t)(n_traps + 1);
     if (prof && prof->enabled) prof->begin(st, "index_fused", (double)n_cap * 28.0);
     hipLaunchKernelGGL(k_index_fused, dim3(fgrid(n_cap, kFBlock)), dim3(kFBlock), lds, st, traps,
-                       trap_start, n_traps, s, key, n_dev, dead_key, keep_dead ? 1 : 0);
+                       starts, n_traps, s, key, n_dev, dead_key, keep_dead ? 1 : 0);
     DSMC_HIP(hipGetLastError());
     if (prof && prof->enabled) prof->end(st);
 }

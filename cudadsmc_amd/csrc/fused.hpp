@@ -138,7 +138,8 @@ int  fused_max_traps();
 void launch_init_fused(const TrapDev *traps, const int *trap_start, int n_traps,
                        const InitParams &ip, const FusedPtrs &s, int n, hipStream_t st,
                        Profiler *prof);
-void launch_index_fused(const TrapDev *traps, const int *trap_start, int n_traps,
+// starts: the traps' first slots, or with keep_dead their first keys.
+void launch_index_fused(const TrapDev *traps, const int *starts, int n_traps,
                         const FusedPtrs &s, uint32_t *key, const int *n_dev, int n_cap,
                         uint32_t dead_key, bool keep_dead, hipStream_t st, Profiler *prof);
 void launch_table_fused(const uint32_t *key, const int *key_base, const TableParams &tp,

@@ -156,21 +156,9 @@ __global__ __launch_bounds__(kRBlock) void k_widen_f(const float *__restrict__ i
     if (i < n) out[i] = (double)in[i];
 }
 
-__global__ __launch_bounds__(kRBlock) void k_widen_flag(const uint8_t *__restrict__ in, long long n,
-                                                        int *__restrict__ out)
-{
-    const long long i = (long long)blockIdx.x * kRBlock + threadIdx.x;
-    if (i < n) out[i] = in[i] ? 1 : 0;
-}
-
 void launch_widen(const float *in, long long n, double *out, hipStream_t st)
 {
     DSMC_READOUT(k_widen_f, n, st, in, n, out);
-}
-
-void launch_widen(const uint8_t *in, long long n, int *out, hipStream_t st)
-{
-    DSMC_READOUT(k_widen_flag, n, st, in, n, out);
 }
 
 __global__ __launch_bounds__(kRBlock) void k_iota(int *__restrict__ out, int n)

@@ -30,7 +30,6 @@ void launch_unpack_columns(const double *in, int ncols, const uint32_t *map, int
                            hipStream_t st);
 // out[i] = in[i], widened.
 void launch_widen(const float *in, long long n, double *out, hipStream_t st);
-void launch_widen(const uint8_t *in, long long n, int *out, hipStream_t st);   // 0 or 1
 void launch_iota(int *out, int n, hipStream_t st);
 // stencil[i] = 1 for slots with the dead key, 0 for the alive ones.
 void launch_dead_stencil(const uint32_t *key, const int *n_dev, int n_cap, uint32_t dead_key,

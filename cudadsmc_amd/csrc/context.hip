@@ -233,6 +233,7 @@ struct dsmc_ctx {
     bool lazy_dead = false;         // removed atoms may still hold slots
     bool acc_stale = false;         // the accelerations in memory are not the state's
     bool tables_stale = false;      // cell table and counts are those of an earlier sort
+    bool up_set = false;            // ps[].up hold the initial flags
     bool index_stale = false;       // key_a is not as the last step's index and sort leave it
     int perm_mask = -1;             // perm's slots count the removed atoms of mask_d2[perm_mask]
     // FP32 form
@@ -1265,7 +1266,11 @@ static void reset_cells(dsmc_ctx *x)
     if (!x->fp32) {
         plain_enter(x);   // what host reads see of the earlier run stays readable
         DSMC_HIP(hipMemsetAsync(x->cc_tagged, 0, sizeof(unsigned long long) * (x->ncells + 1), st));
-        for (int b = 0; b < 2; ++b) DSMC_HIP(hipMemsetAsync(x->ps[b].up, 1, (size_t)x->n_cap, st));
+        // every atom spin up, in both buffers (a move keeps the flags of the
+        // one it writes unless atoms can flip)
+        if (x->cfg.mcwf || !x->up_set)
+            for (int b = 0; b < 2; ++b) DSMC_HIP(hipMemsetAsync(x->ps[b].up, 1, (size_t)x->n_cap, st));
+        x->up_set = true;
     }
     // the double buffers as in a new context: a captured graph stays valid
     x->ssel = x->tsel = x->srt_cur = x->csel = x->mpar = 0;

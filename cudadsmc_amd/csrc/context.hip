@@ -492,13 +492,16 @@ static void build_context(dsmc_ctx *x, const dsmc_config *c, const dsmc_trap *tr
             x->flips = x->alloc<unsigned long long>(1);
         }
         x->ctl = x->alloc<PlainCtl>(2);
-        x->key_f = x->alloc<uint32_t>(N);
+        // few allocations: each costs a small context's creation 4 us
+        const size_t row = ((size_t)N + 63) & ~(size_t)63, words = resort_mask_words(N);
+        x->key_f = x->alloc<uint32_t>(5 * row);
+        uint64_t *const masks = x->alloc<uint64_t>(3 * words);
         for (int b = 0; b < 2; ++b) {
-            x->srt_k[b] = x->alloc<uint32_t>(N);
-            x->srt_v[b] = x->alloc<uint32_t>(N);
-            x->mask_d2[b] = x->alloc<uint64_t>(resort_mask_words(N));
+            x->srt_k[b] = x->key_f + (1 + 2 * b) * row;
+            x->srt_v[b] = x->key_f + (2 + 2 * b) * row;
+            x->mask_d2[b] = masks + b * words;
         }
-        x->mask_last = x->alloc<uint64_t>(resort_mask_words(N));
+        x->mask_last = masks + 2 * words;
         x->rec64 = x->alloc<double>((size_t)std::min(c->lpc, kMaxSub) * kStepRec * step_rec_stride(N));
         x->cc_tagged = x->alloc<unsigned long long>(C1);
     } else {

@@ -843,7 +843,6 @@ static void plain_substeps(dsmc_ctx *x, int L)
     p.decay = decay_params(x);
     p.spin_loss = (x->cfg.evaporation & DSMC_EVAP_SPIN) ? 1 : 0;
     p.energy_cut = (x->cfg.evaporation & DSMC_EVAP_ENERGY) ? 1 : 0;
-    p.mcwf = x->cfg.mcwf;
     p.lpc = lpc;
     p.phase = phase;
     p.L = L;
@@ -1637,17 +1636,15 @@ struct Workspace {
 // ---------------------------------------------------------------------------
 // Scratch of the allocation-free sort (dsmc_sort_by_key_noalloc): a
 // file-scope device array, one copy per device, resident until the process
-// ends.  Layout: the pair count (one word in a 256-byte header), the radix
-// histograms and digit totals for kNoAllocMaxPairs pairs, then the alternate
-// key and value buffers of the passes.  Host code never uses the array's
+// ends.  Layout: the radix digit totals and histograms for kNoAllocMaxPairs
+// pairs, then the alternate key and value buffers of the passes.  Host code never uses the array's
 // name as an address: the address on each device comes from
 // hipGetSymbolAddress with that device current (noalloc_scratch()).
 // ---------------------------------------------------------------------------
 constexpr int kNoAllocMaxPairs = 1 << 20;
-constexpr size_t kNoAllocHdr = 256;
 constexpr size_t kNoAllocSortBytes =
     ((size_t)kRadix * (kNoAllocMaxPairs / kSortTile) * 4 + (size_t)kRadix * 4 + 256 + 255) & ~(size_t)255;
-constexpr size_t kNoAllocBytes = kNoAllocHdr + kNoAllocSortBytes + 2 * (size_t)kNoAllocMaxPairs * 4;
+constexpr size_t kNoAllocBytes = kNoAllocSortBytes + 2 * (size_t)kNoAllocMaxPairs * 4;
 static_assert(kNoAllocMaxPairs % kSortTile == 0, "whole sort tiles");
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
@@ -2257,8 +2254,8 @@ dsmc_status dsmc_sort_by_key_noalloc(unsigned int *d_keys, unsigned int *d_value
     if (n == 0) return DSMC_OK;
     hipStream_t st = (hipStream_t)stream;
     SortScratch s;
-    sort_scratch_bind(s, n, base + kNoAllocHdr, kRadix);
-    uint32_t *tk = (uint32_t *)(base + kNoAllocHdr + kNoAllocSortBytes);
+    sort_scratch_bind(s, n, base, kRadix);
+    uint32_t *tk = (uint32_t *)(base + kNoAllocSortBytes);
     uint32_t *tv = tk + kNoAllocMaxPairs;
     const RadixPlan plan = radix_plan(n, key_bits, kRadixBits);   // its fixed scratch holds 256 digits
     if (plan.passes % 2 == 0) {

@@ -1647,23 +1647,6 @@ void launch_observe_fused(const TrapDev *traps, const int *key_base, int n_traps
     DSMC_HIP(hipGetLastError());
 }
 
-// dst[i] = src[map[i]] for every FP32 state array.
-__global__ __launch_bounds__(kFBlock) void k_gather_fused(FusedPtrs dst, FusedPtrs src,
-                                                          const uint32_t *__restrict__ map,
-                                                          const int *__restrict__ n_dev, int spin)
-{
-    const int i = blockIdx.x * kFBlock + threadIdx.x;
-    if (i >= *n_dev) return;
-    const uint32_t j = map[i];
-    const f4 *q = src.r + rec_index(j);
-    f4 *d = dst.r + rec_index((uint32_t)i);
-#pragma unroll
-    for (int c = 0; c < kRecPlanes; ++c) d[c * kRecTile] = q[c * kRecTile];
-    if (spin)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) dst.s[c][i] = src.s[c][j];
-}
-
 // ---------------------------------------------------------------------------
 // Host launchers.
 // ---------------------------------------------------------------------------
@@ -1974,13 +1957,6 @@ void launch_obs_finalize(int n_traps, int max_trap_atoms, int move_block, double
                        rec.acc_over, coll_accum, step_cur, step_next, obs_log, obs_cap, n_next, work);
     DSMC_HIP(hipGetLastError());
     if (prof && prof->enabled) prof->end(st);
-}
-
-void launch_gather_fused(const FusedPtrs &dst, const FusedPtrs &src, const uint32_t *map,
-                         const int *n_dev, int n_cap, int spin, hipStream_t st, Profiler *prof)
-{
-    DSMC_LAUNCH(prof, "gather_fused", (double)n_cap * (4.0 + 2.0 * (48 + (spin ? 12 : 0))),
-                k_gather_fused, fgrid(n_cap, kFBlock), kFBlock, st, dst, src, map, n_dev, spin);
 }
 
 }  // namespace dsmc

@@ -211,8 +211,6 @@ void launch_obs_finalize(int n_traps, int max_trap_atoms, int move_block, double
 void launch_observe_fused(const TrapDev *traps, const int *key_base, int n_traps, double mass,
                           const FusedPtrs &s, const uint32_t *key, const int *n_dev, int n_cap,
                           uint32_t dead_key, int *first, int *last, double *acc, hipStream_t st);
-void launch_gather_fused(const FusedPtrs &dst, const FusedPtrs &src, const uint32_t *map,
-                         const int *n_dev, int n_cap, int spin, hipStream_t st, Profiler *prof);
 double move_fused_bytes_per_atom(int spin);
 
 }  // namespace dsmc

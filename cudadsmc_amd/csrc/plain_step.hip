@@ -349,8 +349,6 @@ __global__ void k_set_ctl(PlainCtl *ctl, long long step, unsigned coll, const in
     ctl->alive = *n;
 }
 
-__global__ void k_ctl_alive(const PlainCtl *ctl, int *n) { *n = ctl->alive; }
-
 __global__ __launch_bounds__(256) void k_prev_dead_stencil(const uint32_t *__restrict__ key,
                                                            const uint64_t *__restrict__ mask_last,
                                                            const int *__restrict__ n, uint32_t dead_key,
@@ -443,12 +441,6 @@ void launch_step_finalize(const PlainStepParams &p, bool after_sort, const doubl
 void launch_set_ctl(PlainCtl *ctl, long long step, unsigned coll, const int *n, hipStream_t st)
 {
     hipLaunchKernelGGL(k_set_ctl, dim3(1), dim3(1), 0, st, ctl, step, coll, n);
-    DSMC_HIP(hipGetLastError());
-}
-
-void launch_ctl_alive(const PlainCtl *ctl, int *n, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_ctl_alive, dim3(1), dim3(1), 0, st, ctl, n);
     DSMC_HIP(hipGetLastError());
 }
 

@@ -26,7 +26,7 @@ struct PlainStepParams {
     SpinParams  spin;
     FlipParams  flip;
     DecayParams decay;
-    int spin_loss, energy_cut, mcwf;
+    int spin_loss, energy_cut;
     int lpc;          // motion substeps per collision step
     int phase;        // substeps of the collision step already taken
     int L;            // substeps of this launch (<= kMaxSub)
@@ -61,8 +61,6 @@ void launch_step_finalize(const PlainStepParams &p, bool after_sort, const doubl
                           double *evap_accum, dsmc_observables *log, int obs_cap, const ResortWork &work,
                           hipStream_t st, Profiler *prof);
 void launch_set_ctl(PlainCtl *ctl, long long step, unsigned coll, const int *n, hipStream_t st);
-// *n = the alive atoms of ctl.
-void launch_ctl_alive(const PlainCtl *ctl, int *n, hipStream_t st);
 // out[perm[i]] (perm null: out[i]) = key[i], i < *n.
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;   // no key: no such slot
 void launch_keys_by_slot(const uint32_t *key, const uint32_t *perm, const int *n, int n_cap, uint32_t *out,

@@ -27,6 +27,8 @@ struct PlainStepParams {
     FlipParams  flip;
     DecayParams decay;
     int spin_loss, energy_cut;
+    int pad;          // the fields behind it at their places: without it the compiler's move is
+                      // 3 % slower (the reference's run, 500 steps: 2.26 ms instead of 2.19)
     int lpc;          // motion substeps per collision step
     int phase;        // substeps of the collision step already taken
     int L;            // substeps of this launch (<= kMaxSub)

@@ -450,9 +450,6 @@ __device__ __forceinline__ T wave_inclusive_scan(T v)
     return v;
 }
 
-// Exclusive scan over a block of BLOCK threads (one value per thread).  Uses
-// `tmp` (>= BLOCK/64 + 1 entries of LDS).  Returns the exclusive prefix and
-// writes the block total to *total.
 // 32-bit integers: the exchanges as DPP operands of the additions (row shifts
 // of 1, 2, 4 and 8 scan each row of 16 lanes, the last lane of rows 0 and 2
 // goes to rows 1 and 3, then lane 31 to the upper half) instead of LDS
@@ -481,6 +478,9 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v)
     return (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_scan(v), kWave - 1);
 }
 
+// Exclusive scan over a block of BLOCK threads (one value per thread).  Uses
+// `tmp` (BLOCK / 64 entries of LDS).  Returns the exclusive prefix and writes
+// the block total to *total.
 template <int BLOCK, typename T>
 __device__ __forceinline__ T block_exclusive_scan(T v, T *tmp, T *total)
 {

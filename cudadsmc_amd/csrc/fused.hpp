@@ -197,8 +197,8 @@ void launch_collide_edges(const TrapDev *traps, const int *key_base, int n_traps
 // trap loses its atoms removed in this step, which the next sort puts last.
 // trap_next / n_next (when not null): the trap ranges and alive count after
 // the next sort, from the move's per-block removal counts and masks.  step
-// is read from step_cur; step + 1 is written to step_next.  list: the same
-// launch also runs the next incremental re-sort's first phase.
+// is read from step_cur; step + 1 is written to step_next.  work: the same
+// launch also runs the next incremental re-sort's first phase, or all of it.
 void launch_obs_finalize(int n_traps, int max_trap_atoms, int move_block, double mass,
                          const int *trap_start, int *trap_next, const uint32_t *blk_dead,
                          const uint64_t *mask_dead, const ObsRecords &rec,

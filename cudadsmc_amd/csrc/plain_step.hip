@@ -5,16 +5,17 @@
 // motion step spin, move, tag, compaction (with another gather) and sums; 17
 // launches a step at lpc = 1 and 11 to 13 per motion step in the reference's
 // run.  At N = 1e4 that is launch latency (68 and 40 us a motion step), at 1e6
-// the state crosses memory some six times (188 us).  Here a collision step is
-// four launches whatever lpc is (three where the finalize's launch holds the
-// whole sort, up to kScanSlots atoms):
+// the state crosses memory some six times (188 us).  Here a collision step of
+// up to kMaxSub motion substeps is four launches (three where the finalize's
+// launch holds the whole sort, up to kScanSlots atoms); every further kMaxSub
+// substeps are a move and a finalize more:
 //   k_ins_merge                the stable sort by (cell, slot) from the last
 //                              one (primitives.hip): the same permutation as
 //                              the radix sort's
 //   k_collide_step             cells of two or more atoms from the sorted keys,
 //                              velocities through the permutation
 //   k_move_step                gathers the state through the permutation into
-//                              the other buffer and runs all motion substeps
+//                              the other buffer and runs the motion substeps
 //                              up to the next collision step in registers
 //                              (an atom needs no other in between): spin,
 //                              Verlet, losses, sums, flips, next key

@@ -1,9 +1,9 @@
 // readout.hip -- see readout.hpp.  Every kernel here touches each byte once and
 // is bound by the memory it streams; the copy over the host link that
-// follows takes some twenty times longer (24 bytes per atom and field at 18
+// follows takes some forty times longer (24 bytes per atom and field at 39
 // GB/s into pageable memory against 72 bytes at 5 TB/s here).  Before these
 // kernels the host unpacked the records itself, one strided read per
-// component: N = 4e6, position, velocity and labels took 292 ms, now 13 ms.
+// component: N = 4e6, position, velocity and labels took 292 ms, now 6.7 ms.
 #include "readout.hpp"
 
 namespace dsmc {
